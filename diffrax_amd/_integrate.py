@@ -50,41 +50,47 @@ def _scalar_time(x, name):
     return float(x)
 
 
-class _HostCopies:
-    """Host values of device-resident inputs that the host checks (t1, SaveAt ts).
+class _TimeChecks:
+    """The checks of t1, dt0 and SaveAt(ts) when t1 or ts is device-resident
+    (dfx_check_times): queued on the current stream, so that the solve can be queued behind
+    them before their outcome is known; ``bits`` then waits for them only, never for the
+    solve.  t1: a device tensor of one value or one per row, or a number; ts: a device tensor
+    [n], [rows, n] or None."""
 
-    A CPU tensor is read in place.  A device tensor is copied to pinned host memory behind
-    the work already queued on the current stream, so the solve can be queued before the
-    checks run: ``get`` then waits for those copies only, never for the solve."""
+    def __init__(self, t0, t1, dt0, ts, device):
+        per_row = [x for x, nd in ((t1, 1), (ts, 2))
+                   if isinstance(x, torch.Tensor) and x.ndim == nd and (nd == 2 or x.numel() != 1)]
+        rows = per_row[0].shape[0] if per_row else 1
+        n_ts = 0 if ts is None else int(ts.shape[-1])
+        # one block reads 1,024 times and more; 1,024 blocks fill the GPU four times over
+        n_flags = max(1, min(1024, rows * max(n_ts, 1) // 1024))
+        self._dev = torch.empty(n_flags, dtype=torch.int32, device=device)
+        t1_t = t1 if isinstance(t1, torch.Tensor) else None
+        _lib.check(_lib.load().dfx_check_times(
+            t1_t.data_ptr() if t1_t is not None else None, 0.0 if t1_t is not None else float(t1),
+            0 if t1_t is None or t1_t.numel() == 1 else 1,
+            ts.data_ptr() if ts is not None else None, n_ts if ts is not None and ts.ndim == 2 else 0,
+            n_ts, rows, t0, _nan_if_none(dt0), self._dev.data_ptr(), n_flags,
+            torch.cuda.current_stream().cuda_stream), "dfx_check_times")
+        self._host = torch.empty(n_flags, dtype=torch.int32, pin_memory=True)
+        self._host.copy_(self._dev, non_blocking=True)
+        self._event = torch.cuda.Event()
+        self._event.record()
 
-    def __init__(self):
-        self._vals = {}
-        self._event = None
-        self._pending = False
+    def bits(self):
+        self._event.synchronize()
+        return int(np.bitwise_or.reduce(self._host.numpy()))
 
-    def add(self, name, t):
-        if t.device.type == "cpu":
-            self._vals[name] = t.numpy()
-            return
-        h = torch.empty(tuple(t.shape), dtype=t.dtype, pin_memory=True)
-        h.copy_(t, non_blocking=True)
-        self._vals[name] = h
-        self._pending = True
+    def check_ts(self):
+        _raise_ts(self.bits())
 
-    @property
-    def deferred(self):
-        return self._pending
 
-    def seal(self):
-        if self._pending:
-            self._event = torch.cuda.Event()
-            self._event.record()
-
-    def get(self, name):
-        if self._event is not None:
-            self._event.synchronize()
-        v = self._vals[name]
-        return v.numpy() if isinstance(v, torch.Tensor) else v
+def _raise_ts(bits):
+    """saveat.ts must be increasing and lie in [t0, t1] (_integrate.py:1222-1235)."""
+    if bits & 2:
+        raise RuntimeError("saveat.ts must be increasing or decreasing.")
+    if bits & 4:
+        raise RuntimeError("saveat.ts must lie between t0 and t1.")
 
 
 class _Workspace:
@@ -208,17 +214,16 @@ class ErkPlan:
 
 
 def _check_ts(ts, t0, t1_vals, directions):
-    """saveat.ts must be increasing and lie in [t0, t1] (_integrate.py:1222-1235).
-    ts: [n] or [B, n]; t1_vals, directions: [1] or [B] (float64 numpy)."""
+    """_raise_ts of host times; ts: [n] or [B, n]; t1_vals, directions: [1] or [B] (float64
+    numpy)."""
     ts = np.asarray(ts, dtype=np.float64)
     dirs = np.asarray(directions, dtype=np.float64).reshape(-1, 1)
     tn = np.atleast_2d(ts) * dirs
-    if tn.shape[-1] > 1 and bool((tn[:, 1:] < tn[:, :-1]).any()):
-        raise RuntimeError("saveat.ts must be increasing or decreasing.")
+    unsorted = tn.shape[-1] > 1 and bool((tn[:, 1:] < tn[:, :-1]).any())
     t0n = t0 * dirs
     t1n = np.asarray(t1_vals, dtype=np.float64).reshape(-1, 1) * dirs
-    if bool(((tn > t1n) | (tn < t0n)).any()):
-        raise RuntimeError("saveat.ts must lie between t0 and t1.")
+    outside = bool(((tn > t1n) | (tn < t0n)).any())
+    _raise_ts((2 if unsorted else 0) | (4 if outside else 0))
 
 
 def _controller_fields(stepsize_controller, dt0f):
@@ -342,14 +347,14 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
     t0f = _scalar_time(t0, "t0")
     if t0f is None:
         raise ValueError("t0 must be a scalar")
-    host = _HostCopies()
+    on_device = False   # t1 or ts in device memory: checked there (_TimeChecks)
     if isinstance(t1, torch.Tensor) and t1.device.type != "cpu":
         # device-resident t1 (one value or one per instance): read by the kernel in place
         t1_t = t1.to(torch.float64).reshape(-1)
         if t1_t.numel() not in (1, B):
             raise ValueError(f"t1 must be a scalar or have shape [{B}]")
         t1_stride = 0 if t1_t.numel() == 1 else 1
-        host.add("t1", t1_t)
+        on_device = True
     else:
         t1f = _scalar_time(t1, "t1")
         if t1f is not None:
@@ -360,7 +365,6 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
             if t1_t.numel() != B:
                 raise ValueError(f"t1 must be a scalar or have shape [{B}]")
             t1_stride = 1
-        host.add("t1", t1_t)
 
     if dt0 is not None:
         dt0f = _scalar_time(dt0, "dt0")
@@ -402,21 +406,20 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
             ts_stride = n_ts
         else:
             raise ValueError(f"SaveAt(ts) must be [n] or [{B}, n]")
-        host.add("ts", ts_t)
+        on_device = on_device or ts_t.device.type != "cpu"
 
-    def check_times():
-        # _integrate.py:1107-1112 (dt0 sign) and 1222-1235 (ts order and range)
-        t1_host = host.get("t1")
+    # _integrate.py:1107-1112 (dt0 sign) and 1222-1235 (ts order and range)
+    def raise_dt0():
+        raise RuntimeError(
+            f"Must have (t1 - t0) * dt0 >= 0, we instead got t1 with value {t1}, t0 "
+            f"with value {t0}, dt0 with value {dt0}")
+
+    if not on_device:
+        t1_host = t1_t.numpy()
         if dt0f is not None and bool(np.any((t1_host - t0f) * dt0f < 0)):
-            raise RuntimeError(
-                f"Must have (t1 - t0) * dt0 >= 0, we instead got t1 with value {t1}, t0 "
-                f"with value {t0}, dt0 with value {dt0}")
+            raise_dt0()
         if ts_t is not None:
-            _check_ts(host.get("ts"), t0f, t1_host, np.where(t0f < t1_host, 1.0, -1.0))
-
-    host.seal()
-    if not host.deferred:
-        check_times()
+            _check_ts(ts_t.numpy(), t0f, t1_host, np.where(t0f < t1_host, 1.0, -1.0))
 
     clip = None
     if isinstance(stepsize_controller, ClipStepSizeController):
@@ -437,6 +440,14 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
     t1_t = t1_t.to(device).contiguous()
     if ts_t is not None:
         ts_t = ts_t.to(device).contiguous()
+    check_times = None
+    if on_device:
+        checks = _TimeChecks(t0f, t1_t, dt0f, ts_t, device)
+
+        def check_times():
+            if checks.bits() & 1:
+                raise_dt0()
+            checks.check_ts()
     params, param_stride = vfo.pack(args, B, d, y0b.dtype, device)
     prob = _lib.ErkProblem(
         solver=solver.solver_id, vf=vfo.vf_id, precision=precision,
@@ -493,7 +504,7 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
     plan = ErkPlan(prob, tensors, n_out, batched, None if launch == "auto" else launch)
     plan.fsal = bool(solver.tableau.fsal)
     # checks of device-resident times, run by diffeqsolve once the solve is queued
-    plan.deferred_checks = check_times if host.deferred else None
+    plan.deferred_checks = check_times
     return plan
 
 

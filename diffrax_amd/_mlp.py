@@ -264,8 +264,7 @@ def prepare_mlp(terms, solver, t0, t1, dt0, y0, saveat, stepsize_controller, max
     ts = None
     check = None
     if sub.ts is not None:
-        # device-resident ts are checked from a pinned copy once the solve is queued
-        from ._integrate import _HostCopies
+        from ._integrate import _TimeChecks, _check_ts
         ts = torch.as_tensor(sub.ts, dtype=torch.float64)
         if ts.ndim == 2 and ts.shape[0] == y0b.shape[0]:
             pass   # per-trajectory save times [B, n_ts]
@@ -273,21 +272,12 @@ def prepare_mlp(terms, solver, t0, t1, dt0, y0, saveat, stepsize_controller, max
             ts = ts.reshape(-1)
         else:
             raise ValueError(f"SaveAt(ts) must be [n] or [{y0b.shape[0]}, n]")
-        host = _HostCopies()
-        host.add("ts", ts)
-        host.seal()
         t0f, t1f = float(t0), float(t1)
-
-        def check():
-            dirn = 1.0 if t0f < t1f else -1.0
-            tn = host.get("ts") * dirn
-            if tn.shape[-1] > 1 and (tn[..., 1:] < tn[..., :-1]).any():
-                raise RuntimeError("saveat.ts must be increasing or decreasing.")
-            if ((tn > t1f * dirn) | (tn < t0f * dirn)).any():
-                raise RuntimeError("saveat.ts must lie between t0 and t1.")
-        if not host.deferred:
-            check()
-            check = None
+        if ts.device.type == "cpu":
+            _check_ts(ts.numpy(), t0f, [t1f], [1.0 if t0f < t1f else -1.0])
+        else:   # checked on the device, the outcome read once the solve is queued
+            ts = ts.to(device).contiguous()
+            check = _TimeChecks(t0f, t1f, None, ts, device).check_ts
     if not allocate:
         probe = _Probe()
         probe.ts_host = ts

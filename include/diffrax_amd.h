@@ -263,6 +263,16 @@ typedef struct dfx_erk_dense_io {
  * solver's local interpolant (_solver/tsit5.py:103-156, _local_interpolation.py:50-139). */
 int dfx_erk_dense_eval(const dfx_erk_problem* p, const dfx_erk_dense_io* io, void* stream);
 
+/* The reference's checks of t1, dt0 and SaveAt(ts) (_integrate.py:1107-1112, 1222-1235) for
+ * times that are in device memory.  t1 [rows] (t1_stride 1), one value (t1_stride 0), or
+ * null for t1_value; ts [rows, n_ts] (ts_stride n_ts), shared [n_ts] (ts_stride 0), or null;
+ * dt0 NaN: none.  flags [n_flags] out, n_flags in [1, 4096]: every word is written, and
+ * their OR has bit 0 when some (t1 - t0) * dt0 < 0, bit 1 when some row is not sorted in
+ * the direction of its solve, bit 2 when some time lies outside [t0, t1]. */
+int dfx_check_times(const double* t1, double t1_value, int64_t t1_stride, const double* ts,
+                    int64_t ts_stride, int32_t n_ts, int64_t rows, double t0, double dt0,
+                    int32_t* flags, int32_t n_flags, void* stream);
+
 /* ---- SDE: Heun with diagonal noise on the registered OU terms ----------------------- */
 /* dy = theta (mu - y) dt + sigma dW, theta/mu/sigma of length d shared by all paths. */
 typedef struct dfx_sde_problem {
