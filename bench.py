@@ -432,9 +432,9 @@ def bench_sde(steps, warmup, with_cpu, P=262144, d=16, N=1000, cpu_paths=16384):
     k_mean, k_med, wall = _event_time(fwd_grad, steps, warmup)
     out["forward_grad"] = dict(paths_per_s=round(P / (wall * 1e-3), 1),
                                ms_per_solve=round(wall, 4), event_ms_mean=round(k_mean, 4),
-                               checkpoint_every=int(gs.prob.checkpoint_every),
-                               algorithmic_bytes=2 * alg_bytes,
-                               achieved_gbs=round(2 * alg_bytes / (wall * 1e-3) / 1e9, 1))
+                               record_bytes=8 * gs.sens.numel(),
+                               algorithmic_bytes=alg_bytes,
+                               achieved_gbs=round(alg_bytes / (wall * 1e-3) / 1e9, 1))
     out.pop("g", None)
     # Errors on the last 512 paths (dW offsets past 2^31): the forward against the FP64
     # oracle, and the adjoint of sum(w * y(1)) with w nonzero on those paths only against

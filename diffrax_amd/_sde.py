@@ -23,7 +23,7 @@ class SdeProblem(ctypes.Structure):
 class SdeIO(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in
                 ("y0", "theta", "mu", "sigma", "dW", "grid", "ys", "ckpt", "ts", "dense_ys",
-                 "dense_k")]
+                 "dense_k", "sens")]
 
 
 class SdeDenseIO(ctypes.Structure):
@@ -41,6 +41,7 @@ class SdeGradIO(ctypes.Structure):
 _SIGS = {
     "dfx_sde_n_out": ([ctypes.POINTER(SdeProblem)], ctypes.c_int),
     "dfx_sde_n_ckpt": ([ctypes.POINTER(SdeProblem)], ctypes.c_int),
+    "dfx_sde_sens_words": ([ctypes.POINTER(SdeProblem)], ctypes.c_int64),
     "dfx_sde_workspace_bytes": ([ctypes.POINTER(SdeProblem), ctypes.POINTER(ctypes.c_size_t)],
                                 ctypes.c_int),
     "dfx_sde_heun_solve": ([ctypes.POINTER(SdeProblem), ctypes.POINTER(SdeIO), ctypes.c_void_p],
@@ -103,17 +104,23 @@ class _Sde:
                                checkpoint_every=ck, save_t0=int(save_t0), save_t1=int(save_t1),
                                save_steps=int(save_steps),
                                n_ts=0 if ts is None else int(ts.numel()))
+        # the gradient's record: the derivatives of y(t1), or checkpoints where rows between
+        # t0 and t1 carry cotangents too
+        words = int(lib.dfx_sde_sens_words(ctypes.byref(self.prob))) if need_grad else 0
         n_ck = lib.dfx_sde_n_ckpt(ctypes.byref(self.prob)) if need_grad else 0
         self.n_out = int(lib.dfx_sde_n_out(ctypes.byref(self.prob)))
         self.ys = torch.empty((self.P, self.n_out, self.d), dtype=y0.dtype, device=y0.device)
         self.ckpt = (torch.empty((max(n_ck, 1), self.P, self.d), dtype=y0.dtype, device=y0.device)
-                     if need_grad else None)
+                     if need_grad and not words else None)
+        self.sens = (torch.empty(words, dtype=torch.float64, device=y0.device)
+                     if words else None)
         self.keep = (y0, theta, mu, sigma, dW, grid)
         io = SdeIO()
         for n, v in zip(("y0", "theta", "mu", "sigma", "dW", "grid"), self.keep):
             setattr(io, n, v.data_ptr())
         io.ys = self.ys.data_ptr()
         io.ckpt = self.ckpt.data_ptr() if self.ckpt is not None else None
+        io.sens = self.sens.data_ptr() if self.sens is not None else None
         self.ts = ts
         io.ts = ts.data_ptr() if ts is not None and ts.numel() else None
         self.dense = None

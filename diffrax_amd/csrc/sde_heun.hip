@@ -102,6 +102,11 @@ int dfx_sde_n_ckpt(const dfx_sde_problem* p) {
   return (p->num_steps + p->checkpoint_every - 1) / p->checkpoint_every - 1;
 }
 
+int64_t dfx_sde_sens_words(const dfx_sde_problem* p) {
+  if (sde_check(p) != DFX_OK || p->n_ts > 0 || p->save_steps > 0 || p->num_steps < 1) return 0;
+  return 2 * p->paths * p->d + 2 * p->d;
+}
+
 int dfx_sde_workspace_bytes(const dfx_sde_problem* p, size_t* bytes) {
   if (sde_check(p) != DFX_OK || !bytes) return DFX_E_ARG;
   const int64_t nblocks = (sde_threads(p, 1) + kBlock - 1) / kBlock;
@@ -119,17 +124,21 @@ int dfx_sde_heun_solve(const dfx_sde_problem* p, const dfx_sde_io* io, void* str
   if (io->ckpt && p->checkpoint_every <= 0) return DFX_E_ARG;
   if ((io->dense_ys == nullptr) != (io->dense_k == nullptr)) return DFX_E_ARG;
   if (io->dense_ys && (p->checkpoint_every > 0 || io->ckpt || p->num_steps < 1)) return DFX_E_ARG;
+  if (io->sens && (dfx_sde_sens_words(p) == 0 || io->ckpt || io->dense_ys)) return DFX_E_ARG;
   if (p->paths == 0) return DFX_OK;
   SdeArgs a;
   memset(&a, 0, sizeof(a));
   a.y0 = io->y0; a.theta = io->theta; a.mu = io->mu; a.sigma = io->sigma;
-  a.dW = io->dW; a.grid = io->grid; a.ys = io->ys; a.ckpt = io->ckpt;
+  a.dW = io->dW; a.grid = io->grid; a.ys = io->ys; a.ckpt = io->ckpt; a.sens = io->sens;
   a.P = p->paths; a.d = p->d; a.N = p->num_steps; a.CK = p->checkpoint_every > 0 ? p->checkpoint_every : 1;
   a.n_out = dfx_sde_n_out(p);
   a.save_t0 = p->save_t0; a.save_t1 = p->save_t1; a.save_steps = p->save_steps;
   a.n_ts = p->n_ts; a.ts = io->ts;
   a.dense_ys = io->dense_ys; a.dense_k = io->dense_k;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (io->sens)
+    return (p->precision == DFX_F32 ? sde_launch_sens_fwd_f32(a, s)
+                                    : sde_launch_sens_fwd_f64(a, s)) == 0 ? DFX_OK : DFX_E_HIP;
   if ((p->precision == DFX_F32 ? sde_launch_fwd_f32(a, s) : sde_launch_fwd_f64(a, s)) != 0)
     return DFX_E_HIP;
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
@@ -181,9 +190,13 @@ int sde_adjoint_impl(const dfx_sde_problem* p, const dfx_sde_io* io, const dfx_s
   if (!io || !g || !io->y0 || !io->theta || !io->mu || !io->sigma || !io->grid || !g->ys_bar)
     return DFX_E_ARG;
   if (!g->theta_bar || !g->mu_bar || !g->sigma_bar) return DFX_E_ARG;
-  if (p->checkpoint_every != 32 && p->checkpoint_every != 16 && p->checkpoint_every != 8)
-    return DFX_E_ARG;
-  if (dfx_sde_n_ckpt(p) > 0 && !io->ckpt) return DFX_E_ARG;
+  if (io->sens) {
+    if (dfx_sde_sens_words(p) == 0) return DFX_E_ARG;
+  } else {
+    if (p->checkpoint_every != 32 && p->checkpoint_every != 16 && p->checkpoint_every != 8)
+      return DFX_E_ARG;
+    if (dfx_sde_n_ckpt(p) > 0 && !io->ckpt) return DFX_E_ARG;
+  }
   if (p->n_ts > 0 && !io->ts) return DFX_E_ARG;
   size_t need = 0;
   dfx_sde_workspace_bytes(p, &need);
@@ -197,14 +210,23 @@ int sde_adjoint_impl(const dfx_sde_problem* p, const dfx_sde_io* io, const dfx_s
   a.n_out = dfx_sde_n_out(p);
   a.save_t0 = p->save_t0; a.save_t1 = p->save_t1; a.save_steps = p->save_steps;
   a.n_ts = p->n_ts; a.ts = io->ts;
-  const int64_t nb = (sde_threads(p, 1) + kBlock - 1) / kBlock;
+  a.sens = io->sens;
+  int64_t nb = (sde_threads(p, 1) + kBlock - 1) / kBlock;
+  // the sens backward streams its few bytes per path with two workgroups per CU, so that
+  // few partials are left to sum (16,384 of them took 35 us)
+  if (io->sens && nb > 512) nb = 512;
   a.partial = reinterpret_cast<double*>(workspace);
   const size_t lds = (size_t)3 * kBlock * sizeof(double);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->paths > 0) {
-    if ((p->precision == DFX_F32 ? sde_launch_adj_f32(a, nb, lds, s)
-                                 : sde_launch_adj_f64(a, nb, lds, s)) != 0)
-      return DFX_E_HIP;
+    int lrc;
+    if (io->sens)
+      lrc = p->precision == DFX_F32 ? sde_launch_sens_bwd_f32(a, nb, s)
+                                    : sde_launch_sens_bwd_f64(a, nb, s);
+    else
+      lrc = p->precision == DFX_F32 ? sde_launch_adj_f32(a, nb, lds, s)
+                                    : sde_launch_adj_f64(a, nb, lds, s);
+    if (lrc != 0) return DFX_E_HIP;
     const int nout = 3 * p->d;
     hipLaunchKernelGGL(sde_reduce_kernel, dim3(nout), dim3(256), 0, s, a.partial,
                        (int)nb, p->d, g->theta_bar, g->mu_bar, g->sigma_bar);

@@ -24,6 +24,10 @@
 // folded into float64 per thread, per block in LDS, then across blocks in a fixed order
 // (deterministic).
 //
+// When only t0 and t1 are saved the gradient needs no second pass over dW: the forward
+// carries the derivatives of y by theta and sigma (sde_heun_sens_kernel) and the backward
+// is a reduction over them.
+//
 // The float64 instantiations are compiled without FMA contraction (bit parity with the
 // FP64 oracle); the float32 ones with contraction, in their own translation unit.
 #pragma once
@@ -53,6 +57,8 @@ struct SdeArgs {
   const double* ts;       // [n_ts]
   void* dense_ys;         // SaveAt(dense=True): [P, N + 1, d] step-end states (or null)
   void* dense_k;          // [P, N, 2, d] each step's two stage increments
+  double* sens;           // dy(t1)/dtheta [P, d], dy(t1)/dsigma [P, d], then per component
+                          // dy(t1)/dy0 [d] and dy(t1)/dmu [d] (sde_heun_sens_kernel)
 };
 
 // Query side of the SDE dense output: one thread per (path, query, component).
@@ -227,6 +233,158 @@ __global__ void __launch_bounds__(256) sde_heun_fwd_kernel(const SdeArgs a) {
     T* o = ys + (int64_t)sde_t1_row(a) * a.d;
 #pragma unroll
     for (int v = 0; v < V; ++v) o[v] = y[v];
+  }
+}
+
+// Forward solve of the gradient when only t0 and t1 are saved: y as sde_heun_fwd_kernel
+// (the same arithmetic), and with it the derivatives of y by theta and sigma.  With
+// c = dt theta, one Heun step is
+//   dy1/dy     = 1 - c + c^2 / 2                                       (damp)
+//   dy1/dtheta = damp dy/dtheta + dt/2 ((mu - z) + (1 - c) (mu - y))
+//   dy1/dsigma = damp dy/dsigma + (1 - c/2) w
+// and dy/dy0, dy/dmu do not depend on the path (sde_sens_coef_kernel).  The added terms are
+// formed in T, as the reverse sweep forms them; the recursions run in float64 (one fma each,
+// which issues at the float32 rate), where the sweep summed 32-step segments in T.
+// Bound: HBM, 4 bytes of dW per component-step, once: 262,144 paths x 16 x 1,000 steps take
+// 3.00 ms (5.6 TB/s) and the backward 0.035 ms, where the checkpointed pair of kernels reads
+// dW twice, 6.2 ms.  From 1 step up it is no slower (262,144 paths: 78 against 90 us for
+// one step, 165 against 262 for 32), so it serves every solve it can.  Three waves per SIMD
+// (168 VGPRs): two took 3.09 ms, four spilled (5.8 ms); 8 steps of loads in flight 3.04.
+template <class T, int V, int U>
+__global__ void __launch_bounds__(256, 3) sde_heun_sens_kernel(const SdeArgs a) {
+  const int groups = a.d / V;
+  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (tid >= a.P * groups) return;
+  const int64_t p = tid / groups;
+  const int j0 = (int)(tid - p * groups) * V;
+  const T* th_p = reinterpret_cast<const T*>(a.theta) + j0;
+  const T* mu_p = reinterpret_cast<const T*>(a.mu) + j0;
+  const T* sg_p = reinterpret_cast<const T*>(a.sigma) + j0;
+  T th[V], mu[V], sg[V], y[V];
+  double st[V], ss[V], damp[V];
+  T om[V], eh[V];  // 1 - c and 1 - c/2
+  const T* y0 = reinterpret_cast<const T*>(a.y0) + p * a.d + j0;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    th[v] = th_p[v]; mu[v] = mu_p[v]; sg[v] = sg_p[v]; y[v] = y0[v];
+    st[v] = ss[v] = 0.0;
+    damp[v] = 1.0;
+    om[v] = eh[v] = T(1);
+  }
+  T* ys = reinterpret_cast<T*>(a.ys) + p * (int64_t)a.n_out * a.d + j0;
+  if (a.save_t0) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) ys[v] = y[v];
+  }
+  const int64_t slab = a.P * a.d;  // elements per step
+  const float* dwp = a.dW + p * a.d + j0;
+  T dt_last = T(0);
+  for (int n0 = 0; n0 < a.N; n0 += U) {
+    Vec<T, V> w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (n0 + u < a.N) w[u] = load_dw<T, V>(dwp + (int64_t)(n0 + u) * slab);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = n0 + u;
+      if (n < a.N) {
+        const T dt = (T)(a.grid[n + 1] - a.grid[n]);
+        if (dt != dt_last) {  // the same for every thread; in float32 most steps share dt
+          dt_last = dt;
+#pragma unroll
+          for (int v = 0; v < V; ++v) {
+            const double c = (double)dt * (double)th[v];
+            damp[v] = __builtin_fma(0.5 * c, c, 1.0 - c);
+            om[v] = (T)(1.0 - c);
+            eh[v] = (T)(1.0 - 0.5 * c);
+          }
+        }
+        const T hd = T(0.5) * dt;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const T z = y[v] + (dt * (th[v] * (mu[v] - y[v])) + sg[v] * w[u].v[v]);
+          st[v] = __builtin_fma(damp[v], st[v], (double)(hd * ((mu[v] - z) + om[v] * (mu[v] - y[v]))));
+          ss[v] = __builtin_fma(damp[v], ss[v], (double)(eh[v] * w[u].v[v]));
+          y[v] = heun_ou<T>(y[v], dt, th[v], mu[v], sg[v], w[u].v[v]);
+        }
+      }
+    }
+  }
+  double* o = a.sens + p * a.d + j0;
+#pragma unroll
+  for (int v = 0; v < V; ++v) { o[v] = st[v]; o[slab + v] = ss[v]; }
+  if (a.save_t1) {
+    T* r = ys + (int64_t)sde_t1_row(a) * a.d;
+#pragma unroll
+    for (int v = 0; v < V; ++v) r[v] = y[v];
+  }
+}
+
+// The path-independent derivatives, one block per component: dy(t1)/dy0 = prod damp_n, and
+// dy(t1)/dmu by S <- damp S + c (1 - c/2).  Each thread composes the affine maps of a
+// contiguous run of steps, then a tree composes the 256 runs in order.
+template <class T>
+__global__ void __launch_bounds__(256) sde_sens_coef_kernel(const SdeArgs a) {
+  __shared__ double dmp[256], add[256];
+  const int j = blockIdx.x, t = threadIdx.x;
+  const double th = (double)reinterpret_cast<const T*>(a.theta)[j];
+  const int run = (a.N + 255) / 256;
+  const int hi = min((t + 1) * run, a.N);
+  double D = 1.0, M = 0.0;
+  for (int n = t * run; n < hi; ++n) {
+    const double c = (double)(T)(a.grid[n + 1] - a.grid[n]) * th;
+    const double d1 = __builtin_fma(0.5 * c, c, 1.0 - c);
+    D = d1 * D;
+    M = __builtin_fma(d1, M, c * (1.0 - 0.5 * c));
+  }
+  dmp[t] = D;
+  add[t] = M;
+  __syncthreads();
+  for (int w = 1; w < 256; w <<= 1) {
+    const int e = 2 * w * t;  // runs [e, e + w) then [e + w, e + 2w)
+    if (e + w < 256) {
+      add[e] = __builtin_fma(dmp[e + w], add[e], add[e + w]);
+      dmp[e] = dmp[e] * dmp[e + w];
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    double* coef = a.sens + 2 * a.P * a.d;
+    coef[j] = dmp[0];
+    coef[a.d + j] = add[0];
+  }
+}
+
+// Backward of the sens solve: the t1 cotangent times the derivatives, summed over the paths
+// of the block (grid-stride; each thread keeps one component, 256 being a multiple of d).
+template <class T>
+__global__ void __launch_bounds__(256) sde_sens_bwd_kernel(const SdeArgs a) {
+  __shared__ double red[3 * 256];
+  const int64_t n = a.P * a.d;
+  const int j = threadIdx.x % a.d;
+  const double* coef = a.sens + 2 * n;
+  const double dy0 = coef[j], dmu = coef[a.d + j];
+  const T* ysb = reinterpret_cast<const T*>(a.ys_bar);
+  T* y0b = reinterpret_cast<T*>(a.y0_bar);
+  double thb = 0.0, g1 = 0.0, sgb = 0.0;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+    const T* row = ysb + (e / a.d) * (int64_t)a.n_out * a.d + j;
+    const double g = a.save_t1 ? (double)row[(int64_t)sde_t1_row(a) * a.d] : 0.0;
+    thb = __builtin_fma(g, a.sens[e], thb);
+    sgb = __builtin_fma(g, a.sens[n + e], sgb);
+    g1 += g;
+    if (y0b) y0b[e] = a.save_t0 ? (T)(dy0 * g) + row[0] : (T)(dy0 * g);
+  }
+  const int ppb = 256 / a.d, lp = threadIdx.x / a.d;
+  red[(0 * a.d + j) * ppb + lp] = thb;
+  red[(1 * a.d + j) * ppb + lp] = dmu * g1;
+  red[(2 * a.d + j) * ppb + lp] = sgb;
+  __syncthreads();
+  for (int q = threadIdx.x; q < 3 * a.d; q += 256) {
+    double acc = 0.0;
+    for (int i = 0; i < ppb; ++i) acc += red[q * ppb + i];
+    a.partial[(int64_t)blockIdx.x * 3 * a.d + q] = acc;
   }
 }
 
@@ -432,6 +590,10 @@ int sde_launch_fwd_f32(const SdeArgs& a, hipStream_t s);
 int sde_launch_fwd_f64(const SdeArgs& a, hipStream_t s);
 int sde_launch_adj_f32(const SdeArgs& a, int64_t blocks, size_t lds, hipStream_t s);
 int sde_launch_adj_f64(const SdeArgs& a, int64_t blocks, size_t lds, hipStream_t s);
+int sde_launch_sens_fwd_f32(const SdeArgs& a, hipStream_t s);
+int sde_launch_sens_fwd_f64(const SdeArgs& a, hipStream_t s);
+int sde_launch_sens_bwd_f32(const SdeArgs& a, int64_t blocks, hipStream_t s);
+int sde_launch_sens_bwd_f64(const SdeArgs& a, int64_t blocks, hipStream_t s);
 int sde_launch_dense_f32(const SdeDenseArgs& a, hipStream_t s);
 int sde_launch_dense_f64(const SdeDenseArgs& a, hipStream_t s);
 constexpr int kSdeBlock = 256;

@@ -26,6 +26,18 @@ int sde_launch_adj_f64(const SdeArgs& a, int64_t nb, size_t lds, hipStream_t s) 
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+int sde_launch_sens_fwd_f64(const SdeArgs& a, hipStream_t s) {
+  const int64_t nb = (a.P * (a.d / 2) + kSdeBlock - 1) / kSdeBlock;
+  hipLaunchKernelGGL((sde_heun_sens_kernel<double, 2, 16>), dim3((unsigned)nb), dim3(kSdeBlock), 0, s, a);
+  hipLaunchKernelGGL((sde_sens_coef_kernel<double>), dim3(a.d), dim3(256), 0, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int sde_launch_sens_bwd_f64(const SdeArgs& a, int64_t nb, hipStream_t s) {
+  hipLaunchKernelGGL((sde_sens_bwd_kernel<double>), dim3((unsigned)nb), dim3(256), 0, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int sde_launch_dense_f64(const SdeDenseArgs& a, hipStream_t s) {
   const int64_t nb = (a.P * a.n_q * a.d + 255) / 256;
   hipLaunchKernelGGL((sde_dense_eval_kernel<double>), dim3((unsigned)nb), dim3(256), 0, s, a);

@@ -306,6 +306,8 @@ typedef struct dfx_sde_io {
   void* dense_ys;           /* SaveAt(dense=True), both or neither, forward only (no
                                checkpoints): out [P, N + 1, d] the step-end states         */
   void* dense_k;            /* out [P, N, 2, d] each step's two stage increments          */
+  double* sens;             /* out [dfx_sde_sens_words] derivatives of y(t1) carried by the
+                               forward instead of checkpoints, or NULL                     */
 } dfx_sde_io;
 
 /* Query side of the SDE's SaveAt(dense=True): buffers dfx_sde_heun_solve wrote. */
@@ -335,6 +337,10 @@ typedef struct dfx_sde_grad_io {
 int dfx_sde_n_out(const dfx_sde_problem* p);
 /* Number of stored checkpoints: ceil(N / CK) - 1. */
 int dfx_sde_n_ckpt(const dfx_sde_problem* p);
+/* float64 words of dfx_sde_io.sens, or 0 where the gradient needs checkpoints (saves
+ * between t0 and t1, no steps).  With sens the forward carries dy(t1)/dtheta and
+ * dy(t1)/dsigma of every path, and dfx_sde_heun_adjoint reads neither dW nor checkpoints. */
+int64_t dfx_sde_sens_words(const dfx_sde_problem* p);
 /* Workspace of dfx_sde_heun_adjoint (per-block partial sums), bytes. */
 int dfx_sde_workspace_bytes(const dfx_sde_problem* p, size_t* bytes);
 /* Forward Heun solve of P independent paths; writes ys and (if ckpt) the checkpoints.
@@ -348,7 +354,7 @@ int dfx_sde_heun_solve(const dfx_sde_problem* p, const dfx_sde_io* io, void* str
  * with ThirdOrderHermitePolynomialInterpolation (_local_interpolation.py:50-139). */
 int dfx_sde_dense_eval(const dfx_sde_problem* p, const dfx_sde_dense_io* io, void* stream);
 /* Discrete adjoint of dfx_sde_heun_solve: from ys_bar, the cotangents of y0, theta, mu,
- * sigma, replaying each CK-step segment from its checkpoint.
+ * sigma, from the forward's sens or replaying each CK-step segment from its checkpoint.
  * Replaces: reverse-mode through RecursiveCheckpointAdjoint.loop (_adjoint.py:264-312). */
 int dfx_sde_heun_adjoint(const dfx_sde_problem* p, const dfx_sde_io* io,
                          const dfx_sde_grad_io* g, void* workspace, size_t workspace_bytes,
