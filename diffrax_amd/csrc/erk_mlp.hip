@@ -39,15 +39,8 @@ __global__ void mlp_pack_kernel(const float* __restrict__ W, typename P::act_t* 
   const int64_t total = (int64_t)N * K;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= total) return;
-  const int NKS = K / P::KSTEP;
-  const int j = (int)(e % P::KA);
-  const int64_t fr = e / P::KA;
-  const int lane = (int)(fr % 64);
-  const int64_t f2 = fr / 64;
-  const int ks = (int)(f2 % NKS);
-  const int nt = (int)(f2 / NKS);
-  const int n = nt * 32 + (lane & 31);
-  const int k = ks * P::KSTEP + (lane >> 5) * P::KA + j;
+  int n, k;
+  mlp_frag_nk<P>(e, K, n, k);
   const float v = forward ? W[(int64_t)n * K + k] : W[(int64_t)k * N + n];
   out[e] = P::to_act(v);
 }
@@ -60,15 +53,8 @@ __global__ void mlp_pack3_kernel(const float* __restrict__ W, __bf16* __restrict
   const int64_t total = (int64_t)N * K;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= total) return;
-  const int NKS = K / P::KSTEP;
-  const int j = (int)(e % P::KA);
-  const int64_t fr = e / P::KA;
-  const int lane = (int)(fr % 64);
-  const int64_t f2 = fr / 64;
-  const int ks = (int)(f2 % NKS);
-  const int nt = (int)(f2 / NKS);
-  const int n = nt * 32 + (lane & 31);
-  const int k = ks * P::KSTEP + (lane >> 5) * P::KA + j;
+  int n, k;
+  mlp_frag_nk<P>(e, K, n, k);
   const float v = forward ? W[(int64_t)n * K + k] : W[(int64_t)k * N + n];
   split3(v, out[e], out[e + plane], out[e + 2 * plane]);
 }

@@ -8,8 +8,8 @@
 // pass (gradient mode) recorded the accepted (t_n, t_{n+1}) and the state at every C-th
 // accepted step.  The backward walks segments of C steps from the last one; for each
 // segment and each tile of 32 trajectories this kernel
-//   1. recomputes the segment forward from its checkpoint (identical arithmetic to the
-//      forward kernel), keeping every stage's f(z_i) in scratch and its layer inputs
+//   1. recomputes the segment forward from its checkpoint (the three-piece form's
+//      arithmetic), keeping every stage's f(z_i) in scratch and its layer inputs
 //      (z_i, h1, h2) in blocked row buffers;
 //   2. runs the exact reverse sweep: cotangents of the SaveAt(ts) values enter through the
 //      Tsit5 interpolant (k_i gets b_i(theta) ybar_s), the SSAL output y_{n+1} = z_6, and
@@ -66,241 +66,12 @@ __device__ __forceinline__ void rows_out(const typename P::act_t* lds, int ld, i
   }
 }
 
-// Element (row, col) of a blocked row buffer of width Wd.
-template <class P>
-__device__ __forceinline__ float row_val(const typename P::act_t* buf, int Wd, int64_t row,
-                                         int col) {
-  constexpr int KA = P::KA;
-  return (float)buf[((row / KA) * Wd + col) * KA + row % KA];
-}
-
-template <class P, int NW>
-__global__ void __launch_bounds__(64 * NW, 1)
-mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs<P> R) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
-  constexpr bool F = P::fast_math;
-  using Tab = Tsit5Tab;
-  constexpr int S = Tab::S;
-  using WV = MlpWaves<NW>;
-  constexpr int CPT = WV::CPT, GRP = MLP_D / CPT, NT = WV::NT12, NT3 = WV::NT3;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int orow = tid / GRP, c0 = (tid % GRP) * CPT;
-  const int tile = blockIdx.x;
-  const int64_t traj = (int64_t)tile * MLP_TILE + orow;
-  const bool valid = traj < a.B;
-  const int nacc = valid ? a.stats[traj * 3 + 1] : 0;
-  const int n0 = a.seg * a.C;
-  int steps_here = nacc - n0;
-  steps_here = steps_here < 0 ? 0 : (steps_here > a.Cs ? a.Cs : steps_here);
-  const int dir = (a.t0 < a.t1) ? 1 : -1;
-  const double* ts_row = a.ts ? a.ts + (valid ? traj : 0) * a.ts_stride : nullptr;
-  using TL = TabLit<Tab, float>;  // float32 stage algebra: the coefficients as literals
-  float* fs_tile = a.zs + (int64_t)tile * a.Cs * S * MLP_TILE * MLP_D;
-  auto fslot = [&](int q, int i) { return fs_tile + (((int64_t)q * S + i) * MLP_TILE + orow) * MLP_D + c0; };
-  // Rows of stage (q, i) in the segment's row buffers.
-  auto stage_row0 = [&](int q, int i) { return ((int64_t)q * S + i) * a.B_pad + (int64_t)tile * MLP_TILE; };
-  // The forward factors of the weight gradients (layer inputs z, h1, h2) straight from LDS
-  // after the stage's MLP evaluation.
-  auto stash_rows = [&](int q, int i) {
-    const int64_t r0 = stage_row0(q, i);
-    rows_out<P>(L.h1, L.LDH, MLP_H, R.b[3], r0);
-    rows_out<P>(L.h2, L.LDH, MLP_H, R.b[5], r0);
-    rows_out<P>(L.x, L.LDX, MLP_D, R.b[1], r0);
-  };
-
-  // ---- 1. recompute the segment: keep every stage's f (scratch) and its layer inputs (row
-  //      buffers), so that the reverse sweep needs no forward re-evaluation ----
-  float y[CPT], fl[CPT];
-#pragma unroll
-  for (int j = 0; j < CPT; ++j) y[j] = (steps_here > 0) ? a.ckpt[(traj * a.n_ckpt + a.seg) * MLP_D + c0 + j] : 0.0f;
-  for (int q = 0; q < a.Cs; ++q) {
-    const bool act = q < steps_here;
-    const int n = n0 + q;
-    const double ta = act ? a.grid[(traj * a.max_steps + n) * 2 + 0] : 0.0;
-    const double tb = act ? a.grid[(traj * a.max_steps + n) * 2 + 1] : 0.0;
-    const float control = (float)((double)dir * (tb - ta));
-    float k[S][CPT], z[CPT], f[CPT];
-    if (q == 0) {
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) store_input<P>(L, orow, c0 + j, y[j]);
-      __syncthreads();
-      mlp_forward<P, NW>(W, L, wave, lane, orow, c0, fl);
-      stash_rows(0, 0);
-      __syncthreads();
-    }
-    {
-      // stage 0 is the FSAL evaluation: f(y_n), whose rows the previous step's last stage
-      // (same input, z_6 = y_{n+1}) or the evaluation above wrote
-      float* fp = fslot(q, 0);
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) { fp[j] = fl[j]; k[0][j] = control * fl[j]; }
-    }
-    static_for<1, S>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        float kc[S];
-#pragma unroll
-        for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
-        z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        store_input<P>(L, orow, c0 + j, z[j]);
-      }
-      __syncthreads();
-      mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
-      stash_rows(q, i);
-      if constexpr (i == S - 1) {
-        if (q + 1 < a.Cs) stash_rows(q + 1, 0);
-      }
-      __syncthreads();
-      float* fp = fslot(q, i);
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) { fp[j] = f[j]; k[i][j] = control * f[j]; }
-    });
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      if (act) y[j] = z[j];
-      fl[j] = f[j];
-    }
-  }
-
-  // ---- 2. reverse sweep ----
-  float yb[CPT];
-#pragma unroll
-  for (int j = 0; j < CPT; ++j) yb[j] = valid ? a.ybar[traj * MLP_D + c0 + j] : 0.0f;
-  for (int q = a.Cs - 1; q >= 0; --q) {
-    const bool act = q < steps_here;
-    const int n = n0 + q;
-    const double ta = act ? a.grid[(traj * a.max_steps + n) * 2 + 0] : 0.0;
-    const double tb = act ? a.grid[(traj * a.max_steps + n) * 2 + 1] : 0.0;
-    const float control = (float)((double)dir * (tb - ta));
-    float kb[S][CPT], ybn[CPT];
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      ybn[j] = yb[j];
-#pragma unroll
-      for (int m = 0; m < S; ++m) kb[m][j] = 0.0f;
-    }
-    if (act) {
-      // y_{n+1} = z_6 = y_n + sum_j a_6j k_j
-#pragma unroll
-      for (int m = 0; m < S - 1; ++m) {
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) kb[m][j] += TL::v.a[S - 1][m] * yb[j];
-      }
-      // SaveAt(ts) values interpolated inside this step
-      int jlo = 0, jhi = 0;
-      for (int s = 0; s < a.n_ts; ++s) {
-        const double tsn = ts_row[s] * dir;
-        if (n > 0 && tsn <= ta) jlo = s + 1;
-        if (tsn <= tb) jhi = s + 1;
-      }
-      for (int s = jlo; s < jhi; ++s) {
-        const double th = linear_rescale(ta, ts_row[s] * dir, tb);
-        double bb[7];
-        tsit5_weights(th, bb);
-        const float* g = a.ys_bar + (traj * a.n_out + (a.save_t0 ? 1 : 0) + s) * MLP_D + c0;
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-          const float gv = g[j];
-          ybn[j] += gv;
-#pragma unroll
-          for (int m = 0; m < 7; ++m) kb[m][j] += (float)bb[m] * gv;
-        }
-      }
-    }
-    // stages in reverse
-    static_for<0, S>([&](auto ic) {
-      constexpr int i = S - 1 - decltype(ic)::value;
-      const int64_t row0 = stage_row0(q, i);
-      const float* fp = fslot(q, i);
-      // delta3 = fbar * (1 - f^2), fbar = control * kbar_i
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        const float fb = act ? control * kb[i][j] : 0.0f;
-        const float fv = fp[j];
-        L.d3[orow * L.LDX + c0 + j] = P::to_act(fb * (1.0f - fv * fv));
-      }
-      __syncthreads();
-      rows_out<P>(L.d3, L.LDX, MLP_D, R.b[4], row0);
-      // h2bar = d3 . W3 ; delta2 = h2bar * softplus'(.) (h2 from its row buffer)
-      floatx16_t acc[NT];
-      wave_gemm<P, MLP_D / P::KSTEP, NT>(L.d3, L.d3, L.LDX, W.w3t, NT * wave, 0, MLP_D / P::KSTEP,
-                                         acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = row_val<P>(R.b[5], MLP_H, row0 + r, col);
-          L.d[r * L.LDH + col] = P::to_act(acc[t][v] * dsoftplus_from_value<F>(h));
-        }
-      }
-      __syncthreads();
-      // h1bar = d2 . W2 ; delta1 = h1bar * softplus'(.), kept in L.h2
-      wave_gemm<P, MLP_H / P::KSTEP, NT>(L.d, L.d, L.LDH, W.w2t, NT * wave, 0, MLP_H / P::KSTEP,
-                                         acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = row_val<P>(R.b[3], MLP_H, row0 + r, col);
-          L.h2[r * L.LDH + col] = P::to_act(acc[t][v] * dsoftplus_from_value<F>(h));
-        }
-      }
-      __syncthreads();
-      rows_out<P>(L.d, L.LDH, MLP_H, R.b[2], row0);
-      rows_out<P>(L.h2, L.LDH, MLP_H, R.b[0], row0);
-      // zbar = d1 . W1 (split-K over the 256 hidden units)
-      constexpr int KS1 = MLP_H / P::KSTEP;
-      const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-      floatx16_t acc3[NT3];
-      wave_gemm<P, KS1, NT3>(L.h2, L.h2, L.LDH, W.w1t, n3, qk * (KS1 / 4), (qk + 1) * (KS1 / 4),
-                             acc3, lane);
-#pragma unroll
-      for (int t = 0; t < NT3; ++t) {
-        const int col = 32 * (n3 + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) L.part[(qk * MLP_TILE + acc_row(lane, v)) * L.LDP + col] = acc3[t][v];
-      }
-      __syncthreads();
-      float zb[CPT];
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        const int c = c0 + j;
-        float s = L.part[(0 * MLP_TILE + orow) * L.LDP + c];
-        s += L.part[(1 * MLP_TILE + orow) * L.LDP + c];
-        s += L.part[(2 * MLP_TILE + orow) * L.LDP + c];
-        s += L.part[(3 * MLP_TILE + orow) * L.LDP + c];
-        zb[j] = act ? s : 0.0f;
-      }
-      // z_i = y_n + sum_{m<i} a_im k_m
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        ybn[j] += zb[j];
-#pragma unroll
-        for (int m = 0; m < i; ++m) kb[m][j] += TL::v.a[i][m] * zb[j];
-      }
-      __syncthreads();
-    });
-    if (act) {
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) yb[j] = ybn[j];
-    }
-  }
-  if (valid) {
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) a.ybar[traj * MLP_D + c0 + j] = yb[j];
-  }
-}
-
-// ---- the three-piece bfloat16 form's adjoint ----------------------------------------------
-// The recompute and reverse sweep of mlp_adj_segment_kernel with every product on the
-// six-pass three-piece MFMA (wave_gemm3): the deltas are split like the activations, so the
-// gradients are those of the float32-weight model that the forward evaluates.  The row
+// ---- recompute and reverse sweep of one segment ---------------------------------------------
+// Every product runs on the six-pass three-piece MFMA (wave_gemm3) for both matmul forms:
+// the deltas are split like the activations, so the gradients are those of the
+// float32-weight model that both forwards evaluate, and the six bf16 passes take 3/8 of
+// the MFMA time of one float32 pass.  Float32 MFMA throughout took 1.97 ms for the
+// float32 form's segment of 8,192 trajectories and 4 steps.  The row
 // buffers hold float32 values (layer inputs and deltas written before their split into
 // pieces) for the float32 weight-gradient GEMM.  LDS: the forward planes;
 // in the sweep the x planes take delta3, the h1 planes delta2 and then the split-K partials,
@@ -310,7 +81,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs<P> 
 
 template <int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
-mlp_adj_segment3_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
+mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
                         const RowBufs<PolicyF32> R) {
   using P = PolicyBF16x3;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -350,7 +121,8 @@ mlp_adj_segment3_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
     if (k.row0b >= 0) R.b[1][(k.row0b + orow) * MLP_D + c0 + j] = v;
   };
 
-  // ---- 1. recompute the segment (as mlp_adj_segment_kernel) ----
+  // ---- 1. recompute the segment: keep every stage's f (scratch) and its layer inputs (row
+  //      buffers), so that the reverse sweep needs no forward re-evaluation ----
   float y[CPT], fl[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) y[j] = (steps_here > 0) ? a.ckpt[(traj * a.n_ckpt + a.seg) * MLP_D + c0 + j] : 0.0f;
@@ -538,6 +310,22 @@ mlp_adj_segment3_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
 #pragma unroll
     for (int j = 0; j < CPT; ++j) a.ybar[traj * MLP_D + c0 + j] = yb[j];
   }
+}
+
+// Three-piece planes (mlp_pack_layout(3)) of a float32 packed buffer (mlp_pack_layout(1)).
+__global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __restrict__ packed,
+                                                               __bf16* __restrict__ out) {
+  const int K[6] = {MLP_D, MLP_H, MLP_H, MLP_H, MLP_H, MLP_D};
+  const MlpPackLayout src = mlp_pack_layout(1), dst = mlp_pack_layout(3);
+  int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int m = 0;
+  while (m < 6 && e >= src.size[m]) e -= src.size[m++];
+  if (m == 6) return;
+  int n, k;
+  mlp_frag_nk<PolicyBF16x3>(e, K[m], n, k);
+  const float v = packed[src.off[m] + mlp_frag_index<PolicyF32>(n, k, K[m])];
+  __bf16* o = out + dst.off[m] + e;
+  split3(v, o[0], o[dst.size[m]], o[2 * dst.size[m]]);
 }
 
 // ---- weight gradients of one segment ---------------------------------------------------
@@ -1086,14 +874,20 @@ void launch_dw_gemm(const RowBufs<PolicyF32>& R, float* partial, float* partial_
                      0, s, R, partial, partial_db, nch, rscale);
 }
 
-// One segment: the recompute + sweep kernel `kern` with the weights of policy P (float32:
-// mlp_adj_segment_kernel on a float32 buffer; the three-piece bfloat16 form:
-// mlp_adj_segment3_kernel on the three split3 planes of a bf16 buffer), then the float32
+// Floats of the weight-gradient partials of nch chunks, and behind them (float32 form) the
+// three-piece planes of the weights.
+int64_t partial_floats(int64_t nch) {
+  return (nch * ((int64_t)dw_layout().first[3] * 1024 + 2 * MLP_H + MLP_D) + 63) / 64 * 64;
+}
+
+// One segment: the recompute + sweep kernel on three-piece weights (a bf16 buffer as it is;
+// a float32 one split into the tail of io->partial first), then the float32
 // weight-gradient GEMM over its float32 row buffers and the fixed-order reduction.
-template <class P, class Kern>
-int run_segment(Kern kern, int threads, const dfx_mlp_problem* p, const void* packed,
-                const float* b1, const float* b2, const float* b3, const dfx_mlp_adj_io* io,
-                int32_t seg, int32_t seg_steps, hipStream_t s) {
+int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, const float* b2,
+                const float* b3, const dfx_mlp_adj_io* io, int32_t seg, int32_t seg_steps,
+                hipStream_t s) {
+  using P = PolicyBF16x3;
+  constexpr int NW = 8;
   AdjArgs a;
   memset(&a, 0, sizeof(a));
   a.grid = io->grid; a.ckpt = io->ckpt; a.stats = io->stats; a.ts = io->ts; a.ys_bar = io->ys_bar;
@@ -1103,6 +897,14 @@ int run_segment(Kern kern, int threads, const dfx_mlp_problem* p, const void* pa
   a.Cs = seg_steps; a.seg = seg; a.n_ts = p->n_ts; a.ts_stride = p->ts_stride;
   a.n_out = (p->save_t0 ? 1 : 0) + p->n_ts + (p->save_t1 ? 1 : 0);
   a.save_t0 = p->save_t0; a.t0 = p->t0; a.t1 = p->t1;
+  const int nch = (int)seg_chunks(p->batch, seg_steps);
+  if (p->precision == DFX_F32) {
+    __bf16* planes = reinterpret_cast<__bf16*>(io->partial + partial_floats(nch));
+    const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);
+    hipLaunchKernelGGL(mlp_split_packed_kernel, dim3(nb), dim3(256), 0, s,
+                       reinterpret_cast<const float*>(packed), planes);
+    packed = planes;
+  }
   const MlpWeights<P> W = mlp_weights_from<P>(packed, P::PIECES, b1, b2, b3);
   RowBufs<PolicyF32> R;
   const int64_t rows_alloc = seg_chunks(p->batch, seg_steps) * ADJ_CHUNK;
@@ -1111,10 +913,10 @@ int run_segment(Kern kern, int threads, const dfx_mlp_problem* p, const void* pa
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) { R.b[i] = base + off; off += rows_alloc * widths[i]; }
   const unsigned ntiles = (unsigned)(a.B_pad / MLP_TILE);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_adj_segment_kernel<NW>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLds<P>));
-  hipLaunchKernelGGL(kern, dim3(ntiles), dim3(threads), sizeof(MlpLds<P>), s, a, W, R);
-  const int nch = (int)seg_chunks(p->batch, seg_steps);
+  hipLaunchKernelGGL(mlp_adj_segment_kernel<NW>, dim3(ntiles), dim3(64 * NW), sizeof(MlpLds<P>), s,
+                     a, W, R);
   const DwLayout lay = dw_layout();
   float* partial = io->partial;
   float* partial_db = io->partial + (int64_t)nch * lay.first[3] * 1024;
@@ -1139,8 +941,8 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) wsum += widths[i];
   *rows_bytes = (size_t)(rows_alloc * wsum) * sizeof(float);   // float32 rows for both forms
-  const DwLayout lay = dw_layout();
-  *partial_bytes = (size_t)(seg_chunks(p->batch, seg_steps) * ((int64_t)lay.first[3] * 1024 + 2 * MLP_H + MLP_D)) * sizeof(float);
+  *partial_bytes = (size_t)partial_floats(seg_chunks(p->batch, seg_steps)) * sizeof(float);
+  if (p->precision == DFX_F32) *partial_bytes += (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
 }
 
@@ -1246,17 +1048,10 @@ int dfx_mlp_adj_segment(const dfx_mlp_problem* p, const void* packed, const floa
   if (p->ts_stride != 0 && p->ts_stride != p->n_ts) return DFX_E_ARG;
   if (p->batch == 0) return DFX_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // eight waves per tile, two per SIMD: at four the kernels held 415 (float32) and 512 + 93
-  // spilled (three-piece) registers per lane, one wave per SIMD.  The backward of 8,192
-  // trajectories went from 3.11 to 2.86 ms (float32) and from 2.51-2.55 to 2.16-2.17 ms
-  // (three-piece), with bit-identical gradients.
-  if (p->precision == DFX_BF16_F32)
-    return run_segment<PolicyBF16x3>(&mlp_adj_segment3_kernel<8>, 64 * 8, p, packed, b1, b2, b3,
-                                      io, segment, seg_steps, s);
-  if (p->precision == DFX_F32)
-    return run_segment<PolicyF32>(&mlp_adj_segment_kernel<PolicyF32, 8>, 64 * 8, p, packed, b1,
-                                  b2, b3, io, segment, seg_steps, s);
-  return DFX_E_ARG;
+  // eight waves per tile, two per SIMD: at four the kernel held 512 registers per lane, 93
+  // spilled, one wave per SIMD, and the backward of 8,192 trajectories took 2.51-2.55 ms
+  // against 2.16-2.17 (bit-identical gradients).
+  return run_segment(p, packed, b1, b2, b3, io, segment, seg_steps, s);
 }
 
 }  // extern "C"

@@ -120,6 +120,23 @@ __host__ __device__ inline MlpPackLayout mlp_pack_layout(int pieces) {
   return l;
 }
 
+// Element e of a packed matrix with K input columns <-> its (n, k): fragments (n tile,
+// k step) of 64 lanes x KA elements.
+template <class P>
+__host__ __device__ inline void mlp_frag_nk(int64_t e, int K, int& n, int& k) {
+  const int j = (int)(e % P::KA), lane = (int)(e / P::KA % 64);
+  const int64_t f = e / P::KA / 64;
+  const int nks = K / P::KSTEP;
+  n = (int)(f / nks) * 32 + (lane & 31);
+  k = (int)(f % nks) * P::KSTEP + (lane >> 5) * P::KA + j;
+}
+template <class P>
+__host__ __device__ inline int64_t mlp_frag_index(int n, int k, int K) {
+  const int kk = k % P::KSTEP;
+  const int lane = (n & 31) + 32 * (kk / P::KA);
+  return (((int64_t)(n / 32) * (K / P::KSTEP) + k / P::KSTEP) * 64 + lane) * P::KA + kk % P::KA;
+}
+
 // Packed weights of one solve.  Forward fragments: B[k][n] = W[n][k].  Backward fragments
 // (transposed products): B[k][n] = W[k][n].
 template <class P>
