@@ -16,12 +16,13 @@ __global__ void __launch_bounds__(MLP_THREADS, 1) mlp_eval_kernel(const float* _
                                                                   const MlpWeights<P> W) {
   extern __shared__ __align__(16) unsigned char smem[];
   MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int orow = tid >> 3, c0 = (tid & 7) * 8;
   const int64_t row = (int64_t)blockIdx.x * MLP_TILE + orow;
   const bool valid = row < R;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) store_input<P>(L, orow, c0 + j, valid ? Y[row * MLP_D + c0 + j] : 0.0f);
+  for (int j = 0; j < 8; ++j) store_input(L, orow, c0 + j, valid ? Y[row * MLP_D + c0 + j] : 0.0f);
+  mlp_begin<P>(W, L);
   __syncthreads();
   float f[8];
   mlp_forward<P>(W, L, wave, lane, orow, c0, f);
@@ -31,32 +32,26 @@ __global__ void __launch_bounds__(MLP_THREADS, 1) mlp_eval_kernel(const float* _
   }
 }
 
-// Pack a row-major float32 matrix into MFMA B fragments.  forward: B[k][n] = W[n][k]
-// (W is [N][K]); otherwise B[k][n] = W[k][n] (W is [K][N]).
+// Pack the three weight matrices (row-major float32, W1 [256, 64], W2 [256, 256], W3
+// [64, 256]) into MFMA fragments, forward and transposed, all six in one launch (six took 15
+// to 18 us of launches for 0.8 MB).  Three-piece form: element e of plane p holds piece p of
+// split3(v).
 template <class P>
-__global__ void mlp_pack_kernel(const float* __restrict__ W, typename P::act_t* __restrict__ out,
-                                int N, int K, int forward) {
-  const int64_t total = (int64_t)N * K;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
+__global__ void __launch_bounds__(256) mlp_pack_kernel(const float* __restrict__ w1,
+                                                       const float* __restrict__ w2,
+                                                       const float* __restrict__ w3,
+                                                       typename P::act_t* __restrict__ out) {
+  int e = blockIdx.x * 256 + threadIdx.x, m, before;
+  mlp_pack_find(e, m, before);
+  if (m == 6) return;
+  const MlpPackShape sh = mlp_pack_shape(m);
   int n, k;
-  mlp_frag_nk<P>(e, K, n, k);
-  const float v = forward ? W[(int64_t)n * K + k] : W[(int64_t)k * N + n];
-  out[e] = P::to_act(v);
-}
-
-// Three-piece bf16 packing (PolicyBF16x3): fragment element e of plane p holds piece p of
-// split3(v); the planes are `plane` elements apart.
-__global__ void mlp_pack3_kernel(const float* __restrict__ W, __bf16* __restrict__ out, int N,
-                                 int K, int forward, int64_t plane) {
-  using P = PolicyBF16x3;
-  const int64_t total = (int64_t)N * K;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int n, k;
-  mlp_frag_nk<P>(e, K, n, k);
-  const float v = forward ? W[(int64_t)n * K + k] : W[(int64_t)k * N + n];
-  split3(v, out[e], out[e + plane], out[e + 2 * plane]);
+  mlp_frag_nk<P>(e, sh.k, n, k);
+  const float* W = m % 3 == 0 ? w1 : m % 3 == 1 ? w2 : w3;
+  const float v = sh.forward ? W[n * sh.k + k] : W[k * sh.n + n];
+  typename P::act_t* o = out + P::PIECES * before + e;
+  if constexpr (P::PIECES == 3) split3(v, o[0], o[sh.n * sh.k], o[2 * sh.n * sh.k]);
+  else *o = v;
 }
 
 // Dense output of the neural ODE at query times (erk_dense.hpp's evaluation for d = 64):
@@ -170,24 +165,14 @@ int dfx_mlp_pack(int32_t precision, const float* w1, const float* w2, const floa
                  void* stream) {
   if (!w1 || !w2 || !w3 || !packed) return DFX_E_ARG;
   if (precision != DFX_F32 && precision != DFX_BF16_F32) return DFX_E_ARG;
-  const MlpPackLayout lay = mlp_pack_layout(pieces_of(precision));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  struct Job { const float* W; int N, K, fwd; };
-  const Job jobs[6] = {{w1, MLP_H, MLP_D, 1}, {w2, MLP_H, MLP_H, 1}, {w3, MLP_D, MLP_H, 1},
-                       {w1, MLP_D, MLP_H, 0}, {w2, MLP_H, MLP_H, 0}, {w3, MLP_H, MLP_D, 0}};
-  for (int i = 0; i < 6; ++i) {
-    const int64_t n = (int64_t)jobs[i].N * jobs[i].K;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    if (precision == DFX_BF16_F32) {
-      __bf16* o = reinterpret_cast<__bf16*>(packed) + lay.off[i];
-      hipLaunchKernelGGL(mlp_pack3_kernel, dim3(nb), dim3(256), 0, s, jobs[i].W, o, jobs[i].N,
-                         jobs[i].K, jobs[i].fwd, lay.size[i]);
-    } else {
-      float* o = reinterpret_cast<float*>(packed) + lay.off[i];
-      hipLaunchKernelGGL(mlp_pack_kernel<PolicyF32>, dim3(nb), dim3(256), 0, s, jobs[i].W, o,
-                         jobs[i].N, jobs[i].K, jobs[i].fwd);
-    }
-  }
+  const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);  // elements, any planes
+  if (precision == DFX_BF16_F32)
+    hipLaunchKernelGGL(mlp_pack_kernel<PolicyBF16x3>, dim3(nb), dim3(256), 0, s, w1, w2, w3,
+                       reinterpret_cast<__bf16*>(packed));
+  else
+    hipLaunchKernelGGL(mlp_pack_kernel<PolicyF32>, dim3(nb), dim3(256), 0, s, w1, w2, w3,
+                       reinterpret_cast<float*>(packed));
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -281,11 +266,14 @@ int dfx_mlp_solve(const dfx_mlp_problem* p, const void* packed, const float* b1,
   const bool integral = mlp_pid_params(p, a.pid);
   const unsigned nblocks = (unsigned)((p->batch + MLP_TILE - 1) / MLP_TILE);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // waves per tile (MlpWaves): the problem's choice, or by default eight for the
-  // three-piece form (its 436 registers per lane at four waves leave one wave per SIMD; at
-  // eight, two) and four for float32 (0.49 against 0.52 ms per solve of 8,192
-  // trajectories at eight)
-  const int waves = p->waves != 0 ? p->waves : (p->precision == DFX_BF16_F32 ? 8 : 4);
+  // waves per tile (MlpWaves): the problem's choice, or by default eight, two per SIMD, for
+  // the three-piece form (its registers at four waves leave one wave per SIMD) and for
+  // float32 batches of at most one tile per CU; larger float32 batches take four, of which
+  // two workgroups share a CU and fill each other's barriers (solves of 8,192, 10,007 and
+  // 16,384 trajectories: 416, 776 and 785 us at eight, 427, 743 and 756 us at four)
+  constexpr unsigned kCus = 256;
+  const int waves = p->waves != 0 ? p->waves
+                    : (p->precision == DFX_BF16_F32 || nblocks <= kCus) ? 8 : 4;
   const bool g = p->ckpt_every > 0;
   if (p->precision == DFX_BF16_F32)
     launch_erk_mlp_bf16(waves, a, weights_from<PolicyBF16x3>(packed, b1, b2, b3), g, integral,

@@ -60,15 +60,19 @@ struct MlpArgs {
 // the reference (runge_kutta.py:684-690); here the FSAL stage is kept, which is the same
 // value bit for bit: the last stage is evaluated at the new state itself and the field is
 // autonomous.
+// Registers: two waves per SIMD in every build but the three-piece form's four-wave one.  For
+// float32 at four waves that is two workgroups per CU, and faster also at one (8,192
+// trajectories: 427 against 443 us with 256 + 89 registers and one wave per SIMD).
 template <class P, class Tab, bool Grad, int Ctl, int NW, bool Ext = false>
-__global__ void __launch_bounds__(64 * NW, 1) erk_mlp_kernel(const MlpArgs a, const MlpWeights<P> W) {
+__global__ void __launch_bounds__(64 * NW, P::PIECES == 1 && NW == 4 ? 2 : 1)
+erk_mlp_kernel(const MlpArgs a, const MlpWeights<P> W) {
   extern __shared__ __align__(16) unsigned char smem[];
   MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
   constexpr int S = Tab::S;
   constexpr int CPT = MlpWaves<NW>::CPT;  // components per owner
   constexpr int GRP = MLP_D / CPT;         // owners per trajectory
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int orow = tid / GRP;             // trajectory within the tile
   const int c0 = (tid % GRP) * CPT;       // owner's first component
   const int gbase = lane & ~(GRP - 1);    // first lane of this trajectory's owner group
@@ -148,7 +152,8 @@ __global__ void __launch_bounds__(64 * NW, 1) erk_mlp_kernel(const MlpArgs a, co
 
   // ---- first stage of the first step (FSAL seed): f(t0, y0) ----
 #pragma unroll
-  for (int j = 0; j < CPT; ++j) store_input<P>(L, orow, c0 + j, y[j]);
+  for (int j = 0; j < CPT; ++j) store_input(L, orow, c0 + j, y[j]);
+  mlp_begin<P>(W, L);
   __syncthreads();
   mlp_forward<P, NW>(W, L, wave, lane, orow, c0, fsal);
 
@@ -191,7 +196,7 @@ __global__ void __launch_bounds__(64 * NW, 1) erk_mlp_kernel(const MlpArgs a, co
     const double h0 = cond ? 1e-6 : 0.01 * (d0 / (cond ? 1.0 : d1));
     __syncthreads();  // every wave is done with the seed's layer-3 partials
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) store_input<P>(L, orow, c0 + j, y[j] + (float)h0 * fsal[j]);
+    for (int j = 0; j < CPT; ++j) store_input(L, orow, c0 + j, y[j] + (float)h0 * fsal[j]);
     __syncthreads();
     float f1[CPT];
     mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f1);
@@ -267,7 +272,7 @@ __global__ void __launch_bounds__(64 * NW, 1) erk_mlp_kernel(const MlpArgs a, co
 #pragma unroll
         for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
         z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        store_input<P>(L, orow, c0 + j, z[j]);
+        store_input(L, orow, c0 + j, z[j]);
       }
       __syncthreads();
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);

@@ -33,9 +33,8 @@ constexpr int ADJ_CHUNK = 4096;  // rows per split-K chunk of the weight-gradien
 
 // Six row buffers: D1 (width 256), Z (64), D2 (256), H1 (256), D3 (64), H2 (256).
 
-template <class P>
-struct RowBufs {
-  typename P::act_t* b[6];
+struct RowBufs {  // float32 [rows][width]
+  float* b[6];
 };
 
 struct AdjArgs {
@@ -50,21 +49,6 @@ struct AdjArgs {
   int32_t max_steps, n_ckpt, C, Cs, seg, n_ts, n_out, save_t0;
   double t0, t1;
 };
-
-// Copy 32 tile rows of an LDS buffer [32][ld] into a blocked global row buffer of width
-// Wd: element (row, col) at ((row / KA) * Wd + col) * KA + row % KA.
-template <class P>
-__device__ __forceinline__ void rows_out(const typename P::act_t* lds, int ld, int Wd,
-                                         typename P::act_t* dst, int64_t row0) {
-  constexpr int KA = P::KA;
-  const int pairs = (MLP_TILE / KA) * Wd;
-  for (int e = threadIdx.x; e < pairs; e += blockDim.x) {
-    const int rb = e / Wd, col = e - rb * Wd;
-    typename P::act_t* o = dst + ((row0 / KA + rb) * Wd + col) * KA;
-#pragma unroll
-    for (int j = 0; j < KA; ++j) o[j] = lds[(rb * KA + j) * ld + col];
-  }
-}
 
 // ---- recompute and reverse sweep of one segment ---------------------------------------------
 // Every product runs on the six-pass three-piece MFMA (wave_gemm3) for both matmul forms:
@@ -82,7 +66,7 @@ __device__ __forceinline__ void rows_out(const typename P::act_t* lds, int ld, i
 template <int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
 mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
-                        const RowBufs<PolicyF32> R) {
+                        const RowBufs R) {
   using P = PolicyBF16x3;
   extern __shared__ __align__(16) unsigned char smem[];
   MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
@@ -90,7 +74,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
   constexpr int S = Tab::S;
   using WV = MlpWaves<NW>;
   constexpr int CPT = WV::CPT, GRP = MLP_D / CPT, NT = WV::NT12, NT3 = WV::NT3;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int orow = tid / GRP, c0 = (tid % GRP) * CPT;
   const int tile = blockIdx.x;
   const int64_t traj = (int64_t)tile * MLP_TILE + orow;
@@ -137,7 +121,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
       const MlpRowSink k0 = sink_of(0, 0);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        store_input<P>(L, orow, c0 + j, y[j]);
+        store_input(L, orow, c0 + j, y[j]);
         put_x(k0, j, y[j]);
       }
       __syncthreads();
@@ -158,7 +142,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
 #pragma unroll
         for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
         z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        store_input<P>(L, orow, c0 + j, z[j]);
+        store_input(L, orow, c0 + j, z[j]);
         put_x(ki, j, z[j]);
       }
       __syncthreads();
@@ -244,7 +228,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
         for (int v = 0; v < 16; ++v) {
           const int r = acc_row(lane, v);
           const float h = R.b[5][(row0 + r) * MLP_H + col];
-          const float d2 = acc[t][v] * dsoftplus_from_value<true>(h);
+          const float d2 = acc[t][v] * dsoftplus_from_value(h);
           R.b[2][(row0 + r) * MLP_H + col] = d2;
           const int li = r * L.LDH + col;
           split3(d2, L.h1[0][li], L.h1[1][li], L.h1[2][li]);
@@ -261,7 +245,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
         for (int v = 0; v < 16; ++v) {
           const int r = acc_row(lane, v);
           const float h = R.b[3][(row0 + r) * MLP_H + col];
-          const float d1 = acc[t][v] * dsoftplus_from_value<true>(h);
+          const float d1 = acc[t][v] * dsoftplus_from_value(h);
           R.b[0][(row0 + r) * MLP_H + col] = d1;
           const int li = r * L.LDH + col;
           split3(d1, L.h2[0][li], L.h2[1][li], L.h2[2][li]);
@@ -315,17 +299,15 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
 // Three-piece planes (mlp_pack_layout(3)) of a float32 packed buffer (mlp_pack_layout(1)).
 __global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __restrict__ packed,
                                                                __bf16* __restrict__ out) {
-  const int K[6] = {MLP_D, MLP_H, MLP_H, MLP_H, MLP_H, MLP_D};
-  const MlpPackLayout src = mlp_pack_layout(1), dst = mlp_pack_layout(3);
-  int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  int m = 0;
-  while (m < 6 && e >= src.size[m]) e -= src.size[m++];
+  int e = blockIdx.x * 256 + threadIdx.x, m, before;
+  mlp_pack_find(e, m, before);
   if (m == 6) return;
+  const MlpPackShape sh = mlp_pack_shape(m);
   int n, k;
-  mlp_frag_nk<PolicyBF16x3>(e, K[m], n, k);
-  const float v = packed[src.off[m] + mlp_frag_index<PolicyF32>(n, k, K[m])];
-  __bf16* o = out + dst.off[m] + e;
-  split3(v, o[0], o[dst.size[m]], o[2 * dst.size[m]]);
+  mlp_frag_nk<PolicyBF16x3>(e, sh.k, n, k);
+  const float v = packed[before + mlp_frag_index<PolicyF32>(n, k, sh.k)];
+  __bf16* o = out + 3 * before + e;
+  split3(v, o[0], o[sh.n * sh.k], o[2 * sh.n * sh.k]);
 }
 
 // ---- weight gradients of one segment ---------------------------------------------------
@@ -364,13 +346,12 @@ __host__ __device__ inline int dw_blocks_of(int m) {
   return (l.n1[m] / 64) * (l.n2[m] / 64);
 }
 
-template <class P, bool SC = false>
-__global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs<P> R,
+template <bool SC = false>
+__global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs R,
                                                            float* __restrict__ partial,
                                                            float* __restrict__ partial_db,
                                                            int nch,
                                                            const float* __restrict__ rscale = nullptr) {
-  static_assert(!SC || P::KA == 1, "row scales need one row per fragment element");
   const DwLayout lay = dw_layout();
   const int nblk = dw_blocks_of(0) + dw_blocks_of(1) + dw_blocks_of(2);
   const int xcd = (int)(blockIdx.x % kXcds), slot = (int)(blockIdx.x / kXcds);
@@ -381,11 +362,11 @@ __global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs<P> R,
   while (bg >= dw_blocks_of(m)) { bg -= dw_blocks_of(m); ++m; }
   const int nbj = lay.n2[m] / 64;
   const int bi = bg / nbj, bj = bg - bi * nbj;
-  const typename P::act_t* A = R.b[2 * m];       // deltas (width n1)
-  const typename P::act_t* Bm = R.b[2 * m + 1];  // layer inputs (width n2)
+  const float* A = R.b[2 * m];       // deltas (width n1)
+  const float* Bm = R.b[2 * m + 1];  // layer inputs (width n2)
   const int WA = lay.n1[m], WB = lay.n2[m];
   const int lane = threadIdx.x;
-  constexpr int KA = P::KA, KS = P::KSTEP, U = 4;
+  constexpr int KS = 2, U = 4;
   static_assert(ADJ_CHUNK % (KS * U) == 0, "chunk must hold whole k-step groups");
   const bool col_sums = (bj == 0);
   const int64_t r_begin = (int64_t)chunk * ADJ_CHUNK;
@@ -394,15 +375,15 @@ __global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs<P> R,
   for (int x = 0; x < 2; ++x) { acc[x][0] = floatx16_t{}; acc[x][1] = floatx16_t{}; }
   float csum[2] = {0.0f, 0.0f};
   const int ca = bi * 64 + (lane & 31), cb = bj * 64 + (lane & 31);
-  using frag_t = typename P::frag_t;
+  using frag_t = float;
   auto load_group = [&](int64_t r0, frag_t (&fa)[U][2], frag_t (&fb)[U][2]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t rb = (r0 + u * KS) / KA + (lane >> 5);
+      const int64_t rb = r0 + u * KS + (lane >> 5);
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        fa[u][x] = P::load_a(A + (rb * WA + ca + 32 * x) * KA);
-        fb[u][x] = P::load_a(Bm + (rb * WB + cb + 32 * x) * KA);
+        fa[u][x] = A[rb * WA + ca + 32 * x];
+        fb[u][x] = Bm[rb * WB + cb + 32 * x];
       }
       if constexpr (SC) {
         const float w = rscale[rb];
@@ -419,16 +400,9 @@ __global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs<P> R,
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        acc[x][0] = P::mfma(fa[u][x], fb[u][0], acc[x][0]);
-        acc[x][1] = P::mfma(fa[u][x], fb[u][1], acc[x][1]);
-        if (col_sums) {
-          if constexpr (KA == 1) {
-            csum[x] += fa[u][x];
-          } else {
-#pragma unroll
-            for (int j = 0; j < KA; ++j) csum[x] += (float)fa[u][x][j];
-          }
-        }
+        acc[x][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u][x], fb[u][0], acc[x][0], 0, 0, 0);
+        acc[x][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u][x], fb[u][1], acc[x][1], 0, 0, 0);
+        if (col_sums) csum[x] += fa[u][x];
       }
     }
   };
@@ -528,19 +502,37 @@ struct BsArgs {
   PidParams pid;         // the backward controller
 };
 
-template <class P, int NW>
+// The forward's LDS with partials of their own (h1 is read again after layer 3) and the
+// deltas of layers 3 and 2.
+struct MlpLdsBack : MlpLds<PolicyF32> {
+  float d[MLP_TILE * LDH];
+  float d3[MLP_TILE * LDX];
+  float part_[4 * MLP_TILE * LDP];
+  __device__ __forceinline__ float* part() { return part_; }
+};
+static_assert(sizeof(MlpLdsBack) <= 160 * 1024, "one workgroup per CU");
+
+// The tile's rows of an LDS buffer (columns at PolicyF32::pos) to row-major rows of width Wd.
+template <int Wd>
+__device__ __forceinline__ void rows_out(const float* lds, int ld, float* dst, int64_t row0) {
+  for (int e = threadIdx.x; e < MLP_TILE * Wd; e += blockDim.x) {
+    const int r = e / Wd, col = e % Wd;
+    dst[(row0 + r) * Wd + col] = lds[r * ld + PolicyF32::pos(col)];
+  }
+}
+
+template <int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
-mlp_backsolve_kernel(const BsArgs a, const MlpWeights<P> W, const RowBufs<P> R) {
-  static_assert(P::KA == 1, "float32 rows");
+mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBufs R) {
+  using P = PolicyF32;
   extern __shared__ __align__(16) unsigned char smem[];
-  MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
-  constexpr bool F = P::fast_math;
+  MlpLdsBack& L = *reinterpret_cast<MlpLdsBack*>(smem);
   using Tab = Tsit5Tab;
   constexpr int S = Tab::S;
   using TL = TabLit<Tab, float>;
   using WV = MlpWaves<NW>;
   constexpr int CPT = WV::CPT, GRP = MLP_D / CPT, NT = WV::NT12, NT3 = WV::NT3;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int orow = tid / GRP, c0 = (tid % GRP) * CPT, gbase = lane & ~(GRP - 1);
   const bool lead = (tid % GRP) == 0;
   const int tile = blockIdx.x;
@@ -622,6 +614,26 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<P> W, const RowBufs<P> R) 
     }
   }
 
+  mlp_begin<P>(W, L);  // the first iteration's barriers come before its first use
+  const int half = lane >> 5, row = lane & 31;
+  // delta = acc softplus'(h) of the layer whose activations h are given, into dst
+  auto put_delta = [&](const floatx16_t (&acc)[NT], const float* hbuf, float* dst) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int o = row * L.LDH + P::pos(32 * (NT * wave + t) + 8 * i + 4 * half);
+        const float2 he = *reinterpret_cast<const float2*>(hbuf + o);
+        const float2 ho = *reinterpret_cast<const float2*>(hbuf + o + 4);
+        *reinterpret_cast<float2*>(dst + o) =
+            make_float2(acc[t][4 * i] * dsoftplus_from_value(he.x),
+                        acc[t][4 * i + 2] * dsoftplus_from_value(he.y));
+        *reinterpret_cast<float2*>(dst + o + 4) =
+            make_float2(acc[t][4 * i + 1] * dsoftplus_from_value(ho.x),
+                        acc[t][4 * i + 3] * dsoftplus_from_value(ho.y));
+      }
+    }
+  };
   const int64_t rb0 = (int64_t)tile * MLP_TILE + orow;
   auto stage_row0 = [&](int q, int i) { return ((int64_t)q * S + i) * a.B_pad + (int64_t)tile * MLP_TILE; };
   int q = 0;
@@ -649,71 +661,59 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<P> W, const RowBufs<P> R) 
           za[j] = av[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], ca, 0.0f);
         }
         if (!run) { zy[j] = 0.0f; za[j] = 0.0f; }  // idle rows: zero deltas
-        store_input<P>(L, orow, c0 + j, zy[j]);
+        store_input(L, orow, c0 + j, zy[j]);
       }
       __syncthreads();
       float f[CPT];
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
       const int64_t row0 = stage_row0(q, i);
-      rows_out<P>(L.x, L.LDX, MLP_D, R.b[1], row0);
-      rows_out<P>(L.h1, L.LDH, MLP_H, R.b[3], row0);
-      rows_out<P>(L.h2, L.LDH, MLP_H, R.b[5], row0);
+      rows_out<MLP_D>(L.x, L.LDX, R.b[1], row0);
+      rows_out<MLP_H>(L.h1, L.LDH, R.b[3], row0);
+      rows_out<MLP_H>(L.h2, L.LDH, R.b[5], row0);
       // vjp with cotangent w = -a_y of the stage: delta3 = w (1 - f^2)
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) L.d3[orow * L.LDX + c0 + j] = P::to_act(-za[j] * (1.0f - f[j] * f[j]));
+      for (int j = 0; j < CPT; ++j)
+        L.d3[orow * L.LDX + P::pos(c0 + j)] = -za[j] * (1.0f - f[j] * f[j]);
       __syncthreads();
-      rows_out<P>(L.d3, L.LDX, MLP_D, R.b[4], row0);
+      rows_out<MLP_D>(L.d3, L.LDX, R.b[4], row0);
       // delta2 = (delta3 . W3) softplus'(h2)
+      constexpr int F1 = MLP_D / P::KSTEP, F2 = MLP_H / P::KSTEP;
       floatx16_t acc[NT];
-      wave_gemm<P, MLP_D / P::KSTEP, NT>(L.d3, L.d3, L.LDX, W.w3t, NT * wave, 0, MLP_D / P::KSTEP,
-                                         acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = (float)L.h2[r * L.LDH + col];
-          L.d[r * L.LDH + col] = P::to_act(acc[t][v] * dsoftplus_from_value<F>(h));
-        }
-      }
+      GemmF32<F1, NT> g3t;
+      g3t.preload(W.w3t, NT * wave, 0, lane);
+      g3t.template run<F1>(L.d3, L.LDX, 0, acc, lane);
+      put_delta(acc, L.h2, L.d);
       __syncthreads();
       // delta1 = (delta2 . W2) softplus'(h1), into the h2 buffer (h2 is in its row buffer)
-      wave_gemm<P, MLP_H / P::KSTEP, NT>(L.d, L.d, L.LDH, W.w2t, NT * wave, 0, MLP_H / P::KSTEP,
-                                         acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = (float)L.h1[r * L.LDH + col];
-          L.h2[r * L.LDH + col] = P::to_act(acc[t][v] * dsoftplus_from_value<F>(h));
-        }
-      }
+      GemmF32<F2, NT> g2t;
+      g2t.preload(W.w2t, NT * wave, 0, lane);
+      g2t.template run<F2>(L.d, L.LDH, 0, acc, lane);
+      put_delta(acc, L.h1, L.h2);
       __syncthreads();
-      rows_out<P>(L.d, L.LDH, MLP_H, R.b[2], row0);
-      rows_out<P>(L.h2, L.LDH, MLP_H, R.b[0], row0);
+      rows_out<MLP_H>(L.d, L.LDH, R.b[2], row0);
+      rows_out<MLP_H>(L.h2, L.LDH, R.b[0], row0);
       // vjp_y = delta1 . W1 (split-K over the 256 hidden units)
-      constexpr int KS1 = MLP_H / P::KSTEP;
       const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
       floatx16_t acc3[NT3];
-      wave_gemm<P, KS1, NT3>(L.h2, L.h2, L.LDH, W.w1t, n3, qk * (KS1 / 4), (qk + 1) * (KS1 / 4),
-                             acc3, lane);
+      GemmF32<F2, NT3> g1t;
+      g1t.preload(W.w1t, n3, qk * (F2 / 4), lane);
+      g1t.template run<F2 / 4>(L.h2, L.LDH, qk * (F2 / 4), acc3, lane);
+      float* part = L.part();
 #pragma unroll
       for (int t = 0; t < NT3; ++t) {
-        const int col = 32 * (n3 + t) + (lane & 31);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) L.part[(qk * MLP_TILE + acc_row(lane, v)) * L.LDP + col] = acc3[t][v];
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<float4*>(part + (qk * MLP_TILE + row) * L.LDP + 32 * (n3 + t) + 8 * i + 4 * half) =
+              make_float4(acc3[t][4 * i], acc3[t][4 * i + 1], acc3[t][4 * i + 2], acc3[t][4 * i + 3]);
       }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
         const int c = c0 + j;
-        float sv = L.part[(0 * MLP_TILE + orow) * L.LDP + c];
-        sv += L.part[(1 * MLP_TILE + orow) * L.LDP + c];
-        sv += L.part[(2 * MLP_TILE + orow) * L.LDP + c];
-        sv += L.part[(3 * MLP_TILE + orow) * L.LDP + c];
+        float sv = part[(0 * MLP_TILE + orow) * L.LDP + c];
+        sv += part[(1 * MLP_TILE + orow) * L.LDP + c];
+        sv += part[(2 * MLP_TILE + orow) * L.LDP + c];
+        sv += part[(3 * MLP_TILE + orow) * L.LDP + c];
         ky[i][j] = control * f[j];
         ka[i][j] = control * sv;
       }
@@ -866,11 +866,11 @@ __global__ void bs_reset_kernel(int32_t* counters, float* rscale, int64_t used, 
 
 // The weight-gradient GEMM over nch chunks of float32 rows (SC: per-row weights rscale).
 template <bool SC>
-void launch_dw_gemm(const RowBufs<PolicyF32>& R, float* partial, float* partial_db, int nch,
+void launch_dw_gemm(const RowBufs& R, float* partial, float* partial_db, int nch,
                     const float* rscale, hipStream_t s) {
   const int groups = (nch + kXcds - 1) / kXcds;
   const int nblk = dw_blocks_of(0) + dw_blocks_of(1) + dw_blocks_of(2);
-  hipLaunchKernelGGL((mlp_dw_gemm_kernel<PolicyF32, SC>), dim3(kXcds * nblk * groups), dim3(64),
+  hipLaunchKernelGGL((mlp_dw_gemm_kernel<SC>), dim3(kXcds * nblk * groups), dim3(64),
                      0, s, R, partial, partial_db, nch, rscale);
 }
 
@@ -906,7 +906,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
     packed = planes;
   }
   const MlpWeights<P> W = mlp_weights_from<P>(packed, P::PIECES, b1, b2, b3);
-  RowBufs<PolicyF32> R;
+  RowBufs R;
   const int64_t rows_alloc = seg_chunks(p->batch, seg_steps) * ADJ_CHUNK;
   float* base = reinterpret_cast<float*>(io->rows);
   int64_t off = 0;
@@ -995,7 +995,7 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   // for DFX_F32): the bfloat16 form's forward evaluates the float32-weight model too.
   using P = PolicyF32;
   const MlpWeights<P> W = mlp_weights_from<P>(packed, 1, b1, b2, b3);
-  RowBufs<P> R;
+  RowBufs R;
   float* base = reinterpret_cast<float*>(io->rows);
   int64_t off = 0;
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
@@ -1008,10 +1008,10 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   // took 34.9 ms against 19.6 ms for the backsolve of 8,192 trajectories (bit-identical
   // gradients)
   constexpr int NWB = 4;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_backsolve_kernel<P, NWB>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLds<P>));
-  hipLaunchKernelGGL((mlp_backsolve_kernel<P, NWB>), dim3(ntiles), dim3(64 * NWB),
-                     sizeof(MlpLds<P>), s, a, W, R);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_backsolve_kernel<NWB>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLdsBack));
+  hipLaunchKernelGGL((mlp_backsolve_kernel<NWB>), dim3(ntiles), dim3(64 * NWB),
+                     sizeof(MlpLdsBack), s, a, W, R);
   const DwLayout lay = dw_layout();
   float* partial = io->partial;
   float* partial_db = io->partial + (int64_t)nch * lay.first[3] * 1024;

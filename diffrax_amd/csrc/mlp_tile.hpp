@@ -12,8 +12,9 @@
 //  - layers 1 and 2: wave w produces output columns [64w, 64w + 64) (two 32x32 tiles);
 //    layer 3 (64 outputs, K = 256) is split over K: wave w reduces K in [64w, 64w + 64) and
 //    the four partial sums meet in LDS, where the owner threads add them in wave order.
-// Precision policies: BF16 operands with f32 accumulate (v_mfma_f32_32x32x16_bf16), or
-// f32 throughout (v_mfma_f32_32x32x2f32).  Activation functions are evaluated in f32.
+// Precision policies: three-piece BF16 operands with f32 accumulate
+// (v_mfma_f32_32x32x16_bf16), or f32 throughout (v_mfma_f32_32x32x2f32).  Activation
+// functions are evaluated in f32.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -32,20 +33,46 @@ constexpr int MLP_H = 256;
 constexpr int MLP_TILE = 32;
 constexpr int MLP_THREADS = 256;
 
-struct PolicyBF16 {
+// Float32 MFMA.  One fragment is four consecutive k steps of v_mfma_f32_32x32x2_f32 (k = 8g
+// .. 8g + 7 of the sum): a lane holds its four k values together, one 16-byte load from the
+// packed weights and one from LDS for four MFMAs, where a fragment per MFMA (4-byte loads)
+// left the matrix cores waiting on L2 for half of the time (8,192 trajectories: 0.52 ms).
+struct PolicyF32 {
+  using act_t = float;
+  typedef float frag_t __attribute__((ext_vector_type(4)));
+  static constexpr int KSTEP = 8;  // k per fragment
+  static constexpr int KA = 4;     // elements per lane per fragment
+  static constexpr int PIECES = 1;
+  // The k of element j of a lane in half h (lanes 0-31, 32-63) within the fragment: MFMA j
+  // takes k = 2j from half 0 and 2j + 1 from half 1.
+  __host__ __device__ static constexpr int k_of(int h, int j) { return 2 * j + h; }
+  // Where column k of an activation row is stored, so that a lane's four lie together.
+  __host__ __device__ static constexpr int pos(int k) {
+    return (k & ~7) | ((k & 1) << 2) | ((k >> 1) & 3);
+  }
+  __device__ __forceinline__ static floatx16_t mfma(frag_t a, frag_t b, floatx16_t c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], c, 0, 0, 0);
+    return c;
+  }
+};
+
+// BF16 MFMA (float32 accumulate) with every operand carried as three bfloat16 pieces,
+// v = p0 + p1 + p2 exactly for a float32 v (split3).  The six products p_i q_j with
+// i + j <= 2 give each layer sum to ~2^-24 relative, float32 MFMA accuracy, from six bf16
+// MFMA passes: the float32-weight model itself is evaluated (the weights are split, not
+// rounded), and the products of the leading pieces accumulate apart from the five
+// correction products.  bf16 MFMA has 16x the float32 MFMA rate on gfx950.  A single
+// bfloat16 operand (8 bits) would turn f into a step function at the scale of the O(dt f)
+// differences between stages, and the embedded error estimate would measure rounding noise.
+struct PolicyBF16x3 {
   using act_t = __bf16;
   using frag_t = bf16x8_t;
   static constexpr int KSTEP = 16;  // K per MFMA
   static constexpr int KA = 8;      // elements per lane per fragment
   static constexpr int PAD = 8;     // LDS row padding (elements); keeps 16-byte alignment
-  static constexpr bool fast_math = true;
-  // Every layer input (the RK stage value and both hidden activations) is fed as hi + lo
-  // bfloat16 terms, ~16 significant bits.  A single bfloat16 (8 bits) turns f into a step
-  // function at the scale of the O(dt f) differences between stages, and the embedded error
-  // estimate then measures rounding noise instead of truncation error.  Each layer costs two
-  // bfloat16 MFMA passes (float32 accumulate); the weights themselves are bfloat16.
-  static constexpr bool split_input = true;
-  static constexpr int PIECES = 1;  // weight planes read (plane 0 of a three-piece buffer)
+  static constexpr int PIECES = 3;
+  __host__ __device__ static constexpr int k_of(int h, int j) { return 8 * h + j; }
   __device__ __forceinline__ static frag_t load_a(const act_t* p) {
     return *reinterpret_cast<const frag_t*>(p);
   }
@@ -55,40 +82,6 @@ struct PolicyBF16 {
   __device__ __forceinline__ static floatx16_t mfma(frag_t a, frag_t b, floatx16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
-  __device__ __forceinline__ static act_t to_act(float x) { return (act_t)x; }
-};
-
-struct PolicyF32 {
-  using act_t = float;
-  using frag_t = float;
-  static constexpr int KSTEP = 2;
-  static constexpr int KA = 1;
-  static constexpr int PAD = 1;     // odd row stride: conflict-free column reads
-  // Softplus / tanh through the hardware exp2, log2 and reciprocal (about 1 ulp each): the
-  // vector field stays within 8.4e-7 of a float64 evaluation (the libm forms gave 8e-7)
-  // and the forward runs 2x faster, its VALU work having been the larger part of a step.
-  static constexpr bool fast_math = true;
-  static constexpr bool split_input = false;
-  static constexpr int PIECES = 1;
-  __device__ __forceinline__ static frag_t load_a(const act_t* p) { return *p; }
-  __device__ __forceinline__ static frag_t load_b(const act_t* packed, int frag) {
-    return packed[frag];
-  }
-  __device__ __forceinline__ static floatx16_t mfma(frag_t a, frag_t b, floatx16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-  __device__ __forceinline__ static act_t to_act(float x) { return x; }
-};
-
-// BF16 MFMA (float32 accumulate) with every operand carried as three bfloat16 pieces,
-// v = p0 + p1 + p2 exactly for a float32 v (split3).  The six products p_i q_j with
-// i + j <= 2 give each layer sum to ~2^-24 relative, float32 MFMA accuracy, from six bf16
-// MFMA passes: the float32-weight model itself is evaluated (the weights are split, not
-// rounded), and the products of the leading pieces accumulate apart from the five
-// correction products.  bf16 MFMA has 16x the float32 MFMA rate on gfx950.
-struct PolicyBF16x3 : PolicyBF16 {
-  static constexpr bool split_input = false;
-  static constexpr int PIECES = 3;
 };
 
 // v = p0 + p1 + p2 with bfloat16 pieces: each residual is exact in float32 and the last
@@ -120,21 +113,50 @@ __host__ __device__ inline MlpPackLayout mlp_pack_layout(int pieces) {
   return l;
 }
 
+// The packed matrices' input columns K (MFMA reduction lengths), and whether B[k][n] =
+// W[n][k] (forward) or W[k][n] (transposed).
+struct MlpPackShape {
+  int n, k, forward;
+};
+__host__ __device__ constexpr MlpPackShape mlp_pack_shape(int m) {
+  return m == 0   ? MlpPackShape{MLP_H, MLP_D, 1}
+         : m == 1 ? MlpPackShape{MLP_H, MLP_H, 1}
+         : m == 2 ? MlpPackShape{MLP_D, MLP_H, 1}
+         : m == 3 ? MlpPackShape{MLP_D, MLP_H, 0}
+         : m == 4 ? MlpPackShape{MLP_H, MLP_H, 0}
+                  : MlpPackShape{MLP_H, MLP_D, 0};
+}
+
+// The matrix m and element e within it of element `e` of all six, and the number of elements
+// before it (times the pieces: its offset).  m = 6 past the end.
+__host__ __device__ inline void mlp_pack_find(int& e, int& m, int& before) {
+  m = before = 0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const int size = mlp_pack_shape(i).n * mlp_pack_shape(i).k;
+    if (m == i && e >= size) { e -= size; before += size; ++m; }
+  }
+}
+
 // Element e of a packed matrix with K input columns <-> its (n, k): fragments (n tile,
 // k step) of 64 lanes x KA elements.
 template <class P>
-__host__ __device__ inline void mlp_frag_nk(int64_t e, int K, int& n, int& k) {
-  const int j = (int)(e % P::KA), lane = (int)(e / P::KA % 64);
-  const int64_t f = e / P::KA / 64;
-  const int nks = K / P::KSTEP;
-  n = (int)(f / nks) * 32 + (lane & 31);
-  k = (int)(f % nks) * P::KSTEP + (lane >> 5) * P::KA + j;
+__host__ __device__ inline void mlp_frag_nk(int e, int K, int& n, int& k) {
+  const int j = e % P::KA, lane = e / P::KA % 64;
+  const int f = e / P::KA / 64;
+  const int nks = K / P::KSTEP;  // 4, 8, 16 or 32
+  const int nt = f / nks;
+  n = nt * 32 + (lane & 31);
+  k = (f - nt * nks) * P::KSTEP + P::k_of(lane >> 5, j);
 }
 template <class P>
-__host__ __device__ inline int64_t mlp_frag_index(int n, int k, int K) {
+__host__ __device__ inline int mlp_frag_index(int n, int k, int K) {
   const int kk = k % P::KSTEP;
-  const int lane = (n & 31) + 32 * (kk / P::KA);
-  return (((int64_t)(n / 32) * (K / P::KSTEP) + k / P::KSTEP) * 64 + lane) * P::KA + kk % P::KA;
+  int h = 0, j = 0;
+  while (P::k_of(h, j) != kk) {
+    if (++j == P::KA) { j = 0; ++h; }
+  }
+  return ((n / 32 * (K / P::KSTEP) + k / P::KSTEP) * 64 + (n & 31) + 32 * h) * P::KA + j;
 }
 
 // Packed weights of one solve.  Forward fragments: B[k][n] = W[n][k].  Backward fragments
@@ -170,134 +192,99 @@ __host__ __device__ inline MlpWeights<P> mlp_weights_from(const void* packed, in
 }
 
 template <class P>
-struct MlpLds {
-  static constexpr int LDX = MLP_D + P::PAD;
-  static constexpr int LDH = MLP_H + P::PAD;
+struct MlpLds;
+
+// Float32: columns of x, h1 and h2 at P::pos.  The row strides (17 and 65 16-byte units) are
+// odd, so the 16-byte reads of 32 rows are free of bank conflicts.  The split-K partials of
+// layer 3 take the h1 buffer, which nobody reads after layer 2.  79,104 bytes: two
+// workgroups per CU.
+template <>
+struct MlpLds<PolicyF32> {
+  static constexpr int LDX = MLP_D + 4;
+  static constexpr int LDH = MLP_H + 4;
   static constexpr int LDP = MLP_D + 4;
-  typename P::act_t x[MLP_TILE * LDX];    // layer-1 input (stage value), high part
-  typename P::act_t xlo[P::split_input ? MLP_TILE * LDX : 1];  // layer-1 input, low part
-  typename P::act_t h1[MLP_TILE * LDH];   // softplus(layer 1) (high part)
-  typename P::act_t h2[MLP_TILE * LDH];   // softplus(layer 2) (high part)
-  typename P::act_t h1lo[P::split_input ? MLP_TILE * LDH : 1];  // low parts
-  typename P::act_t h2lo[P::split_input ? MLP_TILE * LDH : 1];
-  typename P::act_t d[MLP_TILE * LDH];    // backward: delta of layer 2
-  typename P::act_t d3[MLP_TILE * LDX];   // backward: delta of layer 3
-  float part[4 * MLP_TILE * LDP];         // split-K partial sums of the 64-wide outputs
+  float x[MLP_TILE * LDX];      // layer-1 input (stage value)
+  float h1[4 * MLP_TILE * LDP]; // softplus(layer 1) [32][LDH], then the partials [4][32][LDP]
+  float h2[MLP_TILE * LDH];     // softplus(layer 2)
+  float bias[2 * MLP_H + MLP_D];
+  __device__ __forceinline__ float* part() { return h1; }
 };
-
-// Store one float value of the layer-1 input (row r, column c) in its policy's form.
-template <class P>
-__device__ __forceinline__ void store_input(MlpLds<P>& L, int r, int c, float v) {
-  const typename P::act_t hi = P::to_act(v);
-  L.x[r * L.LDX + c] = hi;
-  if constexpr (P::split_input) L.xlo[r * L.LDX + c] = P::to_act(v - (float)hi);
-}
-
-// Store a hidden activation (hi, and lo for split policies).
-template <class P>
-__device__ __forceinline__ void store_hidden(typename P::act_t* hi_buf, typename P::act_t* lo_buf,
-                                             int idx, float v) {
-  const typename P::act_t hi = P::to_act(v);
-  hi_buf[idx] = hi;
-  if constexpr (P::split_input) lo_buf[idx] = P::to_act(v - (float)hi);
-}
+static_assert(4 * MlpLds<PolicyF32>::LDP >= MlpLds<PolicyF32>::LDH, "h1 fits");
+static_assert(2 * sizeof(MlpLds<PolicyF32>) <= 160 * 1024, "two workgroups per CU");
 
 // ---- activations ------------------------------------------------------------------------
-template <bool Fast>
+// Softplus / tanh through the hardware exp2, log2 and reciprocal (about 1 ulp each): the
+// vector field stays within 8.4e-7 of a float64 evaluation (the libm forms gave 8e-7)
+// and the forward runs 2x faster, its VALU work having been the larger part of a step.
 __device__ __forceinline__ float softplus_f(float x) {
   // jax.nn.softplus(x) = logaddexp(x, 0) = max(x, 0) + log1p(exp(-|x|))
-  if constexpr (Fast) {
-    const float e = __builtin_amdgcn_exp2f(-fabsf(x) * 1.4426950408889634f);
-    return fmaxf(x, 0.0f) + 0.6931471805599453f * __builtin_amdgcn_logf(1.0f + e);
-  } else {
-    return fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x)));
-  }
+  const float e = __builtin_amdgcn_exp2f(-fabsf(x) * 1.4426950408889634f);
+  return fmaxf(x, 0.0f) + 0.6931471805599453f * __builtin_amdgcn_logf(1.0f + e);
 }
-template <bool Fast>
 __device__ __forceinline__ float tanh_f(float x) {
-  if constexpr (Fast) {
-    // tanh(x) = sign(x) (1 - 2 / (exp(2|x|) + 1))
-    const float e = __builtin_amdgcn_exp2f(fminf(2.0f * fabsf(x), 60.0f) * 1.4426950408889634f);
-    const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
-    return copysignf(t, x);
-  } else {
-    return tanhf(x);
-  }
+  // tanh(x) = sign(x) (1 - 2 / (exp(2|x|) + 1))
+  const float e = __builtin_amdgcn_exp2f(fminf(2.0f * fabsf(x), 60.0f) * 1.4426950408889634f);
+  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+  return copysignf(t, x);
 }
 // derivative of softplus from its value h = softplus(s): sigmoid(s) = 1 - exp(-h)
-template <bool Fast>
 __device__ __forceinline__ float dsoftplus_from_value(float h) {
-  if constexpr (Fast) return 1.0f - __builtin_amdgcn_exp2f(-h * 1.4426950408889634f);
-  else return -expm1f(-h);
-}
-
-// ---- one wave's share of a layer --------------------------------------------------------
-// acc[nt] (32x32 f32) = sum over k-steps [ks0, ks1) of A(lds rows, k) * B(fragment (nt0+nt, ks)),
-// where A = a_lds, or a_lds + a_lo (LO: the hi + lo halves of a split operand, two MFMAs per
-// B fragment).  16-byte fragments (bf16) are loaded PF k-steps ahead of their MFMAs through a
-// ring of registers (PF = 4; 8 for layer 2: 7 % faster forward, 12 % faster adjoint than one
-// step ahead); 4-byte fragments (f32, 2 k per MFMA, PF = 0) are left to the compiler's
-// unrolled schedule, where explicit prefetch measured slower.
-template <class P, int NKS, int NT, bool LO = false, int PF = (P::KA == 1 ? 0 : 4)>
-__device__ __forceinline__ void wave_gemm(const typename P::act_t* a_lds,
-                                          const typename P::act_t* a_lo, int lda,
-                                          const typename P::act_t* wp, int nt0, int ks0,
-                                          int ks1, floatx16_t (&acc)[NT], int lane) {
-  using frag_t = typename P::frag_t;
-  const int row = lane & 31;
-  const int kh = (lane >> 5) * P::KA;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = floatx16_t{};
-  if constexpr (P::KA == 1 && PF == 0) {
-    static_assert(!LO, "split operands are bfloat16");
-#pragma unroll 8
-    for (int ks = ks0; ks < ks1; ++ks) {
-      const frag_t a = P::load_a(a_lds + row * lda + ks * P::KSTEP + kh);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const frag_t b = P::load_b(wp, ((nt0 + t) * NKS + ks) * 64 + lane);
-        acc[t] = P::mfma(a, b, acc[t]);
-      }
-    }
-  } else {
-    // B fragments come from L2 (the weights of every layer, shared by all workgroups), whose
-    // latency is several k-steps of MFMA work: PF k-steps are kept in flight.
-    frag_t buf[PF][NT];
-#pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int kp = (ks0 + p < ks1) ? ks0 + p : ks1 - 1;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) buf[p][t] = P::load_b(wp, ((nt0 + t) * NKS + kp) * 64 + lane);
-    }
-    for (int ks = ks0; ks < ks1; ks += PF) {
-#pragma unroll
-      for (int p = 0; p < PF; ++p) {
-        const int k = ks + p;
-        if (k < ks1) {
-          frag_t b[NT];
-          const int kn = (k + PF < ks1) ? k + PF : ks1 - 1;  // the tail re-reads the last one
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            b[t] = buf[p][t];
-            buf[p][t] = P::load_b(wp, ((nt0 + t) * NKS + kn) * 64 + lane);
-          }
-          const frag_t a = P::load_a(a_lds + row * lda + k * P::KSTEP + kh);
-#pragma unroll
-          for (int t = 0; t < NT; ++t) acc[t] = P::mfma(a, b[t], acc[t]);
-          if constexpr (LO) {
-            const frag_t al = P::load_a(a_lo + row * lda + k * P::KSTEP + kh);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) acc[t] = P::mfma(al, b[t], acc[t]);
-          }
-        }
-      }
-    }
-  }
+  return 1.0f - __builtin_amdgcn_exp2f(-h * 1.4426950408889634f);
 }
 
 // C-layout helpers: accumulator element v (= 4i + j) of lane l sits at
 // row 8i + (l/32)*4 + j, column l%32 of the 32x32 tile.
 __device__ __forceinline__ int acc_row(int lane, int v) { return 8 * (v >> 2) + (lane >> 5) * 4 + (v & 3); }
+
+// ---- the float32 form ------------------------------------------------------------------
+// One wave's share of a layer: acc[t] = sum over fragments [g0, g0 + G) of W . x, the weights
+// of output tile nt0 + t as the A operand and the activation rows (LDS) as B, so that a
+// lane's accumulators are four runs of four consecutive outputs of one trajectory (wide
+// LDS stores).  NG: fragments along K of the matrix.  Weights come from L2, whose latency
+// is longer than a fragment's MFMAs: PF fragments are in flight, the first of them loaded
+// by preload() ahead of the barrier that the activations wait for.
+template <int NG, int NT, int PF = 4>
+struct GemmF32 {
+  using P = PolicyF32;
+  using frag_t = P::frag_t;
+  frag_t b[PF][NT];
+  const frag_t* wp;
+  __device__ __forceinline__ void preload(const float* w, int nt0, int g0, int lane) {
+    wp = reinterpret_cast<const frag_t*>(w) + ((int64_t)nt0 * NG + g0) * 64 + lane;
+#pragma unroll
+    for (int p = 0; p < PF; ++p) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b[p][t] = wp[(t * NG + p) * 64];
+    }
+  }
+  // A ring slot is refilled right after its MFMAs (the load may write the registers they
+  // read), so the loop carries no copies that would wait for the loads it just issued.
+  template <int G>
+  __device__ __forceinline__ void run(const float* act, int ld, int g0, floatx16_t (&acc)[NT],
+                                      int lane) {
+    static_assert(G % PF == 0 && G >= PF && PF % 2 == 0, "whole rings");
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = floatx16_t{};
+    const float* ap = act + (lane & 31) * ld + 8 * g0 + 4 * (lane >> 5);
+    auto load_a = [&](int g) { return *reinterpret_cast<const frag_t*>(ap + 8 * g); };
+    frag_t a[2] = {load_a(0), load_a(1)};
+    auto ring = [&](int g, auto last) {
+#pragma unroll
+      for (int p = 0; p < PF; ++p) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = P::mfma(b[p][t], a[p & 1], acc[t]);
+        if (!decltype(last)::value) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) b[p][t] = wp[(t * NG + g + p + PF) * 64];
+        }
+        if (!decltype(last)::value || p + 2 < PF) a[p & 1] = load_a(g + p + 2);
+      }
+    };
+#pragma unroll 1
+    for (int g = 0; g < G - PF; g += PF) ring(g, std::false_type{});
+    ring(G - PF, std::true_type{});
+  }
+};
 
 // ---- the three-piece bf16 form --------------------------------------------------------
 // LDS: the three pieces of the layer-1 input and of both hidden activations (115 KB).  The
@@ -316,11 +303,22 @@ static_assert(4 * MLP_TILE * MlpLds<PolicyBF16x3>::LDP * sizeof(float) <=
                   sizeof(MlpLds<PolicyBF16x3>::h1),
               "layer-3 partials fit in the h1 planes");
 
-template <>
-__device__ __forceinline__ void store_input<PolicyBF16x3>(MlpLds<PolicyBF16x3>& L, int r, int c,
-                                                          float v) {
+// Store one value of the layer-1 input (row r, column c).
+__device__ __forceinline__ void store_input(MlpLds<PolicyBF16x3>& L, int r, int c, float v) {
   const int i = r * L.LDX + c;
   split3(v, L.x[0][i], L.x[1][i], L.x[2][i]);
+}
+__device__ __forceinline__ void store_input(MlpLds<PolicyF32>& L, int r, int c, float v) {
+  L.x[r * L.LDX + PolicyF32::pos(c)] = v;
+}
+
+// Kernels call this once before their first evaluation (a barrier follows it there).
+template <class P>
+__device__ __forceinline__ void mlp_begin(const MlpWeights<P>& W, MlpLds<P>& L) {
+  if constexpr (P::PIECES == 1) {
+    for (int i = threadIdx.x; i < 2 * MLP_H + MLP_D; i += blockDim.x)
+      L.bias[i] = i < MLP_H ? W.b1[i] : (i < 2 * MLP_H ? W.b2[i - MLP_H] : W.b3[i - 2 * MLP_H]);
+  }
 }
 
 // acc[nt] (32x32 f32) = sum over k-steps [ks0, ks1) of A . B with A and B three-piece
@@ -437,7 +435,7 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int i = acc_row(lane, v) * L.LDH + col;
-      const float h = softplus_f<true>(acc[t][v] + bias);
+      const float h = softplus_f(acc[t][v] + bias);
       if (sink.h1) sink.put(sink.h1, acc_row(lane, v), col, h);
       split3(h, L.h1[0][i], L.h1[1][i], L.h1[2][i]);
     }
@@ -453,7 +451,7 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int i = acc_row(lane, v) * L.LDH + col;
-      const float h = softplus_f<true>(acc[t][v] + bias);
+      const float h = softplus_f(acc[t][v] + bias);
       if (sink.h2) sink.put(sink.h2, acc_row(lane, v), col, h);
       split3(h, L.h2[0][i], L.h2[1][i], L.h2[2][i]);
     }
@@ -481,73 +479,78 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
     s += part[(1 * MLP_TILE + owner_row) * L.LDP + c];
     s += part[(2 * MLP_TILE + owner_row) * L.LDP + c];
     s += part[(3 * MLP_TILE + owner_row) * L.LDP + c];
-    fout[j] = tanh_f<true>(s + W.b3[c]);
+    fout[j] = tanh_f(s + W.b3[c]);
   }
 }
 
 // Forward of the MLP on the tile: reads L.x (stage values), leaves softplus activations in
 // L.h1 / L.h2 and returns f for the owner's 32 / NW components in fout (NW waves per tile;
 // MlpWaves).  The three-piece bf16 form runs mlp_forward3.
-template <class P, int NW = 4>
-__device__ __forceinline__ void mlp_forward(const MlpWeights<P>& W, MlpLds<P>& L, int wave,
+template <class P, int NW = 4, class Lds = MlpLds<P>>
+__device__ __forceinline__ void mlp_forward(const MlpWeights<P>& W, Lds& L, int wave,
                                             int lane, int owner_row, int owner_c0,
                                             float (&fout)[MlpWaves<NW>::CPT]) {
   if constexpr (P::PIECES == 3) {
     mlp_forward3<NW>(W, L, wave, lane, owner_row, owner_c0, fout, MlpRowSink{});
   } else {
-  using WV = MlpWaves<NW>;
-  constexpr int NT = WV::NT12;
-  constexpr bool F = P::fast_math;
-  floatx16_t acc[NT];
-  // layer 1: [32 x 64] . W1^T -> [32 x 256], wave's columns [64w, 64w + 64)
-  constexpr bool S = P::split_input;
-  wave_gemm<P, MLP_D / P::KSTEP, NT, S>(L.x, L.xlo, L.LDX, W.w1, NT * wave, 0, MLP_D / P::KSTEP,
-                                        acc, lane);
+    using WV = MlpWaves<NW>;
+    constexpr int NT = WV::NT12, NT3 = WV::NT3;
+    const int half = lane >> 5, row = lane & 31;
+    // softplus of a layer's accumulators into buf: per run of four outputs n .. n + 3, the
+    // even and the odd ones lie together (P::pos)
+    auto put_hidden = [&](const floatx16_t (&acc)[NT], const float* bias, float* buf) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = 32 * (NT * wave + t) + (lane & 31);
-    const float bias = W.b1[col];
+      for (int t = 0; t < NT; ++t) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
-      store_hidden<P>(L.h1, L.h1lo, acc_row(lane, v) * L.LDH + col, softplus_f<F>(acc[t][v] + bias));
-  }
-  __syncthreads();
-  // layer 2: [32 x 256] . W2^T -> [32 x 256]
-  wave_gemm<P, MLP_H / P::KSTEP, NT, S, (P::KA == 1 ? 0 : 8)>(L.h1, L.h1lo, L.LDH, W.w2,
-                                                              NT * wave, 0, MLP_H / P::KSTEP,
-                                                              acc, lane);
+        for (int i = 0; i < 4; ++i) {
+          const int n = 32 * (NT * wave + t) + 8 * i + 4 * half;
+          const float4 bv = *reinterpret_cast<const float4*>(bias + n);
+          const float h0 = softplus_f(acc[t][4 * i] + bv.x), h1 = softplus_f(acc[t][4 * i + 1] + bv.y);
+          const float h2 = softplus_f(acc[t][4 * i + 2] + bv.z), h3 = softplus_f(acc[t][4 * i + 3] + bv.w);
+          float* o = buf + row * L.LDH + P::pos(n);
+          *reinterpret_cast<float2*>(o) = make_float2(h0, h2);
+          *reinterpret_cast<float2*>(o + 4) = make_float2(h1, h3);
+        }
+      }
+    };
+    floatx16_t acc[NT];
+    GemmF32<MLP_D / P::KSTEP, NT> g1;
+    GemmF32<MLP_H / P::KSTEP, NT> g2;
+    GemmF32<MLP_H / P::KSTEP, NT3> g3;
+    g1.preload(W.w1, NT * wave, 0, lane);
+    g1.template run<MLP_D / P::KSTEP>(L.x, L.LDX, 0, acc, lane);
+    g2.preload(W.w2, NT * wave, 0, lane);
+    __builtin_amdgcn_sched_barrier(0);  // issued here, ahead of the epilogue
+    put_hidden(acc, L.bias, L.h1);
+    __syncthreads();
+    g2.template run<MLP_H / P::KSTEP>(L.h1, L.LDH, 0, acc, lane);
+    // layer 3 (split-K): wave w sums a quarter of K
+    constexpr int G3 = MLP_H / P::KSTEP / 4;
+    const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+    g3.preload(W.w3, n3, qk * G3, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    put_hidden(acc, L.bias + MLP_H, L.h2);
+    __syncthreads();
+    floatx16_t acc3[NT3];
+    g3.template run<G3>(L.h2, L.LDH, qk * G3, acc3, lane);
+    float* part = L.part();  // the h1 buffer: layer 2, its last reader, is behind the barrier
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = 32 * (NT * wave + t) + (lane & 31);
-    const float bias = W.b2[col];
+    for (int t = 0; t < NT3; ++t) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
-      store_hidden<P>(L.h2, L.h2lo, acc_row(lane, v) * L.LDH + col, softplus_f<F>(acc[t][v] + bias));
-  }
-  __syncthreads();
-  // layer 3 (split-K): wave w sums K in [64w, 64w + 64) for all 64 outputs
-  constexpr int KS3 = MLP_H / P::KSTEP;
-  constexpr int NT3 = WV::NT3;
-  const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-  floatx16_t acc3[NT3];
-  wave_gemm<P, KS3, NT3, S>(L.h2, L.h2lo, L.LDH, W.w3, n3, qk * (KS3 / 4), (qk + 1) * (KS3 / 4),
-                            acc3, lane);
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(part + (qk * MLP_TILE + row) * L.LDP + 32 * (n3 + t) + 8 * i + 4 * half) =
+            make_float4(acc3[t][4 * i], acc3[t][4 * i + 1], acc3[t][4 * i + 2], acc3[t][4 * i + 3]);
+    }
+    __syncthreads();
 #pragma unroll
-  for (int t = 0; t < NT3; ++t) {
-    const int col = 32 * (n3 + t) + (lane & 31);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) L.part[(qk * MLP_TILE + acc_row(lane, v)) * L.LDP + col] = acc3[t][v];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < WV::CPT; ++j) {
-    const int c = owner_c0 + j;
-    float s = L.part[(0 * MLP_TILE + owner_row) * L.LDP + c];
-    s += L.part[(1 * MLP_TILE + owner_row) * L.LDP + c];
-    s += L.part[(2 * MLP_TILE + owner_row) * L.LDP + c];
-    s += L.part[(3 * MLP_TILE + owner_row) * L.LDP + c];
-    fout[j] = tanh_f<F>(s + W.b3[c]);
-  }
+    for (int j = 0; j < WV::CPT; ++j) {
+      const int c = owner_c0 + j;
+      float s = part[(0 * MLP_TILE + owner_row) * L.LDP + c];
+      s += part[(1 * MLP_TILE + owner_row) * L.LDP + c];
+      s += part[(2 * MLP_TILE + owner_row) * L.LDP + c];
+      s += part[(3 * MLP_TILE + owner_row) * L.LDP + c];
+      fout[j] = tanh_f(s + L.bias[2 * MLP_H + c]);
+    }
   }
 }
 
