@@ -20,11 +20,12 @@ __global__ void __launch_bounds__(MLP_THREADS, 1) mlp_eval_kernel(const float* _
   const int orow = tid >> 3, c0 = (tid & 7) * 8;
   const int64_t row = (int64_t)blockIdx.x * MLP_TILE + orow;
   const bool valid = row < R;
+  float f[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) store_input(L, orow, c0 + j, valid ? Y[row * MLP_D + c0 + j] : 0.0f);
+  for (int j = 0; j < 8; ++j) f[j] = valid ? Y[row * MLP_D + c0 + j] : 0.0f;
+  store_inputs(L, orow, c0, f);
   mlp_begin<P>(W, L);
   __syncthreads();
-  float f[8];
   mlp_forward<P>(W, L, wave, lane, orow, c0, f);
   if (valid) {
 #pragma unroll

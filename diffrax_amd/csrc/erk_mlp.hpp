@@ -151,8 +151,7 @@ erk_mlp_kernel(const MlpArgs a, const MlpWeights<P> W) {
   }
 
   // ---- first stage of the first step (FSAL seed): f(t0, y0) ----
-#pragma unroll
-  for (int j = 0; j < CPT; ++j) store_input(L, orow, c0 + j, y[j]);
+  store_inputs(L, orow, c0, y);
   mlp_begin<P>(W, L);
   __syncthreads();
   mlp_forward<P, NW>(W, L, wave, lane, orow, c0, fsal);
@@ -195,10 +194,11 @@ erk_mlp_kernel(const MlpArgs a, const MlpWeights<P> W) {
     const bool cond = (d0 < 1e-5) || (d1 < 1e-5);
     const double h0 = cond ? 1e-6 : 0.01 * (d0 / (cond ? 1.0 : d1));
     __syncthreads();  // every wave is done with the seed's layer-3 partials
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) store_input(L, orow, c0 + j, y[j] + (float)h0 * fsal[j]);
-    __syncthreads();
     float f1[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) f1[j] = y[j] + (float)h0 * fsal[j];
+    store_inputs(L, orow, c0, f1);
+    __syncthreads();
     mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f1);
     double t2[CPT];
 #pragma unroll
@@ -272,8 +272,8 @@ erk_mlp_kernel(const MlpArgs a, const MlpWeights<P> W) {
 #pragma unroll
         for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
         z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        store_input(L, orow, c0 + j, z[j]);
       }
+      store_inputs(L, orow, c0, z);
       __syncthreads();
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
 #pragma unroll

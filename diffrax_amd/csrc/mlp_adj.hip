@@ -120,10 +120,8 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
     if (q == 0) {
       const MlpRowSink k0 = sink_of(0, 0);
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        store_input(L, orow, c0 + j, y[j]);
-        put_x(k0, j, y[j]);
-      }
+      for (int j = 0; j < CPT; ++j) put_x(k0, j, y[j]);
+      store_inputs(L, orow, c0, y);
       __syncthreads();
       mlp_forward3<NW>(W, L, wave, lane, orow, c0, fl, k0);
       __syncthreads();
@@ -142,9 +140,9 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
 #pragma unroll
         for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
         z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        store_input(L, orow, c0 + j, z[j]);
         put_x(ki, j, z[j]);
       }
+      store_inputs(L, orow, c0, z);
       __syncthreads();
       mlp_forward3<NW>(W, L, wave, lane, orow, c0, f, ki);
       __syncthreads();
@@ -661,8 +659,8 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
           za[j] = av[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], ca, 0.0f);
         }
         if (!run) { zy[j] = 0.0f; za[j] = 0.0f; }  // idle rows: zero deltas
-        store_input(L, orow, c0 + j, zy[j]);
       }
+      store_inputs(L, orow, c0, zy);
       __syncthreads();
       float f[CPT];
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);

@@ -93,6 +93,28 @@ __device__ __forceinline__ void split3(float v, __bf16& p0, __bf16& p1, __bf16& 
   p2 = (__bf16)(r1 - (float)p1);
 }
 
+// split3 of four values, the pieces packed for 8-byte LDS stores.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float floatx2_t __attribute__((ext_vector_type(2)));
+struct Split4 {
+  uint2 p[3];
+};
+__device__ __forceinline__ Split4 split3x4(float a, float b, float c, float d) {
+  Split4 s;
+  floatx2_t lo = {a, b}, hi = {c, d};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const bf16x2_t ql = __builtin_convertvector(lo, bf16x2_t);
+    const bf16x2_t qh = __builtin_convertvector(hi, bf16x2_t);
+    s.p[i] = make_uint2(__builtin_bit_cast(unsigned, ql), __builtin_bit_cast(unsigned, qh));
+    if (i < 2) {
+      lo = lo - __builtin_convertvector(ql, floatx2_t);
+      hi = hi - __builtin_convertvector(qh, floatx2_t);
+    }
+  }
+  return s;
+}
+
 // Packed weight buffer: six matrices (w1, w2, w3 forward; w1t, w2t, w3t transposed), each
 // `pieces` planes of its fragment array (bf16: the three split3 pieces, plane 0 the
 // rounded weight; float32: one plane).  Element offsets of plane 0 and plane sizes.
@@ -278,6 +300,7 @@ struct GemmF32 {
           for (int t = 0; t < NT; ++t) b[p][t] = wp[(t * NG + g + p + PF) * 64];
         }
         if (!decltype(last)::value || p + 2 < PF) a[p & 1] = load_a(g + p + 2);
+        __builtin_amdgcn_sched_barrier(0);  // the loads stay here, ahead of the next MFMAs
       }
     };
 #pragma unroll 1
@@ -297,28 +320,41 @@ struct MlpLds<PolicyBF16x3> {
   __bf16 x[3][MLP_TILE * LDX];
   __bf16 h1[3][MLP_TILE * LDH];
   __bf16 h2[3][MLP_TILE * LDH];
+  float bias[2 * MLP_H + MLP_D];
   __device__ __forceinline__ float* part() { return reinterpret_cast<float*>(&h1[0][0]); }
 };
 static_assert(4 * MLP_TILE * MlpLds<PolicyBF16x3>::LDP * sizeof(float) <=
                   sizeof(MlpLds<PolicyBF16x3>::h1),
               "layer-3 partials fit in the h1 planes");
 
-// Store one value of the layer-1 input (row r, column c).
-__device__ __forceinline__ void store_input(MlpLds<PolicyBF16x3>& L, int r, int c, float v) {
-  const int i = r * L.LDX + c;
-  split3(v, L.x[0][i], L.x[1][i], L.x[2][i]);
+// Store N consecutive values (4 or 8, from a multiple of N) of the layer-1 input's row r.
+template <int N>
+__device__ __forceinline__ void store_inputs(MlpLds<PolicyBF16x3>& L, int r, int c0,
+                                             const float (&v)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; j += 4) {
+    const Split4 s = split3x4(v[j], v[j + 1], v[j + 2], v[j + 3]);
+#pragma unroll
+    for (int pc = 0; pc < 3; ++pc)
+      *reinterpret_cast<uint2*>(&L.x[pc][r * L.LDX + c0 + j]) = s.p[pc];
+  }
 }
-__device__ __forceinline__ void store_input(MlpLds<PolicyF32>& L, int r, int c, float v) {
-  L.x[r * L.LDX + PolicyF32::pos(c)] = v;
+template <int N>
+__device__ __forceinline__ void store_inputs(MlpLds<PolicyF32>& L, int r, int c0,
+                                             const float (&v)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; j += 4) {
+    float* o = L.x + r * L.LDX + PolicyF32::pos(c0 + j);
+    *reinterpret_cast<float2*>(o) = make_float2(v[j], v[j + 2]);
+    *reinterpret_cast<float2*>(o + 4) = make_float2(v[j + 1], v[j + 3]);
+  }
 }
 
 // Kernels call this once before their first evaluation (a barrier follows it there).
 template <class P>
 __device__ __forceinline__ void mlp_begin(const MlpWeights<P>& W, MlpLds<P>& L) {
-  if constexpr (P::PIECES == 1) {
-    for (int i = threadIdx.x; i < 2 * MLP_H + MLP_D; i += blockDim.x)
-      L.bias[i] = i < MLP_H ? W.b1[i] : (i < 2 * MLP_H ? W.b2[i - MLP_H] : W.b3[i - 2 * MLP_H]);
-  }
+  for (int i = threadIdx.x; i < 2 * MLP_H + MLP_D; i += blockDim.x)
+    L.bias[i] = i < MLP_H ? W.b1[i] : (i < 2 * MLP_H ? W.b2[i - MLP_H] : W.b3[i - 2 * MLP_H]);
 }
 
 // acc[nt] (32x32 f32) = sum over k-steps [ks0, ks1) of A . B with A and B three-piece
@@ -388,6 +424,75 @@ __device__ __forceinline__ void wave_gemm3(const __bf16* a0, const __bf16* a1, c
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = big[t] + sml[t];
 }
+
+// wave_gemm3 with the weights as the A operand (a lane's accumulators are four runs of four
+// consecutive outputs of one trajectory) and the ring of GemmF32: PF k steps of weights in
+// flight, the first loaded ahead of the barrier that the activations wait for.  The same
+// products in the same order, so the same bits.  One evaluation of a 32-trajectory tile by
+// eight waves takes 23,000 cycles, 9,200 of them MFMA on every SIMD and 6,700 VALU (softplus
+// and the splits, between the barriers, so that little of it overlaps); with wave_gemm3's
+// copied ring, 2-byte LDS stores and a split per value it took 26,400 and 10,100 VALU
+// (8,192 trajectories: 0.33-0.35 against 0.30 ms; 33: 0.266 against 0.234).
+template <int NKS, int NT, int PF = 2>
+struct Gemm3 {
+  using P = PolicyBF16x3;
+  using frag_t = P::frag_t;
+  frag_t b[PF][3][NT];
+  const frag_t* wp;
+  int plane;
+  __device__ __forceinline__ void load(int p, int k) {
+#pragma unroll
+    for (int pc = 0; pc < 3; ++pc) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b[p][pc][t] = wp[pc * plane + (t * NKS + k) * 64];
+    }
+  }
+  __device__ __forceinline__ void preload(const __bf16* w, int64_t pl, int nt0, int k0, int lane) {
+    wp = reinterpret_cast<const frag_t*>(w) + ((int64_t)nt0 * NKS + k0) * 64 + lane;
+    plane = (int)(pl / P::KA);
+#pragma unroll
+    for (int p = 0; p < PF; ++p) load(p, p);
+  }
+  template <int G>
+  __device__ __forceinline__ void run(const __bf16* act, int aplane, int ld, int k0,
+                                      floatx16_t (&acc)[NT], int lane) {
+    static_assert(G % PF == 0 && G >= PF, "whole rings");
+    floatx16_t sml[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) { acc[t] = floatx16_t{}; sml[t] = floatx16_t{}; }
+    const __bf16* ap = act + (lane & 31) * ld + P::KSTEP * k0 + P::KA * (lane >> 5);
+    frag_t x[2][3];
+    auto load_x = [&](int q, int k) {
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) x[q][pc] = P::load_a(ap + pc * aplane + P::KSTEP * k);
+    };
+    load_x(0, 0);
+    load_x(1, 1);
+    auto ring = [&](int g, auto last) {
+#pragma unroll
+      for (int p = 0; p < PF; ++p) {
+        const int q = p & 1;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          acc[t] = P::mfma(b[p][0][t], x[q][0], acc[t]);
+          sml[t] = P::mfma(b[p][1][t], x[q][0], sml[t]);
+          sml[t] = P::mfma(b[p][0][t], x[q][1], sml[t]);
+          sml[t] = P::mfma(b[p][2][t], x[q][0], sml[t]);
+          sml[t] = P::mfma(b[p][1][t], x[q][1], sml[t]);
+          sml[t] = P::mfma(b[p][0][t], x[q][2], sml[t]);
+        }
+        if (!decltype(last)::value) load(p, g + p + PF);
+        if (!decltype(last)::value || p + 2 < PF) load_x(q, g + p + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+#pragma unroll 1
+    for (int g = 0; g < G - PF; g += PF) ring(g, std::false_type{});
+    ring(G - PF, std::true_type{});
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = acc[t] + sml[t];
+  }
+};
 
 // Float32 copies of the hidden activations for the adjoint's row buffers ([rows][256] each,
 // the tile's rows from row0, and again from row0b when row0b >= 0): written in the layer
@@ -483,6 +588,34 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
   }
 }
 
+// Layer 3's split-K partials (accumulators with the outputs along a lane's runs), which take
+// the h1 buffer (layer 2, its last reader, is behind a barrier), and the output from them.
+template <int NT3>
+__device__ __forceinline__ void put_partials(const floatx16_t (&acc)[NT3], float* part, int ldp,
+                                             int qk, int n3, int lane) {
+#pragma unroll
+  for (int t = 0; t < NT3; ++t) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<float4*>(part + (qk * MLP_TILE + (lane & 31)) * ldp + 32 * (n3 + t) + 8 * i +
+                                 4 * (lane >> 5)) =
+          make_float4(acc[t][4 * i], acc[t][4 * i + 1], acc[t][4 * i + 2], acc[t][4 * i + 3]);
+  }
+}
+template <int CPT>
+__device__ __forceinline__ void sum_partials(const float* part, int ldp, const float* b3,
+                                             int owner_row, int owner_c0, float (&fout)[CPT]) {
+#pragma unroll
+  for (int j = 0; j < CPT; ++j) {
+    const int c = owner_c0 + j;
+    float s = part[(0 * MLP_TILE + owner_row) * ldp + c];
+    s += part[(1 * MLP_TILE + owner_row) * ldp + c];
+    s += part[(2 * MLP_TILE + owner_row) * ldp + c];
+    s += part[(3 * MLP_TILE + owner_row) * ldp + c];
+    fout[j] = tanh_f(s + b3[c]);
+  }
+}
+
 // Forward of the MLP on the tile: reads L.x (stage values), leaves softplus activations in
 // L.h1 / L.h2 and returns f for the owner's 32 / NW components in fout (NW waves per tile;
 // MlpWaves).  The three-piece bf16 form runs mlp_forward3.
@@ -491,7 +624,46 @@ __device__ __forceinline__ void mlp_forward(const MlpWeights<P>& W, Lds& L, int 
                                             int lane, int owner_row, int owner_c0,
                                             float (&fout)[MlpWaves<NW>::CPT]) {
   if constexpr (P::PIECES == 3) {
-    mlp_forward3<NW>(W, L, wave, lane, owner_row, owner_c0, fout, MlpRowSink{});
+    using WV = MlpWaves<NW>;
+    constexpr int NT = WV::NT12, NT3 = WV::NT3, KS1 = MLP_D / 16, KS2 = MLP_H / 16;
+    constexpr int HP = MLP_TILE * Lds::LDH;
+    const int half = lane >> 5, row = lane & 31;
+    auto put_hidden = [&](const floatx16_t (&acc)[NT], const float* bias, __bf16* buf) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int n = 32 * (NT * wave + t) + 8 * i + 4 * half;
+          const float4 bv = *reinterpret_cast<const float4*>(bias + n);
+          const Split4 s = split3x4(softplus_f(acc[t][4 * i] + bv.x), softplus_f(acc[t][4 * i + 1] + bv.y),
+                                    softplus_f(acc[t][4 * i + 2] + bv.z), softplus_f(acc[t][4 * i + 3] + bv.w));
+#pragma unroll
+          for (int pc = 0; pc < 3; ++pc)
+            *reinterpret_cast<uint2*>(buf + pc * HP + row * L.LDH + n) = s.p[pc];
+        }
+      }
+    };
+    floatx16_t acc[NT];
+    Gemm3<KS1, NT> g1;
+    Gemm3<KS2, NT> g2;
+    Gemm3<KS2, NT3> g3;
+    g1.preload(W.w1, W.plane1, NT * wave, 0, lane);
+    g1.template run<KS1>(L.x[0], MLP_TILE * Lds::LDX, L.LDX, 0, acc, lane);
+    g2.preload(W.w2, W.plane2, NT * wave, 0, lane);
+    __builtin_amdgcn_sched_barrier(0);  // issued here, ahead of the epilogue
+    put_hidden(acc, L.bias, L.h1[0]);
+    __syncthreads();
+    g2.template run<KS2>(L.h1[0], HP, L.LDH, 0, acc, lane);
+    const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+    g3.preload(W.w3, W.plane3, n3, qk * (KS2 / 4), lane);
+    __builtin_amdgcn_sched_barrier(0);
+    put_hidden(acc, L.bias + MLP_H, L.h2[0]);
+    __syncthreads();
+    floatx16_t acc3[NT3];
+    g3.template run<KS2 / 4>(L.h2[0], HP, L.LDH, qk * (KS2 / 4), acc3, lane);
+    put_partials<NT3>(acc3, L.part(), L.LDP, qk, n3, lane);
+    __syncthreads();
+    sum_partials<WV::CPT>(L.part(), L.LDP, L.bias + 2 * MLP_H, owner_row, owner_c0, fout);
   } else {
     using WV = MlpWaves<NW>;
     constexpr int NT = WV::NT12, NT3 = WV::NT3;
@@ -533,24 +705,9 @@ __device__ __forceinline__ void mlp_forward(const MlpWeights<P>& W, Lds& L, int 
     __syncthreads();
     floatx16_t acc3[NT3];
     g3.template run<G3>(L.h2, L.LDH, qk * G3, acc3, lane);
-    float* part = L.part();  // the h1 buffer: layer 2, its last reader, is behind the barrier
-#pragma unroll
-    for (int t = 0; t < NT3; ++t) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<float4*>(part + (qk * MLP_TILE + row) * L.LDP + 32 * (n3 + t) + 8 * i + 4 * half) =
-            make_float4(acc3[t][4 * i], acc3[t][4 * i + 1], acc3[t][4 * i + 2], acc3[t][4 * i + 3]);
-    }
+    put_partials<NT3>(acc3, L.part(), L.LDP, qk, n3, lane);
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < WV::CPT; ++j) {
-      const int c = owner_c0 + j;
-      float s = part[(0 * MLP_TILE + owner_row) * L.LDP + c];
-      s += part[(1 * MLP_TILE + owner_row) * L.LDP + c];
-      s += part[(2 * MLP_TILE + owner_row) * L.LDP + c];
-      s += part[(3 * MLP_TILE + owner_row) * L.LDP + c];
-      fout[j] = tanh_f(s + L.bias[2 * MLP_H + c]);
-    }
+    sum_partials<WV::CPT>(L.part(), L.LDP, L.bias + 2 * MLP_H, owner_row, owner_c0, fout);
   }
 }
 
