@@ -426,7 +426,7 @@ def backward_mlp(plan, ys_bar):
                                              ctypes.byref(rows_b), ctypes.byref(part_b)),
                    "dfx_mlp_adj_workspace")
         zs = torch.empty(int(zs_b.value) // 4, dtype=torch.float32, device=dev)
-        rows = torch.zeros(int(rows_b.value), dtype=torch.uint8, device=dev)
+        rows = torch.empty(int(rows_b.value), dtype=torch.uint8, device=dev)
         part = torch.empty(int(part_b.value) // 4, dtype=torch.float32, device=dev)
         io = MlpAdjIO(grid=plan.grid.data_ptr(), ckpt=plan.ckpt.data_ptr(),
                       stats=plan.stats.data_ptr(),
@@ -547,7 +547,7 @@ def backsolve_mlp(plan, back, ys_bar, chunk=BACKSOLVE_CHUNK):
                                                ctypes.byref(rows_b), ctypes.byref(part_b)),
                "dfx_mlp_backsolve_workspace")
     state = torch.zeros(int(st_b.value), dtype=torch.uint8, device=dev)
-    rows = torch.zeros(int(rows_b.value) // 4, dtype=torch.float32, device=dev)
+    rows = torch.empty(int(rows_b.value) // 4, dtype=torch.float32, device=dev)
     part = torch.empty(int(part_b.value) // 4, dtype=torch.float32, device=dev)
     io = MlpBacksolveIO(ys=plan.ys.data_ptr(), ts_out=plan.ts_out.data_ptr(),
                         ys_bar=ys_bar.data_ptr(), state=state.data_ptr(), rows=rows.data_ptr(),

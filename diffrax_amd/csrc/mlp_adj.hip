@@ -33,7 +33,7 @@ constexpr int ADJ_CHUNK = 4096;  // rows per split-K chunk of the weight-gradien
 
 // Six row buffers: D1 (width 256), Z (64), D2 (256), H1 (256), D3 (64), H2 (256).
 
-struct RowBufs {  // float32 [rows][width]
+struct RowBufs {  // float32 blocks of 32 rows, in the order of rows_frag
   float* b[6];
 };
 
@@ -57,7 +57,7 @@ struct AdjArgs {
 // the MFMA time of one float32 pass.  Float32 MFMA throughout took 1.97 ms for the
 // float32 form's segment of 8,192 trajectories and 4 steps.  The row
 // buffers hold float32 values (layer inputs and deltas written before their split into
-// pieces) for the float32 weight-gradient GEMM.  LDS: the forward planes;
+// pieces) for the weight-gradient GEMM.  LDS: the forward planes;
 // in the sweep the x planes take delta3, the h1 planes delta2 and then the split-K partials,
 // the h2 planes delta1 (the activations come back from the row buffers).  NW waves per tile
 // share the products as in the forward (MlpWaves); the arithmetic of every element does not
@@ -88,7 +88,8 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
   using TL = TabLit<Tab, float>;
   float* fs_tile = a.zs + (int64_t)tile * a.Cs * S * MLP_TILE * MLP_D;
   auto fslot = [&](int q, int i) { return fs_tile + (((int64_t)q * S + i) * MLP_TILE + orow) * MLP_D + c0; };
-  auto stage_row0 = [&](int q, int i) { return ((int64_t)q * S + i) * a.B_pad + (int64_t)tile * MLP_TILE; };
+  const int64_t ntiles = a.B_pad / MLP_TILE;
+  auto stage_block = [&](int q, int i) { return ((int64_t)q * S + i) * ntiles + tile; };
   // The layer inputs of stage (q, i) go to the row buffers as they are formed: the stage
   // value by its owner threads, the activations from the forward's epilogues.  The last
   // stage's rows are also the next step's stage-0 rows (FSAL: the same input).
@@ -96,13 +97,13 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
     MlpRowSink k;
     k.h1 = R.b[3];
     k.h2 = R.b[5];
-    k.row0 = stage_row0(q, i);
-    k.row0b = (i == S - 1 && q + 1 < a.Cs) ? stage_row0(q + 1, 0) : -1;
+    k.block = stage_block(q, i);
+    k.block2 = (i == S - 1 && q + 1 < a.Cs) ? stage_block(q + 1, 0) : -1;
     return k;
   };
   auto put_x = [&](const MlpRowSink& k, int j, float v) {
-    R.b[1][(k.row0 + orow) * MLP_D + c0 + j] = v;
-    if (k.row0b >= 0) R.b[1][(k.row0b + orow) * MLP_D + c0 + j] = v;
+    R.b[1][rows_index(k.block, MLP_D, orow, c0 + j)] = v;
+    if (k.block2 >= 0) R.b[1][rows_index(k.block2, MLP_D, orow, c0 + j)] = v;
   };
 
   // ---- 1. recompute the segment: keep every stage's f (scratch) and its layer inputs (row
@@ -202,18 +203,19 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
     }
     static_for<0, S>([&](auto ic) {
       constexpr int i = S - 1 - decltype(ic)::value;
-      const int64_t row0 = stage_row0(q, i);
+      const int64_t block = stage_block(q, i);
       const float* fp = fslot(q, i);
       // delta3 = fbar (1 - f^2), fbar = control * kbar_i: its row, and its pieces in x
+      float d3v[CPT];
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
         const float fb = act ? control * kb[i][j] : 0.0f;
         const float fv = fp[j];
         const float d3 = fb * (1.0f - fv * fv);
-        R.b[4][(row0 + orow) * MLP_D + c0 + j] = d3;
-        const int li = orow * L.LDX + c0 + j;
-        split3(d3, L.x[0][li], L.x[1][li], L.x[2][li]);
+        R.b[4][rows_index(block, MLP_D, orow, c0 + j)] = d3;
+        d3v[j] = d3;
       }
+      store_inputs(L, orow, c0, d3v);
       __syncthreads();
       // delta2 = (delta3 . W3) softplus'(h2): its row, and its pieces in h1
       floatx16_t acc[NT];
@@ -223,13 +225,15 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
       for (int t = 0; t < NT; ++t) {
         const int col = 32 * (NT * wave + t) + (lane & 31);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = R.b[5][(row0 + r) * MLP_H + col];
-          const float d2 = acc[t][v] * dsoftplus_from_value(h);
-          R.b[2][(row0 + r) * MLP_H + col] = d2;
-          const int li = r * L.LDH + col;
-          split3(d2, L.h1[0][li], L.h1[1][li], L.h1[2][li]);
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int64_t fr = rows_frag(block, MLP_H, NT * wave + t, i4, lane);
+          const float4 h = *reinterpret_cast<const float4*>(R.b[5] + fr);
+          const float4 dl = make_float4(acc[t][4 * i4] * dsoftplus_from_value(h.x),
+                                        acc[t][4 * i4 + 1] * dsoftplus_from_value(h.y),
+                                        acc[t][4 * i4 + 2] * dsoftplus_from_value(h.z),
+                                        acc[t][4 * i4 + 3] * dsoftplus_from_value(h.w));
+          *reinterpret_cast<float4*>(R.b[2] + fr) = dl;
+          store_col4(L.h1[0], MLP_TILE * L.LDH, L.LDH, 8 * i4 + 4 * (lane >> 5), col, dl);
         }
       }
       __syncthreads();
@@ -240,13 +244,15 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
       for (int t = 0; t < NT; ++t) {
         const int col = 32 * (NT * wave + t) + (lane & 31);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = acc_row(lane, v);
-          const float h = R.b[3][(row0 + r) * MLP_H + col];
-          const float d1 = acc[t][v] * dsoftplus_from_value(h);
-          R.b[0][(row0 + r) * MLP_H + col] = d1;
-          const int li = r * L.LDH + col;
-          split3(d1, L.h2[0][li], L.h2[1][li], L.h2[2][li]);
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int64_t fr = rows_frag(block, MLP_H, NT * wave + t, i4, lane);
+          const float4 h = *reinterpret_cast<const float4*>(R.b[3] + fr);
+          const float4 dl = make_float4(acc[t][4 * i4] * dsoftplus_from_value(h.x),
+                                        acc[t][4 * i4 + 1] * dsoftplus_from_value(h.y),
+                                        acc[t][4 * i4 + 2] * dsoftplus_from_value(h.z),
+                                        acc[t][4 * i4 + 3] * dsoftplus_from_value(h.w));
+          *reinterpret_cast<float4*>(R.b[0] + fr) = dl;
+          store_col4(L.h2[0], MLP_TILE * L.LDH, L.LDH, 8 * i4 + 4 * (lane >> 5), col, dl);
         }
       }
       __syncthreads();
@@ -321,108 +327,148 @@ __host__ __device__ inline DwLayout dw_layout() {
 }
 
 // Launch order is XCD-aware: workgroups are dealt to the 8 XCDs round-robin by linear id,
-// so block b runs on XCD b % 8; XCD x takes chunks x, x + 8, ... and runs the blocks of a
-// chunk back to back, which then read the chunk's rows through one L2 instead of eight.
+// so workgroup b runs on XCD b % 8; XCD x takes chunks x, x + 8, ... and runs the workgroups
+// of a chunk back to back, which then read the chunk's rows through one L2 instead of eight.
 constexpr int kXcds = 8;
 
-// partial[chunk][tile] = A^T B over one chunk of ADJ_CHUNK rows (A = deltas, B = layer
-// inputs) for every 32 x 32 output tile, each wave on a 2 x 2 block of tiles (a 64 x 64
-// piece of one matrix): per k-step it loads two delta and two input fragments for four
-// MFMAs (a wave per tile, measured before, loaded twice as much per MFMA and took the
-// backward of 8,192 trajectories from 2.84 to 2.91 ms, the backsolve from 19.0 to 19.6 ms,
-// with the same bits).  The fragments come in groups of 4 k-steps held in two register
-// buffers (the next group loads while the current one feeds the MFMAs).  The row buffers
-// are allocated in whole chunks and rows past the segment's last are zero, so every chunk
-// runs its full length.  The 96 tiles of a chunk form 24 blocks (dW1 4 x 1, dW2 4 x 4,
-// dW3 1 x 4); blocks in the first block column of a matrix also produce the chunk's column
-// sums of A (the bias gradient partials, partial_db: [chunk][db1 | db2 | db3]).
-// SC: the delta rows are multiplied by rscale[row] as they load (the backsolve's per-row
-// weights dt * b_i, zero for rejected steps and idle rows; a row of zero weight is dropped
-// from both operands, so a non-finite value in it contributes nothing).  Float32 rows only.
-__host__ __device__ inline int dw_blocks_of(int m) {
+// Chunks of row blocks the GEMM splits K into: 24 one-wave workgroups (64 x 64 output
+// pieces) each, two per SIMD of the chip resident at once, so at most 80 chunks (1,920
+// waves), and no more than there are four-block chunks.
+__host__ __device__ inline int dw_chunks(int64_t blocks) {
+  const int64_t n = (blocks + 3) / 4;
+  return (int)(n < 80 ? (n < 1 ? 1 : n) : 80);
+}
+
+// partial[chunk][tile] = A^T B over one chunk of row blocks (A = deltas, B = layer inputs)
+// for every 32 x 32 output tile, each wave on a 2 x 2 block of tiles (a 64 x 64 piece of one
+// matrix: dW1 4 x 1, dW2 4 x 4, dW3 1 x 4 pieces).  A lane's sixteen values of a block piece
+// are the rows of its two k halves (rows_frag), so fragments go from memory through the
+// split straight to the MFMAs: six bf16 products per pair of fragments, as in wave_gemm3,
+// with float32 accumulation.  The next block's values load while this one's are split.
+// Waves in the first piece column of a matrix also produce the chunk's column sums of A (the
+// bias gradient partials, partial_db: [chunk][db1 | db2 | db3]).
+// SC: the rows of A are multiplied by rscale[row] (the backsolve's per-row weights dt * b_i,
+// zero for rejected steps and idle rows; a row of zero weight is dropped from both operands,
+// so a non-finite value in it contributes nothing).
+// Bound: the rows' HBM reads, 4.6 KB a row: 0.31 ms for the 229,376 rows of 8,192
+// trajectories and 4 steps (3.4 TB/s, 290 TFLOP/s of 6 bf16 passes each), where float32 MFMA
+// with a 4-byte load per operand and MFMA took 0.72 ms (and 0.58 ms for 105,000 rows, now
+// 0.115).  Against float64 the gradients are closer than before (5.6e-7 to 8e-7 of the
+// largest, 1.3e-6 to 1.8e-6 with float32 MFMA).
+__host__ __device__ inline int dw_pieces_of(int m) {
   const DwLayout l = dw_layout();
   return (l.n1[m] / 64) * (l.n2[m] / 64);
 }
 
-template <bool SC = false>
-__global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs R,
-                                                           float* __restrict__ partial,
-                                                           float* __restrict__ partial_db,
-                                                           int nch,
-                                                           const float* __restrict__ rscale = nullptr) {
+template <bool SC>
+__global__ void __launch_bounds__(64, 2)
+mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restrict__ partial_db,
+                   int64_t blocks, int nch, const float* __restrict__ rscale) {
   const DwLayout lay = dw_layout();
-  const int nblk = dw_blocks_of(0) + dw_blocks_of(1) + dw_blocks_of(2);
+  const int npc = dw_pieces_of(0) + dw_pieces_of(1) + dw_pieces_of(2);
   const int xcd = (int)(blockIdx.x % kXcds), slot = (int)(blockIdx.x / kXcds);
-  const int chunk = (slot / nblk) * kXcds + xcd;
-  int bg = slot - (slot / nblk) * nblk;
+  const int chunk = (slot / npc) * kXcds + xcd;
+  int pg = slot - (slot / npc) * npc;
   if (chunk >= nch) return;
   int m = 0;
-  while (bg >= dw_blocks_of(m)) { bg -= dw_blocks_of(m); ++m; }
-  const int nbj = lay.n2[m] / 64;
-  const int bi = bg / nbj, bj = bg - bi * nbj;
-  const float* A = R.b[2 * m];       // deltas (width n1)
-  const float* Bm = R.b[2 * m + 1];  // layer inputs (width n2)
-  const int WA = lay.n1[m], WB = lay.n2[m];
-  const int lane = threadIdx.x;
-  constexpr int KS = 2, U = 4;
-  static_assert(ADJ_CHUNK % (KS * U) == 0, "chunk must hold whole k-step groups");
-  const bool col_sums = (bj == 0);
-  const int64_t r_begin = (int64_t)chunk * ADJ_CHUNK;
+  while (pg >= dw_pieces_of(m)) { pg -= dw_pieces_of(m); ++m; }
+  const int W1 = m == 2 ? MLP_D : MLP_H, W2 = m == 0 ? MLP_D : MLP_H;  // columns of A and B
+  const int npj = W2 / 64;
+  const int pi = pg / npj, pj = pg - pi * npj;
+  const float* A = m == 0 ? R.b[0] : m == 1 ? R.b[2] : R.b[4];
+  const float* Bm = m == 0 ? R.b[1] : m == 1 ? R.b[3] : R.b[5];
+  const int lane = threadIdx.x, half = lane >> 5;
+  const bool col_sums = (pj == 0);
+  const int64_t b0 = blocks * chunk / nch, b1 = blocks * (chunk + 1) / nch;
+  using P = PolicyBF16x3;
+  using frag_t = P::frag_t;
   floatx16_t acc[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x) { acc[x][0] = floatx16_t{}; acc[x][1] = floatx16_t{}; }
   float csum[2] = {0.0f, 0.0f};
-  const int ca = bi * 64 + (lane & 31), cb = bj * 64 + (lane & 31);
-  using frag_t = float;
-  auto load_group = [&](int64_t r0, frag_t (&fa)[U][2], frag_t (&fb)[U][2]) {
+  float4 va[2][4], vb[2][4];
+  auto load = [&](int64_t blk) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t rb = r0 + u * KS + (lane >> 5);
+    for (int x = 0; x < 2; ++x) {
 #pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        fa[u][x] = A[rb * WA + ca + 32 * x];
-        fb[u][x] = Bm[rb * WB + cb + 32 * x];
+      for (int i = 0; i < 4; ++i) {
+        va[x][i] = *reinterpret_cast<const float4*>(A + rows_frag(blk, W1, 2 * pi + x, i, lane));
+        vb[x][i] = *reinterpret_cast<const float4*>(Bm + rows_frag(blk, W2, 2 * pj + x, i, lane));
       }
-      if constexpr (SC) {
-        const float w = rscale[rb];
+    }
+  };
+  if (b0 < b1) load(b0);
+  for (int64_t blk = b0; blk < b1; ++blk) {
+    if constexpr (SC) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 w = *reinterpret_cast<const float4*>(rscale + blk * 32 + 8 * i + 4 * half);
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-          fa[u][x] = (w != 0.0f) ? fa[u][x] * w : 0.0f;
-          fb[u][x] = (w != 0.0f) ? fb[u][x] : 0.0f;
+          auto sc = [](float wt, float& da, float& db) {
+            da = (wt != 0.0f) ? da * wt : 0.0f;
+            db = (wt != 0.0f) ? db : 0.0f;
+          };
+          sc(w.x, va[x][i].x, vb[x][i].x);
+          sc(w.y, va[x][i].y, vb[x][i].y);
+          sc(w.z, va[x][i].z, vb[x][i].z);
+          sc(w.w, va[x][i].w, vb[x][i].w);
         }
       }
     }
-  };
-  auto mma_group = [&](const frag_t (&fa)[U][2], const frag_t (&fb)[U][2]) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
+    if (col_sums) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        acc[x][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u][x], fb[u][0], acc[x][0], 0, 0, 0);
-        acc[x][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u][x], fb[u][1], acc[x][1], 0, 0, 0);
-        if (col_sums) csum[x] += fa[u][x];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          csum[x] += (va[x][i].x + va[x][i].y) + (va[x][i].z + va[x][i].w);
       }
     }
-  };
-  constexpr int G = ADJ_CHUNK / (KS * U);
-  static_assert(G % 2 == 0, "groups are processed in pairs");
-  frag_t a0[U][2], b0[U][2], a1[U][2], b1[U][2];
-  load_group(r_begin, a0, b0);
-  for (int g = 0; g < G; g += 2) {
-    load_group(r_begin + (int64_t)(g + 1) * KS * U, a1, b1);
-    mma_group(a0, b0);
-    load_group(r_begin + (int64_t)min(g + 2, G - 1) * KS * U, a0, b0);
-    mma_group(a1, b1);
+    // k half s: the rows 16 s .. 16 s + 15 of the block, in the same order for both operands
+    frag_t fa[2][2][3], fb[2][2][3];  // [s][x][piece]
+    auto split = [&](const float4& u, const float4& v, frag_t (&f)[3]) {
+      const Split4 s0 = split3x4(u.x, u.y, u.z, u.w), s1 = split3x4(v.x, v.y, v.z, v.w);
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) {
+        const uint4 q = make_uint4(s0.p[pc].x, s0.p[pc].y, s1.p[pc].x, s1.p[pc].y);
+        f[pc] = __builtin_bit_cast(frag_t, q);
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        split(va[x][2 * s], va[x][2 * s + 1], fa[s][x]);
+        split(vb[x][2 * s], vb[x][2 * s + 1], fb[s][x]);
+      }
+    }
+    if (blk + 1 < b1) load(blk + 1);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int pq = 0; pq < 6; ++pq) {  // p0q0, p0q1, p1q0, p0q2, p1q1, p2q0
+        constexpr int pa[6] = {0, 0, 1, 0, 1, 2}, pb[6] = {0, 1, 0, 2, 1, 0};
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+            acc[x][y] = P::mfma(fa[s][x][pa[pq]], fb[s][y][pb[pq]], acc[x][y]);
+        }
+      }
+    }
   }
-  const int ntj = lay.n2[m] / 32;
+  const int ntj = W2 / 32;
+  const int first = m == 0 ? lay.first[0] : m == 1 ? lay.first[1] : lay.first[2];
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
-      const int tg = lay.first[m] + (2 * bi + x) * ntj + (2 * bj + y);
-      float* o = partial + ((int64_t)chunk * lay.first[3] + tg) * 1024 + lane * 16;
+      const int tg = first + (2 * pi + x) * ntj + (2 * pj + y);
+      float4* o = reinterpret_cast<float4*>(partial + ((int64_t)chunk * lay.first[3] + tg) * 1024);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) o[v] = acc[x][y][v];
+      for (int i = 0; i < 4; ++i)
+        o[i * 64 + lane] = make_float4(acc[x][y][4 * i], acc[x][y][4 * i + 1], acc[x][y][4 * i + 2],
+                                       acc[x][y][4 * i + 3]);
     }
   }
   if (col_sums) {
@@ -430,35 +476,65 @@ __global__ void __launch_bounds__(64) mlp_dw_gemm_kernel(const RowBufs R,
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
       const float c = csum[x] + __shfl_xor(csum[x], 32);
-      if (lane < 32) partial_db[(int64_t)chunk * (2 * MLP_H + MLP_D) + off + ca + 32 * x] = c;
+      if (lane < 32)
+        partial_db[(int64_t)chunk * (2 * MLP_H + MLP_D) + off + pi * 64 + 32 * x + lane] = c;
     }
   }
 }
 
-// dw_acc (dW1 | dW2 | dW3 | db1 | db2 | db3, row-major) += partials summed in chunk order.
-__global__ void mlp_dw_reduce_kernel(const float* __restrict__ partial,
-                                     const float* __restrict__ partial_db, int nchunks,
-                                     float* __restrict__ dw_acc) {
+// dw_acc (dW1 | dW2 | dW3 | db1 | db2 | db3, row-major) += partials over the chunks.  A
+// workgroup takes 64 float4 of the partials; its four waves sum every fourth chunk each and
+// the four sums are added in order.  (One thread per output over all chunks, its loads one
+// behind the other and 64 bytes apart: 34 us.)
+__global__ void __launch_bounds__(256) mlp_dw_reduce_kernel(const float* __restrict__ partial,
+                                                            const float* __restrict__ partial_db,
+                                                            int nchunks,
+                                                            float* __restrict__ dw_acc) {
+  __shared__ float4 sum[4][64];
   const DwLayout lay = dw_layout();
-  const int nW = MLP_H * MLP_D + MLP_H * MLP_H + MLP_D * MLP_H;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nW + 2 * MLP_H + MLP_D) return;
-  float s = 0.0f;
-  if (e < nW) {
-    int m = 0, off = e;
-    const int sz[3] = {MLP_H * MLP_D, MLP_H * MLP_H, MLP_D * MLP_H};
-    while (off >= sz[m]) { off -= sz[m]; ++m; }
-    const int n1 = off / lay.n2[m], n2 = off - (off / lay.n2[m]) * lay.n2[m];
-    const int tg = lay.first[m] + (n1 / 32) * (lay.n2[m] / 32) + n2 / 32;
-    const int r = n1 % 32, c = n2 % 32;
-    const int lane = c + 32 * ((r % 8) / 4);
-    const int v = 4 * (r / 8) + (r % 4);
-    for (int ch = 0; ch < nchunks; ++ch) s += partial[((int64_t)ch * lay.first[3] + tg) * 1024 + lane * 16 + v];
-  } else {
-    const int col = e - nW;
-    for (int ch = 0; ch < nchunks; ++ch) s += partial_db[(int64_t)ch * (2 * MLP_H + MLP_D) + col];
+  const int ntile = lay.first[3], nb = (2 * MLP_H + MLP_D) / 4;
+  const int col = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int blk = blockIdx.x;
+  const bool weights = blk < ntile * 4;  // then the bias partials, 144 float4
+  const int e = weights ? blk * 64 + col : (blk - ntile * 4) * 64 + col;
+  const bool live = weights || e < nb;
+  const int64_t stride = weights ? (int64_t)ntile * 256 : nb;
+  const float4* src = reinterpret_cast<const float4*>(weights ? partial : partial_db) + e;
+  float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (live) {
+#pragma unroll 4
+    for (int ch = part; ch < nchunks; ch += 4) {
+      const float4 v = src[ch * stride];
+      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    }
   }
-  dw_acc[e] += s;
+  sum[part][col] = s;
+  __syncthreads();
+  if (part != 0 || !live) return;
+#pragma unroll
+  for (int q = 1; q < 4; ++q) {
+    const float4 v = sum[q][col];
+    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  }
+  const int nW = MLP_H * MLP_D + MLP_H * MLP_H + MLP_D * MLP_H;
+  const float sv[4] = {s.x, s.y, s.z, s.w};
+  if (!weights) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dw_acc[nW + 4 * e + j] += sv[j];
+    return;
+  }
+  // float4 i of tile tg, lane col: rows 8i + 4(col/32) + j, column col%32
+  const int tg = blk >> 2, i = blk & 3;
+  int m = 0;
+  while (tg >= lay.first[m + 1]) ++m;
+  const int W2 = m == 0 ? MLP_D : MLP_H, ntj = W2 / 32;
+  const int off = m == 0 ? 0 : m == 1 ? MLP_H * MLP_D : MLP_H * MLP_D + MLP_H * MLP_H;
+  const int ti = (tg - lay.first[m]) / ntj, tj = (tg - lay.first[m]) % ntj;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = 32 * ti + 8 * i + 4 * (col >> 5) + j;
+    dw_acc[off + r * W2 + 32 * tj + (col & 31)] += sv[j];
+  }
 }
 
 // ---- BacksolveAdjoint of the neural ODE ---------------------------------------------
@@ -510,12 +586,14 @@ struct MlpLdsBack : MlpLds<PolicyF32> {
 };
 static_assert(sizeof(MlpLdsBack) <= 160 * 1024, "one workgroup per CU");
 
-// The tile's rows of an LDS buffer (columns at PolicyF32::pos) to row-major rows of width Wd.
+// The tile's rows of an LDS buffer (columns at PolicyF32::pos) to a block of a row buffer.
 template <int Wd>
-__device__ __forceinline__ void rows_out(const float* lds, int ld, float* dst, int64_t row0) {
-  for (int e = threadIdx.x; e < MLP_TILE * Wd; e += blockDim.x) {
-    const int r = e / Wd, col = e % Wd;
-    dst[(row0 + r) * Wd + col] = lds[r * ld + PolicyF32::pos(col)];
+__device__ __forceinline__ void rows_out(const float* lds, int ld, float* dst, int64_t block) {
+  for (int e = threadIdx.x; e < MLP_TILE * Wd / 4; e += blockDim.x) {
+    const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
+    const float* p = lds + (8 * i + 4 * (l >> 5)) * ld + PolicyF32::pos(32 * t + (l & 31));
+    *reinterpret_cast<float4*>(dst + rows_frag(block, Wd, t, i, l)) =
+        make_float4(p[0], p[ld], p[2 * ld], p[3 * ld]);
   }
 }
 
@@ -633,7 +711,7 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
     }
   };
   const int64_t rb0 = (int64_t)tile * MLP_TILE + orow;
-  auto stage_row0 = [&](int q, int i) { return ((int64_t)q * S + i) * a.B_pad + (int64_t)tile * MLP_TILE; };
+  const int64_t ntiles = a.B_pad / MLP_TILE;
   int q = 0;
   for (; q < a.Q; ++q) {
     const bool run = !st.done;
@@ -664,16 +742,16 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
       __syncthreads();
       float f[CPT];
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
-      const int64_t row0 = stage_row0(q, i);
-      rows_out<MLP_D>(L.x, L.LDX, R.b[1], row0);
-      rows_out<MLP_H>(L.h1, L.LDH, R.b[3], row0);
-      rows_out<MLP_H>(L.h2, L.LDH, R.b[5], row0);
+      const int64_t block = ((int64_t)q * S + i) * ntiles + tile;
+      rows_out<MLP_D>(L.x, L.LDX, R.b[1], block);
+      rows_out<MLP_H>(L.h1, L.LDH, R.b[3], block);
+      rows_out<MLP_H>(L.h2, L.LDH, R.b[5], block);
       // vjp with cotangent w = -a_y of the stage: delta3 = w (1 - f^2)
 #pragma unroll
       for (int j = 0; j < CPT; ++j)
         L.d3[orow * L.LDX + P::pos(c0 + j)] = -za[j] * (1.0f - f[j] * f[j]);
       __syncthreads();
-      rows_out<MLP_D>(L.d3, L.LDX, R.b[4], row0);
+      rows_out<MLP_D>(L.d3, L.LDX, R.b[4], block);
       // delta2 = (delta3 . W3) softplus'(h2)
       constexpr int F1 = MLP_D / P::KSTEP, F2 = MLP_H / P::KSTEP;
       floatx16_t acc[NT];
@@ -688,8 +766,8 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
       g2t.template run<F2>(L.d, L.LDH, 0, acc, lane);
       put_delta(acc, L.h1, L.h2);
       __syncthreads();
-      rows_out<MLP_H>(L.d, L.LDH, R.b[2], row0);
-      rows_out<MLP_H>(L.h2, L.LDH, R.b[0], row0);
+      rows_out<MLP_H>(L.d, L.LDH, R.b[2], block);
+      rows_out<MLP_H>(L.h2, L.LDH, R.b[0], block);
       // vjp_y = delta1 . W1 (split-K over the 256 hidden units)
       const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
       floatx16_t acc3[NT3];
@@ -862,20 +940,26 @@ __global__ void bs_reset_kernel(int32_t* counters, float* rscale, int64_t used, 
   for (int64_t r = used + threadIdx.x; r < nrow; r += blockDim.x) rscale[r] = 0.0f;
 }
 
-// The weight-gradient GEMM over nch chunks of float32 rows (SC: per-row weights rscale).
+// The weight gradients of `blocks` row blocks (SC: per-row weights rscale) added to dw.
 template <bool SC>
-void launch_dw_gemm(const RowBufs& R, float* partial, float* partial_db, int nch,
-                    const float* rscale, hipStream_t s) {
+void launch_dw(const RowBufs& R, float* partial, int64_t blocks, const float* rscale, float* dw,
+               hipStream_t s) {
+  const int nch = dw_chunks(blocks);
+  const DwLayout lay = dw_layout();
+  float* partial_db = partial + (int64_t)nch * lay.first[3] * 1024;
   const int groups = (nch + kXcds - 1) / kXcds;
-  const int nblk = dw_blocks_of(0) + dw_blocks_of(1) + dw_blocks_of(2);
-  hipLaunchKernelGGL((mlp_dw_gemm_kernel<SC>), dim3(kXcds * nblk * groups), dim3(64),
-                     0, s, R, partial, partial_db, nch, rscale);
+  const int npc = dw_pieces_of(0) + dw_pieces_of(1) + dw_pieces_of(2);
+  hipLaunchKernelGGL((mlp_dw_gemm_kernel<SC>), dim3(kXcds * npc * groups), dim3(64), 0, s, R,
+                     partial, partial_db, blocks, nch, rscale);
+  const int nblk = lay.first[3] * 4 + ((2 * MLP_H + MLP_D) / 4 + 63) / 64;
+  hipLaunchKernelGGL(mlp_dw_reduce_kernel, dim3(nblk), dim3(256), 0, s, partial, partial_db, nch,
+                     dw);
 }
 
-// Floats of the weight-gradient partials of nch chunks, and behind them (float32 form) the
-// three-piece planes of the weights.
-int64_t partial_floats(int64_t nch) {
-  return (nch * ((int64_t)dw_layout().first[3] * 1024 + 2 * MLP_H + MLP_D) + 63) / 64 * 64;
+// Floats of the weight-gradient partials of `blocks` row blocks; behind them (float32 form)
+// come the three-piece planes of the weights.
+int64_t partial_floats(int64_t blocks) {
+  return (dw_chunks(blocks) * ((int64_t)dw_layout().first[3] * 1024 + 2 * MLP_H + MLP_D) + 63) / 64 * 64;
 }
 
 // One segment: the recompute + sweep kernel on three-piece weights (a bf16 buffer as it is;
@@ -895,9 +979,9 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   a.Cs = seg_steps; a.seg = seg; a.n_ts = p->n_ts; a.ts_stride = p->ts_stride;
   a.n_out = (p->save_t0 ? 1 : 0) + p->n_ts + (p->save_t1 ? 1 : 0);
   a.save_t0 = p->save_t0; a.t0 = p->t0; a.t1 = p->t1;
-  const int nch = (int)seg_chunks(p->batch, seg_steps);
+  const int64_t blocks = seg_rows(p->batch, seg_steps) / MLP_TILE;
   if (p->precision == DFX_F32) {
-    __bf16* planes = reinterpret_cast<__bf16*>(io->partial + partial_floats(nch));
+    __bf16* planes = reinterpret_cast<__bf16*>(io->partial + partial_floats(blocks));
     const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);
     hipLaunchKernelGGL(mlp_split_packed_kernel, dim3(nb), dim3(256), 0, s,
                        reinterpret_cast<const float*>(packed), planes);
@@ -915,13 +999,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLds<P>));
   hipLaunchKernelGGL(mlp_adj_segment_kernel<NW>, dim3(ntiles), dim3(64 * NW), sizeof(MlpLds<P>), s,
                      a, W, R);
-  const DwLayout lay = dw_layout();
-  float* partial = io->partial;
-  float* partial_db = io->partial + (int64_t)nch * lay.first[3] * 1024;
-  launch_dw_gemm<false>(R, partial, partial_db, nch, nullptr, s);
-  const int nout = MLP_H * MLP_D + MLP_H * MLP_H + MLP_D * MLP_H + 2 * MLP_H + MLP_D;
-  hipLaunchKernelGGL(mlp_dw_reduce_kernel, dim3((nout + 255) / 256), dim3(256), 0, s, partial,
-                     partial_db, nch, io->dw);
+  launch_dw<false>(R, io->partial, blocks, nullptr, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -939,7 +1017,7 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) wsum += widths[i];
   *rows_bytes = (size_t)(rows_alloc * wsum) * sizeof(float);   // float32 rows for both forms
-  *partial_bytes = (size_t)partial_floats(seg_chunks(p->batch, seg_steps)) * sizeof(float);
+  *partial_bytes = (size_t)partial_floats(seg_rows(p->batch, seg_steps) / MLP_TILE) * sizeof(float);
   if (p->precision == DFX_F32) *partial_bytes += (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
 }
@@ -954,9 +1032,7 @@ int dfx_mlp_backsolve_workspace(const dfx_mlp_problem* p, int32_t chunk_iters,
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) wsum += widths[i];
   *rows_bytes = (size_t)(nrow * wsum) * sizeof(float);
-  const DwLayout lay = dw_layout();
-  *partial_bytes = (size_t)(seg_chunks(p->batch, chunk_iters) *
-                            ((int64_t)lay.first[3] * 1024 + 2 * MLP_H + MLP_D)) * sizeof(float);
+  *partial_bytes = (size_t)partial_floats(seg_rows(p->batch, chunk_iters) / MLP_TILE) * sizeof(float);
   return DFX_OK;
 }
 
@@ -1010,13 +1086,8 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLdsBack));
   hipLaunchKernelGGL((mlp_backsolve_kernel<NWB>), dim3(ntiles), dim3(64 * NWB),
                      sizeof(MlpLdsBack), s, a, W, R);
-  const DwLayout lay = dw_layout();
-  float* partial = io->partial;
-  float* partial_db = io->partial + (int64_t)nch * lay.first[3] * 1024;
-  launch_dw_gemm<true>(R, partial, partial_db, nch, a.rscale, s);
-  const int nout = MLP_H * MLP_D + MLP_H * MLP_H + MLP_D * MLP_H + 2 * MLP_H + MLP_D;
-  hipLaunchKernelGGL(mlp_dw_reduce_kernel, dim3((nout + 255) / 256), dim3(256), 0, s, partial,
-                     partial_db, nch, io->dw);
+  launch_dw<true>(R, io->partial, seg_rows(back->batch, chunk_iters) / MLP_TILE, a.rscale, io->dw,
+                  s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 

@@ -494,18 +494,43 @@ struct Gemm3 {
   }
 };
 
-// Float32 copies of the hidden activations for the adjoint's row buffers ([rows][256] each,
-// the tile's rows from row0, and again from row0b when row0b >= 0): written in the layer
-// epilogues, before layer 3's partials reuse the h1 planes.
+// The adjoint's row buffers hold float32 rows in blocks of 32 (one tile's rows of one stage),
+// each 32-column piece of a block in the accumulator order of its MFMA tile: the four rows
+// 8i + 4(l/32) + j, j = 0..3, of column l%32 are one float4 of lane l.  The epilogues that
+// produce a block store it in whole lines, and a lane's sixteen values are the k values of
+// two MFMA operands of the weight-gradient product (whose k are the rows).
+__host__ __device__ inline int64_t rows_frag(int64_t block, int width, int t, int i, int lane) {
+  return (((block * (width / 32) + t) * 4 + i) * 64 + lane) * 4;
+}
+__host__ __device__ inline int64_t rows_index(int64_t block, int width, int row, int col) {
+  return rows_frag(block, width, col / 32, row / 8, col % 32 + 32 * (row % 8 / 4)) + row % 4;
+}
+
+// Where the hidden activations of an evaluation go in the row buffers (block, and again at
+// block2 when that is not negative).
 struct MlpRowSink {
   float* h1 = nullptr;
   float* h2 = nullptr;
-  int64_t row0 = 0, row0b = -1;
-  __device__ __forceinline__ void put(float* dst, int r, int col, float v) const {
-    dst[(row0 + r) * MLP_H + col] = v;
-    if (row0b >= 0) dst[(row0b + r) * MLP_H + col] = v;
+  int64_t block = 0, block2 = -1;
+  __device__ __forceinline__ void put(float* dst, int t, int i, int lane, float4 v) const {
+    *reinterpret_cast<float4*>(dst + rows_frag(block, MLP_H, t, i, lane)) = v;
+    if (block2 >= 0) *reinterpret_cast<float4*>(dst + rows_frag(block2, MLP_H, t, i, lane)) = v;
   }
 };
+
+// Store four rows r .. r + 3 of one column in the three planes of an LDS buffer.
+__device__ __forceinline__ void store_col4(__bf16* buf, int plane, int ld, int r, int col,
+                                           const float4 v) {
+  const Split4 s = split3x4(v.x, v.y, v.z, v.w);
+#pragma unroll
+  for (int pc = 0; pc < 3; ++pc) {
+    unsigned short* o = reinterpret_cast<unsigned short*>(buf + pc * plane + r * ld + col);
+    o[0] = (unsigned short)s.p[pc].x;
+    o[ld] = (unsigned short)(s.p[pc].x >> 16);
+    o[2 * ld] = (unsigned short)s.p[pc].y;
+    o[3 * ld] = (unsigned short)(s.p[pc].y >> 16);
+  }
+}
 
 // The tile's waves split the work: layers 1 and 2 by output columns (NT12 tiles of 32 per
 // wave), layer 3 by K quarters (four waves: both 32-column tiles of one quarter; eight
@@ -538,11 +563,11 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
     const int col = 32 * (NT * wave + t) + (lane & 31);
     const float bias = W.b1[col];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int i = acc_row(lane, v) * L.LDH + col;
-      const float h = softplus_f(acc[t][v] + bias);
-      if (sink.h1) sink.put(sink.h1, acc_row(lane, v), col, h);
-      split3(h, L.h1[0][i], L.h1[1][i], L.h1[2][i]);
+    for (int i = 0; i < 4; ++i) {
+      const float4 h = make_float4(softplus_f(acc[t][4 * i] + bias), softplus_f(acc[t][4 * i + 1] + bias),
+                                   softplus_f(acc[t][4 * i + 2] + bias), softplus_f(acc[t][4 * i + 3] + bias));
+      sink.put(sink.h1, NT * wave + t, i, lane, h);
+      store_col4(L.h1[0], MLP_TILE * L.LDH, L.LDH, 8 * i + 4 * (lane >> 5), col, h);
     }
   }
   __syncthreads();
@@ -554,11 +579,11 @@ __device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
     const int col = 32 * (NT * wave + t) + (lane & 31);
     const float bias = W.b2[col];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int i = acc_row(lane, v) * L.LDH + col;
-      const float h = softplus_f(acc[t][v] + bias);
-      if (sink.h2) sink.put(sink.h2, acc_row(lane, v), col, h);
-      split3(h, L.h2[0][i], L.h2[1][i], L.h2[2][i]);
+    for (int i = 0; i < 4; ++i) {
+      const float4 h = make_float4(softplus_f(acc[t][4 * i] + bias), softplus_f(acc[t][4 * i + 1] + bias),
+                                   softplus_f(acc[t][4 * i + 2] + bias), softplus_f(acc[t][4 * i + 3] + bias));
+      sink.put(sink.h2, NT * wave + t, i, lane, h);
+      store_col4(L.h2[0], MLP_TILE * L.LDH, L.LDH, 8 * i + 4 * (lane >> 5), col, h);
     }
   }
   __syncthreads();

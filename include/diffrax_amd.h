@@ -501,7 +501,7 @@ typedef struct dfx_mlp_backsolve_io {
   const double* ts_out;     /* [B, n_out] their times                                      */
   const float* ys_bar;      /* [B, n_out, 64] cotangent of the saved states                 */
   void* state;              /* scratch, dfx_mlp_backsolve_workspace state_bytes             */
-  void* rows;               /* scratch, rows_bytes; zero it once before the first launch   */
+  void* rows;               /* scratch, rows_bytes                                          */
   float* partial;           /* scratch, partial_bytes                                      */
   float* dw;                /* in/out accumulator: dW1 | dW2 | dW3 | db1 | db2 | db3
                                (float32, row-major, 98880 values); zero it first           */
