@@ -45,6 +45,7 @@ struct AdjArgs {
   const float* ys_bar;
   float* ybar;
   float* zs;
+  int32_t* evals;  // out [tiles]: evaluations (row blocks) of each tile
   int64_t B, B_pad, ts_stride;
   int32_t max_steps, n_ckpt, C, Cs, seg, n_ts, n_out, save_t0;
   double t0, t1;
@@ -63,10 +64,20 @@ struct AdjArgs {
 // share the products as in the forward (MlpWaves); the arithmetic of every element does not
 // depend on NW.
 
+// Evaluations of a tile: its first state (slot 0), then six per step (slot 1 + 6q + i - 1 for
+// stage i of step q).  A step's last stage is the next one's first (FSAL: f at the same
+// point), so the sweep adds the two cotangents of f there and pulls them back once, and the
+// weight-gradient GEMM sees one row block for both.  A tile runs as many steps as its
+// longest trajectory has; evals[tile] tells the GEMM how many of its E = 1 + 6 Cs slots
+// (block tile * E + slot) hold rows.
+// One segment of 8,192 trajectories and up to 4 steps: 0.69 ms; 0.92 ms with seven
+// pull-backs a step, idle steps run, and the products' loads waited for in the K loop (and
+// the GEMM 0.26 against 0.31 ms for the rows that went).  15 us per evaluation: MFMA, the
+// splits and the LDS stores of one column at a time, one after the other, bound it, not the
+// 1.3 GB of rows.
 template <int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
-mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
-                        const RowBufs R) {
+mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const RowBufs R) {
   using P = PolicyBF16x3;
   extern __shared__ __align__(16) unsigned char smem[];
   MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
@@ -75,228 +86,231 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W,
   using WV = MlpWaves<NW>;
   constexpr int CPT = WV::CPT, GRP = MLP_D / CPT, NT = WV::NT12, NT3 = WV::NT3;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int orow = tid / GRP, c0 = (tid % GRP) * CPT;
+  const int orow = tid / GRP, c0 = (tid % GRP) * CPT, gbase = lane & ~(GRP - 1);
   const int tile = blockIdx.x;
   const int64_t traj = (int64_t)tile * MLP_TILE + orow;
   const bool valid = traj < a.B;
   const int nacc = valid ? a.stats[traj * 3 + 1] : 0;
   const int n0 = a.seg * a.C;
-  int steps_here = nacc - n0;
-  steps_here = steps_here < 0 ? 0 : (steps_here > a.Cs ? a.Cs : steps_here);
+  const int steps_here = min(max(nacc - n0, 0), a.Cs);
+  int tile_steps = 0;
+  while (__syncthreads_or(tile_steps < steps_here)) ++tile_steps;
+  if (tid == 0) a.evals[tile] = tile_steps > 0 ? 1 + 6 * tile_steps : 0;
+  if (tile_steps == 0) return;
   const int dir = (a.t0 < a.t1) ? 1 : -1;
   const double* ts_row = a.ts ? a.ts + (valid ? traj : 0) * a.ts_stride : nullptr;
   using TL = TabLit<Tab, float>;
-  float* fs_tile = a.zs + (int64_t)tile * a.Cs * S * MLP_TILE * MLP_D;
-  auto fslot = [&](int q, int i) { return fs_tile + (((int64_t)q * S + i) * MLP_TILE + orow) * MLP_D + c0; };
-  const int64_t ntiles = a.B_pad / MLP_TILE;
-  auto stage_block = [&](int q, int i) { return ((int64_t)q * S + i) * ntiles + tile; };
-  // The layer inputs of stage (q, i) go to the row buffers as they are formed: the stage
-  // value by its owner threads, the activations from the forward's epilogues.  The last
-  // stage's rows are also the next step's stage-0 rows (FSAL: the same input).
-  auto sink_of = [&](int q, int i) {
-    MlpRowSink k;
-    k.h1 = R.b[3];
-    k.h2 = R.b[5];
-    k.block = stage_block(q, i);
-    k.block2 = (i == S - 1 && q + 1 < a.Cs) ? stage_block(q + 1, 0) : -1;
-    return k;
+  const int64_t slot0 = (int64_t)tile * (1 + 6 * a.Cs);
+  auto slot_of = [&](int q, int i) { return slot0 + 6 * q + i; };  // stage i >= 1, or (0, 0)
+  auto fslot = [&](int64_t slot) { return a.zs + (slot * MLP_TILE + orow) * MLP_D + c0; };
+  // The layer inputs of an evaluation go to its row block as they are formed: the stage value
+  // by its owner threads, the activations from the forward's epilogues.
+  auto put_cols = [&](float* rows, int64_t slot, const float (&v)[CPT]) {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) rows[rows_index(slot, MLP_D, orow, c0 + j)] = v[j];
   };
-  auto put_x = [&](const MlpRowSink& k, int j, float v) {
-    R.b[1][rows_index(k.block, MLP_D, orow, c0 + j)] = v;
-    if (k.block2 >= 0) R.b[1][rows_index(k.block2, MLP_D, orow, c0 + j)] = v;
+  auto step_times = [&](int q, double& ta, double& tb) {
+    const bool act = q < steps_here;
+    const double* g = a.grid + (traj * a.max_steps + n0 + q) * 2;
+    ta = act ? g[0] : 0.0;
+    tb = act ? g[1] : 0.0;
+    return act;
   };
+  mlp_begin<P>(W, L);
 
-  // ---- 1. recompute the segment: keep every stage's f (scratch) and its layer inputs (row
-  //      buffers), so that the reverse sweep needs no forward re-evaluation ----
-  float y[CPT], fl[CPT];
+  // ---- 1. recompute the segment: keep every evaluation's f (scratch) and its layer inputs
+  //      (row buffers), so that the reverse sweep needs no forward re-evaluation ----
+  auto forward = [&](int64_t slot, const float (&z)[CPT],
+                     float (&f)[CPT]) __attribute__((always_inline)) {
+    put_cols(R.b[1], slot, z);
+    store_inputs(L, orow, c0, z);
+    __syncthreads();
+    mlp_forward_rows<NW>(W, L, wave, lane, orow, c0, f, R.b[3], R.b[5], slot);
+    float* fp = fslot(slot);
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) fp[j] = f[j];
+  };
+  float y[CPT], f[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) y[j] = (steps_here > 0) ? a.ckpt[(traj * a.n_ckpt + a.seg) * MLP_D + c0 + j] : 0.0f;
-  for (int q = 0; q < a.Cs; ++q) {
-    const bool act = q < steps_here;
-    const int n = n0 + q;
-    const double ta = act ? a.grid[(traj * a.max_steps + n) * 2 + 0] : 0.0;
-    const double tb = act ? a.grid[(traj * a.max_steps + n) * 2 + 1] : 0.0;
+  forward(slot0, y, f);
+  for (int q = 0; q < tile_steps; ++q) {
+    double ta, tb;
+    const bool act = step_times(q, ta, tb);
     const float control = (float)((double)dir * (tb - ta));
-    float k[S][CPT], z[CPT], f[CPT];
-    if (q == 0) {
-      const MlpRowSink k0 = sink_of(0, 0);
+    float k[S][CPT], z[CPT];
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) put_x(k0, j, y[j]);
-      store_inputs(L, orow, c0, y);
-      __syncthreads();
-      mlp_forward3<NW>(W, L, wave, lane, orow, c0, fl, k0);
-      __syncthreads();
-    }
-    {
-      float* fp = fslot(q, 0);
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) { fp[j] = fl[j]; k[0][j] = control * fl[j]; }
-    }
+    for (int j = 0; j < CPT; ++j) k[0][j] = control * f[j];
     static_for<1, S>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      const MlpRowSink ki = sink_of(q, i);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
         float kc[S];
 #pragma unroll
         for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : 0.0f;
         z[j] = y[j] + comb<Tab, 0, i, 0, i, false>(TL::v.a[i], kc, 0.0f);
-        put_x(ki, j, z[j]);
       }
-      store_inputs(L, orow, c0, z);
-      __syncthreads();
-      mlp_forward3<NW>(W, L, wave, lane, orow, c0, f, ki);
-      __syncthreads();
-      float* fp = fslot(q, i);
+      forward(slot_of(q, i), z, f);
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) { fp[j] = f[j]; k[i][j] = control * f[j]; }
+      for (int j = 0; j < CPT; ++j) k[i][j] = control * f[j];
     });
+    if (act) {
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      if (act) y[j] = z[j];
-      fl[j] = f[j];
+      for (int j = 0; j < CPT; ++j) y[j] = z[j];
     }
   }
 
   // ---- 2. reverse sweep ----
-  float yb[CPT];
+  // Pull the cotangent fb of an evaluation's f back to its input: delta3 = fb (1 - f^2),
+  // delta2 = (delta3 . W3) softplus'(h2), delta1 = (delta2 . W2) softplus'(h1), zb = delta1 .
+  // W1, the deltas to their row blocks.  LDS: delta3 in the x planes, delta2 in h1, delta1 in
+  // h2, then the split-K partials in h1; every buffer's last readers are behind a barrier
+  // when it is written.
+  auto pull_back = [&](int64_t slot, const float (&fb)[CPT],
+                       float (&zb)[CPT]) __attribute__((always_inline)) {
+    constexpr int KS1 = MLP_D / 16, KS2 = MLP_H / 16, HP = MLP_TILE * MlpLds<P>::LDH;
+    float4 h[NT][4];
+    auto load_h = [&](const float* rows) {  // ahead of the product it follows
 #pragma unroll
-  for (int j = 0; j < CPT; ++j) yb[j] = valid ? a.ybar[traj * MLP_D + c0 + j] : 0.0f;
-  for (int q = a.Cs - 1; q >= 0; --q) {
-    const bool act = q < steps_here;
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          h[t][i] = *reinterpret_cast<const float4*>(rows + rows_frag(slot, MLP_H, NT * wave + t, i, lane));
+      }
+    };
+    floatx16_t acc[NT];
+    auto delta = [&](int t, int i) {
+      return make_float4(acc[t][4 * i] * dsoftplus_from_value(h[t][i].x),
+                         acc[t][4 * i + 1] * dsoftplus_from_value(h[t][i].y),
+                         acc[t][4 * i + 2] * dsoftplus_from_value(h[t][i].z),
+                         acc[t][4 * i + 3] * dsoftplus_from_value(h[t][i].w));
+    };
+    Gemm3<KS1, NT, false> g3;
+    Gemm3<KS2, NT, false> g2;
+    Gemm3<KS2, NT3> g1;
+    const float* fp = fslot(slot);
+    float d3[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) d3[j] = fb[j] * (1.0f - fp[j] * fp[j]);
+    g3.preload(W.w3t, W.plane3, NT * wave, 0, lane);
+    load_h(R.b[5]);
+    __builtin_amdgcn_sched_barrier(0);
+    put_cols(R.b[4], slot, d3);
+    store_inputs(L, orow, c0, d3);
+    __syncthreads();
+    g3.template run<KS1>(L.x[0], MLP_TILE * MlpLds<P>::LDX, L.LDX, 0, acc, lane);
+    g2.preload(W.w2t, W.plane2, NT * wave, 0, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    put_rows<NW>(L, L.h1[0], R.b[2], slot, wave, lane, delta);
+    load_h(R.b[3]);
+    __syncthreads();
+    g2.template run<KS2>(L.h1[0], HP, L.LDH, 0, acc, lane);
+    const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+    g1.preload(W.w1t, W.plane1, n3, qk * (KS2 / 4), lane);
+    __builtin_amdgcn_sched_barrier(0);
+    put_rows<NW>(L, L.h2[0], R.b[0], slot, wave, lane, delta);
+    __syncthreads();
+    floatx16_t acc3[NT3];
+    g1.template run<KS2 / 4>(L.h2[0], HP, L.LDH, qk * (KS2 / 4), acc3, lane);
+    float* part = L.part();
+    put_partials<NT3>(acc3, part, L.LDP, qk, n3, lane);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int c = c0 + j;
+      float s = part[(0 * MLP_TILE + orow) * L.LDP + c];
+      s += part[(1 * MLP_TILE + orow) * L.LDP + c];
+      s += part[(2 * MLP_TILE + orow) * L.LDP + c];
+      s += part[(3 * MLP_TILE + orow) * L.LDP + c];
+      zb[j] = s;
+    }
+  };
+  // yb: cotangent of the state at the end of step q; fb: of f there, from the next step's
+  // first stage.
+  float yb[CPT], fb[CPT], zb[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; ++j) {
+    yb[j] = valid ? a.ybar[traj * MLP_D + c0 + j] : 0.0f;
+    fb[j] = 0.0f;
+  }
+  for (int q = tile_steps - 1; q >= 0; --q) {
+    double ta, tb;
+    const bool act = step_times(q, ta, tb);
     const int n = n0 + q;
-    const double ta = act ? a.grid[(traj * a.max_steps + n) * 2 + 0] : 0.0;
-    const double tb = act ? a.grid[(traj * a.max_steps + n) * 2 + 1] : 0.0;
     const float control = (float)((double)dir * (tb - ta));
     float kb[S][CPT], ybn[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
       ybn[j] = yb[j];
 #pragma unroll
-      for (int m = 0; m < S; ++m) kb[m][j] = 0.0f;
+      for (int m = 0; m < S; ++m) kb[m][j] = (act && m < S - 1) ? TL::v.a[S - 1][m] * yb[j] : 0.0f;
     }
-    if (act) {
-#pragma unroll
-      for (int m = 0; m < S - 1; ++m) {
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) kb[m][j] += TL::v.a[S - 1][m] * yb[j];
-      }
+    if (act && a.n_ts > 0) {
+      // SaveAt(ts) rows interpolated inside this step, (ta, tb] (from the start for the
+      // solve's first step): counted and weighted by the owner group, one time per owner
+      // (the weights pass through the h2 planes, idle here)
+      const int qo = lane & (GRP - 1);
       int jlo = 0, jhi = 0;
-      for (int s = 0; s < a.n_ts; ++s) {
-        const double tsn = ts_row[s] * dir;
-        if (n > 0 && tsn <= ta) jlo = s + 1;
-        if (tsn <= tb) jhi = s + 1;
+      for (int s0 = 0; s0 < a.n_ts; s0 += GRP) {
+        const double t = s0 + qo < a.n_ts ? ts_row[s0 + qo] * dir : __builtin_inf();
+        const unsigned grp = (unsigned)((1ull << GRP) - 1);
+        jlo += __builtin_popcount((unsigned)(__ballot(n > 0 && t <= ta) >> gbase) & grp);
+        jhi += __builtin_popcount((unsigned)(__ballot(t <= tb) >> gbase) & grp);
       }
-      for (int s = jlo; s < jhi; ++s) {
-        const double th = linear_rescale(ta, ts_row[s] * dir, tb);
-        double bb[7];
-        tsit5_weights(th, bb);
-        const float* g = a.ys_bar + (traj * a.n_out + (a.save_t0 ? 1 : 0) + s) * MLP_D + c0;
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-          const float gv = g[j];
-          ybn[j] += gv;
-#pragma unroll
-          for (int m = 0; m < 7; ++m) kb[m][j] += (float)bb[m] * gv;
+      float* wts = reinterpret_cast<float*>(L.h2[0]) + orow * GRP * 8;
+      for (int s0 = jlo; s0 < jhi; s0 += GRP) {
+        const int cnt = min(GRP, jhi - s0);
+        {
+          double bb[7];
+          tsit5_weights(linear_rescale(ta, ts_row[min(s0 + qo, jhi - 1)] * dir, tb), bb);
+          float4* o = reinterpret_cast<float4*>(wts + 8 * qo);
+          o[0] = make_float4((float)bb[0], (float)bb[1], (float)bb[2], (float)bb[3]);
+          o[1] = make_float4((float)bb[4], (float)bb[5], (float)bb[6], 0.0f);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const float* g = a.ys_bar + (traj * a.n_out + (a.save_t0 ? 1 : 0) + s0) * MLP_D + c0;
+        for (int e = 0; e < cnt; ++e) {
+          const float4 w0 = reinterpret_cast<const float4*>(wts)[2 * e];
+          const float4 w1 = reinterpret_cast<const float4*>(wts)[2 * e + 1];
+          const float bb[7] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z};
+#pragma unroll
+          for (int j = 0; j < CPT; ++j) {
+            const float gv = g[e * MLP_D + j];
+            ybn[j] += gv;
+#pragma unroll
+            for (int m = 0; m < 7; ++m) kb[m][j] += bb[m] * gv;
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
     }
-    static_for<0, S>([&](auto ic) {
+    // stages 6 .. 1: z_i = y_n + sum_{m<i} a_im k_m
+    static_for<0, S - 1>([&](auto ic) {
       constexpr int i = S - 1 - decltype(ic)::value;
-      const int64_t block = stage_block(q, i);
-      const float* fp = fslot(q, i);
-      // delta3 = fbar (1 - f^2), fbar = control * kbar_i: its row, and its pieces in x
-      float d3v[CPT];
+      float fbi[CPT];
+#pragma unroll
+      for (int j = 0; j < CPT; ++j)
+        fbi[j] = (act ? control * kb[i][j] : 0.0f) + (i == S - 1 ? fb[j] : 0.0f);
+      pull_back(slot_of(q, i), fbi, zb);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        const float fb = act ? control * kb[i][j] : 0.0f;
-        const float fv = fp[j];
-        const float d3 = fb * (1.0f - fv * fv);
-        R.b[4][rows_index(block, MLP_D, orow, c0 + j)] = d3;
-        d3v[j] = d3;
+        const float z = act ? zb[j] : 0.0f;
+        ybn[j] += z;
+#pragma unroll
+        for (int m = 0; m < i; ++m) kb[m][j] += TL::v.a[i][m] * z;
       }
-      store_inputs(L, orow, c0, d3v);
-      __syncthreads();
-      // delta2 = (delta3 . W3) softplus'(h2): its row, and its pieces in h1
-      floatx16_t acc[NT];
-      wave_gemm3<MLP_D / 16, NT>(L.x[0], L.x[1], L.x[2], L.LDX, W.w3t, W.plane3, NT * wave, 0,
-                                 MLP_D / 16, acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          const int64_t fr = rows_frag(block, MLP_H, NT * wave + t, i4, lane);
-          const float4 h = *reinterpret_cast<const float4*>(R.b[5] + fr);
-          const float4 dl = make_float4(acc[t][4 * i4] * dsoftplus_from_value(h.x),
-                                        acc[t][4 * i4 + 1] * dsoftplus_from_value(h.y),
-                                        acc[t][4 * i4 + 2] * dsoftplus_from_value(h.z),
-                                        acc[t][4 * i4 + 3] * dsoftplus_from_value(h.w));
-          *reinterpret_cast<float4*>(R.b[2] + fr) = dl;
-          store_col4(L.h1[0], MLP_TILE * L.LDH, L.LDH, 8 * i4 + 4 * (lane >> 5), col, dl);
-        }
-      }
-      __syncthreads();
-      // delta1 = (delta2 . W2) softplus'(h1): its row, and its pieces in h2
-      wave_gemm3<MLP_H / 16, NT>(L.h1[0], L.h1[1], L.h1[2], L.LDH, W.w2t, W.plane2, NT * wave, 0,
-                                 MLP_H / 16, acc, lane);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * (NT * wave + t) + (lane & 31);
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          const int64_t fr = rows_frag(block, MLP_H, NT * wave + t, i4, lane);
-          const float4 h = *reinterpret_cast<const float4*>(R.b[3] + fr);
-          const float4 dl = make_float4(acc[t][4 * i4] * dsoftplus_from_value(h.x),
-                                        acc[t][4 * i4 + 1] * dsoftplus_from_value(h.y),
-                                        acc[t][4 * i4 + 2] * dsoftplus_from_value(h.z),
-                                        acc[t][4 * i4 + 3] * dsoftplus_from_value(h.w));
-          *reinterpret_cast<float4*>(R.b[0] + fr) = dl;
-          store_col4(L.h2[0], MLP_TILE * L.LDH, L.LDH, 8 * i4 + 4 * (lane >> 5), col, dl);
-        }
-      }
-      __syncthreads();
-      // zbar = delta1 . W1 (split-K over the 256 hidden units); the partials take the h1
-      // planes, whose last readers (the delta1 products) are behind the barrier above
-      constexpr int KS1 = MLP_H / 16;
-      const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-      floatx16_t acc3[NT3];
-      wave_gemm3<KS1, NT3>(L.h2[0], L.h2[1], L.h2[2], L.LDH, W.w1t, W.plane1, n3,
-                           qk * (KS1 / 4), (qk + 1) * (KS1 / 4), acc3, lane);
-      float* part = L.part();
-#pragma unroll
-      for (int t = 0; t < NT3; ++t) {
-        const int col = 32 * (n3 + t) + (lane & 31);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) part[(qk * MLP_TILE + acc_row(lane, v)) * L.LDP + col] = acc3[t][v];
-      }
-      __syncthreads();
-      float zb[CPT];
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        const int c = c0 + j;
-        float sv = part[(0 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(1 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(2 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(3 * MLP_TILE + orow) * L.LDP + c];
-        zb[j] = act ? sv : 0.0f;
-      }
-#pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        ybn[j] += zb[j];
-#pragma unroll
-        for (int m = 0; m < i; ++m) kb[m][j] += TL::v.a[i][m] * zb[j];
-      }
-      __syncthreads();
     });
-    if (act) {
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) yb[j] = ybn[j];
+    for (int j = 0; j < CPT; ++j) {
+      fb[j] = act ? control * kb[0][j] : 0.0f;
+      yb[j] = act ? ybn[j] : yb[j];
     }
   }
+  pull_back(slot0, fb, zb);
   if (valid) {
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) a.ybar[traj * MLP_D + c0 + j] = yb[j];
+    for (int j = 0; j < CPT; ++j)
+      a.ybar[traj * MLP_D + c0 + j] = steps_here > 0 ? yb[j] + zb[j] : yb[j];
   }
 }
 
@@ -347,6 +361,7 @@ __host__ __device__ inline int dw_chunks(int64_t blocks) {
 // with float32 accumulation.  The next block's values load while this one's are split.
 // Waves in the first piece column of a matrix also produce the chunk's column sums of A (the
 // bias gradient partials, partial_db: [chunk][db1 | db2 | db3]).
+// evals: of every `slots` blocks (a tile) only the first evals[tile] hold rows (null: all do).
 // SC: the rows of A are multiplied by rscale[row] (the backsolve's per-row weights dt * b_i,
 // zero for rejected steps and idle rows; a row of zero weight is dropped from both operands,
 // so a non-finite value in it contributes nothing).
@@ -363,7 +378,8 @@ __host__ __device__ inline int dw_pieces_of(int m) {
 template <bool SC>
 __global__ void __launch_bounds__(64, 2)
 mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restrict__ partial_db,
-                   int64_t blocks, int nch, const float* __restrict__ rscale) {
+                   int64_t blocks, int nch, const int32_t* __restrict__ evals, int slots,
+                   const float* __restrict__ rscale) {
   const DwLayout lay = dw_layout();
   const int npc = dw_pieces_of(0) + dw_pieces_of(1) + dw_pieces_of(2);
   const int xcd = (int)(blockIdx.x % kXcds), slot = (int)(blockIdx.x / kXcds);
@@ -397,8 +413,24 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
       }
     }
   };
-  if (b0 < b1) load(b0);
-  for (int64_t blk = b0; blk < b1; ++blk) {
+  // the first block with rows at or after blk (b1: none); lim: the end of its tile's
+  int64_t lim = evals ? b0 : b1;
+  auto next = [&](int64_t blk) {
+    while (blk >= lim && blk < b1) {
+      const int64_t tile = blk / slots;
+      lim = min(tile * slots + evals[tile], b1);
+      if (blk >= lim) {
+        blk = min((tile + 1) * slots, b1);
+        lim = blk;
+      }
+    }
+    return blk;
+  };
+  int64_t nxt = next(b0);
+  if (nxt < b1) load(nxt);
+  while (nxt < b1) {
+    const int64_t blk = nxt;
+    nxt = next(blk + 1);
     if constexpr (SC) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -442,7 +474,7 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
         split(vb[x][2 * s], vb[x][2 * s + 1], fb[s][x]);
       }
     }
-    if (blk + 1 < b1) load(blk + 1);
+    if (nxt < b1) load(nxt);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -942,22 +974,22 @@ __global__ void bs_reset_kernel(int32_t* counters, float* rscale, int64_t used, 
 
 // The weight gradients of `blocks` row blocks (SC: per-row weights rscale) added to dw.
 template <bool SC>
-void launch_dw(const RowBufs& R, float* partial, int64_t blocks, const float* rscale, float* dw,
-               hipStream_t s) {
+void launch_dw(const RowBufs& R, float* partial, int64_t blocks, const int32_t* evals, int slots,
+               const float* rscale, float* dw, hipStream_t s) {
   const int nch = dw_chunks(blocks);
   const DwLayout lay = dw_layout();
   float* partial_db = partial + (int64_t)nch * lay.first[3] * 1024;
   const int groups = (nch + kXcds - 1) / kXcds;
   const int npc = dw_pieces_of(0) + dw_pieces_of(1) + dw_pieces_of(2);
   hipLaunchKernelGGL((mlp_dw_gemm_kernel<SC>), dim3(kXcds * npc * groups), dim3(64), 0, s, R,
-                     partial, partial_db, blocks, nch, rscale);
+                     partial, partial_db, blocks, nch, evals, slots, rscale);
   const int nblk = lay.first[3] * 4 + ((2 * MLP_H + MLP_D) / 4 + 63) / 64;
   hipLaunchKernelGGL(mlp_dw_reduce_kernel, dim3(nblk), dim3(256), 0, s, partial, partial_db, nch,
                      dw);
 }
 
-// Floats of the weight-gradient partials of `blocks` row blocks; behind them (float32 form)
-// come the three-piece planes of the weights.
+// Floats of the weight-gradient partials of `blocks` row blocks; behind them, for a segment,
+// come its tiles' evaluation counts and (float32 form) the three-piece planes of the weights.
 int64_t partial_floats(int64_t blocks) {
   return (dw_chunks(blocks) * ((int64_t)dw_layout().first[3] * 1024 + 2 * MLP_H + MLP_D) + 63) / 64 * 64;
 }
@@ -969,7 +1001,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
                 const float* b3, const dfx_mlp_adj_io* io, int32_t seg, int32_t seg_steps,
                 hipStream_t s) {
   using P = PolicyBF16x3;
-  constexpr int NW = 8;
+  constexpr int NW = 8;  // two waves per SIMD; four (one per SIMD) took a sixth longer
   AdjArgs a;
   memset(&a, 0, sizeof(a));
   a.grid = io->grid; a.ckpt = io->ckpt; a.stats = io->stats; a.ts = io->ts; a.ys_bar = io->ys_bar;
@@ -979,9 +1011,11 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   a.Cs = seg_steps; a.seg = seg; a.n_ts = p->n_ts; a.ts_stride = p->ts_stride;
   a.n_out = (p->save_t0 ? 1 : 0) + p->n_ts + (p->save_t1 ? 1 : 0);
   a.save_t0 = p->save_t0; a.t0 = p->t0; a.t1 = p->t1;
-  const int64_t blocks = seg_rows(p->batch, seg_steps) / MLP_TILE;
+  const int slots = 1 + 6 * seg_steps;
+  const int64_t ntiles64 = a.B_pad / MLP_TILE, blocks = ntiles64 * slots;
+  a.evals = reinterpret_cast<int32_t*>(io->partial + partial_floats(blocks));
   if (p->precision == DFX_F32) {
-    __bf16* planes = reinterpret_cast<__bf16*>(io->partial + partial_floats(blocks));
+    __bf16* planes = reinterpret_cast<__bf16*>(a.evals + (ntiles64 + 63) / 64 * 64);
     const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);
     hipLaunchKernelGGL(mlp_split_packed_kernel, dim3(nb), dim3(256), 0, s,
                        reinterpret_cast<const float*>(packed), planes);
@@ -994,12 +1028,12 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   int64_t off = 0;
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) { R.b[i] = base + off; off += rows_alloc * widths[i]; }
-  const unsigned ntiles = (unsigned)(a.B_pad / MLP_TILE);
+  const unsigned ntiles = (unsigned)ntiles64;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_adj_segment_kernel<NW>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLds<P>));
   hipLaunchKernelGGL(mlp_adj_segment_kernel<NW>, dim3(ntiles), dim3(64 * NW), sizeof(MlpLds<P>), s,
                      a, W, R);
-  launch_dw<false>(R, io->partial, blocks, nullptr, io->dw, s);
+  launch_dw<false>(R, io->partial, blocks, a.evals, slots, nullptr, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -1017,7 +1051,9 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) wsum += widths[i];
   *rows_bytes = (size_t)(rows_alloc * wsum) * sizeof(float);   // float32 rows for both forms
-  *partial_bytes = (size_t)partial_floats(seg_rows(p->batch, seg_steps) / MLP_TILE) * sizeof(float);
+  const int64_t ntiles = Bp / MLP_TILE;
+  *partial_bytes = (size_t)(partial_floats(ntiles * (1 + 6 * seg_steps)) + (ntiles + 63) / 64 * 64) *
+                   sizeof(float);
   if (p->precision == DFX_F32) *partial_bytes += (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
 }
@@ -1086,8 +1122,8 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLdsBack));
   hipLaunchKernelGGL((mlp_backsolve_kernel<NWB>), dim3(ntiles), dim3(64 * NWB),
                      sizeof(MlpLdsBack), s, a, W, R);
-  launch_dw<true>(R, io->partial, seg_rows(back->batch, chunk_iters) / MLP_TILE, a.rscale, io->dw,
-                  s);
+  launch_dw<true>(R, io->partial, seg_rows(back->batch, chunk_iters) / MLP_TILE, nullptr, 0,
+                  a.rscale, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -1117,9 +1153,6 @@ int dfx_mlp_adj_segment(const dfx_mlp_problem* p, const void* packed, const floa
   if (p->ts_stride != 0 && p->ts_stride != p->n_ts) return DFX_E_ARG;
   if (p->batch == 0) return DFX_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // eight waves per tile, two per SIMD: at four the kernel held 512 registers per lane, 93
-  // spilled, one wave per SIMD, and the backward of 8,192 trajectories took 2.51-2.55 ms
-  // against 2.16-2.17 (bit-identical gradients).
   return run_segment(p, packed, b1, b2, b3, io, segment, seg_steps, s);
 }
 

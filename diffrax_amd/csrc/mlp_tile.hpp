@@ -357,89 +357,30 @@ __device__ __forceinline__ void mlp_begin(const MlpWeights<P>& W, MlpLds<P>& L) 
     L.bias[i] = i < MLP_H ? W.b1[i] : (i < 2 * MLP_H ? W.b2[i - MLP_H] : W.b3[i - 2 * MLP_H]);
 }
 
-// acc[nt] (32x32 f32) = sum over k-steps [ks0, ks1) of A . B with A and B three-piece
-// operands: A from LDS planes a0..a2, B fragment (nt0 + nt, ks) from planes wp + p * plane.
-// The leading products a0 b0 accumulate in `big`, the five corrections (a0 b1, a1 b0, a0 b2,
-// a1 b1, a2 b0) in `sml`, added at the end.  B fragments are loaded PF k-steps ahead.
-template <int NKS, int NT, int PF = 1>
-__device__ __forceinline__ void wave_gemm3(const __bf16* a0, const __bf16* a1, const __bf16* a2,
-                                           int lda, const __bf16* wp, int64_t plane, int nt0,
-                                           int ks0, int ks1, floatx16_t (&acc)[NT], int lane) {
-  using P = PolicyBF16x3;
-  using frag_t = P::frag_t;
-  const int row = lane & 31;
-  const int kh = (lane >> 5) * P::KA;
-  floatx16_t big[NT], sml[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) { big[t] = floatx16_t{}; sml[t] = floatx16_t{}; }
-  auto bfrag = [&](int pc, int t, int k) {
-    return P::load_b(wp + pc * plane, ((nt0 + t) * NKS + k) * 64 + lane);
-  };
-  frag_t buf[PF][3][NT];
-#pragma unroll
-  for (int p = 0; p < PF; ++p) {
-    const int kp = (ks0 + p < ks1) ? ks0 + p : ks1 - 1;
-#pragma unroll
-    for (int pc = 0; pc < 3; ++pc) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) buf[p][pc][t] = bfrag(pc, t, kp);
-    }
-  }
-  // one PF-step group per iteration: a fully unrolled K loop (seven inlined evaluations per
-  // step) lets the scheduler hoist loads until the registers spill
-#pragma unroll 1
-  for (int ks = ks0; ks < ks1; ks += PF) {
-#pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int k = ks + p;
-      if (k < ks1) {
-        frag_t b[3][NT];
-#pragma unroll
-        for (int pc = 0; pc < 3; ++pc) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) b[pc][t] = buf[p][pc][t];
-        }
-        if (k + PF < ks1) {
-#pragma unroll
-          for (int pc = 0; pc < 3; ++pc) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) buf[p][pc][t] = bfrag(pc, t, k + PF);
-          }
-        }
-        const int ao = row * lda + k * P::KSTEP + kh;
-        const frag_t x0 = P::load_a(a0 + ao), x1 = P::load_a(a1 + ao), x2 = P::load_a(a2 + ao);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) big[t] = P::mfma(x0, b[0][t], big[t]);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          sml[t] = P::mfma(x0, b[1][t], sml[t]);
-          sml[t] = P::mfma(x1, b[0][t], sml[t]);
-          sml[t] = P::mfma(x0, b[2][t], sml[t]);
-          sml[t] = P::mfma(x1, b[1][t], sml[t]);
-          sml[t] = P::mfma(x2, b[0][t], sml[t]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = big[t] + sml[t];
-}
-
-// wave_gemm3 with the weights as the A operand (a lane's accumulators are four runs of four
-// consecutive outputs of one trajectory) and the ring of GemmF32: PF k steps of weights in
-// flight, the first loaded ahead of the barrier that the activations wait for.  The same
-// products in the same order, so the same bits.  One evaluation of a 32-trajectory tile by
-// eight waves takes 23,000 cycles, 9,200 of them MFMA on every SIMD and 6,700 VALU (softplus
-// and the splits, between the barriers, so that little of it overlaps); with wave_gemm3's
-// copied ring, 2-byte LDS stores and a split per value it took 26,400 and 10,100 VALU
-// (8,192 trajectories: 0.33-0.35 against 0.30 ms; 33: 0.266 against 0.234).
-template <int NKS, int NT, int PF = 2>
+// The three-piece product of one wave: acc[t] (32x32 f32) = sum over k steps of W . x, both
+// operands in three pieces: the activation rows from LDS planes, the weights of output tile
+// nt0 + t from L2.  The leading products w0 x0 accumulate in acc, the five corrections (w1
+// x0, w0 x1, w2 x0, w1 x1, w0 x2) apart, added at the end.
+// WA: the weights are the A operand, so that a lane's accumulators are four runs of four
+// consecutive outputs of one trajectory; else the activations are, and the runs are four
+// consecutive trajectories of one output.  Either way the same bits.
+// PF k steps of weights are in flight, the first loaded by preload() ahead of the barrier
+// that the activations wait for; a ring slot is refilled right after its MFMAs, and the
+// loads are pinned there.  One evaluation of a 32-trajectory tile by eight waves takes 23,000
+// cycles, 9,200 of them MFMA on every SIMD and 6,700 VALU (softplus and the splits, between
+// the barriers, so that little of it overlaps); with a ring that was copied (and so waited
+// for), 2-byte LDS stores and a split per value it took 26,400 and 10,100 VALU (8,192
+// trajectories: 0.33-0.35 against 0.30 ms; 33: 0.266 against 0.234).
+template <int NKS, int NT, bool WA = true, int PF = 2>
 struct Gemm3 {
   using P = PolicyBF16x3;
   using frag_t = P::frag_t;
   frag_t b[PF][3][NT];
   const frag_t* wp;
   int plane;
+  __device__ __forceinline__ static floatx16_t mm(frag_t w, frag_t x, floatx16_t c) {
+    return WA ? P::mfma(w, x, c) : P::mfma(x, w, c);
+  }
   __device__ __forceinline__ void load(int p, int k) {
 #pragma unroll
     for (int pc = 0; pc < 3; ++pc) {
@@ -474,12 +415,12 @@ struct Gemm3 {
         const int q = p & 1;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          acc[t] = P::mfma(b[p][0][t], x[q][0], acc[t]);
-          sml[t] = P::mfma(b[p][1][t], x[q][0], sml[t]);
-          sml[t] = P::mfma(b[p][0][t], x[q][1], sml[t]);
-          sml[t] = P::mfma(b[p][2][t], x[q][0], sml[t]);
-          sml[t] = P::mfma(b[p][1][t], x[q][1], sml[t]);
-          sml[t] = P::mfma(b[p][0][t], x[q][2], sml[t]);
+          acc[t] = mm(b[p][0][t], x[q][0], acc[t]);
+          sml[t] = mm(b[p][1][t], x[q][0], sml[t]);
+          sml[t] = mm(b[p][0][t], x[q][1], sml[t]);
+          sml[t] = mm(b[p][2][t], x[q][0], sml[t]);
+          sml[t] = mm(b[p][1][t], x[q][1], sml[t]);
+          sml[t] = mm(b[p][0][t], x[q][2], sml[t]);
         }
         if (!decltype(last)::value) load(p, g + p + PF);
         if (!decltype(last)::value || p + 2 < PF) load_x(q, g + p + 2);
@@ -505,18 +446,6 @@ __host__ __device__ inline int64_t rows_frag(int64_t block, int width, int t, in
 __host__ __device__ inline int64_t rows_index(int64_t block, int width, int row, int col) {
   return rows_frag(block, width, col / 32, row / 8, col % 32 + 32 * (row % 8 / 4)) + row % 4;
 }
-
-// Where the hidden activations of an evaluation go in the row buffers (block, and again at
-// block2 when that is not negative).
-struct MlpRowSink {
-  float* h1 = nullptr;
-  float* h2 = nullptr;
-  int64_t block = 0, block2 = -1;
-  __device__ __forceinline__ void put(float* dst, int t, int i, int lane, float4 v) const {
-    *reinterpret_cast<float4*>(dst + rows_frag(block, MLP_H, t, i, lane)) = v;
-    if (block2 >= 0) *reinterpret_cast<float4*>(dst + rows_frag(block2, MLP_H, t, i, lane)) = v;
-  }
-};
 
 // Store four rows r .. r + 3 of one column in the three planes of an LDS buffer.
 __device__ __forceinline__ void store_col4(__bf16* buf, int plane, int ld, int r, int col,
@@ -546,73 +475,6 @@ struct MlpWaves {
   __device__ static int quarter(int wave) { return NW == 4 ? wave : (wave >> 1); }
 };
 
-template <int NW = 4>
-__device__ __forceinline__ void mlp_forward3(const MlpWeights<PolicyBF16x3>& W,
-                                             MlpLds<PolicyBF16x3>& L, int wave, int lane,
-                                             int owner_row, int owner_c0,
-                                             float (&fout)[MlpWaves<NW>::CPT],
-                                             const MlpRowSink& sink) {
-  using WV = MlpWaves<NW>;
-  constexpr int NT = WV::NT12;
-  constexpr int KS1 = MLP_D / 16, KS2 = MLP_H / 16;
-  floatx16_t acc[NT];
-  // layer 1: [32 x 64] . W1^T -> [32 x 256], wave's columns [64w, 64w + 64)
-  wave_gemm3<KS1, NT>(L.x[0], L.x[1], L.x[2], L.LDX, W.w1, W.plane1, NT * wave, 0, KS1, acc, lane);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = 32 * (NT * wave + t) + (lane & 31);
-    const float bias = W.b1[col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 h = make_float4(softplus_f(acc[t][4 * i] + bias), softplus_f(acc[t][4 * i + 1] + bias),
-                                   softplus_f(acc[t][4 * i + 2] + bias), softplus_f(acc[t][4 * i + 3] + bias));
-      sink.put(sink.h1, NT * wave + t, i, lane, h);
-      store_col4(L.h1[0], MLP_TILE * L.LDH, L.LDH, 8 * i + 4 * (lane >> 5), col, h);
-    }
-  }
-  __syncthreads();
-  // layer 2: [32 x 256] . W2^T -> [32 x 256]
-  wave_gemm3<KS2, NT>(L.h1[0], L.h1[1], L.h1[2], L.LDH, W.w2, W.plane2, NT * wave, 0, KS2, acc,
-                      lane);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = 32 * (NT * wave + t) + (lane & 31);
-    const float bias = W.b2[col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 h = make_float4(softplus_f(acc[t][4 * i] + bias), softplus_f(acc[t][4 * i + 1] + bias),
-                                   softplus_f(acc[t][4 * i + 2] + bias), softplus_f(acc[t][4 * i + 3] + bias));
-      sink.put(sink.h2, NT * wave + t, i, lane, h);
-      store_col4(L.h2[0], MLP_TILE * L.LDH, L.LDH, 8 * i + 4 * (lane >> 5), col, h);
-    }
-  }
-  __syncthreads();
-  // layer 3 (split-K): wave w sums K in [64w, 64w + 64) for all 64 outputs; the partials go
-  // to the h1 planes (layer 2, their last reader, finished before the barrier above)
-  constexpr int NT3 = WV::NT3;
-  const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-  floatx16_t acc3[NT3];
-  wave_gemm3<KS2, NT3>(L.h2[0], L.h2[1], L.h2[2], L.LDH, W.w3, W.plane3, n3, qk * (KS2 / 4),
-                       (qk + 1) * (KS2 / 4), acc3, lane);
-  float* part = L.part();
-#pragma unroll
-  for (int t = 0; t < NT3; ++t) {
-    const int col = 32 * (n3 + t) + (lane & 31);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) part[(qk * MLP_TILE + acc_row(lane, v)) * L.LDP + col] = acc3[t][v];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < WV::CPT; ++j) {
-    const int c = owner_c0 + j;
-    float s = part[(0 * MLP_TILE + owner_row) * L.LDP + c];
-    s += part[(1 * MLP_TILE + owner_row) * L.LDP + c];
-    s += part[(2 * MLP_TILE + owner_row) * L.LDP + c];
-    s += part[(3 * MLP_TILE + owner_row) * L.LDP + c];
-    fout[j] = tanh_f(s + W.b3[c]);
-  }
-}
-
 // Layer 3's split-K partials (accumulators with the outputs along a lane's runs), which take
 // the h1 buffer (layer 2, its last reader, is behind a barrier), and the output from them.
 template <int NT3>
@@ -639,6 +501,66 @@ __device__ __forceinline__ void sum_partials(const float* part, int ldp, const f
     s += part[(3 * MLP_TILE + owner_row) * ldp + c];
     fout[j] = tanh_f(s + b3[c]);
   }
+}
+
+// A row-buffered layer's values (unsplit accumulator runs: four trajectories of one output):
+// to the block's pieces in `rows`, and split to the three planes of `buf`.
+template <int NW, class F>
+__device__ __forceinline__ void put_rows(MlpLds<PolicyBF16x3>& L, __bf16* buf, float* rows,
+                                         int64_t block, int wave, int lane, F&& value) {
+  constexpr int NT = MlpWaves<NW>::NT12;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tn = NT * wave + t;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 v = value(t, i);
+      *reinterpret_cast<float4*>(rows + rows_frag(block, MLP_H, tn, i, lane)) = v;
+      store_col4(buf, MLP_TILE * L.LDH, L.LDH, 8 * i + 4 * (lane >> 5), 32 * tn + (lane & 31), v);
+    }
+  }
+}
+
+// The forward of the three-piece form with its hidden activations kept in row buffers as well
+// (the adjoint's recompute): mlp_forward's bits.
+template <int NW>
+__device__ __forceinline__ void mlp_forward_rows(const MlpWeights<PolicyBF16x3>& W,
+                                                 MlpLds<PolicyBF16x3>& L, int wave, int lane,
+                                                 int owner_row, int owner_c0,
+                                                 float (&fout)[MlpWaves<NW>::CPT], float* h1_rows,
+                                                 float* h2_rows, int64_t block) {
+  using WV = MlpWaves<NW>;
+  using LD = MlpLds<PolicyBF16x3>;
+  constexpr int NT = WV::NT12, NT3 = WV::NT3, KS1 = MLP_D / 16, KS2 = MLP_H / 16;
+  constexpr int HP = MLP_TILE * LD::LDH;
+  floatx16_t acc[NT];
+  auto hidden = [&](const float* bias) {
+    return [&, bias](int t, int i) {
+      const float b = bias[32 * (NT * wave + t) + (lane & 31)];
+      return make_float4(softplus_f(acc[t][4 * i] + b), softplus_f(acc[t][4 * i + 1] + b),
+                         softplus_f(acc[t][4 * i + 2] + b), softplus_f(acc[t][4 * i + 3] + b));
+    };
+  };
+  Gemm3<KS1, NT, false> g1;
+  Gemm3<KS2, NT, false> g2;
+  Gemm3<KS2, NT3> g3;
+  g1.preload(W.w1, W.plane1, NT * wave, 0, lane);
+  g1.template run<KS1>(L.x[0], MLP_TILE * LD::LDX, L.LDX, 0, acc, lane);
+  g2.preload(W.w2, W.plane2, NT * wave, 0, lane);
+  __builtin_amdgcn_sched_barrier(0);  // issued here, ahead of the epilogue
+  put_rows<NW>(L, L.h1[0], h1_rows, block, wave, lane, hidden(L.bias));
+  __syncthreads();
+  g2.template run<KS2>(L.h1[0], HP, L.LDH, 0, acc, lane);
+  const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+  g3.preload(W.w3, W.plane3, n3, qk * (KS2 / 4), lane);
+  __builtin_amdgcn_sched_barrier(0);
+  put_rows<NW>(L, L.h2[0], h2_rows, block, wave, lane, hidden(L.bias + MLP_H));
+  __syncthreads();
+  floatx16_t acc3[NT3];
+  g3.template run<KS2 / 4>(L.h2[0], HP, L.LDH, qk * (KS2 / 4), acc3, lane);
+  put_partials<NT3>(acc3, L.part(), L.LDP, qk, n3, lane);
+  __syncthreads();
+  sum_partials<WV::CPT>(L.part(), L.LDP, L.bias + 2 * MLP_H, owner_row, owner_c0, fout);
 }
 
 // Forward of the MLP on the tile: reads L.x (stage values), leaves softplus activations in
