@@ -139,7 +139,7 @@ class ErkPlan:
         for name in ("y0", "t1", "ts", "params", "ys", "ts_out", "stats", "result", "grid",
                      "dense_ts", "dense_ys", "dense_k", "step_ts", "jump_ts",
                      "event_coeffs", "event_flags", "event_mask", "grid_y", "rtol", "atol",
-                     "ckpt", "state_in", "state_out"):
+                     "ckpt", "state_in", "state_out", "tape", "tape_y"):
             v = self.t.get(name)
             setattr(self.io, name, v.data_ptr() if v is not None else None)
 
@@ -158,8 +158,9 @@ class ErkPlan:
         """Store the lane state every K accepted steps, the restart points of the discrete
         adjoint: K = ceil(max_steps / checkpoints), checkpoints = ceil(sqrt(max_steps)) when
         None (RecursiveCheckpointAdjoint.checkpoints, _adjoint.py:264-329).  Memory is
-        [B, ceil(max_steps / K), d + 8] float64 here and [B, K] records of (2 + d) values in
-        the adjoint's workspace."""
+        [B, ceil(max_steps / K), d + 8] float64 and a tape of up to 8K attempted steps
+        (``_tape_steps``) here, and [B, 2K] records of (2 + d) values in the adjoint's
+        workspace."""
         M = max(int(self.problem.max_steps), 1)
         c = int(math.ceil(math.sqrt(M))) if checkpoints is None else int(checkpoints)
         if c < 1:
@@ -169,10 +170,48 @@ class ErkPlan:
         lib = _lib.load()
         _lib.check(lib.dfx_erk_ckpt_layout(ctypes.byref(self.problem), ctypes.byref(n_ck),
                                            ctypes.byref(words)), "dfx_erk_ckpt_layout")
-        B = self.t["y0"].shape[0]
+        y0 = self.t["y0"]
+        B, d = y0.shape
         self.t["ckpt"] = torch.empty((B, n_ck.value, words.value), dtype=torch.float64,
-                                     device=self.t["y0"].device)
+                                     device=y0.device)
+        n = self._tape_steps(M)
+        self.problem.tape_steps = n
+        W = -(-B // 64)
+        self.t["tape"] = (torch.empty((W, n, 64, 2), dtype=torch.float64, device=y0.device)
+                          if n else None)
+        self.t["tape_y"] = (torch.empty((W, n, 64, d), dtype=y0.dtype, device=y0.device)
+                            if n else None)
         self._bind()
+
+    # The tape: what a sweep needs of an attempted step (16 + d * itemsize bytes).  A solve
+    # that fits on it is swept without replaying its steps; a longer one replays from the
+    # checkpoints.  8K steps keep the memory at O(B sqrt(max_steps)) by default.
+    TAPE_BYTES = 4 << 30          # of one solve
+    TAPE_SMALL_BYTES = 64 << 20   # below this, taken without asking the driver
+
+    def _tape_steps(self, max_steps):
+        """Records per instance: min(max_steps, 8K) within TAPE_BYTES, or 0 where that is
+        less than two segments or would leave under 3/4 of the device's memory free (the
+        tape is a convenience: a program near the card's memory runs as without it)."""
+        y0 = self.t["y0"]
+        B, d = y0.shape
+        if self.problem.n_step_ts or self.problem.n_jump_ts:
+            return 0      # clipped solves replay
+        B = -(-B // 64) * 64
+        K = int(self.problem.ckpt_every)
+        rec = 16 + d * y0.element_size()
+        n = min(max_steps, 8 * K, self.TAPE_BYTES // max(B * rec, 1))
+        if n < min(max_steps, 2 * K):
+            return 0
+        if B * n * rec > self.TAPE_SMALL_BYTES:
+            if torch.cuda.is_current_stream_capturing():
+                return 0
+            free, total = torch.cuda.mem_get_info(y0.device)
+            free += (torch.cuda.memory_reserved(y0.device)
+                     - torch.cuda.memory_allocated(y0.device))
+            if free - B * n * rec < total * 3 // 4:
+                return 0
+        return n
 
     def adjoint(self, ys_bar, y0_bar, params_bar, workspace=None, stream=None):
         """dfx_erk_adjoint over this plan's checkpoints (after launch()): cotangents of

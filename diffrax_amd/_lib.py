@@ -40,6 +40,7 @@ class ErkProblem(ctypes.Structure):
         ("n_step_ts", ctypes.c_int32), ("n_jump_ts", ctypes.c_int32),
         ("n_events", ctypes.c_int32), ("event_root_find", ctypes.c_int32),
         ("ckpt_every", ctypes.c_int32), ("resume", ctypes.c_int32),
+        ("tape_steps", ctypes.c_int32),
     ]
 
 
@@ -54,6 +55,7 @@ class ErkIO(ctypes.Structure):
         ("event_mask", ctypes.c_void_p), ("grid_y", ctypes.c_void_p),
         ("rtol", ctypes.c_void_p), ("atol", ctypes.c_void_p), ("ckpt", ctypes.c_void_p),
         ("state_in", ctypes.c_void_p), ("state_out", ctypes.c_void_p),
+        ("tape", ctypes.c_void_p), ("tape_y", ctypes.c_void_p),
     ]
 
 

@@ -107,7 +107,8 @@ int fill_erk_inputs(const dfx_erk_problem* p, const dfx_erk_io* io, ErkKArgs& a)
   if (p->batch < 0 || p->n_ts < 0 || p->max_steps < 0 || p->save_steps < 0) return DFX_E_ARG;
   if (p->t1_stride < 0 || p->ts_stride < 0 || p->param_stride < 0) return DFX_E_ARG;
   if (p->controller == DFX_CONSTANT && isnan(p->dt0)) return DFX_E_ARG;
-  if (p->ckpt_every < 0) return DFX_E_ARG;
+  if (p->ckpt_every < 0 || p->tape_steps < 0) return DFX_E_ARG;
+  if (p->tape_steps > 0 && p->ckpt_every == 0) return DFX_E_ARG;
   if (p->n_step_ts < 0 || p->n_jump_ts < 0) return DFX_E_ARG;
   if ((p->n_step_ts > 0 || p->n_jump_ts > 0) && p->controller != DFX_PID) return DFX_E_ARG;
   if (p->n_events < 0 || p->n_events > kMaxEvents) return DFX_E_ARG;
@@ -272,6 +273,12 @@ int dfx_erk_solve(const dfx_erk_problem* p, const dfx_erk_io* io, void* workspac
     a.ckpt = io->ckpt;
     a.ckpt_every = p->ckpt_every;
     a.n_ckpt = ckpt_count(p);
+    if (p->tape_steps > 0) {
+      if (!io->tape || !io->tape_y) return DFX_E_ARG;
+      a.tape = io->tape;
+      a.tape_y = io->tape_y;
+      a.tape_steps = p->tape_steps;
+    }
   }
   a.counter = reinterpret_cast<unsigned int*>(workspace);
   if (p->resume != 0) {
@@ -376,6 +383,15 @@ int dfx_erk_adjoint(const dfx_erk_problem* p, const dfx_erk_io* fwd,
   b.ys_bar = io->ys_bar;
   b.y0_bar = io->y0_bar;
   b.q_bar = io->params_bar;
+  b.tape = nullptr;
+  b.tape_y = nullptr;
+  b.tape_steps = 0;
+  if (p->tape_steps > 0) {
+    if (!fwd->tape || !fwd->tape_y) return DFX_E_ARG;
+    b.tape = fwd->tape;
+    b.tape_y = fwd->tape_y;
+    b.tape_steps = p->tape_steps;
+  }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->precision == DFX_F64) return erk_adjoint_f64(p->solver, p->vf, p->d, a, ra, b, s);
   return erk_adjoint_f32(p->solver, p->vf, p->d, a, ra, b, s);

@@ -13,6 +13,14 @@
 // constants of the gradient (pid.py:374, 498-530) and rejected steps contribute nothing,
 // so only the accepted steps enter the sweep.
 //
+// With a tape (ErkKArgs::tape, 8K attempts by default) the forward also records what the
+// sweep reads, and a workgroup whose solves fit on it replays nothing: the same records,
+// so the same bits.  The replay, its rejected steps and controller included, was the larger
+// half of this kernel: 65,536 Van der Pol solves with 64 saves (879 attempts at most)
+// 2.35 -> 1.10 ms, for 0.09 ms of stores in the forward; 64 solves 1.23 -> 0.90 ms.  What
+// is left is bound by instruction issue: one wave per SIMD, about 300 instructions per
+// attempt and 110 per save of the lane with the most.
+//
 // Per accepted step, newest first (one lane per instance):
 //   - its stages are recomputed from the recorded start state, exactly as the forward
 //     computes them (z_i = y0 + sum_l a_il k_l, k_i = control * f(z_i));
@@ -34,6 +42,9 @@ struct DiscreteAdjArgs {
   const void* ys_bar;     // [B, n_out, D] cotangents of the saved rows
   void* y0_bar;           // out [B, D]
   void* q_bar;            // out [B, P] per instance
+  const double* tape;     // the forward's record of its first tape_steps attempted steps
+  const void* tape_y;     // (ErkKArgs::tape; none: tape_steps = 0)
+  int32_t tape_steps;
 };
 
 // Transpose of erk_interp: for out = interp(y0, y1, k, t) and cotangent g, adds the
@@ -94,21 +105,22 @@ struct AdjSweep {
   TabRegs<Tab> tr;
   T q[P], gq[P];
   int64_t id;
-  int dir, n, c_last, ksave;
+  int dir, n, ksave;
   double T0, T1;
   const T* g;
   const double* tsr;
   T ab[D];    // cotangent of the state at the end of the step being processed
-  T grow[D];  // cotangent of save row r, loaded one row ahead
+  // Cotangent of save row r and time of save ti, and those one before (grow2, tsv2), loaded a
+  // save ahead: the loop over a step's saves tests the next time at once, and a load issued
+  // there made every save wait on memory (65,536 solves with 64 saves: 0.56 of 1.26 ms).
+  T grow[D], grow2[D];
   int r, ti;
-  double tsv;
+  double tsv, tsv2;
 
-  __device__ void setup(const ErkKArgs& a, const DiscreteAdjArgs& b, int64_t id_, int n_,
-                        int K) {
+  __device__ void setup(const ErkKArgs& a, const DiscreteAdjArgs& b, int64_t id_, int n_) {
     tr.load();
     id = id_;
     n = n_;
-    c_last = n > 0 ? (n - 1) / K : -1;
     ksave = a.save_steps;
     const T* qp = reinterpret_cast<const T*>(a.params) + id * a.param_stride;
 #pragma unroll
@@ -120,10 +132,10 @@ struct AdjSweep {
     g = reinterpret_cast<const T*>(b.ys_bar) + id * (int64_t)a.n_out * D;
     tsr = a.ts ? a.ts + id * a.ts_stride : nullptr;
 #pragma unroll
-    for (int j = 0; j < D; ++j) { ab[j] = T(0); grow[j] = T(0); }
+    for (int j = 0; j < D; ++j) { ab[j] = T(0); grow[j] = grow2[j] = T(0); }
     r = -1;
     ti = -1;
-    tsv = -__builtin_inf();
+    tsv = tsv2 = -__builtin_inf();
     if (n == 0) setup_rows(a, -__builtin_inf());
   }
 
@@ -143,20 +155,31 @@ struct AdjSweep {
     }
     r -= 1;           // the last row a step wrote
     ti = (T0 == T1) ? -1 : n_saved - 1;  // the last ts index saved
-    if (r >= 0) {
-#pragma unroll
-      for (int j = 0; j < D; ++j) grow[j] = g[(int64_t)r * D + j];
-    }
+    load_row(r, grow);
+    load_row(r - 1, grow2);
     tsv = (ti >= 0) ? tsr[ti] * dir : -__builtin_inf();
+    tsv2 = (ti >= 1) ? tsr[ti - 1] : -__builtin_inf();
   }
 
-  // Accepted steps [c K, min((c + 1) K, n)) of segment c, newest first, from their records
-  // sg (t_start, t_end) and sy (start state); tl is the end of the step before the segment.
-  __device__ void segment(const ErkKArgs& a, int c, int K, const double* sg, const T* sy,
+  __device__ __forceinline__ void load_row(int row, T (&v)[D]) const {
+    if (row >= 0) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) v[j] = g[(int64_t)row * D + j];
+    }
+  }
+  // To the row before: the one loaded ahead, and the load of the one before that.
+  __device__ __forceinline__ void next_row() {
+    --r;
+#pragma unroll
+    for (int j = 0; j < D; ++j) grow[j] = grow2[j];
+    load_row(r - 1, grow2);
+  }
+
+  // Accepted steps [lo, hi), newest first, from their records sg (t_start, t_end) and sy
+  // (start state); tl is the end of the step before lo.
+  __device__ void segment(const ErkKArgs& a, int lo, int hi, const double* sg, const T* sy,
                           double tl) {
-    const int lo = c * K;
-    const int hi = min(lo + K, n);
-    if (c == c_last) setup_rows(a, sg[(int64_t)(hi - 1 - lo) * 2 + 1]);
+    if (hi == n) setup_rows(a, sg[(int64_t)(hi - 1 - lo) * 2 + 1]);
     // The records are read one step ahead: a lane walks them serially, so a load issued
     // where it is used would expose its full latency once per step.
     double nts0 = sg[(int64_t)(hi - 1 - lo) * 2];
@@ -167,7 +190,7 @@ struct AdjSweep {
     for (int s = hi - 1; s >= lo; --s) {
       const int i = s - lo;
       const double ts0 = nts0, ts1 = nts1;
-      T y0[D], zs[S][D], k[S][D];
+      T y0[D];
 #pragma unroll
       for (int j = 0; j < D; ++j) y0[j] = ny0[j];
       if (i > 0) {
@@ -176,85 +199,127 @@ struct AdjSweep {
 #pragma unroll
         for (int j = 0; j < D; ++j) ny0[j] = sy[(int64_t)(i - 1) * D + j];
       }
-      const double prev_end = i > 0 ? nts1 : tl;  // end of the previous accepted step
-      const double dt = ts1 - ts0;
-      const T control = T((double)dir * dt);
-      // the step's stages, as the forward computes them
-      static_for<0, S>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-          T kc[S];
-#pragma unroll
-          for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : T(0);
-          zs[i][j] = y0[j] + comb<Tab, 0, i, 0, i, false>(tr.a[i], kc, T(0));
-        }
-        constexpr double ci = Tab::c[i];
-        const double tsi = (ci == 1.0) ? ts1 : ts0 + ci * dt;
-        T f[D];
-        VF::eval(tsi * dir, zs[i], q, f);
-#pragma unroll
-        for (int j = 0; j < D; ++j) k[i][j] = control * f[j];
-      });
-      T gy1[D], gy0[D], gk[S][D];
+      step(a, s, ts0, ts1, y0, i > 0 ? nts1 : tl);
+    }
+  }
+
+  // Transposes accepted step s of the instance: from (ts0, ts1, y0), with the save rows in
+  // (prev_end, ts1]; prev_end is the end of step s - 1 (-inf for the first).
+  __device__ __forceinline__ void step(const ErkKArgs& a, int s, double ts0, double ts1,
+                                       const T (&y0)[D], double prev_end) {
+    T zs[S][D], k[S][D];
+    const double dt = ts1 - ts0;
+    const T control = T((double)dir * dt);
+    // the step's stages, as the forward computes them
+    static_for<0, S>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
 #pragma unroll
       for (int j = 0; j < D; ++j) {
-        gy1[j] = ab[j];
-        gy0[j] = T(0);
+        T kc[S];
 #pragma unroll
-        for (int m = 0; m < S; ++m) gk[m][j] = T(0);
+        for (int m = 0; m < S; ++m) kc[m] = (m < i) ? k[m][j] : T(0);
+        zs[i][j] = y0[j] + comb<Tab, 0, i, 0, i, false>(tr.a[i], kc, T(0));
       }
-      if (ksave > 0 && (s + 1) % ksave == 0) {  // the step's end state (SaveAt(steps=k))
+      constexpr double ci = Tab::c[i];
+      const double tsi = (ci == 1.0) ? ts1 : ts0 + ci * dt;
+      T f[D];
+      VF::eval(tsi * dir, zs[i], q, f);
 #pragma unroll
-        for (int j = 0; j < D; ++j) gy1[j] = gy1[j] + grow[j];
-        --r;
-        if (r >= 0) {
+      for (int j = 0; j < D; ++j) k[i][j] = control * f[j];
+    });
+    T gy1[D], gy0[D], gk[S][D];
 #pragma unroll
-          for (int j = 0; j < D; ++j) grow[j] = g[(int64_t)r * D + j];
-        }
+    for (int j = 0; j < D; ++j) {
+      gy1[j] = ab[j];
+      gy0[j] = T(0);
+#pragma unroll
+      for (int m = 0; m < S; ++m) gk[m][j] = T(0);
+    }
+    if (ksave > 0 && (s + 1) % ksave == 0) {  // the step's end state (SaveAt(steps=k))
+#pragma unroll
+      for (int j = 0; j < D; ++j) gy1[j] = gy1[j] + grow[j];
+      next_row();
+    }
+    // SaveAt(ts) rows inside this step: t in (end of the previous step, ts1]
+    while (ti >= 0 && tsv > prev_end) {
+      erk_interp_vjp<Tab, T, D>(ts0, ts1, tsv, grow, gy0, gy1, gk);
+      --ti;
+      tsv = (ti >= 0) ? tsv2 * dir : -__builtin_inf();
+      tsv2 = (ti >= 1) ? tsr[ti - 1] : -__builtin_inf();
+      next_row();
+    }
+    // y1 = y0 + sum_m b_m k_m
+#pragma unroll
+    for (int j = 0; j < D; ++j) gy0[j] = gy0[j] + gy1[j];
+    static_for<0, S>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      if constexpr (Tab::b[m] != 0.0) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) gk[m][j] = fma_t(T(Tab::b[m]), gy1[j], gk[m][j]);
       }
-      // SaveAt(ts) rows inside this step: t in (end of the previous step, ts1]
-      while (ti >= 0 && tsv > prev_end) {
-        erk_interp_vjp<Tab, T, D>(ts0, ts1, tsv, grow, gy0, gy1, gk);
-        --ti;
-        --r;
-        tsv = (ti >= 0) ? tsr[ti] * dir : -__builtin_inf();
-        if (r >= 0) {
+    });
+    // stages, last first
+    static_for<0, S>([&](auto ic) {
+      constexpr int i = S - 1 - decltype(ic)::value;
+      T w[D], gz[D], gqi[P];
 #pragma unroll
-          for (int j = 0; j < D; ++j) grow[j] = g[(int64_t)r * D + j];
-        }
-      }
-      // y1 = y0 + sum_m b_m k_m
+      for (int j = 0; j < D; ++j) w[j] = control * gk[i][j];
+      VF::vjp(zs[i], q, w, gz, gqi);
 #pragma unroll
-      for (int j = 0; j < D; ++j) gy0[j] = gy0[j] + gy1[j];
-      static_for<0, S>([&](auto mc) {
-        constexpr int m = decltype(mc)::value;
-        if constexpr (Tab::b[m] != 0.0) {
+      for (int m = 0; m < P; ++m) gq[m] = gq[m] + gqi[m];
 #pragma unroll
-          for (int j = 0; j < D; ++j) gk[m][j] = fma_t(T(Tab::b[m]), gy1[j], gk[m][j]);
+      for (int j = 0; j < D; ++j) gy0[j] = gy0[j] + gz[j];
+      static_for<0, i>([&](auto lc) {
+        constexpr int l = decltype(lc)::value;
+        if constexpr (Tab::a[i][l] != 0.0) {
+#pragma unroll
+          for (int j = 0; j < D; ++j) gk[l][j] = fma_t(T(Tab::a[i][l]), gz[j], gk[l][j]);
         }
       });
-      // stages, last first
-      static_for<0, S>([&](auto ic) {
-        constexpr int i = S - 1 - decltype(ic)::value;
-        T w[D], gz[D], gqi[P];
+    });
 #pragma unroll
-        for (int j = 0; j < D; ++j) w[j] = control * gk[i][j];
-        VF::vjp(zs[i], q, w, gz, gqi);
+    for (int j = 0; j < D; ++j) ab[j] = gy0[j];
+  }
+
+  // The whole solve from the forward's tape: `tried` attempts of this instance, `rows` the
+  // most of the workgroup's.  The lanes walk the attempts together, newest first, so a row
+  // of the tape is one contiguous load (read two rows ahead) and a lane idles in the
+  // attempts it rejected or had not reached.  Without step clipping a step starts where
+  // the previous one ended, so ts0 is also the end of the step before.
+  __device__ void tape(const ErkKArgs& a, const DiscreteAdjArgs& b, int tried, int rows) {
+    const int64_t at0 = (id >> 6) * (int64_t)b.tape_steps * 64 + (id & 63);
+    const double* tt = b.tape + at0 * 2;
+    const T* ty = reinterpret_cast<const T*>(b.tape_y) + at0 * D;
+    if (n > 0) {
+      int last = tried - 1;  // the newest accepted attempt
+      while (last > 0 && tt[(int64_t)last * 128 + 1] == -__builtin_inf()) --last;
+      setup_rows(a, tt[(int64_t)last * 128 + 1]);
+    }
+    double c0 = 0.0, c1 = 0.0, n0 = 0.0, n1 = 0.0;  // rows it and it - 1
+    T cy[D], ny[D];
+    auto load = [&](int it, double& t0, double& t1, T (&y)[D]) {
+      if (it >= 0 && it < tried) {
+        t0 = tt[(int64_t)it * 128];
+        t1 = tt[(int64_t)it * 128 + 1];
 #pragma unroll
-        for (int m = 0; m < P; ++m) gq[m] = gq[m] + gqi[m];
+        for (int j = 0; j < D; ++j) y[j] = ty[(int64_t)it * 64 * D + j];
+      }
+    };
+    load(rows - 1, c0, c1, cy);
+    load(rows - 2, n0, n1, ny);
+    int s = n - 1;
+    for (int it = rows - 1; it >= 0; --it) {
+      const double ts0 = c0, ts1 = c1;
+      T y0[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) gy0[j] = gy0[j] + gz[j];
-        static_for<0, i>([&](auto lc) {
-          constexpr int l = decltype(lc)::value;
-          if constexpr (Tab::a[i][l] != 0.0) {
-#pragma unroll
-            for (int j = 0; j < D; ++j) gk[l][j] = fma_t(T(Tab::a[i][l]), gz[j], gk[l][j]);
-          }
-        });
-      });
-#pragma unroll
-      for (int j = 0; j < D; ++j) ab[j] = gy0[j];
+      for (int j = 0; j < D; ++j) { y0[j] = cy[j]; cy[j] = ny[j]; }
+      c0 = n0;
+      c1 = n1;
+      load(it - 2, n0, n1, ny);
+      if (it < tried && s >= 0 && ts1 != -__builtin_inf()) {
+        step(a, s, ts0, ts1, y0, s > 0 ? ts0 : -__builtin_inf());
+        --s;
+      }
     }
   }
 
@@ -298,12 +363,32 @@ __global__ void __launch_bounds__(128) erk_adjoint_kernel(const ErkKArgs a, cons
   const int K = a.ckpt_every;
   const int n = live ? min(max(b.stats[id * 3 + 1], 0), a.max_steps) : 0;
   const int c_last = n > 0 ? (n - 1) / K : -1;
-  __shared__ int s_cmax;
-  if (threadIdx.x == 0) s_cmax = -1;
+  __shared__ int s_nmax;
+  if (threadIdx.x == 0) s_nmax = 0;
   __syncthreads();
-  if (role == 0 && c_last >= 0) atomicMax(&s_cmax, c_last);
+  if constexpr (!Extras) {
+    if (b.tape_steps > 0) {
+      const int tried = live ? min(max(b.stats[id * 3], 0), a.max_steps) : 0;
+      if (role == 0) atomicMax(&s_nmax, tried);
+      __syncthreads();
+      const int rows = __builtin_amdgcn_readfirstlane(s_nmax);
+      if (rows <= b.tape_steps) {  // block-uniform: every attempt is on the tape
+        if (role == 1 && live) {
+          AdjSweep<Tab, VF, T> W;
+          W.setup(a, b, id, n);
+          W.tape(a, b, tried, rows);
+          W.finish(a, b);
+        }
+        return;
+      }
+      __syncthreads();
+      if (threadIdx.x == 0) s_nmax = 0;
+      __syncthreads();
+    }
+  }
+  if (role == 0) atomicMax(&s_nmax, n);
   __syncthreads();
-  const int nstages = s_cmax + 2;  // the replay of the oldest segment, then its sweep
+  const int nstages = (s_nmax - 1) / K + 2;  // the replay of the oldest segment, then its sweep
   if (role == 0) {
     ErkLane<Tab, VF, T, Ctl, Extras> L;
     if (live) L.replay_setup(ra, id);
@@ -319,13 +404,13 @@ __global__ void __launch_bounds__(128) erk_adjoint_kernel(const ErkKArgs a, cons
     }
   } else {
     AdjSweep<Tab, VF, T> W;
-    if (live) W.setup(a, b, id, n, K);
+    if (live) W.setup(a, b, id, n);
     for (int s = 0; s < nstages; ++s) {
       const int c = c_last - s + 1;
       if (live && c >= 0 && c <= c_last) {
         const int64_t base = id * ra.grid_stride + (int64_t)(c & 1) * K;
         const double tl = b.ckpt[(id * a.n_ckpt + c) * (D + 8) + D + 4];
-        W.segment(a, c, K, ra.grid + base * 2, reinterpret_cast<const T*>(ra.grid_y) + base * D,
+        W.segment(a, c * K, min(c * K + K, n), ra.grid + base * 2, reinterpret_cast<const T*>(ra.grid_y) + base * D,
                   tl);
       }
       __syncthreads();

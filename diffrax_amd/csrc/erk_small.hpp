@@ -30,6 +30,9 @@ struct ErkKArgs {
   void* grid_y;       // [B, grid_stride, D] start state of each accepted step (with grid)
   double* ckpt;       // [B, n_ckpt, D + 8] lane state every ckpt_every accepted steps
                       // (ErkLane::write_ckpt), the restart points of the discrete adjoint
+  double* tape;       // [ceil(B / 64), tape_steps, 64, 2] (t_start, t_end) of the first
+                      // attempted steps, t_end = -inf on a rejected one, and
+  void* tape_y;       // [ceil(B / 64), tape_steps, 64, D] their start states
   const double* rtol_b;  // per-instance PIDController tolerances [B], or null for pid.rtol
   const double* atol_b;
   double* dense_ts;   // SaveAt(dense=True): [B, max_steps + 1] accepted-step ends (t0 first)
@@ -45,7 +48,8 @@ struct ErkKArgs {
   unsigned int* counter;
   int64_t B, t1_stride, ts_stride, param_stride;
   int64_t grid_stride;  // records per instance in grid / grid_y
-  int32_t ckpt_every, n_ckpt, resume;  // resume: DFX_RESUME_* parts of state_in taken
+  int32_t ckpt_every, n_ckpt, tape_steps;
+  int32_t resume;  // resume: DFX_RESUME_* parts of state_in taken
   int32_t n_step_ts, n_jump_ts, n_events, event_root_find;
   int32_t n_ts, n_out, save_t0, save_t1, save_steps, max_steps, has_dt0, controller;
   double t0, dt0, error_order;
@@ -568,6 +572,11 @@ struct ErkLane {
     ri[5] = cs_completed;
   }
 
+  // Index of this instance's tape record of attempt `step`.
+  __device__ __forceinline__ int64_t tape_at(const ErkKArgs& a, int32_t step) const {
+    return ((traj >> 6) * a.tape_steps + step) * 64 + (traj & 63);
+  }
+
   // The per-instance set-up a replay needs (no initial step, no saves, no events).
   __device__ void replay_setup(const ErkKArgs& a, int64_t id) {
     tr.load();
@@ -842,6 +851,20 @@ struct ErkLane {
 
     ++num_steps;
     if (keep) ++num_acc; else ++num_rej;
+    if constexpr (Ck && !Extras) {
+      // The adjoint's tape.  Indexed by the attempt, which the lanes of a wave share, so the
+      // 64 records are one contiguous store; records of 64 lanes each in its own row (by
+      // accepted step) held up every later load of the loop: 65,536 Van der Pol solves took
+      // 1.92 ms that way.
+      if (num_steps <= a.tape_steps) {
+        const int64_t rec = tape_at(a, num_steps - 1);
+        a.tape[rec * 2] = ts0;
+        a.tape[rec * 2 + 1] = keep ? ts1 : -__builtin_inf();
+        T* ty = reinterpret_cast<T*>(a.tape_y) + rec * D;
+#pragma unroll
+        for (int j = 0; j < D; ++j) ty[j] = y[j];
+      }
+    }
     if (result == DFX_SUCCESSFUL) result = code;
 
     bool event_now = false;

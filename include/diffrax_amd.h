@@ -85,6 +85,10 @@ typedef struct dfx_erk_problem {
    * controller's init is skipped); with dt0 NaN the initial step is selected as usual.
    * Not with step_ts / jump_ts clipping, checkpoints or the adjoints. */
   int32_t resume;
+  /* With ckpt_every > 0: records per instance of dfx_erk_io.tape, 0 for none.  Solves
+   * that attempt no more steps are swept from the tape by dfx_erk_adjoint, without a replay.
+   * Not written with step_ts / jump_ts clipping. */
+  int32_t tape_steps;
 } dfx_erk_problem;
 
 enum { DFX_RESUME_SOLVER = 1, DFX_RESUME_CONTROLLER = 2, DFX_RESUME_MADE_JUMP = 4 };
@@ -143,6 +147,11 @@ typedef struct dfx_erk_io {
                              controller state and made_jump (SaveAt(solver_state=True,
                              controller_state=True, made_jump=True), _integrate.py:
                              1489-1500); NULL to skip                                   */
+  double* tape;         /* out [ceil(B / 64), tape_steps, 64, 2] when tape_steps > 0, else NULL:
+                           (t_start, t_end) of the first attempted steps, direction-
+                           normalised, t_end = -inf on a rejected one                      */
+  void* tape_y;         /* out [ceil(B / 64), tape_steps, 64, d] state dtype: the start states
+                           of those steps (with tape)                                     */
 } dfx_erk_io;
 
 /* Launch shape (NULL: block 64, one lane per instance).  Fewer lanes than instances
@@ -233,6 +242,8 @@ int dfx_erk_adjoint_workspace_bytes(const dfx_erk_problem* p, size_t* bytes);
  * reference.  p and fwd are the forward's problem and buffers (its inputs are read: t1,
  * ts, params, rtol / atol, step_ts / jump_ts; its outputs are not touched); p: LV, VdP,
  * linear with d <= 4, no events, no dense output, ckpt_every > 0.
+ * Where 64 neighbouring instances have all attempted at most tape_steps steps, these come
+ * from fwd's tape (same values, so the same gradients) and nothing is replayed.
  * Replaces: RecursiveCheckpointAdjoint.loop (_adjoint.py:264-312) differentiating the
  * accepted steps of _integrate.py:302-662 (AbstractRungeKutta.step,
  * _solver/runge_kutta.py:446-1203, and the save interpolation, _integrate.py:456-491),
