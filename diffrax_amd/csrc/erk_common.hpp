@@ -128,6 +128,29 @@ __host__ __device__ inline double jclip(double x, double lo, double hi) { return
 __device__ __forceinline__ double jmax_nonneg(double a, double b) {
   return (a != a || b != b) ? __builtin_nan("") : __builtin_fmax(a, b);
 }
+// One instruction each: of two numbers the larger / smaller, of a number and a NaN the number.
+// (From __builtin_fmax the compiler first quiets each operand by an instruction of its own.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ double num_max(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double num_min(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double num_max_abs(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+#else
+__device__ double num_max(double a, double b);
+__device__ double num_min(double a, double b);
+__device__ double num_max_abs(double a, double b);
+#endif
 __device__ __forceinline__ double jclip_pos(double x, double lo, double hi) {
   return (x != x) ? __builtin_nan("") : __builtin_fmin(__builtin_fmax(x, lo), hi);
 }
@@ -172,18 +195,13 @@ __host__ __device__ inline unsigned long long double_to_bits(double x) {
   return b;
 }
 
-__host__ __device__ inline double cr_pow_fifth(double x_in) {
+// x^0.2 for a positive normal x scaled by 2^(-5 adj) (below).
+__host__ __device__ inline double cr_fifth_core(double x, int adj) {
 #pragma clang fp contract(off)
-  // Zero, negative, NaN and infinite inputs are resolved by one select at the end and the
-  // arithmetic runs on a stand-in for them, so the device code has no branches.
-  const bool finite_pos = (x_in > 0.0) && (x_in < __builtin_inf());
-  const bool sub = x_in < 2.2250738585072014e-308;  // subnormal: scale by 2^100
-  double x = finite_pos ? x_in : 1.0;
-  x = sub ? x * 1.2676506002282294e30 : x;
-  const int adj = sub ? -20 : 0;
   const unsigned long long bx = double_to_bits(x);
   const int E = (int)((bx >> 52) & 0x7ff) - 1023;
-  const int k = (E >= 0) ? E / 5 : -((4 - E) / 5);
+  // floor(E / 5) for E in [-1023, 1024], by an unsigned product (no branch, no mask logic)
+  const int k = (int)(((unsigned)(E + 1025) * 52429u) >> 18) - 205;
   const int j = E - 5 * k;  // 0..4
   const double f = bits_to_double((bx & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);  // [1,2)
   const double m = f * (double)(1 << j);  // x = m * 2^(5k), m in [1, 32)
@@ -232,9 +250,24 @@ __host__ __device__ inline double cr_pow_fifth(double x_in) {
   const double eps = 1.1102230246251565e-17;  // 0.2 (float64) - 1/5
   const double corr = r * (eps * lnx);
   const double out = r + (delta + corr);
-  const double scale = bits_to_double((unsigned long long)(1023 + k + adj) << 52);
-  const double special = (x_in == 0.0) ? 0.0 : ((x_in > 0.0) ? x_in : __builtin_nan(""));
-  return finite_pos ? out * scale : special;
+  return out * bits_to_double((unsigned long long)(1023 + k + adj) << 52);
+}
+
+__host__ __device__ inline double cr_pow_fifth(double x_in) {
+#pragma clang fp contract(off)
+  // Zero, negative, NaN and infinite inputs are resolved by one select at the end and the
+  // arithmetic runs on a stand-in for them, so the device code has no branches.
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool finite_pos = __builtin_amdgcn_class(x_in, 0x180);  // positive normal or subnormal
+#else
+  const bool finite_pos = (x_in > 0.0) && (x_in < __builtin_inf());
+#endif
+  const bool sub = x_in < 2.2250738585072014e-308;  // subnormal: scale by 2^100
+  double x = finite_pos ? x_in : 1.0;
+  x = sub ? x * 1.2676506002282294e30 : x;
+  const double out = cr_fifth_core(x, sub ? -20 : 0);
+  const double special = (x_in >= 0.0) ? x_in + 0.0 : __builtin_nan("");  // -0 + 0 is 0
+  return finite_pos ? out : special;
 }
 
 // Exponents other than 0.2 / 0.5 / 1 (non-default PID coefficients or error orders) use
@@ -306,14 +339,33 @@ struct PidState {
 //                exponent 0.2, 0.5 or 1 chosen at run time: factor2 = factor3 = 1;
 //   PID_FIFTH    the integral-only controller with exponent 0.2 (the default for the
 //                fifth-order embedded pairs): the correctly rounded fifth root inline,
-//                with no run-time dispatch and no branches.
-enum : int { PID_INTEGRAL = 0, PID_GENERIC = 1, PID_FIFTH = 2 };
+//                with no run-time dispatch and no branches;
+//   PID_PLAIN    PID_FIFTH without dtmin and dtmax, for bounds on the factor that make the
+//                root of zero, subnormal and infinite inputs irrelevant (pid_is_plain) and
+//                with no controller state to keep: 45 instructions fewer per step.
+enum : int { PID_INTEGRAL = 0, PID_GENERIC = 1, PID_FIFTH = 2, PID_PLAIN = 3 };
 
 template <int Ctl>
 __device__ __forceinline__ bool pid_adapt(const PidParams& p, double scaled, double tprev,
                                           double tnext, PidState& st, double& ntprev,
                                           double& ntnext, int& code) {
   const double prev_dt = tnext - tprev;
+  if constexpr (Ctl == PID_PLAIN) {
+    const bool keep = scaled < 1.0;
+    const double inv = 1.0 / scaled;
+    // scaled >= 0 or NaN.  Outside the normal numbers the core returns about 2^-205 (0,
+    // subnormal) or 2^205 (inf) for the root, which the bounds turn into the same factor.
+    const double root = cr_fifth_core(inv, 0);
+    const double lo = keep ? 1.0 : p.factormin;
+    const double hi = keep ? p.factormax : p.safety;
+    const double factor =
+        (inv != inv) ? __builtin_nan("") : num_min(num_max(p.safety * root, lo), hi);
+    ntprev = keep ? tnext : tprev;
+    const double dt = prev_dt * factor;  // (a product of its own also where the build contracts)
+    ntnext = ntprev + dt;
+    code = 0;
+    return keep;
+  }
   bool keep = scaled < 1.0;
   if (p.has_dtmin) keep = keep || st.at_dtmin;
   double inv = 1.0 / scaled;
@@ -361,6 +413,13 @@ inline bool pid_is_integral(const PidParams& p) {
 // Whether the PID_FIFTH controller path reproduces these coefficients.
 inline bool pid_is_fifth(const PidParams& p) {
   return p.coeff2 == 0.0 && p.coeff3 == 0.0 && p.coeff1 == 0.2;
+}
+
+// Whether PID_PLAIN does.
+inline bool pid_is_plain(const PidParams& p) {
+  constexpr double lo = 7.888609052210118e-31, hi = 1.2676506002282294e30;  // 2^-100, 2^100
+  return pid_is_fifth(p) && !p.has_dtmin && !p.has_dtmax && p.factormin >= lo &&
+         p.factormax <= hi && p.safety >= lo && p.safety <= hi;
 }
 
 // optimistix.rms_norm restated: sqrt(sum x^2)/sqrt(n), |x| when n == 1.

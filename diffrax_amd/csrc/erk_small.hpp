@@ -358,8 +358,19 @@ __device__ __forceinline__ unsigned int lane_rank(unsigned long long mask) {
 // Ck: the step loop writes the discrete adjoint's checkpoints when a.ckpt is set.  The
 // plain kernels are built without and with it, so a forward solve that records none runs
 // no code of theirs; the extras kernels always carry it.
+// Ctl = PID_PLAIN is the default solve on a lane per instance: PIDController with exponent
+// 0.2 and no dtmin or dtmax, no grid record and no SaveAt(steps), save times in LDS.  What
+// bounds these kernels is the number of instructions: a wave alone on its SIMD takes 4.5
+// cycles for each one, vector or scalar, 5.5 where an 8-byte one is not 8-byte aligned, so
+// this build resolves what it can at compile time (about 300 instructions a step and 86 a
+// save in place of 430 and 93).  Kernel times, general build then this one: Van der Pol, 64
+// saves, float64, 64 / 4,096 / 65,536 instances 919 / 1,079 / 1,330 -> 711 / 833 / 1,010 us;
+// float32 state, 20,011 instances 1,250 -> 990 us; Lotka-Volterra, 100 saves, 1 / 1,024
+// instances 128 / 206 -> 114 / 157 us.  The same bits.
 template <class Tab, class VF, class T, int Ctl, bool Extras, bool Ck = Extras>
 struct ErkLane {
+  static constexpr bool Plain = Ctl == PID_PLAIN;
+  static_assert(!(Plain && Extras), "the extras are not part of the plain solve");
   static constexpr int D = VF::D;
   static constexpr int P = VF::P;
   static constexpr int S = Tab::S;
@@ -387,11 +398,42 @@ struct ErkLane {
   int32_t num_steps, num_acc, num_rej, result;
   int32_t ck_left;    // accepted steps until the next checkpoint (INT32_MAX: none recorded)
   int32_t save_index, ts_index;
-  double next_ts;    // normalised save time ts[ts_index], +inf when none left
+  double next_ts;    // normalised save time ts[ts_index], NaN when none left
   double after_raw;  // ts[min(ts_index + 1, n_ts - 1)] as stored, loaded one save ahead
                      // and used only when the next save is reached, so a save never
                      // waits on memory
   const double* ts_row;
+
+  // Plain: the save times in LDS, index k of this lane at win[k * win_step], NaN in the two
+  // entries after the last, and after_raw the one after next_ts.  Loads from memory inside
+  // the step loop waited for the stores of the rows before them (one counter for both), and
+  // their clamped indexes were a sixth of a save's instructions.
+  const double* win;
+  int32_t win_step;
+  // One row for the wave where the batch shares its times, else one per lane; `live` lanes.
+  __device__ __forceinline__ void load_times(const ErkKArgs& a, double* lds, int lane, int live) {
+    const double* row = a.ts + traj * a.ts_stride;
+    if (a.ts_stride == 0) {
+      for (int i = lane; i < a.n_ts + 2; i += live)
+        lds[i] = i < a.n_ts ? row[i] : __builtin_nan("");
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      win = lds;
+      win_step = 1;
+    } else {
+      for (int i = 0; i < a.n_ts + 2; i += 8) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = row[min(i + k, a.n_ts - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (i + k < a.n_ts + 2) lds[(i + k) * 64 + lane] = i + k < a.n_ts ? v[k] : __builtin_nan("");
+      }
+      win = lds + lane;
+      win_step = 64;
+    }
+  }
 
   // Unconditional (no branch for the compiler to sink the previous value's use past): the
   // index is clamped into the row, and without save times ts_row points at t1, which is
@@ -400,13 +442,27 @@ struct ErkLane {
     after_raw = ts_row[max(min(ts_index + 1, a.n_ts - 1), 0)];
   }
   __device__ __forceinline__ void first_ts(const ErkKArgs& a) {
-    next_ts = (a.ts != nullptr && a.n_ts > 0) ? ts_row[0] * (double)dir : __builtin_inf();
+    if constexpr (Plain) {
+      next_ts = after_raw = __builtin_nan("");
+      if (a.n_ts > 0) {
+        next_ts = win[0] * (double)dir;
+        after_raw = win[win_step];
+      }
+      return;
+    }
+    next_ts = (a.ts != nullptr && a.n_ts > 0) ? ts_row[0] * (double)dir : __builtin_nan("");
     after_raw = 0.0;
     prefetch_ts(a);
   }
-  // After ++ts_index: the prefetched time becomes the next one (+inf past the last).
+  // After ++ts_index: the prefetched time becomes the next one (NaN past the last).
   __device__ __forceinline__ void load_next_ts(const ErkKArgs& a) {
-    next_ts = (ts_index < a.n_ts) ? after_raw * (double)dir : __builtin_inf();
+    if constexpr (Plain) {
+      next_ts = after_raw * (double)dir;
+      win += win_step;
+      after_raw = win[win_step];
+      return;
+    }
+    next_ts = (ts_index < a.n_ts) ? after_raw * (double)dir : __builtin_nan("");
     prefetch_ts(a);
   }
 
@@ -539,8 +595,8 @@ struct ErkLane {
     begin_times(a, t0r, t1r);
     save_index = 0;
     ts_index = 0;
-    ts_row = a.t1;  // no save times (next_ts = +inf keeps the save loop from running)
-    next_ts = after_raw = __builtin_inf();
+    ts_row = a.t1;  // no save times (next_ts = NaN keeps the save loop from running)
+    next_ts = after_raw = __builtin_nan("");
     ev_mask = 0;
     while (running(a)) step(a);
     if (tprev < T1 && result == DFX_SUCCESSFUL) result = DFX_MAX_STEPS_REACHED;
@@ -566,7 +622,7 @@ struct ErkLane {
     int32_t* ri = reinterpret_cast<int32_t*>(r + D + 5);
     ri[0] = pid.at_dtmin | (made_jump ? 2 : 0);
     ri[1] = num_steps;
-    ri[2] = num_rej;
+    ri[2] = Plain ? num_steps - num_acc : num_rej;
     ri[3] = step_index;
     ri[4] = jump_index;
     ri[5] = cs_completed;
@@ -586,7 +642,7 @@ struct ErkLane {
     save_index = 0;
     ts_index = 0;
     ts_row = a.t1;
-    next_ts = after_raw = __builtin_inf();
+    next_ts = after_raw = __builtin_nan("");
     ev_mask = 0;
   }
 
@@ -704,6 +760,10 @@ struct ErkLane {
     ts_index = 0;
     ts_row = a.ts ? a.ts + id * a.ts_stride : a.t1;
     first_ts(a);
+    if constexpr (Plain) {
+      out_y = reinterpret_cast<T*>(a.ys) + traj * a.n_out * D;
+      out_t = a.ts_out + traj * a.n_out;
+    }
     if (a.save_t0) {
       write_save(a, T0, y);
     }
@@ -733,7 +793,17 @@ struct ErkLane {
     }
   }
 
+  T* out_y;       // Plain: the next row to save, in place of save_index
+  double* out_t;
   __device__ __forceinline__ void write_save(const ErkKArgs& a, double t_norm, const T (&v)[D]) {
+    if constexpr (Plain) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) out_y[j] = v[j];
+      *out_t = t_norm * (double)dir;
+      out_y += D;
+      ++out_t;
+      return;
+    }
     T* row = reinterpret_cast<T*>(a.ys) + (traj * a.n_out + save_index) * D;
 #pragma unroll
     for (int j = 0; j < D; ++j) row[j] = v[j];
@@ -742,6 +812,7 @@ struct ErkLane {
   }
 
   __device__ __forceinline__ bool running(const ErkKArgs& a) const {
+    if constexpr (Plain) return tprev < T1 && num_steps < a.max_steps;  // no result until the end
     return tprev < T1 && result == DFX_SUCCESSFUL && num_steps < a.max_steps;
   }
 
@@ -800,7 +871,7 @@ struct ErkLane {
     bool keep;
     double ntprev, ntnext;
     int code = 0;
-    if (a.controller == DFX_PID) {
+    if (Plain || a.controller == DFX_PID) {
       bool anynan = false;
 #pragma unroll
       for (int j = 0; j < D; ++j) anynan = anynan || (y1[j] != y1[j]);
@@ -808,7 +879,9 @@ struct ErkLane {
 #pragma unroll
       for (int j = 0; j < D; ++j) {
         const double y1c = anynan ? (double)y[j] : (double)y1[j];
-        const double yy = jmax_nonneg(fabs((double)y[j]), fabs(y1c));
+        // a NaN y makes y1 NaN, so y1c is NaN with it: the plain maximum has two NaNs or none
+        const double yy = Plain ? num_max_abs((double)y[j], y1c)
+                                : jmax_nonneg(fabs((double)y[j]), fabs(y1c));
         e[j] = (double)yerr[j] / (pv.atol + yy * pv.rtol);
       }
       double scaled;
@@ -846,11 +919,16 @@ struct ErkLane {
       }
     }
     if (Extras && keep) made_jump = mj;
-    ntprev = jmin(ntprev, T1);
+    if constexpr (!Plain) ntprev = jmin(ntprev, T1);  // plain: tnext <= T1 or NaN already
     if (ntnext > floor_t1) ntnext = keep ? T1 : ntprev + 0.5 * (T1 - ntprev);
 
     ++num_steps;
-    if (keep) ++num_acc; else ++num_rej;
+    if constexpr (Plain) {
+      num_acc += keep ? 1 : 0;  // num_rej = num_steps - num_acc (finish, write_ckpt)
+    } else {
+      if (keep) ++num_acc; else ++num_rej;
+      if (result == DFX_SUCCESSFUL) result = code;
+    }
     if constexpr (Ck && !Extras) {
       // The adjoint's tape.  Indexed by the attempt, which the lanes of a wave share, so the
       // 64 records are one contiguous store; records of 64 lanes each in its own row (by
@@ -865,7 +943,6 @@ struct ErkLane {
         for (int j = 0; j < D; ++j) ty[j] = y[j];
       }
     }
-    if (result == DFX_SUCCESSFUL) result = code;
 
     bool event_now = false;
     if (Extras && a.n_events > 0) {
@@ -899,7 +976,7 @@ struct ErkLane {
     }
 
     if (keep) {
-      if (a.grid) {
+      if (!Plain && a.grid) {
         const int64_t rec = traj * a.grid_stride + (num_acc - 1);
         double* g = a.grid + rec * 2;
         g[0] = ts0;
@@ -931,7 +1008,7 @@ struct ErkLane {
         T v[D];
         interp(ts0, ts1, y, y1, k, next_ts, v);
         write_save(a, next_ts, v);
-        ++ts_index;
+        if (!Plain) ++ts_index;
         load_next_ts(a);
       }
 #pragma unroll
@@ -943,7 +1020,7 @@ struct ErkLane {
         for (int j = 0; j < D; ++j) fsal_f[j] = f[j];
       }
       // SaveAt(steps=k): every k-th accepted step (_integrate.py:493-527)
-      if (a.save_steps && num_acc % a.save_steps == 0 && !(Extras && event_now && ntprev > tfinal))
+      if (!Plain && a.save_steps && num_acc % a.save_steps == 0 && !(Extras && event_now && ntprev > tfinal))
         write_save(a, ntprev, y);
     }
     tprev = ntprev;
@@ -968,9 +1045,12 @@ struct ErkLane {
   // Loop exit bookkeeping (_integrate.py:823-883) and output of counters.
   __device__ void finish(const ErkKArgs& a) {
     const double T0 = a.t0 * dir;
+    // (opaque: the loop need not carry its last test of tprev < T1 in a mask for the use here)
+    if constexpr (Plain) asm volatile("" : "+v"(tprev));
     if (T0 == T1) {
       for (int r = 0; r < a.n_ts; ++r) write_save(a, T0, y);
     }
+    if constexpr (Plain) save_index = (int32_t)(out_t - (a.ts_out + traj * a.n_out));
     if (Extras && result == DFX_EVENT_OCCURRED) {  // the solve ends at the event
       tprev = tfinal;
 #pragma unroll
@@ -982,7 +1062,10 @@ struct ErkLane {
     const bool via_steps = a.save_steps && num_acc % a.save_steps == 0;
     const bool root = Extras && a.n_events > 0 && a.event_root_find;
     const bool t1_pred = root ? (a.save_t1 || via_steps) : (a.save_t1 && !via_steps);
-    if (t1_pred && save_index < a.n_out) write_save(a, tprev, y);
+    if (t1_pred && save_index < a.n_out) {
+      write_save(a, tprev, y);
+      if (Plain) ++save_index;
+    }
     if (tprev < T1 && result == DFX_SUCCESSFUL) result = DFX_MAX_STEPS_REACHED;
     if (Extras && a.n_events > 0 && a.event_mask) {
       for (int i = 0; i < a.n_events; ++i) a.event_mask[traj * a.n_events + i] = (ev_mask >> i) & 1;
@@ -998,7 +1081,7 @@ struct ErkLane {
     }
     a.stats[traj * 3 + 0] = num_steps;
     a.stats[traj * 3 + 1] = num_acc;
-    a.stats[traj * 3 + 2] = num_rej;
+    a.stats[traj * 3 + 2] = Plain ? num_steps - num_acc : num_rej;
     a.result[traj] = result;
     if (Extras && a.state_out) write_state(a);
   }
@@ -1075,11 +1158,24 @@ __global__ void __launch_bounds__(256) erk_backsolve_kernel(const ErkKArgs a, co
 // One trajectory per lane, no work queue: used when the launch has a lane for every
 // instance.  Lanes whose trajectory has finished idle (masked) until the wave's last lane
 // is done.
+// LDS doubles of a wave's save times in the plain kernels (ErkLane::load_times).
+__host__ __device__ inline int64_t plain_lds_doubles(const ErkKArgs& a) {
+  return a.n_ts > 0 ? (a.n_ts + 2ll) * (a.ts_stride == 0 ? 1 : 64) : 0;
+}
+
 template <class Tab, class VF, class T, int Ctl, bool Extras, bool Ck = Extras>
 __global__ void __launch_bounds__(256) erk_small_kernel(const ErkKArgs a) {
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= a.B) return;
   ErkLane<Tab, VF, T, Ctl, Extras, Ck> L;
+  if constexpr (Ctl == PID_PLAIN) {
+    extern __shared__ double times[];
+    const int lane = threadIdx.x & 63;
+    L.traj = id;
+    if (a.n_ts > 0)
+      L.load_times(a, times + (threadIdx.x >> 6) * plain_lds_doubles(a), lane,
+                   (int)min((int64_t)64, a.B - (id - lane)));
+  }
   L.start(a, id);
   while (L.running(a)) L.step(a);
   L.finish(a);
