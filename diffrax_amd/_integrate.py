@@ -93,6 +93,21 @@ def _raise_ts(bits):
         raise RuntimeError("saveat.ts must lie between t0 and t1.")
 
 
+def raise_unless_okay(result, okay=int(RESULTS.event_occurred)):
+    """throw=True: waits for the solve that writes result ([B] int32 on the GPU) and raises for
+    the first code that is neither successful nor ``okay``."""
+    stream = torch.cuda.current_stream(result.device)
+    n = result.numel()
+    first = torch.empty(max(1, min(256, n // 4096)), dtype=torch.int32, pin_memory=True)
+    _lib.check(_lib.load().dfx_check_results(result.data_ptr(), n, okay, first.data_ptr(),
+                                             first.numel(), stream.cuda_stream),
+               "dfx_check_results")
+    stream.synchronize()
+    codes = first.numpy()
+    if codes.any():
+        raise RuntimeError(RESULTS[int(codes[codes != 0][0])])
+
+
 class _Workspace:
     """Per-device scratch buffers owned by the caller side (torch allocator)."""
 
@@ -563,11 +578,7 @@ def _finish(plan, t0, t1, max_steps, throw, ys=None, saveat=None):
         ys, ts, result = ys[0], ts[0], result[0]
         stats = {k: (v[0] if isinstance(v, torch.Tensor) else v) for k, v in stats.items()}
     if throw:
-        codes = T["result"]
-        bad = (codes != 0) & (codes != int(RESULTS.event_occurred))   # is_okay
-        if bool(bad.any()):
-            first = int(codes[bad][0].item())
-            raise RuntimeError(RESULTS[first])
+        raise_unless_okay(T["result"])
     res = result
     interp = DenseInterpolation(plan) if T.get("dense_ts") is not None else None
     if plan.problem.n_ts == 0 and not (plan.problem.save_t0 or plan.problem.save_t1 or
@@ -918,8 +929,8 @@ class _ErkBacksolve(torch.autograd.Function):
         _lib.check(lib.dfx_erk_backsolve(ctypes.byref(back), ctypes.byref(io),
                                          ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
                    "dfx_erk_backsolve")
-        if ctx.throw and bool((result != 0).any()):
-            raise RuntimeError(RESULTS[int(result[result != 0][0].item())])
+        if ctx.throw:
+            raise_unless_okay(result, okay=0)
         gparams = params_bar.sum(0) if plan.problem.param_stride == 0 else params_bar
         return None, None, None, y0_bar, gparams.reshape(T["params"].shape)
 

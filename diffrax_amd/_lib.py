@@ -105,6 +105,8 @@ _SIGS = {
                          ctypes.c_int64, ctypes.c_int32, ctypes.c_int64, ctypes.c_double,
                          ctypes.c_double, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
                         ctypes.c_int),
+    "dfx_check_results": ([ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p,
+                           ctypes.c_int32, ctypes.c_void_p], ctypes.c_int),
     "dfx_erk_backsolve": ([ctypes.POINTER(ErkProblem), ctypes.POINTER(BacksolveIO),
                            ctypes.c_void_p], ctypes.c_int),
     "dfx_erk_ckpt_layout": ([ctypes.POINTER(ErkProblem), ctypes.POINTER(ctypes.c_int32),

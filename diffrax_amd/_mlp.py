@@ -313,7 +313,8 @@ def _state_outputs(plan, saveat):
 
 
 def _solution(plan, t0, t1, max_steps, throw, ys, saveat=None):
-    from ._solution import RESULTS, Solution
+    from ._integrate import raise_unless_okay
+    from ._solution import Solution
     if getattr(plan, "deferred_checks", None) is not None:
         plan.deferred_checks()
     st = plan.stats
@@ -324,9 +325,7 @@ def _solution(plan, t0, t1, max_steps, throw, ys, saveat=None):
         ys, ts, result = ys[0], ts[0], result[0]
         stats = {k: (v[0] if isinstance(v, torch.Tensor) else v) for k, v in stats.items()}
     if throw:
-        bad = (plan.result != 0) & (plan.result != int(RESULTS.event_occurred))   # is_okay
-        if bool(bad.any()):
-            raise RuntimeError(RESULTS[int(plan.result[bad][0].item())])
+        raise_unless_okay(plan.result)
     event_mask = None
     if getattr(plan, "event_mask", None) is not None:
         m = plan.event_mask.bool()
@@ -606,14 +605,12 @@ class _MlpBacksolve(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, ys_bar, *_):
-        from ._solution import RESULTS
+        from ._integrate import raise_unless_okay
         ctx.saved_tensors   # the version check of the saved ys
         ys_bar = torch.zeros_like(ctx.plan.ys) if ys_bar is None else ys_bar
         grads, result = backsolve_mlp(ctx.plan, ctx.back, ys_bar)
         if ctx.throw:
-            bad = result != 0
-            if bool(bad.any()):
-                raise RuntimeError(RESULTS[int(result[bad][0].item())])
+            raise_unless_okay(result, okay=0)
         out = [g.to(dt) if need else None
                for g, dt, need in zip(grads, ctx.dtypes, ctx.needs_input_grad[:7])]
         return (*out, None)

@@ -61,6 +61,26 @@ __global__ void __launch_bounds__(256) check_times_kernel(const double* t1, doub
   if (threadIdx.x == 0) flags[blockIdx.x] = any;
 }
 
+// The first failure of each block's run of result codes, written where the host reads it.
+// Bound by its launch: comparing, masking and reducing the codes as tensors was five launches
+// and a copy, 30 us of a call whose solve takes 110 us.  A block reads 4,096 codes and more.
+__global__ void __launch_bounds__(256) check_results_kernel(const int32_t* result, int64_t n,
+                                                            int32_t ok_code, int32_t* first) {
+  const int64_t len = (n + gridDim.x - 1) / gridDim.x;
+  const int64_t lo = blockIdx.x * len, hi = min(n, lo + len);
+  __shared__ unsigned long long at;
+  if (threadIdx.x == 0) at = ~0ull;
+  __syncthreads();
+  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+    if (result[i] != 0 && result[i] != ok_code) {
+      atomicMin(&at, (unsigned long long)i);
+      break;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) first[blockIdx.x] = at == ~0ull ? 0 : result[at];
+}
+
 int solver_order(int solver) { return solver == DFX_HEUN ? 2 : 5; }
 
 bool small_vf_supported(int vf, int d) {
@@ -439,6 +459,14 @@ int dfx_check_times(const double* t1, double t1_value, int64_t t1_stride, const 
   hipLaunchKernelGGL(check_times_kernel, dim3((unsigned)n_flags), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), t1, t1_value, t1_stride,
                      n_ts > 0 ? ts : nullptr, ts_stride, n_ts, rows, t0, dt0, flags);
+  return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
+}
+
+int dfx_check_results(const int32_t* result, int64_t n, int32_t ok_code, int32_t* first,
+                      int32_t n_first, void* stream) {
+  if (!first || n_first < 1 || n_first > 4096 || n < 0 || (n > 0 && !result)) return DFX_E_ARG;
+  hipLaunchKernelGGL(check_results_kernel, dim3((unsigned)n_first), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), result, n, ok_code, first);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 

@@ -284,6 +284,12 @@ int dfx_check_times(const double* t1, double t1_value, int64_t t1_stride, const 
                     int64_t ts_stride, int32_t n_ts, int64_t rows, double t0, double dt0,
                     int32_t* flags, int32_t n_flags, void* stream);
 
+/* The throw=True check of a solve's result codes: result [n] is split into n_first
+ * (in [1, 4096]) runs of equal length, and first[i] (device memory or pinned host memory)
+ * becomes the first code of run i that is neither 0 nor ok_code, or 0. */
+int dfx_check_results(const int32_t* result, int64_t n, int32_t ok_code, int32_t* first,
+                      int32_t n_first, void* stream);
+
 /* ---- SDE: Heun with diagonal noise on the registered OU terms ----------------------- */
 /* dy = theta (mu - y) dt + sigma dW, theta/mu/sigma of length d shared by all paths. */
 typedef struct dfx_sde_problem {
