@@ -18,7 +18,7 @@ from . import _lib
 from ._adjoint import AbstractAdjoint, BacksolveAdjoint, RecursiveCheckpointAdjoint
 from ._saveat import SaveAt, SubSaveAt, save_y
 from ._solution import RESULTS, Solution
-from ._solver import AbstractERK, AbstractSolver
+from ._solver import AbstractERK, AbstractSolver, _device_fsal
 from ._step_size_controller import (ClipStepSizeController, ConstantStepSize, PIDController,
                                     rms_norm)
 from ._term import ControlTerm, IncrementPath, MultiTerm, ODETerm
@@ -491,9 +491,14 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
 
     device = _require_gpu()
     y0b = y0b.to(device).contiguous()
-    t1_t = t1_t.to(device).contiguous()
-    if ts_t is not None:
-        ts_t = ts_t.to(device).contiguous()
+    if ts_t is not None and t1_t.device.type == "cpu" and ts_t.device.type == "cpu":
+        # one copy for both (a small copy from pageable memory costs the host 10 us)
+        both = torch.cat((ts_t.reshape(-1), t1_t)).to(device)
+        ts_t, t1_t = both[:ts_t.numel()].view(ts_t.shape), both[ts_t.numel():]
+    else:
+        t1_t = t1_t.to(device).contiguous()
+        if ts_t is not None:
+            ts_t = ts_t.to(device).contiguous()
     check_times = None
     if on_device:
         checks = _TimeChecks(t0f, t1_t, dt0f, ts_t, device)
@@ -556,7 +561,7 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
             dense_ys=torch.empty((B, int(max_steps) + 1, d), dtype=y0b.dtype, device=device),
             dense_k=torch.empty((B, int(max_steps), S, d), dtype=y0b.dtype, device=device))
     plan = ErkPlan(prob, tensors, n_out, batched, None if launch == "auto" else launch)
-    plan.fsal = bool(solver.tableau.fsal)
+    plan.fsal = _device_fsal(solver.solver_id)
     # checks of device-resident times, run by diffeqsolve once the solve is queued
     plan.deferred_checks = check_times
     return plan

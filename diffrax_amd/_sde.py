@@ -66,19 +66,26 @@ def constant_grid(t0: float, t1: float, dt0: float):
     floor = t1
     for _ in range(100):
         floor = float(np.nextafter(floor, -math.inf))
-    ts = [t0]
-    tnext = min(t0 + dt0, t1)
-    completed = 1
-    tprev = t0
-    while tprev < t1:
-        ts.append(tnext)
-        completed += 1
-        tn = t0 + (t1 - t0) * (completed / num)
-        if completed == num:
-            tn = t1
-        tprev = min(tnext, t1)
-        tnext = t1 if tn > floor else tn
-    return np.array(ts, dtype=np.float64)
+    # step n ends at t0 + (t1 - t0) (n / num), the first at t0 + dt0; ends within 100 ulps of
+    # t1 are t1, and the first end that reaches t1 is the last
+    ends = t0 + (t1 - t0) * (np.arange(1, num + 2, dtype=np.float64) / num)
+    ends[num - 1:] = t1
+    ends[1:][ends[1:] > floor] = t1
+    ends[0] = min(t0 + dt0, t1)
+    last = int(np.argmax(ends >= t1))
+    return np.concatenate(([t0], ends[:last + 1]))
+
+
+def _row_times(grid, ts, save_t0, save_t1, k, t0, t1):
+    """Times of the saved rows, in the kernels' order: t0; per step, the ts inside it and then
+    its end when k divides the step count; t1 unless the last step was saved."""
+    N = len(grid) - 1
+    t = np.empty(0) if ts is None else ts[:np.searchsorted(ts, grid[N], side="right")]
+    at = np.arange(k, N + 1, k) if k else np.empty(0, dtype=np.int64)
+    steps = np.concatenate((np.maximum(np.searchsorted(grid, t, side="left"), 1), at))
+    body = np.concatenate((t, grid[at]))[np.argsort(steps, kind="stable")]
+    return np.concatenate(([t0] if save_t0 else [], body,
+                           [t1] if save_t1 and not (k and N % k == 0) else []))
 
 
 def _ck_for(num_steps, checkpoints):
@@ -223,7 +230,6 @@ def solve_sde(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controller,
     if dW.dtype != torch.float32:
         raise ValueError("dW must be float32")
     dW = dW.to(device).contiguous()
-    grid = torch.tensor(grid_np, dtype=torch.float64, device=device)
     ckpts = adjoint.checkpoints if hasattr(adjoint, "checkpoints") else None
     sub_none = sub is None
     if sub_none:   # dense output only: no saved rows
@@ -240,7 +246,13 @@ def solve_sde(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controller,
             raise RuntimeError("saveat.ts must be increasing (the SDE path runs forward).")
         if ts_np.size and (ts_np[0] < t0f or ts_np[-1] > t1f):
             raise RuntimeError("saveat.ts must lie between t0 and t1.")
-        ts_dev = torch.tensor(ts_np, dtype=torch.float64, device=device)
+    # the grid, the saved rows' times and the save times in one copy
+    rows_np = _row_times(grid_np, ts_np, bool(sub.t0), bool(sub.t1), k, t0f, t1f)
+    parts = [grid_np, rows_np] + ([] if ts_np is None else [ts_np])
+    times = torch.from_numpy(np.concatenate(parts)).to(device)
+    grid, rows = times[:N + 1], times[N + 1:N + 1 + rows_np.size]
+    if ts_np is not None:
+        ts_dev = times[N + 1 + rows_np.size:]
     if saveat.dense:
         if torch.is_grad_enabled() and (y0b.requires_grad or any(
                 a.requires_grad for a in (theta, mu, sigma))):
@@ -256,20 +268,7 @@ def solve_sde(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controller,
         ys = _SdeFunction.apply(y0b, theta, mu, sigma, dW, grid, bool(sub.t0), bool(sub.t1),
                                 ckpts, k, ts_dev)
         interp = None
-    # rows: t0; per step, the ts inside it and then its end when k divides the step count;
-    # t1 unless the last step was saved (the kernels' order)
-    ts_list = [t0f] if sub.t0 else []
-    i = 0
-    n_ts = 0 if ts_np is None else ts_np.size
-    for n in range(N):
-        while i < n_ts and ts_np[i] <= grid_np[n + 1]:
-            ts_list.append(float(ts_np[i]))
-            i += 1
-        if k and (n + 1) % k == 0:
-            ts_list.append(float(grid_np[n + 1]))
-    if sub.t1 and not (k and N % k == 0):
-        ts_list.append(t1f)
-    ts = torch.tensor(ts_list, dtype=torch.float64, device=device).expand(P, len(ts_list))
+    ts = rows.expand(P, rows.numel())
     if not batched:
         ys, ts = ys[0], ts[0]
     if sub_none:

@@ -5,6 +5,7 @@ library (erk_common.hpp) and are read back through dfx_tableau for inspection.""
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -39,6 +40,11 @@ def _device_tableau(solver_id: int) -> ButcherTableau:
         c=np.array(c[1:S]), b_sol=np.array(b[:S]), b_error=np.array(be[:S]),
         a_lower=tuple(A[i, :i].copy() for i in range(1, S)), fsal=bool(info[1]),
         ssal=bool(info[2]), num_stages=S)
+
+
+@functools.lru_cache(maxsize=None)
+def _device_fsal(solver_id: int) -> bool:
+    return _device_tableau(solver_id).fsal
 
 
 class AbstractSolver:

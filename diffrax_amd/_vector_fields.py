@@ -18,6 +18,9 @@ from . import _lib
 
 def _as_batched(values, batch, dtype, device):
     """Stack scalars / [B] tensors into a [P] (shared) or [B, P] (per-instance) tensor."""
+    values = list(values)
+    if all(type(v) in (int, float) for v in values):   # plain numbers: one copy for them all
+        return torch.tensor(values, dtype=dtype, device=device), 0
     cols = [torch.as_tensor(v, dtype=dtype, device=device) for v in values]
     if all(c.ndim == 0 for c in cols):
         return torch.stack(cols).contiguous(), 0
