@@ -17,9 +17,10 @@
 // sweep reads, and a workgroup whose solves fit on it replays nothing: the same records,
 // so the same bits.  The replay, its rejected steps and controller included, was the larger
 // half of this kernel: 65,536 Van der Pol solves with 64 saves (879 attempts at most)
-// 2.35 -> 1.10 ms, for 0.09 ms of stores in the forward; 64 solves 1.23 -> 0.90 ms.  What
-// is left is bound by instruction issue: one wave per SIMD, about 300 instructions per
-// attempt and 110 per save of the lane with the most.
+// 2.35 -> 1.10 ms, for 0.1 ms of stores in the forward.  With branchless loads in the save
+// loop and the tape's loads two rows at a time behind the saves (AdjSweep::tape) 0.73 ms;
+// 64 solves 1.23 -> 0.70 ms.  What is left is bound by instruction issue: one wave per
+// SIMD, about 330 instructions per attempt and 97 per save of the lane with the most.
 //
 // Per accepted step, newest first (one lane per instance):
 //   - its stages are recomputed from the recorded start state, exactly as the forward
@@ -172,7 +173,9 @@ struct AdjSweep {
     --r;
 #pragma unroll
     for (int j = 0; j < D; ++j) grow[j] = grow2[j];
-    load_row(r - 1, grow2);
+    const T* row = g + (int64_t)max(r - 1, 0) * D;  // (a row of its own where r - 1 < 0: unused)
+#pragma unroll
+    for (int j = 0; j < D; ++j) grow2[j] = row[j];
   }
 
   // Accepted steps [lo, hi), newest first, from their records sg (t_start, t_end) and sy
@@ -199,14 +202,40 @@ struct AdjSweep {
 #pragma unroll
         for (int j = 0; j < D; ++j) ny0[j] = sy[(int64_t)(i - 1) * D + j];
       }
-      step(a, s, ts0, ts1, y0, i > 0 ? nts1 : tl);
+      step_saves(a, s, ts0, ts1, i > 0 ? nts1 : tl);
+      step_stages(ts0, ts1, y0);
     }
   }
 
-  // Transposes accepted step s of the instance: from (ts0, ts1, y0), with the save rows in
-  // (prev_end, ts1]; prev_end is the end of step s - 1 (-inf for the first).
-  __device__ __forceinline__ void step(const ErkKArgs& a, int s, double ts0, double ts1,
-                                       const T (&y0)[D], double prev_end) {
+  // Cotangents of a step's end state, start state and stage increments.
+  T gy1[D], gy0[D], gk[S][D];
+  // The transpose of accepted step s over (ts0, ts1), in two parts: the cotangents of the
+  // rows saved in (prev_end, ts1], where prev_end is the end of step s - 1 (-inf for the
+  // first), and then of the step itself from its start state y0.
+  __device__ __forceinline__ void step_saves(const ErkKArgs& a, int s, double ts0, double ts1,
+                                             double prev_end) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      gy1[j] = ab[j];
+      gy0[j] = T(0);
+#pragma unroll
+      for (int m = 0; m < S; ++m) gk[m][j] = T(0);
+    }
+    if (ksave > 0 && (s + 1) % ksave == 0) {  // the step's end state (SaveAt(steps=k))
+#pragma unroll
+      for (int j = 0; j < D; ++j) gy1[j] = gy1[j] + grow[j];
+      next_row();
+    }
+    // SaveAt(ts) rows inside this step: t in (end of the previous step, ts1]
+    while (tsv > prev_end) {  // (-inf after the last: never)
+      erk_interp_vjp<Tab, T, D>(ts0, ts1, tsv, grow, gy0, gy1, gk);
+      --ti;
+      tsv = (ti >= 0) ? tsv2 * dir : -__builtin_inf();
+      tsv2 = tsr[max(ti - 1, 0)];
+      next_row();
+    }
+  }
+  __device__ __forceinline__ void step_stages(double ts0, double ts1, const T (&y0)[D]) {
     T zs[S][D], k[S][D];
     const double dt = ts1 - ts0;
     const T control = T((double)dir * dt);
@@ -227,27 +256,6 @@ struct AdjSweep {
 #pragma unroll
       for (int j = 0; j < D; ++j) k[i][j] = control * f[j];
     });
-    T gy1[D], gy0[D], gk[S][D];
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      gy1[j] = ab[j];
-      gy0[j] = T(0);
-#pragma unroll
-      for (int m = 0; m < S; ++m) gk[m][j] = T(0);
-    }
-    if (ksave > 0 && (s + 1) % ksave == 0) {  // the step's end state (SaveAt(steps=k))
-#pragma unroll
-      for (int j = 0; j < D; ++j) gy1[j] = gy1[j] + grow[j];
-      next_row();
-    }
-    // SaveAt(ts) rows inside this step: t in (end of the previous step, ts1]
-    while (ti >= 0 && tsv > prev_end) {
-      erk_interp_vjp<Tab, T, D>(ts0, ts1, tsv, grow, gy0, gy1, gk);
-      --ti;
-      tsv = (ti >= 0) ? tsv2 * dir : -__builtin_inf();
-      tsv2 = (ti >= 1) ? tsr[ti - 1] : -__builtin_inf();
-      next_row();
-    }
     // y1 = y0 + sum_m b_m k_m
 #pragma unroll
     for (int j = 0; j < D; ++j) gy0[j] = gy0[j] + gy1[j];
@@ -295,31 +303,37 @@ struct AdjSweep {
       while (last > 0 && tt[(int64_t)last * 128 + 1] == -__builtin_inf()) --last;
       setup_rows(a, tt[(int64_t)last * 128 + 1]);
     }
-    double c0 = 0.0, c1 = 0.0, n0 = 0.0, n1 = 0.0;  // rows it and it - 1
-    T cy[D], ny[D];
-    auto load = [&](int it, double& t0, double& t1, T (&y)[D]) {
-      if (it >= 0 && it < tried) {
-        t0 = tt[(int64_t)it * 128];
-        t1 = tt[(int64_t)it * 128 + 1];
+    struct Row { double t0, t1; T y[D]; };
+    // (the row is the wave's, so its offset is scalar; a lane that had not reached it, or a
+    // row before the first, loads a record that it does not use)
+    auto load = [&](int row, Row& r) {
+      const int it = max(row, 0);
+      r.t0 = tt[(int64_t)it * 128];
+      r.t1 = tt[(int64_t)it * 128 + 1];
 #pragma unroll
-        for (int j = 0; j < D; ++j) y[j] = ty[(int64_t)it * 64 * D + j];
-      }
+      for (int j = 0; j < D; ++j) r.y[j] = ty[(int64_t)it * 64 * D + j];
     };
-    load(rows - 1, c0, c1, cy);
-    load(rows - 2, n0, n1, ny);
     int s = n - 1;
-    for (int it = rows - 1; it >= 0; --it) {
-      const double ts0 = c0, ts1 = c1;
-      T y0[D];
-#pragma unroll
-      for (int j = 0; j < D; ++j) { y0[j] = cy[j]; cy[j] = ny[j]; }
-      c0 = n0;
-      c1 = n1;
-      load(it - 2, n0, n1, ny);
-      if (it < tried && s >= 0 && ts1 != -__builtin_inf()) {
-        step(a, s, ts0, ts1, y0, s > 0 ? ts0 : -__builtin_inf());
+    auto row_step = [&](int it, const Row& r, auto&& ahead) __attribute__((always_inline)) {
+      const bool accepted = it < tried && s >= 0 && r.t1 != -__builtin_inf();
+      if (accepted) step_saves(a, s, r.t0, r.t1, s > 0 ? r.t0 : -__builtin_inf());
+      ahead();
+      if (accepted) {
+        step_stages(r.t0, r.t1, r.y);
         --s;
       }
+    };
+    if (rows == 0) return;
+    Row r0, r1, n0, n1;
+    load(rows - 1, r0);
+    load(rows - 2, r1);
+    // Two rows a turn, the next two loaded between the first one's saves and its stages: a
+    // save waits for every load before it, also those it does not use.
+    for (int it = rows - 1; it >= 0; it -= 2) {
+      row_step(it, r0, [&] { load(it - 2, n0); load(it - 3, n1); });
+      if (it > 0) row_step(it - 1, r1, [] {});
+      r0 = n0;
+      r1 = n1;
     }
   }
 
