@@ -530,7 +530,8 @@ def bench_vdp_grad(mu, y0, t1, ts, steps, warmup, with_cpu, forms=("f64", "f32")
         y0_bar = torch.empty((B, 2), dtype=dtype, device=dev)
         mu_bar = torch.empty((B, 1), dtype=dtype, device=dev)
         ws = torch.empty(plan.adjoint_workspace_bytes(), dtype=torch.uint8, device=dev)
-        extra_bytes = T["ckpt"].numel() * 8 + ws.numel()
+        extra_bytes = T["ckpt"].numel() * 8 + ws.numel() + sum(
+            T[k].numel() * T[k].element_size() for k in ("tape", "tape_y") if T[k] is not None)
 
         def adjoint():
             plan.adjoint(gys, y0_bar, mu_bar, workspace=ws)
