@@ -18,8 +18,9 @@
 // so the same bits.  The replay, its rejected steps and controller included, was the larger
 // half of this kernel: 65,536 Van der Pol solves with 64 saves (879 attempts at most)
 // 2.35 -> 1.10 ms, for 0.1 ms of stores in the forward.  With branchless loads in the save
-// loop and the tape's loads two rows at a time behind the saves (AdjSweep::tape) 0.73 ms;
-// 64 solves 1.23 -> 0.70 ms.  What is left is bound by instruction issue: one wave per
+// loop and the tape's loads two rows at a time behind the saves (AdjSweep::tape) 0.73 ms
+// (64 solves 1.23 -> 0.70 ms), 1.26 ms behind the forward and a kernel on its rows; on a
+// SIMD of its own (erk_tape_adjoint_kernel) 0.71 ms there as well.  What is left is bound by instruction issue: one wave per
 // SIMD, about 330 instructions per attempt and 97 per save of the lane with the most.
 //
 // Per accepted step, newest first (one lane per instance):
@@ -357,6 +358,34 @@ struct AdjSweep {
   }
 };
 
+// The most attempts of the 64 instances from `first` on, or -1 where they are not all on the
+// tape (a wave's question: the same for all of its lanes).
+__device__ __forceinline__ int on_tape(const ErkKArgs& a, const DiscreteAdjArgs& b,
+                                       int64_t first) {
+  if (b.tape_steps == 0) return -1;
+  const int64_t id = first + (threadIdx.x & 63);
+  int most = id < a.B ? min(max(b.stats[id * 3], 0), a.max_steps) : 0;
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) most = max(most, __shfl_xor(most, m));
+  most = __builtin_amdgcn_readfirstlane(most);
+  return most <= b.tape_steps ? most : -1;
+}
+
+// The sweep of the workgroups whose solves are on the tape, a wave per 64 instances.  A kernel
+// of its own: as the second wave of the replay's workgroups the sweeps of a CU shared two of
+// its four SIMDs.  Alone as in erk_small_kernel.
+template <class Tab, class VF, class T, bool Alone>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, Alone ? 1 : 8)))
+erk_tape_adjoint_kernel(const ErkKArgs a, const DiscreteAdjArgs b) {
+  const int rows = on_tape(a, b, (int64_t)blockIdx.x * 64);
+  const int64_t id = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (rows < 0 || id >= a.B) return;
+  AdjSweep<Tab, VF, T> W;
+  W.setup(a, b, id, min(max(b.stats[id * 3 + 1], 0), a.max_steps));
+  W.tape(a, b, min(max(b.stats[id * 3], 0), a.max_steps), rows);
+  W.finish(a, b);
+}
+
 // One workgroup of two waves per 64 instances: wave 0 replays, wave 1 sweeps, one segment
 // apart.  At stage s the replay wave restarts segment c_last - s of each of its instances
 // from the checkpoint and records its accepted steps in half (c & 1) of the instance's
@@ -377,29 +406,12 @@ __global__ void __launch_bounds__(128) erk_adjoint_kernel(const ErkKArgs a, cons
   const int K = a.ckpt_every;
   const int n = live ? min(max(b.stats[id * 3 + 1], 0), a.max_steps) : 0;
   const int c_last = n > 0 ? (n - 1) / K : -1;
+  if constexpr (!Extras) {
+    if (on_tape(a, b, (int64_t)blockIdx.x * 64) >= 0) return;  // erk_tape_adjoint_kernel's
+  }
   __shared__ int s_nmax;
   if (threadIdx.x == 0) s_nmax = 0;
   __syncthreads();
-  if constexpr (!Extras) {
-    if (b.tape_steps > 0) {
-      const int tried = live ? min(max(b.stats[id * 3], 0), a.max_steps) : 0;
-      if (role == 0) atomicMax(&s_nmax, tried);
-      __syncthreads();
-      const int rows = __builtin_amdgcn_readfirstlane(s_nmax);
-      if (rows <= b.tape_steps) {  // block-uniform: every attempt is on the tape
-        if (role == 1 && live) {
-          AdjSweep<Tab, VF, T> W;
-          W.setup(a, b, id, n);
-          W.tape(a, b, tried, rows);
-          W.finish(a, b);
-        }
-        return;
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) s_nmax = 0;
-      __syncthreads();
-    }
-  }
   if (role == 0) atomicMax(&s_nmax, n);
   __syncthreads();
   const int nstages = (s_nmax - 1) / K + 2;  // the replay of the oldest segment, then its sweep
@@ -437,6 +449,16 @@ template <class Tab, class VF, class T, int Ctl, bool X>
 static int launch_adjoint_v(const ErkKArgs& a, const ErkKArgs& ra, const DiscreteAdjArgs& b,
                             hipStream_t s) {
   const int64_t nb = (a.B + 63) / 64;
+  if (!X && b.tape_steps > 0) {
+    if (waves_alone(a.B))
+      hipLaunchKernelGGL((erk_tape_adjoint_kernel<Tab, VF, T, true>), dim3((unsigned)nb), dim3(64),
+                         0, s, a, b);
+    else
+      hipLaunchKernelGGL((erk_tape_adjoint_kernel<Tab, VF, T, false>), dim3((unsigned)nb),
+                         dim3(64), 0, s, a, b);
+    if (b.tape_steps >= a.max_steps)  // no solve can outgrow the tape
+      return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
+  }
   hipLaunchKernelGGL((erk_adjoint_kernel<Tab, VF, T, Ctl, X>), dim3((unsigned)nb), dim3(128), 0,
                      s, a, ra, b);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;

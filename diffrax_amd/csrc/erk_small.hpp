@@ -1158,13 +1158,21 @@ __global__ void __launch_bounds__(256) erk_backsolve_kernel(const ErkKArgs a, co
 // One trajectory per lane, no work queue: used when the launch has a lane for every
 // instance.  Lanes whose trajectory has finished idle (masked) until the wave's last lane
 // is done.
+// Whether a batch's waves get a SIMD each (256 CUs of 4).
+inline bool waves_alone(int64_t batch) { return batch <= 64 * 1024; }
+
 // LDS doubles of a wave's save times in the plain kernels (ErkLane::load_times).
 __host__ __device__ inline int64_t plain_lds_doubles(const ErkKArgs& a) {
   return a.n_ts > 0 ? (a.n_ts + 2ll) * (a.ts_stride == 0 ? 1 : 64) : 0;
 }
 
-template <class Tab, class VF, class T, int Ctl, bool Extras, bool Ck = Extras>
-__global__ void __launch_bounds__(256) erk_small_kernel(const ErkKArgs a) {
+// Alone: at most one wave on a SIMD (the build's registers are padded for it).  Of 1,024
+// waves on 1,024 SIMDs the dispatcher put two on 80 to 100 SIMDs whenever a kernel that
+// writes much had run before, and the launch then takes as long as a pair of the longest:
+// 65,536 Van der Pol solves 1.01 ms behind themselves, 1.34 ms behind a 64 MB fill.
+template <class Tab, class VF, class T, int Ctl, bool Extras, bool Ck = Extras, bool Alone = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, Alone ? 1 : 8)))
+erk_small_kernel(const ErkKArgs a) {
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= a.B) return;
   ErkLane<Tab, VF, T, Ctl, Extras, Ck> L;

@@ -14,15 +14,15 @@ static bool plain_fits(const ErkKArgs& a, int block) {
   const int64_t waves = std::min<int64_t>(8, std::max<int64_t>((a.B + 64 * 256 - 1) / (64 * 256), block / 64));
   return wave * (block / 64) <= (64 << 10) && wave * waves <= (160 << 10);
 }
-template <class Tab, class VF, class T>
+template <class Tab, class VF, class T, bool Alone>
 static void launch_small_plain(const ErkKArgs& a, int block, hipStream_t s) {
   const int64_t nb = (a.B + block - 1) / block;
   const size_t lds = (size_t)plain_lds_doubles(a) * 8 * (block / 64);
   if (a.ckpt)
-    hipLaunchKernelGGL((erk_small_kernel<Tab, VF, T, PID_PLAIN, false, true>), dim3((unsigned)nb),
+    hipLaunchKernelGGL((erk_small_kernel<Tab, VF, T, PID_PLAIN, false, true, Alone>), dim3((unsigned)nb),
                        dim3(block), lds, s, a);
   else
-    hipLaunchKernelGGL((erk_small_kernel<Tab, VF, T, PID_PLAIN, false, false>), dim3((unsigned)nb),
+    hipLaunchKernelGGL((erk_small_kernel<Tab, VF, T, PID_PLAIN, false, false, Alone>), dim3((unsigned)nb),
                        dim3(block), lds, s, a);
 }
 
@@ -57,7 +57,8 @@ static int launch_small(const ErkKArgs& a, int block, int64_t lanes, hipStream_t
                  a.resume != 0 || a.state_out != nullptr;
   if (!x && a.controller == DFX_PID && pid_is_plain(a.pid) && !a.grid &&
       a.save_steps == 0 && (a.ckpt || lanes >= a.B) && plain_fits(a, block)) {
-    launch_small_plain<Tab, VF, T>(a, block, s);
+    if (waves_alone(a.B)) launch_small_plain<Tab, VF, T, true>(a, block, s);
+    else launch_small_plain<Tab, VF, T, false>(a, block, s);
   } else if (g) {
     if (x) launch_small_g<Tab, VF, T, PID_GENERIC, true>(a, block, lanes, s);
     else launch_small_g<Tab, VF, T, PID_GENERIC, false>(a, block, lanes, s);
