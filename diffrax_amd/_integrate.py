@@ -878,8 +878,8 @@ def _backsolve_problem(prob, adjoint, stepsize_controller):
 
 class _ErkDiscreteAdjoint(torch.autograd.Function):
     """ys of a small-system solve, with reverse mode through the accepted steps
-    (dfx_erk_adjoint, replaying each segment from the forward's checkpoints) as its
-    backward."""
+    (dfx_erk_adjoint, sweeping the forward's tape or replaying each segment from its
+    checkpoints) as its backward."""
 
     @staticmethod
     def forward(ctx, plan, y0, params):

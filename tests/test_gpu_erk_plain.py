@@ -61,3 +61,17 @@ def test_shared_times_same_bits_as_general(cuda, B, n_ts):
     a, b = (_solve(cuda, torch.float64, dfx.Dopri5(), y0, mu, t1, ts, 4096, m, False)
             for m in (None, np.inf))
     assert a == b
+
+
+def test_more_waves_than_simds(cuda):
+    """One instance past 65,536: the build without a SIMD per wave."""
+    B = 65537
+    rng = np.random.default_rng(7)
+    y0 = rng.uniform(-2.0, 2.0, (B, 2))
+    mu = rng.uniform(0.1, 2.0, B)
+    t1 = rng.uniform(0.5, 2.0, B)
+    ts = np.stack([np.zeros(B), 0.5 * t1, t1], axis=1)
+    for ckpt in (False, True):
+        a, b = (_solve(cuda, torch.float64, dfx.Tsit5(), y0, mu, t1, ts, 256, m, ckpt)
+                for m in (None, np.inf))
+        assert a == b, ckpt

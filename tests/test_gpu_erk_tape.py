@@ -52,3 +52,29 @@ def test_tape_and_replay_same_bits(cuda, solver, B):
     fwd = oracle.solve(y0, t1, mu, ts=ts, save_t0=True, save_t1=True, record_grid=True, **kw)
     ryb, rqb = oracle.adjoint(t1, mu, fwd, 2.0 * fwd["ys"], ts=ts, save_t0=True, save_t1=True, **kw)
     assert np.array_equal(grads[0][0], ryb) and np.array_equal(grads[0][1], rqb)
+
+
+@pytest.mark.parametrize("B", [65536, 65537])
+def test_tape_one_and_two_waves_per_simd(cuda, B):
+    """The sweep's builds with and without a SIMD per wave, against the replay."""
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    y0 = torch.rand(B, 2, generator=gen, device=cuda, dtype=torch.float64) * 2 - 1
+    mu = torch.rand(B, generator=gen, device=cuda, dtype=torch.float64) + 0.2
+    t1 = torch.rand(B, generator=gen, device=cuda, dtype=torch.float64) + 0.5
+    out = []
+    for tape in (True, False):
+        plan = dfx._integrate._prepare_erk(
+            dfx.ODETerm(dfx.VanDerPol()), dfx.Tsit5(), 0.0, t1, 0.1, y0, mu,
+            dfx.SaveAt(ts=torch.stack([0.5 * t1, t1], 1)), dfx.PIDController(rtol=1e-5, atol=1e-7),
+            256, None)
+        plan.record_checkpoints()
+        assert plan.problem.tape_steps == 128
+        if not tape:
+            plan.problem.tape_steps = 0
+        plan.launch()
+        yb = torch.empty((B, 2), dtype=torch.float64, device=cuda)
+        qb = torch.empty((B, 1), dtype=torch.float64, device=cuda)
+        plan.adjoint((2.0 * plan.t["ys"]).contiguous(), yb, qb)
+        out.append((yb, qb))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert bool(torch.isfinite(out[0][0]).all())
