@@ -2,8 +2,8 @@
 
 RecursiveCheckpointAdjoint is the discretise-then-optimise gradient: reverse mode through
 the accepted step sequence, with the step-size factors treated as constants
-(pid.py:498-530).  In diffrax_amd it is realised by hand-written backward kernels that
-replay the recorded accepted-step grid from sqrt(N)-spaced checkpoints.
+(pid.py:498-530).  In diffrax_amd it is realised by hand-written backward kernels over the
+recorded accepted steps, or their replay from sqrt(N)-spaced checkpoints.
 
 BacksolveAdjoint is the optimise-then-discretise gradient: the continuous adjoint
 equations solved backwards in time between consecutive save times, one lane per
@@ -23,10 +23,12 @@ class RecursiveCheckpointAdjoint(AbstractAdjoint):
     checkpoints: number of stored states per trajectory.  The small-system solves
     (LotkaVolterra, VanDerPol, LinearField) store the full step state every
     K = ceil(max_steps / checkpoints) accepted steps, checkpoints = ceil(sqrt(max_steps))
-    when None; the backward pass replays each K-step segment from its checkpoint and
-    sweeps it in reverse, so memory is O(checkpoints + K) per trajectory.  The neural-ODE
-    solve stores a state every K accepted steps by the same rule.  The reference picks ~log(max_steps) checkpoints for its
-    online binomial scheme (_adjoint.py:315-329); both bound memory, the device kernels
+    when None, and the first 8 K attempted steps themselves; the backward pass sweeps those
+    in reverse, or, in longer solves, replays each K-step segment from its checkpoint and
+    sweeps it, so memory is O(checkpoints + K) per trajectory.  The neural-ODE solve stores a
+    state every K accepted steps by the same rule.  The SDE solve saving at t0 and t1 only
+    carries forward sensitivities instead of checkpoints.  The reference picks
+    ~log(max_steps) checkpoints for its online binomial scheme (_adjoint.py:315-329); both bound memory, the device kernels
     use uniform spacing."""
 
     def __init__(self, checkpoints: Optional[int] = None):
