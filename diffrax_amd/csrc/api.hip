@@ -297,7 +297,9 @@ int dfx_erk_solve(const dfx_erk_problem* p, const dfx_erk_io* io, void* workspac
       if (!io->tape || !io->tape_y) return DFX_E_ARG;
       a.tape = io->tape;
       a.tape_y = io->tape_y;
-      a.tape_steps = p->tape_steps;
+      // clipped solves replay (launch_adjoint): a step of theirs may start past the end of
+      // the one before
+      a.tape_steps = p->n_step_ts > 0 || p->n_jump_ts > 0 ? 0 : p->tape_steps;
     }
   }
   a.counter = reinterpret_cast<unsigned int*>(workspace);

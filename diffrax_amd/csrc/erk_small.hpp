@@ -929,8 +929,10 @@ struct ErkLane {
       if (keep) ++num_acc; else ++num_rej;
       if (result == DFX_SUCCESSFUL) result = code;
     }
-    if constexpr (Ck && !Extras) {
-      // The adjoint's tape.  Indexed by the attempt, which the lanes of a wave share, so the
+    if constexpr (Ck) {
+      // The adjoint's tape, in every build that can record checkpoints: the extras builds run
+      // solves that also export their state or dense output, and dfx_erk_adjoint sweeps
+      // whatever tape the problem declares (tape_steps = 0 here with step clipping).  Indexed by the attempt, which the lanes of a wave share, so the
       // 64 records are one contiguous store; records of 64 lanes each in its own row (by
       // accepted step) held up every later load of the loop: 65,536 Van der Pol solves took
       // 1.92 ms that way.

@@ -87,7 +87,8 @@ typedef struct dfx_erk_problem {
   int32_t resume;
   /* With ckpt_every > 0: records per instance of dfx_erk_io.tape, 0 for none.  Solves
    * that attempt no more steps are swept from the tape by dfx_erk_adjoint, without a replay.
-   * Not written with step_ts / jump_ts clipping. */
+   * Every forward with checkpoints writes it, also one that exports its state or dense
+   * output; only with step_ts / jump_ts clipping it is neither written nor read. */
   int32_t tape_steps;
 } dfx_erk_problem;
 
