@@ -512,7 +512,7 @@ def backsolve_problem(plan, adjoint):
     f = plan.prob
     back = MlpProblem()
     ctypes.memmove(ctypes.byref(back), ctypes.byref(f), ctypes.sizeof(f))
-    back.precision = _lib.F32   # float32 MFMA for the backward products (both matmul forms)
+    back.precision = _lib.F32   # float32 MFMA for the backward solves (both matmul forms)
     back.ckpt_every = 0
     back.dt0 = float(kw["dt0"]) if "dt0" in kw else -float(f.dt0)
     back.max_steps = int(kw.get("max_steps", f.max_steps))
@@ -529,7 +529,8 @@ def backsolve_problem(plan, adjoint):
 def backsolve_mlp(plan, back, ys_bar, chunk=BACKSOLVE_CHUNK):
     """Gradients (y0, W1, b1, W2, b2, W3, b3) of sum(ys * ys_bar) by the continuous adjoint
     (dfx_mlp_backsolve), and the backward solves' result codes.  The weights pack for
-    float32 products (the backward runs them in float32 MFMA for either matmul form)."""
+    float32 products (the backward solves run on float32 MFMA for either matmul form; the
+    weight gradients are summed from their rows as the discrete adjoint sums them)."""
     lib = _lib.load()
     dev = plan.ys.device
     B = plan.ys.shape[0]

@@ -151,9 +151,14 @@ class MLPField(RegisteredVectorField):
     """Neural vector field f(t, y) = tanh(W3 softplus(W2 softplus(W1 y + b1) + b2) + b3)
     with d = 64, width 256, depth 2 -- what eqx.nn.MLP(64, 64, 256, 2, activation=softplus,
     final_activation=tanh) computes.  W1 [256, 64], W2 [256, 256], W3 [64, 256] (torch
-    Linear layout: out x in).  ``matmul`` selects the device form: "f32" (float32 MFMA) or
-    "bf16" (bfloat16 MFMA operands, float32 accumulate); the RK algebra is float32 in both
-    and time / step control float64."""
+    Linear layout: out x in).  ``matmul`` selects the device form of the solve's products:
+    "f32" (float32 MFMA) or "bf16" (bfloat16 MFMA on operands in three pieces, float32
+    accumulate); the RK algebra is float32 in both and time / step control float64.  Gradient
+    products are float32 too: in both forms those of RecursiveCheckpointAdjoint and every
+    weight gradient run on three exact bfloat16 pieces of each operand (their errors against
+    float64 are half of float32 MFMA's), and on float32 MFMA where a value is outside the
+    pieces' range (nonzero below 2^-100, or 2^56 and more); with "bf16" the pull-backs of
+    RecursiveCheckpointAdjoint stay in pieces there, as its solve does."""
 
     vf_id = _lib.VF_MLP
     name = "mlp"

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
+#include <type_traits>
 
 #include "../../include/diffrax_amd.h"
 #include "erk_small.hpp"
@@ -45,18 +46,122 @@ struct AdjArgs {
   const float* ys_bar;
   float* ybar;
   float* zs;
-  int32_t* evals;  // out [tiles]: evaluations (row blocks) of each tile
+  int32_t* evals;  // out [tiles]: evaluations (row blocks) of each tile, negative where some
+                   // value is outside the range of the three-piece products (SplitRange)
+  const int32_t* wflags;  // float32 form: nonzero where a weight is outside (kWeightFlags), and
+                          // such tiles are left to the float32 kernel; else null
   int64_t B, B_pad, ts_stride;
   int32_t max_steps, n_ckpt, C, Cs, seg, n_ts, n_out, save_t0;
   double t0, t1;
 };
 
+// The float32 form's LDS: the forward's with partials of their own (h1 is read again after
+// layer 3) and the deltas of layers 3 and 2.
+struct MlpLdsBack : MlpLds<PolicyF32> {
+  float d[MLP_TILE * LDH];
+  float d3[MLP_TILE * LDX];
+  float part_[4 * MLP_TILE * LDP];
+  __device__ __forceinline__ float* part() { return part_; }
+};
+static_assert(sizeof(MlpLdsBack) <= 160 * 1024, "one workgroup per CU");
+
+// The tile's rows of an LDS buffer (columns at PolicyF32::pos) to a block of a row buffer, and
+// back.
+template <int Wd>
+__device__ __forceinline__ void rows_out(const float* lds, int ld, float* dst, int64_t block) {
+  for (int e = threadIdx.x; e < MLP_TILE * Wd / 4; e += blockDim.x) {
+    const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
+    const float* p = lds + (8 * i + 4 * (l >> 5)) * ld + PolicyF32::pos(32 * t + (l & 31));
+    *reinterpret_cast<float4*>(dst + rows_frag(block, Wd, t, i, l)) =
+        make_float4(p[0], p[ld], p[2 * ld], p[3 * ld]);
+  }
+}
+template <int Wd>
+__device__ __forceinline__ void rows_in(float* lds, int ld, const float* src, int64_t block) {
+  for (int e = threadIdx.x; e < MLP_TILE * Wd / 4; e += blockDim.x) {
+    const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
+    float* p = lds + (8 * i + 4 * (l >> 5)) * ld + PolicyF32::pos(32 * t + (l & 31));
+    const float4 v = *reinterpret_cast<const float4*>(src + rows_frag(block, Wd, t, i, l));
+    p[0] = v.x; p[ld] = v.y; p[2 * ld] = v.z; p[3 * ld] = v.w;
+  }
+}
+
+// The vector-Jacobian product of one evaluation on float32 MFMA: from delta3 (L.d3) and the
+// activations (L.h1, L.h2), just stored, to the owners' zb; the deltas to their row block.
+// Leaves delta1 in L.h2.
+template <int NW>
+__device__ __forceinline__ void pull_back_f32(const MlpWeights<PolicyF32>& W, MlpLdsBack& L,
+                                              const RowBufs& R, int64_t block, int wave, int lane,
+                                              int orow, int c0, float (&zb)[MlpWaves<NW>::CPT]) {
+  using P = PolicyF32;
+  using WV = MlpWaves<NW>;
+  constexpr int NT = WV::NT12, NT3 = WV::NT3, F1 = MLP_D / P::KSTEP, F2 = MLP_H / P::KSTEP;
+  const int half = lane >> 5, row = lane & 31;
+  // delta = acc softplus'(h) of the layer whose activations h are given, into dst
+  auto put_delta = [&](const floatx16_t (&acc)[NT], const float* hbuf, float* dst) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int o = row * L.LDH + P::pos(32 * (NT * wave + t) + 8 * i + 4 * half);
+        const float2 he = *reinterpret_cast<const float2*>(hbuf + o);
+        const float2 ho = *reinterpret_cast<const float2*>(hbuf + o + 4);
+        *reinterpret_cast<float2*>(dst + o) =
+            make_float2(acc[t][4 * i] * dsoftplus_from_value(he.x),
+                        acc[t][4 * i + 2] * dsoftplus_from_value(he.y));
+        *reinterpret_cast<float2*>(dst + o + 4) =
+            make_float2(acc[t][4 * i + 1] * dsoftplus_from_value(ho.x),
+                        acc[t][4 * i + 3] * dsoftplus_from_value(ho.y));
+      }
+    }
+  };
+  __syncthreads();
+  rows_out<MLP_D>(L.d3, L.LDX, R.b[4], block);
+  // delta2 = (delta3 . W3) softplus'(h2)
+  floatx16_t acc[NT];
+  GemmF32<F1, NT> g3t;
+  g3t.preload(W.w3t, NT * wave, 0, lane);
+  g3t.template run<F1>(L.d3, L.LDX, 0, acc, lane);
+  put_delta(acc, L.h2, L.d);
+  __syncthreads();
+  // delta1 = (delta2 . W2) softplus'(h1), into the h2 buffer (h2 is in its row buffer)
+  GemmF32<F2, NT> g2t;
+  g2t.preload(W.w2t, NT * wave, 0, lane);
+  g2t.template run<F2>(L.d, L.LDH, 0, acc, lane);
+  put_delta(acc, L.h1, L.h2);
+  __syncthreads();
+  rows_out<MLP_H>(L.d, L.LDH, R.b[2], block);
+  rows_out<MLP_H>(L.h2, L.LDH, R.b[0], block);
+  // zb = delta1 . W1 (split-K over the 256 hidden units)
+  const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+  floatx16_t acc3[NT3];
+  GemmF32<F2, NT3> g1t;
+  g1t.preload(W.w1t, n3, qk * (F2 / 4), lane);
+  g1t.template run<F2 / 4>(L.h2, L.LDH, qk * (F2 / 4), acc3, lane);
+  float* part = L.part();
+  put_partials<NT3>(acc3, part, L.LDP, qk, n3, lane);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < WV::CPT; ++j) {
+    const int c = c0 + j;
+    float sv = part[(0 * MLP_TILE + orow) * L.LDP + c];
+    sv += part[(1 * MLP_TILE + orow) * L.LDP + c];
+    sv += part[(2 * MLP_TILE + orow) * L.LDP + c];
+    sv += part[(3 * MLP_TILE + orow) * L.LDP + c];
+    zb[j] = sv;
+  }
+}
+
 // ---- recompute and reverse sweep of one segment ---------------------------------------------
-// Every product runs on the six-pass three-piece MFMA (wave_gemm3) for both matmul forms:
-// the deltas are split like the activations, so the gradients are those of the
+// P = PolicyBF16x3: every product runs on the six-pass three-piece MFMA (Gemm3) for both matmul
+// forms: the deltas are split like the activations, so the gradients are those of the
 // float32-weight model that both forwards evaluate, and the six bf16 passes take 3/8 of
 // the MFMA time of one float32 pass.  Float32 MFMA throughout took 1.97 ms for the
-// float32 form's segment of 8,192 trajectories and 4 steps.  The row
+// float32 form's segment of 8,192 trajectories and 4 steps.
+// P = PolicyF32, launched behind it by the float32 form: the tiles that the first pass marked,
+// because some weight, layer input or delta of theirs is outside the pieces' range
+// (SplitRange), from their start again on float32 MFMA; every other workgroup ends at once.
+// The row
 // buffers hold float32 values (layer inputs and deltas written before their split into
 // pieces) for the weight-gradient GEMM.  LDS: the forward planes;
 // in the sweep the x planes take delta3, the h1 planes delta2 and then the split-K partials,
@@ -70,17 +175,23 @@ struct AdjArgs {
 // weight-gradient GEMM sees one row block for both.  A tile runs as many steps as its
 // longest trajectory has; evals[tile] tells the GEMM how many of its E = 1 + 6 Cs slots
 // (block tile * E + slot) hold rows.
-// One segment of 8,192 trajectories and up to 4 steps: 0.69 ms; 0.92 ms with seven
+// One segment of 8,192 trajectories and up to 4 steps: 0.70 ms (the range checks 0.01 of
+// it, and 5 us for the float32 launch that finds no tile marked); 0.92 ms with seven
 // pull-backs a step, idle steps run, and the products' loads waited for in the K loop (and
 // the GEMM 0.26 against 0.31 ms for the rows that went).  15 us per evaluation: MFMA, the
 // splits and the LDS stores of one column at a time, one after the other, bound it, not the
 // 1.3 GB of rows.
-template <int NW>
+constexpr int kWeightFlags = MLP_H * (2 * MLP_D + MLP_H) / 256;  // one per 256 weights
+template <class P>
+using AdjLds = std::conditional_t<P::PIECES == 3, MlpLds<P>, MlpLdsBack>;
+
+template <class P, int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
-mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const RowBufs R) {
-  using P = PolicyBF16x3;
+mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) {
+  constexpr bool Pieces = P::PIECES == 3;
+  static_assert(kWeightFlags <= 64 * NW, "a thread per flag");
   extern __shared__ __align__(16) unsigned char smem[];
-  MlpLds<P>& L = *reinterpret_cast<MlpLds<P>*>(smem);
+  AdjLds<P>& L = *reinterpret_cast<AdjLds<P>*>(smem);
   using Tab = Tsit5Tab;
   constexpr int S = Tab::S;
   using WV = MlpWaves<NW>;
@@ -93,10 +204,19 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
   const int nacc = valid ? a.stats[traj * 3 + 1] : 0;
   const int n0 = a.seg * a.C;
   const int steps_here = min(max(nacc - n0, 0), a.Cs);
+  if (!Pieces && a.evals[tile] >= 0) return;
   int tile_steps = 0;
   while (__syncthreads_or(tile_steps < steps_here)) ++tile_steps;
-  if (tid == 0) a.evals[tile] = tile_steps > 0 ? 1 + 6 * tile_steps : 0;
-  if (tile_steps == 0) return;
+  const int evals = tile_steps > 0 ? 1 + 6 * tile_steps : 0;
+  if (Pieces) {
+    const bool weights_out =
+        __syncthreads_or(a.wflags != nullptr && tid < kWeightFlags && a.wflags[tid] != 0);
+    if (tile_steps == 0 || weights_out) {
+      if (tid == 0) a.evals[tile] = -evals;
+      return;
+    }
+  }
+  SplitRange rng;
   const int dir = (a.t0 < a.t1) ? 1 : -1;
   const double* ts_row = a.ts ? a.ts + (valid ? traj : 0) * a.ts_stride : nullptr;
   using TL = TabLit<Tab, float>;
@@ -125,7 +245,15 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
     put_cols(R.b[1], slot, z);
     store_inputs(L, orow, c0, z);
     __syncthreads();
-    mlp_forward_rows<NW>(W, L, wave, lane, orow, c0, f, R.b[3], R.b[5], slot);
+    if constexpr (Pieces) {
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) rng.see(z[j], z[j + 1], z[j + 2], z[j + 3]);
+      mlp_forward_rows<NW>(W, L, wave, lane, orow, c0, f, R.b[3], R.b[5], slot, rng);
+    } else {
+      mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
+      rows_out<MLP_H>(L.h1, L.LDH, R.b[3], slot);
+      rows_out<MLP_H>(L.h2, L.LDH, R.b[5], slot);
+    }
     float* fp = fslot(slot);
 #pragma unroll
     for (int j = 0; j < CPT; ++j) fp[j] = f[j];
@@ -168,61 +296,74 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
   // when it is written.
   auto pull_back = [&](int64_t slot, const float (&fb)[CPT],
                        float (&zb)[CPT]) __attribute__((always_inline)) {
-    constexpr int KS1 = MLP_D / 16, KS2 = MLP_H / 16, HP = MLP_TILE * MlpLds<P>::LDH;
-    float4 h[NT][4];
-    auto load_h = [&](const float* rows) {  // ahead of the product it follows
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          h[t][i] = *reinterpret_cast<const float4*>(rows + rows_frag(slot, MLP_H, NT * wave + t, i, lane));
-      }
-    };
-    floatx16_t acc[NT];
-    auto delta = [&](int t, int i) {
-      return make_float4(acc[t][4 * i] * dsoftplus_from_value(h[t][i].x),
-                         acc[t][4 * i + 1] * dsoftplus_from_value(h[t][i].y),
-                         acc[t][4 * i + 2] * dsoftplus_from_value(h[t][i].z),
-                         acc[t][4 * i + 3] * dsoftplus_from_value(h[t][i].w));
-    };
-    Gemm3<KS1, NT, false> g3;
-    Gemm3<KS2, NT, false> g2;
-    Gemm3<KS2, NT3> g1;
     const float* fp = fslot(slot);
     float d3[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) d3[j] = fb[j] * (1.0f - fp[j] * fp[j]);
-    g3.preload(W.w3t, W.plane3, NT * wave, 0, lane);
-    load_h(R.b[5]);
-    __builtin_amdgcn_sched_barrier(0);
-    put_cols(R.b[4], slot, d3);
-    store_inputs(L, orow, c0, d3);
-    __syncthreads();
-    g3.template run<KS1>(L.x[0], MLP_TILE * MlpLds<P>::LDX, L.LDX, 0, acc, lane);
-    g2.preload(W.w2t, W.plane2, NT * wave, 0, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    put_rows<NW>(L, L.h1[0], R.b[2], slot, wave, lane, delta);
-    load_h(R.b[3]);
-    __syncthreads();
-    g2.template run<KS2>(L.h1[0], HP, L.LDH, 0, acc, lane);
-    const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-    g1.preload(W.w1t, W.plane1, n3, qk * (KS2 / 4), lane);
-    __builtin_amdgcn_sched_barrier(0);
-    put_rows<NW>(L, L.h2[0], R.b[0], slot, wave, lane, delta);
-    __syncthreads();
-    floatx16_t acc3[NT3];
-    g1.template run<KS2 / 4>(L.h2[0], HP, L.LDH, qk * (KS2 / 4), acc3, lane);
-    float* part = L.part();
-    put_partials<NT3>(acc3, part, L.LDP, qk, n3, lane);
-    __syncthreads();
+    if constexpr (!Pieces) {
+      __syncthreads();  // the save weights of other rows lie in the h2 buffer
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const int c = c0 + j;
-      float s = part[(0 * MLP_TILE + orow) * L.LDP + c];
-      s += part[(1 * MLP_TILE + orow) * L.LDP + c];
-      s += part[(2 * MLP_TILE + orow) * L.LDP + c];
-      s += part[(3 * MLP_TILE + orow) * L.LDP + c];
-      zb[j] = s;
+      for (int j = 0; j < CPT; ++j) L.d3[orow * L.LDX + P::pos(c0 + j)] = d3[j];
+      rows_in<MLP_H>(L.h1, L.LDH, R.b[3], slot);
+      rows_in<MLP_H>(L.h2, L.LDH, R.b[5], slot);
+      pull_back_f32<NW>(W, L, R, slot, wave, lane, orow, c0, zb);
+    } else {
+      constexpr int KS1 = MLP_D / 16, KS2 = MLP_H / 16, HP = MLP_TILE * MlpLds<P>::LDH;
+      float4 h[NT][4];
+      auto load_h = [&](const float* rows) {  // ahead of the product it follows
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            h[t][i] = *reinterpret_cast<const float4*>(rows + rows_frag(slot, MLP_H, NT * wave + t, i, lane));
+        }
+      };
+      floatx16_t acc[NT];
+      auto delta = [&](int t, int i) {
+        const float4 v = make_float4(acc[t][4 * i] * dsoftplus_from_value(h[t][i].x),
+                                     acc[t][4 * i + 1] * dsoftplus_from_value(h[t][i].y),
+                                     acc[t][4 * i + 2] * dsoftplus_from_value(h[t][i].z),
+                                     acc[t][4 * i + 3] * dsoftplus_from_value(h[t][i].w));
+        rng.see(v.x, v.y, v.z, v.w);
+        return v;
+      };
+      Gemm3<KS1, NT, false> g3;
+      Gemm3<KS2, NT, false> g2;
+      Gemm3<KS2, NT3> g1;
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) rng.see(d3[j], d3[j + 1], d3[j + 2], d3[j + 3]);
+      g3.preload(W.w3t, W.plane3, NT * wave, 0, lane);
+      load_h(R.b[5]);
+      __builtin_amdgcn_sched_barrier(0);
+      put_cols(R.b[4], slot, d3);
+      store_inputs(L, orow, c0, d3);
+      __syncthreads();
+      g3.template run<KS1>(L.x[0], MLP_TILE * MlpLds<P>::LDX, L.LDX, 0, acc, lane);
+      g2.preload(W.w2t, W.plane2, NT * wave, 0, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      put_rows<NW>(L, L.h1[0], R.b[2], slot, wave, lane, delta);
+      load_h(R.b[3]);
+      __syncthreads();
+      g2.template run<KS2>(L.h1[0], HP, L.LDH, 0, acc, lane);
+      const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
+      g1.preload(W.w1t, W.plane1, n3, qk * (KS2 / 4), lane);
+      __builtin_amdgcn_sched_barrier(0);
+      put_rows<NW>(L, L.h2[0], R.b[0], slot, wave, lane, delta);
+      __syncthreads();
+      floatx16_t acc3[NT3];
+      g1.template run<KS2 / 4>(L.h2[0], HP, L.LDH, qk * (KS2 / 4), acc3, lane);
+      float* part = L.part();
+      put_partials<NT3>(acc3, part, L.LDP, qk, n3, lane);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) {
+        const int c = c0 + j;
+        float s = part[(0 * MLP_TILE + orow) * L.LDP + c];
+        s += part[(1 * MLP_TILE + orow) * L.LDP + c];
+        s += part[(2 * MLP_TILE + orow) * L.LDP + c];
+        s += part[(3 * MLP_TILE + orow) * L.LDP + c];
+        zb[j] = s;
+      }
     }
   };
   // yb: cotangent of the state at the end of step q; fb: of f there, from the next step's
@@ -257,7 +398,7 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
         jlo += __builtin_popcount((unsigned)(__ballot(n > 0 && t <= ta) >> gbase) & grp);
         jhi += __builtin_popcount((unsigned)(__ballot(t <= tb) >> gbase) & grp);
       }
-      float* wts = reinterpret_cast<float*>(L.h2[0]) + orow * GRP * 8;
+      float* wts = reinterpret_cast<float*>(&L.h2[0]) + orow * GRP * 8;
       for (int s0 = jlo; s0 < jhi; s0 += GRP) {
         const int cnt = min(GRP, jhi - s0);
         {
@@ -307,6 +448,11 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
     }
   }
   pull_back(slot0, fb, zb);
+  if constexpr (Pieces) {
+    const bool out = __syncthreads_or(rng.outside());
+    if (tid == 0) a.evals[tile] = out ? -evals : evals;
+    if (out && a.wflags) return;  // left to the float32 kernel
+  }
   if (valid) {
 #pragma unroll
     for (int j = 0; j < CPT; ++j)
@@ -314,9 +460,11 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<PolicyBF16x3> W, const 
   }
 }
 
-// Three-piece planes (mlp_pack_layout(3)) of a float32 packed buffer (mlp_pack_layout(1)).
+// Three-piece planes (mlp_pack_layout(3)) of a float32 packed buffer (mlp_pack_layout(1)), and
+// per workgroup of the first three matrices whether a weight is outside the pieces' range.
 __global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __restrict__ packed,
-                                                               __bf16* __restrict__ out) {
+                                                               __bf16* __restrict__ out,
+                                                               int32_t* __restrict__ wflags) {
   int e = blockIdx.x * 256 + threadIdx.x, m, before;
   mlp_pack_find(e, m, before);
   if (m == 6) return;
@@ -326,6 +474,12 @@ __global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __re
   const float v = packed[before + mlp_frag_index<PolicyF32>(n, k, sh.k)];
   __bf16* o = out + 3 * before + e;
   split3(v, o[0], o[sh.n * sh.k], o[2 * sh.n * sh.k]);
+  if (m < 3) {  // (whole workgroups: the matrices are multiples of 256)
+    SplitRange rng;
+    rng.see(v);
+    const int outside = __syncthreads_or(rng.outside());
+    if (threadIdx.x == 0) wflags[blockIdx.x] = outside;
+  }
 }
 
 // ---- weight gradients of one segment ---------------------------------------------------
@@ -357,11 +511,14 @@ __host__ __device__ inline int dw_chunks(int64_t blocks) {
 // for every 32 x 32 output tile, each wave on a 2 x 2 block of tiles (a 64 x 64 piece of one
 // matrix: dW1 4 x 1, dW2 4 x 4, dW3 1 x 4 pieces).  A lane's sixteen values of a block piece
 // are the rows of its two k halves (rows_frag), so fragments go from memory through the
-// split straight to the MFMAs: six bf16 products per pair of fragments, as in wave_gemm3,
+// split straight to the MFMAs: six bf16 products per pair of fragments, as in Gemm3,
 // with float32 accumulation.  The next block's values load while this one's are split.
 // Waves in the first piece column of a matrix also produce the chunk's column sums of A (the
 // bias gradient partials, partial_db: [chunk][db1 | db2 | db3]).
-// evals: of every `slots` blocks (a tile) only the first evals[tile] hold rows (null: all do).
+// evals: of every `slots` blocks (a tile) only the first |evals[tile]| hold rows (null: all do).
+// A block with values outside the pieces' range (SplitRange) takes float32 MFMA, its rows as
+// the k of v_mfma_f32_32x32x2 (row 8i + j from lane half 0, 8i + 4 + j from half 1): blocks of
+// a tile with negative evals, or, with SC, found here.
 // SC: the rows of A are multiplied by rscale[row] (the backsolve's per-row weights dt * b_i,
 // zero for rejected steps and idle rows; a row of zero weight is dropped from both operands,
 // so a non-finite value in it contributes nothing).
@@ -413,12 +570,16 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
       }
     }
   };
-  // the first block with rows at or after blk (b1: none); lim: the end of its tile's
+  // the first block with rows of tiles marked so, at or after blk (b1: none); lim: the end of
+  // its tile's; found: whether a block outside the pieces' range has been seen
   int64_t lim = evals ? b0 : b1;
-  auto next = [&](int64_t blk) {
+  bool found = false;
+  auto next = [&](int64_t blk, bool marked) {
     while (blk >= lim && blk < b1) {
       const int64_t tile = blk / slots;
-      lim = min(tile * slots + evals[tile], b1);
+      const int n = evals[tile];
+      found = found || n < 0;
+      lim = (n < 0) == marked ? min(tile * slots + abs(n), b1) : blk;
       if (blk >= lim) {
         blk = min((tile + 1) * slots, b1);
         lim = blk;
@@ -426,28 +587,29 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
     }
     return blk;
   };
-  int64_t nxt = next(b0);
-  if (nxt < b1) load(nxt);
-  while (nxt < b1) {
-    const int64_t blk = nxt;
-    nxt = next(blk + 1);
-    if constexpr (SC) {
+  // the loaded block's rows times their weights (SC), and whether it is outside the range then
+  auto scale = [&](int64_t blk) {
+    SplitRange rng;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 w = *reinterpret_cast<const float4*>(rscale + blk * 32 + 8 * i + 4 * half);
+    for (int i = 0; i < 4; ++i) {
+      const float4 w = *reinterpret_cast<const float4*>(rscale + blk * 32 + 8 * i + 4 * half);
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          auto sc = [](float wt, float& da, float& db) {
-            da = (wt != 0.0f) ? da * wt : 0.0f;
-            db = (wt != 0.0f) ? db : 0.0f;
-          };
-          sc(w.x, va[x][i].x, vb[x][i].x);
-          sc(w.y, va[x][i].y, vb[x][i].y);
-          sc(w.z, va[x][i].z, vb[x][i].z);
-          sc(w.w, va[x][i].w, vb[x][i].w);
-        }
+      for (int x = 0; x < 2; ++x) {
+        auto sc = [](float wt, float& da, float& db) {
+          da = (wt != 0.0f) ? da * wt : 0.0f;
+          db = (wt != 0.0f) ? db : 0.0f;
+        };
+        sc(w.x, va[x][i].x, vb[x][i].x);
+        sc(w.y, va[x][i].y, vb[x][i].y);
+        sc(w.z, va[x][i].z, vb[x][i].z);
+        sc(w.w, va[x][i].w, vb[x][i].w);
+        rng.see(va[x][i].x, va[x][i].y, va[x][i].z, va[x][i].w);
+        rng.see(vb[x][i].x, vb[x][i].y, vb[x][i].z, vb[x][i].w);
       }
     }
+    return (bool)__any(rng.outside());
+  };
+  auto add_columns = [&]() {
     if (col_sums) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
@@ -456,6 +618,20 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
           csum[x] += (va[x][i].x + va[x][i].y) + (va[x][i].z + va[x][i].w);
       }
     }
+  };
+  int64_t nxt = next(b0, false);
+  if (nxt < b1) load(nxt);
+  while (nxt < b1) {
+    const int64_t blk = nxt;
+    nxt = next(blk + 1, false);
+    if constexpr (SC) {
+      if (scale(blk)) {  // left to the loop below
+        found = true;
+        if (nxt < b1) load(nxt);
+        continue;
+      }
+    }
+    add_columns();
     // k half s: the rows 16 s .. 16 s + 15 of the block, in the same order for both operands
     frag_t fa[2][2][3], fb[2][2][3];  // [s][x][piece]
     auto split = [&](const float4& u, const float4& v, frag_t (&f)[3]) {
@@ -485,6 +661,33 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
 #pragma unroll
           for (int y = 0; y < 2; ++y)
             acc[x][y] = P::mfma(fa[s][x][pa[pq]], fb[s][y][pb[pq]], acc[x][y]);
+        }
+      }
+    }
+  }
+  if (found) {  // the blocks outside the range (in a loop of their own: beside the pieces'
+                // registers they would spill)
+    lim = evals ? b0 : b1;
+    for (int64_t blk = next(b0, true); blk < b1; blk = next(blk + 1, true)) {
+      load(blk);
+      if constexpr (SC) {
+        if (!scale(blk)) continue;
+      }
+      add_columns();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            auto mm = [&](float p, float q) {
+              acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(p, q, acc[x][y], 0, 0, 0);
+            };
+            mm(va[x][i].x, vb[y][i].x);
+            mm(va[x][i].y, vb[y][i].y);
+            mm(va[x][i].z, vb[y][i].z);
+            mm(va[x][i].w, vb[y][i].w);
+          }
         }
       }
     }
@@ -608,27 +811,6 @@ struct BsArgs {
   PidParams pid;         // the backward controller
 };
 
-// The forward's LDS with partials of their own (h1 is read again after layer 3) and the
-// deltas of layers 3 and 2.
-struct MlpLdsBack : MlpLds<PolicyF32> {
-  float d[MLP_TILE * LDH];
-  float d3[MLP_TILE * LDX];
-  float part_[4 * MLP_TILE * LDP];
-  __device__ __forceinline__ float* part() { return part_; }
-};
-static_assert(sizeof(MlpLdsBack) <= 160 * 1024, "one workgroup per CU");
-
-// The tile's rows of an LDS buffer (columns at PolicyF32::pos) to a block of a row buffer.
-template <int Wd>
-__device__ __forceinline__ void rows_out(const float* lds, int ld, float* dst, int64_t block) {
-  for (int e = threadIdx.x; e < MLP_TILE * Wd / 4; e += blockDim.x) {
-    const int l = e & 63, i = (e >> 6) & 3, t = e >> 8;
-    const float* p = lds + (8 * i + 4 * (l >> 5)) * ld + PolicyF32::pos(32 * t + (l & 31));
-    *reinterpret_cast<float4*>(dst + rows_frag(block, Wd, t, i, l)) =
-        make_float4(p[0], p[ld], p[2 * ld], p[3 * ld]);
-  }
-}
-
 template <int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
 mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBufs R) {
@@ -723,25 +905,6 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
   }
 
   mlp_begin<P>(W, L);  // the first iteration's barriers come before its first use
-  const int half = lane >> 5, row = lane & 31;
-  // delta = acc softplus'(h) of the layer whose activations h are given, into dst
-  auto put_delta = [&](const floatx16_t (&acc)[NT], const float* hbuf, float* dst) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int o = row * L.LDH + P::pos(32 * (NT * wave + t) + 8 * i + 4 * half);
-        const float2 he = *reinterpret_cast<const float2*>(hbuf + o);
-        const float2 ho = *reinterpret_cast<const float2*>(hbuf + o + 4);
-        *reinterpret_cast<float2*>(dst + o) =
-            make_float2(acc[t][4 * i] * dsoftplus_from_value(he.x),
-                        acc[t][4 * i + 2] * dsoftplus_from_value(he.y));
-        *reinterpret_cast<float2*>(dst + o + 4) =
-            make_float2(acc[t][4 * i + 1] * dsoftplus_from_value(ho.x),
-                        acc[t][4 * i + 3] * dsoftplus_from_value(ho.y));
-      }
-    }
-  };
   const int64_t rb0 = (int64_t)tile * MLP_TILE + orow;
   const int64_t ntiles = a.B_pad / MLP_TILE;
   int q = 0;
@@ -782,48 +945,12 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
 #pragma unroll
       for (int j = 0; j < CPT; ++j)
         L.d3[orow * L.LDX + P::pos(c0 + j)] = -za[j] * (1.0f - f[j] * f[j]);
-      __syncthreads();
-      rows_out<MLP_D>(L.d3, L.LDX, R.b[4], block);
-      // delta2 = (delta3 . W3) softplus'(h2)
-      constexpr int F1 = MLP_D / P::KSTEP, F2 = MLP_H / P::KSTEP;
-      floatx16_t acc[NT];
-      GemmF32<F1, NT> g3t;
-      g3t.preload(W.w3t, NT * wave, 0, lane);
-      g3t.template run<F1>(L.d3, L.LDX, 0, acc, lane);
-      put_delta(acc, L.h2, L.d);
-      __syncthreads();
-      // delta1 = (delta2 . W2) softplus'(h1), into the h2 buffer (h2 is in its row buffer)
-      GemmF32<F2, NT> g2t;
-      g2t.preload(W.w2t, NT * wave, 0, lane);
-      g2t.template run<F2>(L.d, L.LDH, 0, acc, lane);
-      put_delta(acc, L.h1, L.h2);
-      __syncthreads();
-      rows_out<MLP_H>(L.d, L.LDH, R.b[2], block);
-      rows_out<MLP_H>(L.h2, L.LDH, R.b[0], block);
-      // vjp_y = delta1 . W1 (split-K over the 256 hidden units)
-      const int qk = WV::quarter(wave), n3 = WV::nt3(wave);
-      floatx16_t acc3[NT3];
-      GemmF32<F2, NT3> g1t;
-      g1t.preload(W.w1t, n3, qk * (F2 / 4), lane);
-      g1t.template run<F2 / 4>(L.h2, L.LDH, qk * (F2 / 4), acc3, lane);
-      float* part = L.part();
-#pragma unroll
-      for (int t = 0; t < NT3; ++t) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<float4*>(part + (qk * MLP_TILE + row) * L.LDP + 32 * (n3 + t) + 8 * i + 4 * half) =
-              make_float4(acc3[t][4 * i], acc3[t][4 * i + 1], acc3[t][4 * i + 2], acc3[t][4 * i + 3]);
-      }
-      __syncthreads();
+      float sv[CPT];
+      pull_back_f32<NW>(W, L, R, block, wave, lane, orow, c0, sv);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        const int c = c0 + j;
-        float sv = part[(0 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(1 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(2 * MLP_TILE + orow) * L.LDP + c];
-        sv += part[(3 * MLP_TILE + orow) * L.LDP + c];
         ky[i][j] = control * f[j];
-        ka[i][j] = control * sv;
+        ka[i][j] = control * sv[j];
       }
       __syncthreads();
     });
@@ -989,7 +1116,7 @@ void launch_dw(const RowBufs& R, float* partial, int64_t blocks, const int32_t* 
 }
 
 // Floats of the weight-gradient partials of `blocks` row blocks; behind them, for a segment,
-// come its tiles' evaluation counts and (float32 form) the three-piece planes of the weights.
+// come its tiles' evaluation counts and (float32 form) the weights' flags and three-piece planes.
 int64_t partial_floats(int64_t blocks) {
   return (dw_chunks(blocks) * ((int64_t)dw_layout().first[3] * 1024 + 2 * MLP_H + MLP_D) + 63) / 64 * 64;
 }
@@ -1014,14 +1141,18 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   const int slots = 1 + 6 * seg_steps;
   const int64_t ntiles64 = a.B_pad / MLP_TILE, blocks = ntiles64 * slots;
   a.evals = reinterpret_cast<int32_t*>(io->partial + partial_floats(blocks));
-  if (p->precision == DFX_F32) {
-    __bf16* planes = reinterpret_cast<__bf16*>(a.evals + (ntiles64 + 63) / 64 * 64);
+  const bool f32 = p->precision == DFX_F32;
+  const void* pieces = packed;
+  if (f32) {
+    int32_t* wflags = a.evals + (ntiles64 + 63) / 64 * 64;
+    __bf16* planes = reinterpret_cast<__bf16*>(wflags + kWeightFlags);
     const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);
     hipLaunchKernelGGL(mlp_split_packed_kernel, dim3(nb), dim3(256), 0, s,
-                       reinterpret_cast<const float*>(packed), planes);
-    packed = planes;
+                       reinterpret_cast<const float*>(packed), planes, wflags);
+    pieces = planes;
+    a.wflags = wflags;
   }
-  const MlpWeights<P> W = mlp_weights_from<P>(packed, P::PIECES, b1, b2, b3);
+  const MlpWeights<P> W = mlp_weights_from<P>(pieces, P::PIECES, b1, b2, b3);
   RowBufs R;
   const int64_t rows_alloc = seg_chunks(p->batch, seg_steps) * ADJ_CHUNK;
   float* base = reinterpret_cast<float*>(io->rows);
@@ -1029,10 +1160,15 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
   for (int i = 0; i < 6; ++i) { R.b[i] = base + off; off += rows_alloc * widths[i]; }
   const unsigned ntiles = (unsigned)ntiles64;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_adj_segment_kernel<NW>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLds<P>));
-  hipLaunchKernelGGL(mlp_adj_segment_kernel<NW>, dim3(ntiles), dim3(64 * NW), sizeof(MlpLds<P>), s,
-                     a, W, R);
+  auto sweep = [&](auto policy, auto&& w) {
+    using Q = decltype(policy);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_adj_segment_kernel<Q, NW>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(AdjLds<Q>));
+    hipLaunchKernelGGL((mlp_adj_segment_kernel<Q, NW>), dim3(ntiles), dim3(64 * NW),
+                       sizeof(AdjLds<Q>), s, a, w, R);
+  };
+  sweep(P{}, W);
+  if (f32) sweep(PolicyF32{}, mlp_weights_from<PolicyF32>(packed, 1, b1, b2, b3));
   launch_dw<false>(R, io->partial, blocks, a.evals, slots, nullptr, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
@@ -1054,7 +1190,8 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
   const int64_t ntiles = Bp / MLP_TILE;
   *partial_bytes = (size_t)(partial_floats(ntiles * (1 + 6 * seg_steps)) + (ntiles + 63) / 64 * 64) *
                    sizeof(float);
-  if (p->precision == DFX_F32) *partial_bytes += (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
+  if (p->precision == DFX_F32)
+    *partial_bytes += kWeightFlags * sizeof(int32_t) + (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
 }
 
@@ -1101,8 +1238,8 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   a.n_out = n_out; a.save_t0 = back->save_t0; a.max_steps = back->max_steps;
   a.Q = chunk_iters; a.first = first ? 1 : 0;
   a.t0 = back->t0; a.dt0 = back->dt0;
-  // The products run in float32 MFMA for both matmul forms (the caller packs the weights
-  // for DFX_F32): the bfloat16 form's forward evaluates the float32-weight model too.
+  // The backward solves run on float32 MFMA for both matmul forms (the caller packs the
+  // weights for DFX_F32): the bfloat16 form's forward evaluates the float32-weight model too.
   using P = PolicyF32;
   const MlpWeights<P> W = mlp_weights_from<P>(packed, 1, b1, b2, b3);
   RowBufs R;
