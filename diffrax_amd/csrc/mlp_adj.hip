@@ -500,11 +500,14 @@ __host__ __device__ inline DwLayout dw_layout() {
 constexpr int kXcds = 8;
 
 // Chunks of row blocks the GEMM splits K into: 24 one-wave workgroups (64 x 64 output
-// pieces) each, two per SIMD of the chip resident at once, so at most 80 chunks (1,920
-// waves), and no more than there are four-block chunks.
+// pieces) each, two per SIMD of the chip resident at once, so 80 chunks (1,920 waves), but no
+// more than there are four-block chunks, and enough that none has more than 128 blocks: the
+// float32 accumulators' rounding grows with their 4,096 rows (8,192 trajectories and 64 steps,
+// 98,560 blocks: 770 chunks; with 80 the sums were off by 6e-6 of the largest, now by 1.4e-6).
 __host__ __device__ inline int dw_chunks(int64_t blocks) {
-  const int64_t n = (blocks + 3) / 4;
-  return (int)(n < 80 ? (n < 1 ? 1 : n) : 80);
+  const int64_t few = (blocks + 3) / 4, most = (blocks + 127) / 128;
+  const int64_t n = few < 80 ? few : (most > 80 ? most : 80);
+  return (int)(n < 1 ? 1 : n);
 }
 
 // partial[chunk][tile] = A^T B over one chunk of row blocks (A = deltas, B = layer inputs)
