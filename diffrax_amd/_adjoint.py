@@ -23,9 +23,11 @@ class RecursiveCheckpointAdjoint(AbstractAdjoint):
     checkpoints: number of stored states per trajectory.  The small-system solves
     (LotkaVolterra, VanDerPol, LinearField) store the full step state every
     K = ceil(max_steps / checkpoints) accepted steps, checkpoints = ceil(sqrt(max_steps))
-    when None, and the first 8 K attempted steps themselves; the backward pass sweeps those
-    in reverse, or, in longer solves, replays each K-step segment from its checkpoint and
-    sweeps it, so memory is O(checkpoints + K) per trajectory.  The neural-ODE solve stores a
+    when None, and the first 8 K attempted steps themselves (with a given number as many of
+    them as take the checkpoints' bytes, and none if that is less than 2 K); the backward
+    pass sweeps those in reverse, or, in longer solves, replays each K-step segment from its
+    checkpoint and sweeps it, so memory is O(checkpoints + K) per trajectory, O(checkpoints)
+    of it from the forward solve until its graph is freed.  The neural-ODE solve stores a
     state every K accepted steps by the same rule.  The SDE solve saving at t0 and t1 only
     carries forward sensitivities instead of checkpoints.  The reference picks
     ~log(max_steps) checkpoints for its online binomial scheme (_adjoint.py:315-329); both bound memory, the device kernels

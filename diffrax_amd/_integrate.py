@@ -174,8 +174,8 @@ class ErkPlan:
         adjoint: K = ceil(max_steps / checkpoints), checkpoints = ceil(sqrt(max_steps)) when
         None (RecursiveCheckpointAdjoint.checkpoints, _adjoint.py:264-329).  Memory is
         [B, ceil(max_steps / K), d + 8] float64 and a tape of up to 8K attempted steps
-        (``_tape_steps``) here, and [B, 2K] records of (2 + d) values in the adjoint's
-        workspace."""
+        (``_tape_steps``; with a given count no larger than the checkpoints) here, as long as
+        this plan lives, and [B, 2K] records of (2 + d) values in the adjoint's workspace."""
         M = max(int(self.problem.max_steps), 1)
         c = int(math.ceil(math.sqrt(M))) if checkpoints is None else int(checkpoints)
         if c < 1:
@@ -189,7 +189,7 @@ class ErkPlan:
         B, d = y0.shape
         self.t["ckpt"] = torch.empty((B, n_ck.value, words.value), dtype=torch.float64,
                                      device=y0.device)
-        n = self._tape_steps(M)
+        n = self._tape_steps(M, None if checkpoints is None else n_ck.value * words.value * 8)
         self.problem.tape_steps = n
         W = -(-B // 64)
         self.t["tape"] = (torch.empty((W, n, 64, 2), dtype=torch.float64, device=y0.device)
@@ -200,14 +200,17 @@ class ErkPlan:
 
     # The tape: what a sweep needs of an attempted step (16 + d * itemsize bytes).  A solve
     # that fits on it is swept without replaying its steps; a longer one replays from the
-    # checkpoints.  8K steps keep the memory at O(B sqrt(max_steps)) by default.
+    # checkpoints.  8K steps keep the memory at O(B sqrt(max_steps)) by default; a caller who
+    # gives a number of checkpoints bounds the memory by it, and K grows as they get fewer,
+    # so the tape then takes no more bytes than they do.
     TAPE_BYTES = 4 << 30          # of one solve
     TAPE_SMALL_BYTES = 64 << 20   # below this, taken without asking the driver
 
-    def _tape_steps(self, max_steps):
-        """Records per instance: min(max_steps, 8K) within TAPE_BYTES, or 0 where that is
-        less than two segments or would leave under 3/4 of the device's memory free (the
-        tape is a convenience: a program near the card's memory runs as without it)."""
+    def _tape_steps(self, max_steps, limit=None):
+        """Records per instance: min(max_steps, 8K) within TAPE_BYTES and ``limit`` bytes per
+        instance, or 0 where that is less than two segments or would leave under 3/4 of the
+        device's memory free (the tape is a convenience: a program near the card's memory runs
+        as without it)."""
         y0 = self.t["y0"]
         B, d = y0.shape
         if self.problem.n_step_ts or self.problem.n_jump_ts:
@@ -216,6 +219,8 @@ class ErkPlan:
         K = int(self.problem.ckpt_every)
         rec = 16 + d * y0.element_size()
         n = min(max_steps, 8 * K, self.TAPE_BYTES // max(B * rec, 1))
+        if limit is not None:
+            n = min(n, limit // rec)
         if n < min(max_steps, 2 * K):
             return 0
         if B * n * rec > self.TAPE_SMALL_BYTES:
