@@ -190,12 +190,16 @@ class ErkPlan:
         self.t["ckpt"] = torch.empty((B, n_ck.value, words.value), dtype=torch.float64,
                                      device=y0.device)
         n = self._tape_steps(M, None if checkpoints is None else n_ck.value * words.value * 8)
+        tape = tape_y = None
+        if n:
+            W = -(-B // 64)
+            try:
+                tape = torch.empty((W, n, 64, 2), dtype=torch.float64, device=y0.device)
+                tape_y = torch.empty((W, n, 64, d), dtype=y0.dtype, device=y0.device)
+            except torch.OutOfMemoryError:
+                n, tape, tape_y = 0, None, None   # replayed instead
         self.problem.tape_steps = n
-        W = -(-B // 64)
-        self.t["tape"] = (torch.empty((W, n, 64, 2), dtype=torch.float64, device=y0.device)
-                          if n else None)
-        self.t["tape_y"] = (torch.empty((W, n, 64, d), dtype=y0.dtype, device=y0.device)
-                            if n else None)
+        self.t["tape"], self.t["tape_y"] = tape, tape_y
         self._bind()
 
     # The tape: what a sweep needs of an attempted step (16 + d * itemsize bytes).  A solve
@@ -209,8 +213,9 @@ class ErkPlan:
     def _tape_steps(self, max_steps, limit=None):
         """Records per instance: min(max_steps, 8K) within TAPE_BYTES and ``limit`` bytes per
         instance, or 0 where that is less than two segments or would leave under 3/4 of the
-        device's memory free (the tape is a convenience: a program near the card's memory runs
-        as without it)."""
+        device's memory, or of this process's share of it, free (the tape is a convenience: a
+        program near the card's memory, or near the fraction that it may use, runs as without
+        it)."""
         y0 = self.t["y0"]
         B, d = y0.shape
         if self.problem.n_step_ts or self.problem.n_jump_ts:
@@ -223,13 +228,14 @@ class ErkPlan:
             n = min(n, limit // rec)
         if n < min(max_steps, 2 * K):
             return 0
-        if B * n * rec > self.TAPE_SMALL_BYTES:
+        share = torch.cuda.get_per_process_memory_fraction(y0.device)
+        if B * n * rec > self.TAPE_SMALL_BYTES or share < 1.0:
             if torch.cuda.is_current_stream_capturing():
                 return 0
             free, total = torch.cuda.mem_get_info(y0.device)
-            free += (torch.cuda.memory_reserved(y0.device)
-                     - torch.cuda.memory_allocated(y0.device))
-            if free - B * n * rec < total * 3 // 4:
+            used = torch.cuda.memory_allocated(y0.device)
+            free = min(free + torch.cuda.memory_reserved(y0.device) - used, share * total - used)
+            if free - B * n * rec < 0.75 * share * total:
                 return 0
         return n
 
