@@ -29,7 +29,8 @@ class RecursiveCheckpointAdjoint(AbstractAdjoint):
     checkpoint and sweeps it, so memory is O(checkpoints + K) per trajectory, O(checkpoints)
     of it from the forward solve until its graph is freed.  The neural-ODE solve stores a
     state every K accepted steps by the same rule.  The SDE solve saving at t0 and t1 only
-    carries forward sensitivities instead of checkpoints.  The reference picks
+    carries forward sensitivities instead of checkpoints, unless the given number of these
+    takes less memory.  The reference picks
     ~log(max_steps) checkpoints for its online binomial scheme (_adjoint.py:315-329); both bound memory, the device kernels
     use uniform spacing."""
 

@@ -112,9 +112,12 @@ class _Sde:
                                save_steps=int(save_steps),
                                n_ts=0 if ts is None else int(ts.numel()))
         # the gradient's record: the derivatives of y(t1), or checkpoints where rows between
-        # t0 and t1 carry cotangents too
+        # t0 and t1 carry cotangents too, or where the caller asked for fewer of them than the
+        # derivatives take (16 bytes per component: four float32 states, two float64 ones)
         words = int(lib.dfx_sde_sens_words(ctypes.byref(self.prob))) if need_grad else 0
         n_ck = lib.dfx_sde_n_ckpt(ctypes.byref(self.prob)) if need_grad else 0
+        if checkpoints is not None and words * 8 > n_ck * y0.numel() * y0.element_size():
+            words = 0
         self.n_out = int(lib.dfx_sde_n_out(ctypes.byref(self.prob)))
         self.ys = torch.empty((self.P, self.n_out, self.d), dtype=y0.dtype, device=y0.device)
         self.ckpt = (torch.empty((max(n_ck, 1), self.P, self.d), dtype=y0.dtype, device=y0.device)
