@@ -12,6 +12,8 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdiffrax_amd.so")
 
+VERSION = 200   # DFX_VERSION of the header that the structures below follow
+
 # enums (include/diffrax_amd.h)
 TSIT5, DOPRI5, HEUN = 0, 1, 2
 PID, CONSTANT = 0, 1
@@ -141,6 +143,10 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = restype
+    if lib.dfx_version() != VERSION:
+        raise LibraryMissing(
+            f"{LIB_PATH} has version {lib.dfx_version()}, this package needs {VERSION}: build "
+            "it again with `make -C diffrax_amd/csrc` (or __graft_entry__.build()).")
     _lib = lib
     return lib
 

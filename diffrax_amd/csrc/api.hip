@@ -179,7 +179,7 @@ int fill_erk_inputs(const dfx_erk_problem* p, const dfx_erk_io* io, ErkKArgs& a)
 
 extern "C" {
 
-int dfx_version(void) { return 100; }
+int dfx_version(void) { return DFX_VERSION; }
 
 const char* dfx_strerror(int code) {
   switch (code) {

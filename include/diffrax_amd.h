@@ -29,6 +29,13 @@
 extern "C" {
 #endif
 
+/* Version of this interface: major*10000 + minor*100 + patch.  The minor number grows with
+ * every change of a struct's layout or of a packed buffer's: a program is for the library
+ * whose dfx_version() returns the DFX_VERSION that it was compiled with, and passes structs
+ * that are too short to a later one.  0.2.0: dfx_erk_problem.tape_steps, dfx_erk_io.tape and
+ * tape_y, dfx_sde_io.sens, the float32 packing of dfx_mlp_pack. */
+#define DFX_VERSION 200
+
 /* ---- enums ---------------------------------------------------------------------- */
 enum { DFX_TSIT5 = 0, DFX_DOPRI5 = 1, DFX_HEUN = 2 };          /* solver              */
 enum { DFX_PID = 0, DFX_CONSTANT = 1 };                         /* stepsize controller */
@@ -162,7 +169,7 @@ typedef struct dfx_launch {
   int32_t lanes;        /* total persistent lanes (trajectory slots); 0 = batch      */
 } dfx_launch;
 
-/* Library version: major*10000 + minor*100 + patch. */
+/* The DFX_VERSION that the library was built with. */
 int dfx_version(void);
 const char* dfx_strerror(int code);
 /* Number of saved rows per instance: t0 + n_ts + (steps ? max_steps : 0) + t1
