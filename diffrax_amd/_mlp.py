@@ -628,9 +628,9 @@ def checkpoint_every(adjoint, max_steps):
 
 def set_waves(plan, launch):
     """The tile's wave count from diffeqsolve's ``launch``: None keeps the library default
-    (8; 4 for float32 batches of more than 256 tiles), 4 or 8 selects it, "auto" times both
-    once per problem signature and device (_autotune.tune_mlp).  The results are the same
-    bits either way."""
+    (8; 4 for float32 batches of more than a tile per compute unit), 4 or 8 selects it, "auto"
+    times both once per problem signature and device (_autotune.tune_mlp).  The results are
+    the same bits either way."""
     if launch is None:
         return
     if launch == "auto":

@@ -35,6 +35,7 @@
 // its derivative is that of f(y0) of the next step.
 #pragma once
 #include "erk_small.hpp"
+#include "launch_rules.hpp"
 
 namespace dfx {
 
@@ -450,7 +451,7 @@ static int launch_adjoint_v(const ErkKArgs& a, const ErkKArgs& ra, const Discret
                             hipStream_t s) {
   const int64_t nb = (a.B + 63) / 64;
   if (!X && b.tape_steps > 0) {
-    if (waves_alone(a.B))
+    if (waves_alone(a.B, device_cus()))
       hipLaunchKernelGGL((erk_tape_adjoint_kernel<Tab, VF, T, true>), dim3((unsigned)nb), dim3(64),
                          0, s, a, b);
     else

@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include "erk_mlp.hpp"
+#include "launch_rules.hpp"
 
 namespace dfx {
 
@@ -267,14 +268,8 @@ int dfx_mlp_solve(const dfx_mlp_problem* p, const void* packed, const float* b1,
   const bool integral = mlp_pid_params(p, a.pid);
   const unsigned nblocks = (unsigned)((p->batch + MLP_TILE - 1) / MLP_TILE);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // waves per tile (MlpWaves): the problem's choice, or by default eight, two per SIMD, for
-  // the three-piece form (its registers at four waves leave one wave per SIMD) and for
-  // float32 batches of at most one tile per CU; larger float32 batches take four, of which
-  // two workgroups share a CU and fill each other's barriers (solves of 8,192, 10,007 and
-  // 16,384 trajectories: 416, 776 and 785 us at eight, 427, 743 and 756 us at four)
-  constexpr unsigned kCus = 256;
   const int waves = p->waves != 0 ? p->waves
-                    : (p->precision == DFX_BF16_F32 || nblocks <= kCus) ? 8 : 4;
+                                  : mlp_tile_waves(p->precision == DFX_BF16_F32, nblocks, device_cus());
   const bool g = p->ckpt_every > 0;
   if (p->precision == DFX_BF16_F32)
     launch_erk_mlp_bf16(waves, a, weights_from<PolicyBF16x3>(packed, b1, b2, b3), g, integral,

@@ -1157,17 +1157,14 @@ __global__ void __launch_bounds__(256) erk_backsolve_kernel(const ErkKArgs a, co
   b.result[id] = res;
 }
 
-// One trajectory per lane, no work queue: used when the launch has a lane for every
-// instance.  Lanes whose trajectory has finished idle (masked) until the wave's last lane
-// is done.
-// Whether a batch's waves get a SIMD each (256 CUs of 4).
-inline bool waves_alone(int64_t batch) { return batch <= 64 * 1024; }
-
 // LDS doubles of a wave's save times in the plain kernels (ErkLane::load_times).
 __host__ __device__ inline int64_t plain_lds_doubles(const ErkKArgs& a) {
   return a.n_ts > 0 ? (a.n_ts + 2ll) * (a.ts_stride == 0 ? 1 : 64) : 0;
 }
 
+// One trajectory per lane, no work queue: used when the launch has a lane for every
+// instance.  Lanes whose trajectory has finished idle (masked) until the wave's last lane
+// is done.
 // Alone: at most one wave on a SIMD (the build's registers are padded for it).  Of 1,024
 // waves on 1,024 SIMDs the dispatcher put two on 80 to 100 SIMDs whenever a kernel that
 // writes much had run before, and the launch then takes as long as a pair of the longest:

@@ -1,19 +1,12 @@
 // erk_small_dispatch.hpp -- instantiates the small-system kernel for one state type and
 // maps (solver, vector field, d) to a kernel.  Included once per precision build.
 #pragma once
-#include <algorithm>
 #include "erk_small.hpp"
+#include "launch_rules.hpp"
 
 namespace dfx {
 
-// The default solve on a lane per instance (PID_PLAIN), where the save times of the waves
-// that a CU holds at once (by the batch; 8 by registers) fit in its LDS: with fewer resident
-// 131,072 instances with 64 saves take 2.2 ms, in the general build 1.9 ms.
-static bool plain_fits(const ErkKArgs& a, int block) {
-  const int64_t wave = plain_lds_doubles(a) * 8;
-  const int64_t waves = std::min<int64_t>(8, std::max<int64_t>((a.B + 64 * 256 - 1) / (64 * 256), block / 64));
-  return wave * (block / 64) <= (64 << 10) && wave * waves <= (160 << 10);
-}
+// The default solve on a lane per instance (PID_PLAIN).
 template <class Tab, class VF, class T, bool Alone>
 static void launch_small_plain(const ErkKArgs& a, int block, hipStream_t s) {
   const int64_t nb = (a.B + block - 1) / block;
@@ -55,9 +48,11 @@ static int launch_small(const ErkKArgs& a, int block, int64_t lanes, hipStream_t
   const bool g = a.controller == DFX_PID && !pid_is_fifth(a.pid);
   const bool x = a.dense_ts != nullptr || a.n_step_ts > 0 || a.n_jump_ts > 0 || a.n_events > 0 ||
                  a.resume != 0 || a.state_out != nullptr;
+  const int cus = device_cus();
   if (!x && a.controller == DFX_PID && pid_is_plain(a.pid) && !a.grid &&
-      a.save_steps == 0 && (a.ckpt || lanes >= a.B) && plain_fits(a, block)) {
-    if (waves_alone(a.B)) launch_small_plain<Tab, VF, T, true>(a, block, s);
+      a.save_steps == 0 && (a.ckpt || lanes >= a.B) &&
+      save_times_fit(plain_lds_doubles(a) * 8, a.B, block, cus)) {
+    if (waves_alone(a.B, cus)) launch_small_plain<Tab, VF, T, true>(a, block, s);
     else launch_small_plain<Tab, VF, T, false>(a, block, s);
   } else if (g) {
     if (x) launch_small_g<Tab, VF, T, PID_GENERIC, true>(a, block, lanes, s);

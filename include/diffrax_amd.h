@@ -419,7 +419,7 @@ typedef struct dfx_mlp_problem {
   double factormin, factormax, safety, error_order;
   int32_t waves;            /* wavefronts per 32-trajectory workgroup of dfx_mlp_solve: 4
                                or 8; 0 picks 8, or 4 for DFX_F32 batches of more than
-                               256 tiles (no effect on the results: the same bits)      */
+                               a tile per compute unit (the same bits either way)       */
   int32_t save_steps;       /* SaveAt(steps=k): k > 0 also saves every k-th accepted step
                                (rows in time order with the ts rows; forward only)      */
   int64_t ts_stride;        /* 0: ts[n_ts] shared by the batch; n_ts: ts[B, n_ts] per
