@@ -6,15 +6,27 @@ trajectory slots (all instances, or half with the refill queue), for the neural-
 kernel the wavefronts per 32-trajectory tile (4 or 8; the tile's LDS layout is the same,
 the waves split its output columns and state components).  Results are cached in memory
 and, if DIFFRAX_AMD_TUNE_CACHE names a file, as JSON keyed by (kernel signature, batch,
-device name)."""
+device name, build of the library)."""
 from __future__ import annotations
 
+import functools
+import hashlib
 import json
 import os
 
 import torch
 
+from . import _lib
+
 _CACHE: dict = {}
+
+
+@functools.lru_cache(maxsize=None)
+def _build():
+    """The build of the library that the times belong to: a choice that an earlier build made
+    can be a slow one in this (25 ms, once in a process that tunes)."""
+    with open(_lib.LIB_PATH, "rb") as f:
+        return hashlib.blake2b(f.read(), digest_size=8).hexdigest()
 
 
 def _key(plan):
@@ -22,7 +34,7 @@ def _key(plan):
     the (solver, field, precision, d) kernel, the controller kind (PID coefficients) and
     tolerances (shared or per instance), the save layout (ts count and sharing, t0 / t1 /
     every-k-th-step rows), max_steps, the dense / clipping / event variant, step and
-    checkpoint recording, and the batch and device."""
+    checkpoint recording, the batch and device, and the build."""
     p = plan.problem
     io = getattr(plan, "io", None)
     has = lambda f: int(bool(io is not None and getattr(io, f)))
@@ -34,7 +46,7 @@ def _key(plan):
     extras = (f"{p.n_step_ts}/{p.n_jump_ts}/{p.n_events}/{has('dense_ts')}/{has('grid')}/"
               f"{p.ckpt_every}")
     return (f"erk:{p.solver}:{p.vf}:{p.precision}:{p.d}:{p.controller}:{pid}:{tol}:{save}:"
-            f"{extras}:{p.batch}:{name}")
+            f"{extras}:{p.batch}:{name}:{_build()}")
 
 
 def _load_file():
@@ -111,13 +123,13 @@ def tune(plan, verbose=False):
 
 def _key_mlp(plan):
     """The neural-ODE kernel variant (precision, controller kind, gradient recording, dt0
-    given or selected), its save layout and tolerances, the batch and the device."""
+    given or selected), its save layout and tolerances, the batch, the device and the build."""
     p = plan.prob
     name = torch.cuda.get_device_name(torch.cuda.current_device())
     pid = f"{p.pcoeff}/{p.icoeff}/{p.dcoeff}/{p.error_order}/{p.rtol!r}/{p.atol!r}"
     return (f"mlp:{p.precision}:{pid}:{int(p.dt0 == p.dt0)}:{p.n_ts}/{int(p.ts_stride != 0)}/"
             f"{p.save_t0}/{p.save_t1}/{p.save_steps}:"
-            f"{p.max_steps}:{p.ckpt_every}:{p.t0!r}/{p.t1!r}:{p.batch}:{name}")
+            f"{p.max_steps}:{p.ckpt_every}:{p.t0!r}/{p.t1!r}:{p.batch}:{name}:{_build()}")
 
 
 def tune_mlp(plan, verbose=False):
