@@ -78,9 +78,10 @@ def constant_grid(t0: float, t1: float, dt0: float):
 
 def _row_times(grid, ts, save_t0, save_t1, k, t0, t1):
     """Times of the saved rows, in the kernels' order: t0; per step, the ts inside it and then
-    its end when k divides the step count; t1 unless the last step was saved."""
+    its end when k divides the step count; t1 unless the last step was saved.  A NaN among
+    the ts is in no step, and neither are those after it."""
     N = len(grid) - 1
-    t = np.empty(0) if ts is None else ts[:np.searchsorted(ts, grid[N], side="right")]
+    t = np.empty(0) if ts is None else ts[:np.argmin(np.append(ts <= grid[N], False))]
     at = np.arange(k, N + 1, k) if k else np.empty(0, dtype=np.int64)
     steps = np.concatenate((np.maximum(np.searchsorted(grid, t, side="left"), 1), at))
     body = np.concatenate((t, grid[at]))[np.argsort(steps, kind="stable")]
