@@ -63,6 +63,8 @@ def constant_grid(t0: float, t1: float, dt0: float):
     """ConstantStepSize step times (constant.py:30-104) with the loop's end clipping
     (_integrate.py:278-284, 319-322).  Forward time only."""
     num = int(math.ceil((t1 - t0) / float(np.nextafter(dt0, math.inf))))
+    if num < 1:
+        raise ValueError(f"dt0 = {dt0} is too large for constant steps from {t0} to {t1}")
     floor = t1
     for _ in range(100):
         floor = float(np.nextafter(floor, -math.inf))
