@@ -278,6 +278,17 @@ class ErkPlan:
         _lib.check(rc, "dfx_erk_solve")
 
 
+def _refuse_time_gradients(*times):
+    """t1 and SaveAt(ts) are read as numbers: a gradient asked for on them would be dropped.
+    (Device times under no_grad are read as they are; host times go through numpy, which
+    refuses them there as well.)"""
+    for t in times:
+        if t is not None and t.requires_grad and (t.device.type == "cpu" or
+                                                  torch.is_grad_enabled()):
+            raise RuntimeError("gradients with respect to t1 and SaveAt(ts) are not provided: "
+                               "pass these times detached")
+
+
 def _check_ts(ts, t0, t1_vals, directions):
     """_raise_ts of host times; ts: [n] or [B, n]; t1_vals, directions: [1] or [B] (float64
     numpy)."""
@@ -479,6 +490,7 @@ def _prepare_erk(terms, solver, t0, t1, dt0, y0, args, saveat, stepsize_controll
             f"Must have (t1 - t0) * dt0 >= 0, we instead got t1 with value {t1}, t0 "
             f"with value {t0}, dt0 with value {dt0}")
 
+    _refuse_time_gradients(t1_t, ts_t)
     if not on_device:
         t1_host = t1_t.numpy()
         if dt0f is not None and bool(np.any((t1_host - t0f) * dt0f < 0)):

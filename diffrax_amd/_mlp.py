@@ -264,7 +264,7 @@ def prepare_mlp(terms, solver, t0, t1, dt0, y0, saveat, stepsize_controller, max
     ts = None
     check = None
     if sub.ts is not None:
-        from ._integrate import _TimeChecks, _check_ts
+        from ._integrate import _TimeChecks, _check_ts, _refuse_time_gradients
         ts = torch.as_tensor(sub.ts, dtype=torch.float64)
         if ts.ndim == 2 and ts.shape[0] == y0b.shape[0]:
             pass   # per-trajectory save times [B, n_ts]
@@ -272,6 +272,7 @@ def prepare_mlp(terms, solver, t0, t1, dt0, y0, saveat, stepsize_controller, max
             ts = ts.reshape(-1)
         else:
             raise ValueError(f"SaveAt(ts) must be [n] or [{y0b.shape[0]}, n]")
+        _refuse_time_gradients(ts)
         t0f, t1f = float(t0), float(t1)
         if ts.device.type == "cpu":
             _check_ts(ts.numpy(), t0f, [t1f], [1.0 if t0f < t1f else -1.0])
