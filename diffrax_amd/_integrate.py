@@ -218,8 +218,9 @@ class ErkPlan:
         it)."""
         y0 = self.t["y0"]
         B, d = y0.shape
-        if self.problem.n_step_ts or self.problem.n_jump_ts:
-            return 0      # clipped solves replay
+        if (self.problem.n_step_ts or self.problem.n_jump_ts or self.problem.n_events
+                or self.t.get("state_out") is not None or self.t.get("dense_ts") is not None):
+            return 0      # their builds write no tape: replayed
         B = -(-B // 64) * 64
         K = int(self.problem.ckpt_every)
         rec = 16 + d * y0.element_size()

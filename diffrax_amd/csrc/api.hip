@@ -297,9 +297,10 @@ int dfx_erk_solve(const dfx_erk_problem* p, const dfx_erk_io* io, void* workspac
       if (!io->tape || !io->tape_y) return DFX_E_ARG;
       a.tape = io->tape;
       a.tape_y = io->tape_y;
-      // clipped solves replay (launch_adjoint): a step of theirs may start past the end of
-      // the one before
-      a.tape_steps = p->n_step_ts > 0 || p->n_jump_ts > 0 ? 0 : p->tape_steps;
+      a.tape_steps = p->tape_steps;
+      // These solves run a build that writes no tape, and dfx_erk_adjoint would sweep it all
+      // the same (clipped solves do too, but their adjoint always replays).
+      if (io->state_out || dense != 0) return DFX_E_ARG;
     }
   }
   a.counter = reinterpret_cast<unsigned int*>(workspace);

@@ -929,13 +929,13 @@ struct ErkLane {
       if (keep) ++num_acc; else ++num_rej;
       if (result == DFX_SUCCESSFUL) result = code;
     }
-    if constexpr (Ck) {
-      // The adjoint's tape, in every build that can record checkpoints: the extras builds run
-      // solves that also export their state or dense output, and dfx_erk_adjoint sweeps
-      // whatever tape the problem declares (tape_steps = 0 here with step clipping).  Indexed by the attempt, which the lanes of a wave share, so the
-      // 64 records are one contiguous store; records of 64 lanes each in its own row (by
-      // accepted step) held up every later load of the loop: 65,536 Van der Pol solves took
-      // 1.92 ms that way.
+    if constexpr (Ck && !Extras) {
+      // The adjoint's tape.  Not in the extras builds: with these lines in their step loop
+      // 65,536 solves that export their state took 1.29 ms in place of 0.79 and clipped ones
+      // 2.25 in place of 1.55, also with no tape to write.  Indexed by the attempt, which the
+      // lanes of a wave share, so the 64 records are one contiguous store; records of 64 lanes
+      // each in its own row (by accepted step) held up every later load of the loop: 65,536
+      // Van der Pol solves took 1.92 ms that way.
       if (num_steps <= a.tape_steps) {
         const int64_t rec = tape_at(a, num_steps - 1);
         a.tape[rec * 2] = ts0;

@@ -94,8 +94,9 @@ typedef struct dfx_erk_problem {
   int32_t resume;
   /* With ckpt_every > 0: records per instance of dfx_erk_io.tape, 0 for none.  Solves
    * that attempt no more steps are swept from the tape by dfx_erk_adjoint, without a replay.
-   * Every forward with checkpoints writes it, also one that exports its state or dense
-   * output; only with step_ts / jump_ts clipping it is neither written nor read. */
+   * DFX_E_ARG from dfx_erk_solve with io.state_out or dense output, whose solves write no
+   * tape: pass 0 there, and the adjoint replays.  With step_ts / jump_ts clipping it is
+   * neither written nor read. */
   int32_t tape_steps;
 } dfx_erk_problem;
 
