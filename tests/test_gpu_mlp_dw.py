@@ -56,7 +56,7 @@ def test_weight_gradient_of_the_rows(cuda, matmul, B, steps):
     below the result's largest) of every accumulation of one accumulator, six products of 16
     rows each, independent of one another, so their root; no accumulator sums more than 4,096
     rows; and 8 units for the chunks' sum and the products of pieces left out.  Without the
-    third pieces a product would be off by 3e-6."""
+    third pieces the sums would be off by 6e-6."""
     rows, dw, blocks = _segment(cuda, matmul, B, steps)
     per_chunk = max(min(4, blocks), min(128, math.ceil(blocks / 80)))
     tol = (8.0 + math.sqrt(per_chunk * 32 / 16 * 6)) * 2.0 ** -24
