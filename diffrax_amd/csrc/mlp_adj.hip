@@ -30,9 +30,9 @@
 
 namespace dfx {
 
-constexpr int ADJ_CHUNK = 4096;  // rows per split-K chunk of the weight-gradient GEMM
-
 // Six row buffers: D1 (width 256), Z (64), D2 (256), H1 (256), D3 (64), H2 (256).
+constexpr int kRowWidths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
+constexpr int kRowFloats = 4 * MLP_H + 2 * MLP_D;
 
 struct RowBufs {  // float32 blocks of 32 rows, in the order of rows_frag
   float* b[6];
@@ -50,7 +50,7 @@ struct AdjArgs {
                    // value is outside the range of the three-piece products (SplitRange)
   const int32_t* wflags;  // float32 form: nonzero where a weight is outside (kWeightFlags), and
                           // such tiles are left to the float32 kernel; else null
-  int64_t B, B_pad, ts_stride;
+  int64_t B, ts_stride;
   int32_t max_steps, n_ckpt, C, Cs, seg, n_ts, n_out, save_t0;
   double t0, t1;
 };
@@ -824,7 +824,7 @@ mlp_backsolve_kernel(const BsArgs a, const MlpWeights<PolicyF32> W, const RowBuf
   constexpr int S = Tab::S;
   using TL = TabLit<Tab, float>;
   using WV = MlpWaves<NW>;
-  constexpr int CPT = WV::CPT, GRP = MLP_D / CPT, NT = WV::NT12, NT3 = WV::NT3;
+  constexpr int CPT = WV::CPT, GRP = MLP_D / CPT;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int orow = tid / GRP, c0 = (tid % GRP) * CPT, gbase = lane & ~(GRP - 1);
   const bool lead = (tid % GRP) == 0;
@@ -1073,14 +1073,20 @@ namespace {
 
 int64_t padded_batch(int64_t B) { return (B + MLP_TILE - 1) / MLP_TILE * MLP_TILE; }
 
-int64_t seg_rows(int64_t B, int32_t seg_steps) { return (int64_t)seg_steps * 7 * padded_batch(B); }
+// Rows of the row buffers: an evaluation of every trajectory each (a segment's 1 + 6 per step,
+// a backsolve launch's 7 per iteration).
+int64_t seg_rows(int64_t B, int32_t seg_steps) { return padded_batch(B) * (1 + 6 * (int64_t)seg_steps); }
+int64_t bs_rows(int64_t B, int32_t iters) { return padded_batch(B) * 7 * (int64_t)iters; }
 
-int64_t seg_chunks(int64_t B, int32_t seg_steps) {
-  return (seg_rows(B, seg_steps) + ADJ_CHUNK - 1) / ADJ_CHUNK;
+RowBufs row_bufs(void* rows, int64_t nrow) {
+  RowBufs R;
+  float* base = reinterpret_cast<float*>(rows);
+  for (int i = 0; i < 6; base += nrow * kRowWidths[i], ++i) R.b[i] = base;
+  return R;
 }
 
 // The backsolve's state buffer: ya [B_pad, 128] floats, rows [B_pad] BsRow, rscale [nrow]
-// floats (every row of the allocated row buffers), counters [2] int32; 256-byte aligned.
+// floats (every row of the row buffers), counters [2] int32; 256-byte aligned.
 struct BsStateLayout {
   size_t ya, rows, rscale, counters, total;
 };
@@ -1095,11 +1101,9 @@ BsStateLayout bs_state_layout(int64_t Bp, int64_t nrow) {
   return l;
 }
 
-// Zero the launch counters and the row weights past the kernel's rows (the padding of the
-// last split-K chunk), which the kernel never writes.
-__global__ void bs_reset_kernel(int32_t* counters, float* rscale, int64_t used, int64_t nrow) {
+// Zero the launch counters.
+__global__ void bs_reset_kernel(int32_t* counters) {
   if (threadIdx.x < 2) counters[threadIdx.x] = 0;
-  for (int64_t r = used + threadIdx.x; r < nrow; r += blockDim.x) rscale[r] = 0.0f;
 }
 
 // The weight gradients of `blocks` row blocks (SC: per-row weights rscale) added to dw.
@@ -1136,13 +1140,14 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   memset(&a, 0, sizeof(a));
   a.grid = io->grid; a.ckpt = io->ckpt; a.stats = io->stats; a.ts = io->ts; a.ys_bar = io->ys_bar;
   a.ybar = io->ybar; a.zs = io->zs;
-  a.B = p->batch; a.B_pad = padded_batch(p->batch);
+  a.B = p->batch;
   a.max_steps = p->max_steps; a.n_ckpt = dfx_mlp_n_ckpt(p); a.C = p->ckpt_every;
   a.Cs = seg_steps; a.seg = seg; a.n_ts = p->n_ts; a.ts_stride = p->ts_stride;
   a.n_out = (p->save_t0 ? 1 : 0) + p->n_ts + (p->save_t1 ? 1 : 0);
   a.save_t0 = p->save_t0; a.t0 = p->t0; a.t1 = p->t1;
   const int slots = 1 + 6 * seg_steps;
-  const int64_t ntiles64 = a.B_pad / MLP_TILE, blocks = ntiles64 * slots;
+  const int64_t nrow = seg_rows(p->batch, seg_steps), blocks = nrow / MLP_TILE;
+  const int64_t ntiles64 = padded_batch(p->batch) / MLP_TILE;
   a.evals = reinterpret_cast<int32_t*>(io->partial + partial_floats(blocks));
   const bool f32 = p->precision == DFX_F32;
   const void* pieces = packed;
@@ -1156,12 +1161,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
     a.wflags = wflags;
   }
   const MlpWeights<P> W = mlp_weights_from<P>(pieces, P::PIECES, b1, b2, b3);
-  RowBufs R;
-  const int64_t rows_alloc = seg_chunks(p->batch, seg_steps) * ADJ_CHUNK;
-  float* base = reinterpret_cast<float*>(io->rows);
-  int64_t off = 0;
-  const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
-  for (int i = 0; i < 6; ++i) { R.b[i] = base + off; off += rows_alloc * widths[i]; }
+  const RowBufs R = row_bufs(io->rows, nrow);
   const unsigned ntiles = (unsigned)ntiles64;
   auto sweep = [&](auto policy, auto&& w) {
     using Q = decltype(policy);
@@ -1184,15 +1184,10 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
                           size_t* rows_bytes, size_t* partial_bytes) {
   if (!p || seg_steps <= 0 || !zs_bytes || !rows_bytes || !partial_bytes) return DFX_E_ARG;
   const int64_t Bp = padded_batch(p->batch);
-  *zs_bytes = (size_t)(Bp * seg_steps * 7 * MLP_D) * sizeof(float);
-  const int64_t rows_alloc = seg_chunks(p->batch, seg_steps) * ADJ_CHUNK;
-  int64_t wsum = 0;
-  const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
-  for (int i = 0; i < 6; ++i) wsum += widths[i];
-  *rows_bytes = (size_t)(rows_alloc * wsum) * sizeof(float);   // float32 rows for both forms
-  const int64_t ntiles = Bp / MLP_TILE;
-  *partial_bytes = (size_t)(partial_floats(ntiles * (1 + 6 * seg_steps)) + (ntiles + 63) / 64 * 64) *
-                   sizeof(float);
+  const int64_t nrow = seg_rows(p->batch, seg_steps), ntiles = Bp / MLP_TILE;
+  *zs_bytes = (size_t)(nrow * MLP_D) * sizeof(float);
+  *rows_bytes = (size_t)(nrow * kRowFloats) * sizeof(float);   // float32 rows for both forms
+  *partial_bytes = (size_t)(partial_floats(nrow / MLP_TILE) + (ntiles + 63) / 64 * 64) * sizeof(float);
   if (p->precision == DFX_F32)
     *partial_bytes += kWeightFlags * sizeof(int32_t) + (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
@@ -1202,13 +1197,10 @@ int dfx_mlp_backsolve_workspace(const dfx_mlp_problem* p, int32_t chunk_iters,
                                 size_t* state_bytes, size_t* rows_bytes, size_t* partial_bytes) {
   if (!p || chunk_iters <= 0 || !state_bytes || !rows_bytes || !partial_bytes) return DFX_E_ARG;
   const int64_t Bp = padded_batch(p->batch);
-  const int64_t nrow = seg_chunks(p->batch, chunk_iters) * ADJ_CHUNK;
+  const int64_t nrow = bs_rows(p->batch, chunk_iters);
   *state_bytes = bs_state_layout(Bp, nrow).total;
-  int64_t wsum = 0;
-  const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
-  for (int i = 0; i < 6; ++i) wsum += widths[i];
-  *rows_bytes = (size_t)(nrow * wsum) * sizeof(float);
-  *partial_bytes = (size_t)partial_floats(seg_rows(p->batch, chunk_iters) / MLP_TILE) * sizeof(float);
+  *rows_bytes = (size_t)(nrow * kRowFloats) * sizeof(float);
+  *partial_bytes = (size_t)partial_floats(nrow / MLP_TILE) * sizeof(float);
   return DFX_OK;
 }
 
@@ -1228,8 +1220,8 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   memset(&a, 0, sizeof(a));
   if (!mlp_pid_params(back, a.pid)) return DFX_E_ARG;
   const int64_t Bp = padded_batch(back->batch);
-  const int nch = (int)seg_chunks(back->batch, chunk_iters);
-  const BsStateLayout sl = bs_state_layout(Bp, (int64_t)nch * ADJ_CHUNK);
+  const int64_t nrow = bs_rows(back->batch, chunk_iters);
+  const BsStateLayout sl = bs_state_layout(Bp, nrow);
   unsigned char* sb = reinterpret_cast<unsigned char*>(io->state);
   a.ys = io->ys; a.ts_out = io->ts_out; a.ys_bar = io->ys_bar;
   a.ya = reinterpret_cast<float*>(sb + sl.ya);
@@ -1245,14 +1237,9 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   // weights for DFX_F32): the bfloat16 form's forward evaluates the float32-weight model too.
   using P = PolicyF32;
   const MlpWeights<P> W = mlp_weights_from<P>(packed, 1, b1, b2, b3);
-  RowBufs R;
-  float* base = reinterpret_cast<float*>(io->rows);
-  int64_t off = 0;
-  const int widths[6] = {MLP_H, MLP_D, MLP_H, MLP_H, MLP_D, MLP_H};
-  for (int i = 0; i < 6; ++i) { R.b[i] = base + off; off += (int64_t)nch * ADJ_CHUNK * widths[i]; }
+  const RowBufs R = row_bufs(io->rows, nrow);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(bs_reset_kernel, dim3(1), dim3(64), 0, s, a.counters, a.rscale,
-                     (int64_t)chunk_iters * 7 * Bp, (int64_t)nch * ADJ_CHUNK);
+  hipLaunchKernelGGL(bs_reset_kernel, dim3(1), dim3(64), 0, s, a.counters);
   const unsigned ntiles = (unsigned)(Bp / MLP_TILE);
   // four waves per tile: at eight the kernel spills 193 VGPRs per lane (at four, 76) and
   // took 34.9 ms against 19.6 ms for the backsolve of 8,192 trajectories (bit-identical
@@ -1262,8 +1249,7 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLdsBack));
   hipLaunchKernelGGL((mlp_backsolve_kernel<NWB>), dim3(ntiles), dim3(64 * NWB),
                      sizeof(MlpLdsBack), s, a, W, R);
-  launch_dw<true>(R, io->partial, seg_rows(back->batch, chunk_iters) / MLP_TILE, nullptr, 0,
-                  a.rscale, io->dw, s);
+  launch_dw<true>(R, io->partial, nrow / MLP_TILE, nullptr, 0, a.rscale, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -1271,7 +1257,7 @@ int dfx_mlp_backsolve_status(const dfx_mlp_problem* back, int32_t chunk_iters,
                              const void* state, const int32_t** counters) {
   if (!back || chunk_iters <= 0 || !state || !counters) return DFX_E_ARG;
   const int64_t Bp = padded_batch(back->batch);
-  const BsStateLayout sl = bs_state_layout(Bp, seg_chunks(back->batch, chunk_iters) * ADJ_CHUNK);
+  const BsStateLayout sl = bs_state_layout(Bp, bs_rows(back->batch, chunk_iters));
   *counters = reinterpret_cast<const int32_t*>(reinterpret_cast<const unsigned char*>(state) +
                                                sl.counters);
   return DFX_OK;

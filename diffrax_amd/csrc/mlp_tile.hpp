@@ -76,9 +76,6 @@ struct PolicyBF16x3 {
   __device__ __forceinline__ static frag_t load_a(const act_t* p) {
     return *reinterpret_cast<const frag_t*>(p);
   }
-  __device__ __forceinline__ static frag_t load_b(const act_t* packed, int frag) {
-    return reinterpret_cast<const frag_t*>(packed)[frag];
-  }
   __device__ __forceinline__ static floatx16_t mfma(frag_t a, frag_t b, floatx16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
@@ -280,9 +277,8 @@ __device__ __forceinline__ float dsoftplus_from_value(float h) {
   return 1.0f - __builtin_amdgcn_exp2f(-h * 1.4426950408889634f);
 }
 
-// C-layout helpers: accumulator element v (= 4i + j) of lane l sits at
-// row 8i + (l/32)*4 + j, column l%32 of the 32x32 tile.
-__device__ __forceinline__ int acc_row(int lane, int v) { return 8 * (v >> 2) + (lane >> 5) * 4 + (v & 3); }
+// C layout: accumulator element v (= 4i + j) of lane l sits at row 8i + (l/32)*4 + j, column
+// l%32 of the 32x32 tile.
 
 // ---- the float32 form ------------------------------------------------------------------
 // One wave's share of a layer: acc[t] = sum over fragments [g0, g0 + G) of W . x, the weights
