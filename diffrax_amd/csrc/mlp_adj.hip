@@ -1073,10 +1073,11 @@ namespace {
 
 int64_t padded_batch(int64_t B) { return (B + MLP_TILE - 1) / MLP_TILE * MLP_TILE; }
 
-// Rows of the row buffers: an evaluation of every trajectory each (a segment's 1 + 6 per step,
-// a backsolve launch's 7 per iteration).
-int64_t seg_rows(int64_t B, int32_t seg_steps) { return padded_batch(B) * (1 + 6 * (int64_t)seg_steps); }
-int64_t bs_rows(int64_t B, int32_t iters) { return padded_batch(B) * 7 * (int64_t)iters; }
+// Rows that the row buffers are sized for: seven evaluations of every trajectory per step of a
+// segment (which writes 1 + 6 per step) or per iteration of a backsolve launch, in whole
+// blocks of 4,096, the sizes that callers of dfx_mlp_*_workspace know.
+int64_t step_rows(int64_t B, int32_t steps) { return padded_batch(B) * 7 * (int64_t)steps; }
+int64_t alloc_rows(int64_t B, int32_t steps) { return (step_rows(B, steps) + 4095) / 4096 * 4096; }
 
 RowBufs row_bufs(void* rows, int64_t nrow) {
   RowBufs R;
@@ -1129,8 +1130,9 @@ int64_t partial_floats(int64_t blocks) {
 }
 
 // One segment: the recompute + sweep kernel on three-piece weights (a bf16 buffer as it is;
-// a float32 one split into the tail of io->partial first), then the float32
-// weight-gradient GEMM over its float32 row buffers and the fixed-order reduction.
+// a float32 one split into the tail of io->partial first), the same on float32 MFMA for the
+// tiles that it marked (float32 form), then the weight-gradient GEMM over the float32 row
+// buffers and the fixed-order reduction.
 int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, const float* b2,
                 const float* b3, const dfx_mlp_adj_io* io, int32_t seg, int32_t seg_steps,
                 hipStream_t s) {
@@ -1146,8 +1148,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   a.n_out = (p->save_t0 ? 1 : 0) + p->n_ts + (p->save_t1 ? 1 : 0);
   a.save_t0 = p->save_t0; a.t0 = p->t0; a.t1 = p->t1;
   const int slots = 1 + 6 * seg_steps;
-  const int64_t nrow = seg_rows(p->batch, seg_steps), blocks = nrow / MLP_TILE;
-  const int64_t ntiles64 = padded_batch(p->batch) / MLP_TILE;
+  const int64_t ntiles64 = padded_batch(p->batch) / MLP_TILE, blocks = ntiles64 * slots;
   a.evals = reinterpret_cast<int32_t*>(io->partial + partial_floats(blocks));
   const bool f32 = p->precision == DFX_F32;
   const void* pieces = packed;
@@ -1161,7 +1162,7 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
     a.wflags = wflags;
   }
   const MlpWeights<P> W = mlp_weights_from<P>(pieces, P::PIECES, b1, b2, b3);
-  const RowBufs R = row_bufs(io->rows, nrow);
+  const RowBufs R = row_bufs(io->rows, alloc_rows(p->batch, seg_steps));
   const unsigned ntiles = (unsigned)ntiles64;
   auto sweep = [&](auto policy, auto&& w) {
     using Q = decltype(policy);
@@ -1184,10 +1185,11 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
                           size_t* rows_bytes, size_t* partial_bytes) {
   if (!p || seg_steps <= 0 || !zs_bytes || !rows_bytes || !partial_bytes) return DFX_E_ARG;
   const int64_t Bp = padded_batch(p->batch);
-  const int64_t nrow = seg_rows(p->batch, seg_steps), ntiles = Bp / MLP_TILE;
-  *zs_bytes = (size_t)(nrow * MLP_D) * sizeof(float);
-  *rows_bytes = (size_t)(nrow * kRowFloats) * sizeof(float);   // float32 rows for both forms
-  *partial_bytes = (size_t)(partial_floats(nrow / MLP_TILE) + (ntiles + 63) / 64 * 64) * sizeof(float);
+  const int64_t ntiles = Bp / MLP_TILE;
+  *zs_bytes = (size_t)(step_rows(p->batch, seg_steps) * MLP_D) * sizeof(float);
+  *rows_bytes = (size_t)(alloc_rows(p->batch, seg_steps) * kRowFloats) * sizeof(float);
+  *partial_bytes = (size_t)(partial_floats(ntiles * (1 + 6 * (int64_t)seg_steps)) +
+                            (ntiles + 63) / 64 * 64) * sizeof(float);
   if (p->precision == DFX_F32)
     *partial_bytes += kWeightFlags * sizeof(int32_t) + (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
@@ -1197,10 +1199,10 @@ int dfx_mlp_backsolve_workspace(const dfx_mlp_problem* p, int32_t chunk_iters,
                                 size_t* state_bytes, size_t* rows_bytes, size_t* partial_bytes) {
   if (!p || chunk_iters <= 0 || !state_bytes || !rows_bytes || !partial_bytes) return DFX_E_ARG;
   const int64_t Bp = padded_batch(p->batch);
-  const int64_t nrow = bs_rows(p->batch, chunk_iters);
+  const int64_t nrow = alloc_rows(p->batch, chunk_iters);
   *state_bytes = bs_state_layout(Bp, nrow).total;
   *rows_bytes = (size_t)(nrow * kRowFloats) * sizeof(float);
-  *partial_bytes = (size_t)partial_floats(nrow / MLP_TILE) * sizeof(float);
+  *partial_bytes = (size_t)partial_floats(step_rows(p->batch, chunk_iters) / MLP_TILE) * sizeof(float);
   return DFX_OK;
 }
 
@@ -1220,7 +1222,7 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   memset(&a, 0, sizeof(a));
   if (!mlp_pid_params(back, a.pid)) return DFX_E_ARG;
   const int64_t Bp = padded_batch(back->batch);
-  const int64_t nrow = bs_rows(back->batch, chunk_iters);
+  const int64_t nrow = alloc_rows(back->batch, chunk_iters);
   const BsStateLayout sl = bs_state_layout(Bp, nrow);
   unsigned char* sb = reinterpret_cast<unsigned char*>(io->state);
   a.ys = io->ys; a.ts_out = io->ts_out; a.ys_bar = io->ys_bar;
@@ -1241,15 +1243,15 @@ int dfx_mlp_backsolve(const dfx_mlp_problem* back, const void* packed, const flo
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(bs_reset_kernel, dim3(1), dim3(64), 0, s, a.counters);
   const unsigned ntiles = (unsigned)(Bp / MLP_TILE);
-  // four waves per tile: at eight the kernel spills 193 VGPRs per lane (at four, 76) and
-  // took 34.9 ms against 19.6 ms for the backsolve of 8,192 trajectories (bit-identical
-  // gradients)
+  // four waves per tile: 256 VGPRs without spills (eight spill 2 per lane; calls with 8,192
+  // trajectories take 12.4 ms at four and 11.9 at eight, the same bits)
   constexpr int NWB = 4;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_backsolve_kernel<NWB>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpLdsBack));
   hipLaunchKernelGGL((mlp_backsolve_kernel<NWB>), dim3(ntiles), dim3(64 * NWB),
                      sizeof(MlpLdsBack), s, a, W, R);
-  launch_dw<true>(R, io->partial, nrow / MLP_TILE, nullptr, 0, a.rscale, io->dw, s);
+  launch_dw<true>(R, io->partial, step_rows(back->batch, chunk_iters) / MLP_TILE, nullptr, 0,
+                  a.rscale, io->dw, s);
   return hipGetLastError() == hipSuccess ? DFX_OK : DFX_E_HIP;
 }
 
@@ -1257,7 +1259,7 @@ int dfx_mlp_backsolve_status(const dfx_mlp_problem* back, int32_t chunk_iters,
                              const void* state, const int32_t** counters) {
   if (!back || chunk_iters <= 0 || !state || !counters) return DFX_E_ARG;
   const int64_t Bp = padded_batch(back->batch);
-  const BsStateLayout sl = bs_state_layout(Bp, bs_rows(back->batch, chunk_iters));
+  const BsStateLayout sl = bs_state_layout(Bp, alloc_rows(back->batch, chunk_iters));
   *counters = reinterpret_cast<const int32_t*>(reinterpret_cast<const unsigned char*>(state) +
                                                sl.counters);
   return DFX_OK;
