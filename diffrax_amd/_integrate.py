@@ -62,7 +62,8 @@ class _TimeChecks:
                    if isinstance(x, torch.Tensor) and x.ndim == nd and (nd == 2 or x.numel() != 1)]
         rows = per_row[0].shape[0] if per_row else 1
         n_ts = 0 if ts is None else int(ts.shape[-1])
-        # one block reads 1,024 times and more; 1,024 blocks fill the GPU four times over
+        # one block up to 2,047 times, then at least 1,024 a block; 1,024 blocks fill the GPU
+        # four times over
         n_flags = max(1, min(1024, rows * max(n_ts, 1) // 1024))
         self._dev = torch.empty(n_flags, dtype=torch.int32, device=device)
         t1_t = t1 if isinstance(t1, torch.Tensor) else None

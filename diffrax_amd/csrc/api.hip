@@ -63,7 +63,8 @@ __global__ void __launch_bounds__(256) check_times_kernel(const double* t1, doub
 
 // The first failure of each block's run of result codes, written where the host reads it.
 // Bound by its launch: comparing, masking and reducing the codes as tensors was five launches
-// and a copy, 30 us of a call whose solve takes 110 us.  A block reads 4,096 codes and more.
+// and a copy, 30 us of a call whose solve takes 110 us.  One block up to 8,191 codes, then at
+// least 4,096 codes a block.
 __global__ void __launch_bounds__(256) check_results_kernel(const int32_t* result, int64_t n,
                                                             int32_t ok_code, int32_t* first) {
   const int64_t len = (n + gridDim.x - 1) / gridDim.x;

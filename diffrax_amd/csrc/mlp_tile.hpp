@@ -1,17 +1,21 @@
 // mlp_tile.hpp -- the registered neural vector field f(y) = tanh(W3 sp(W2 sp(W1 y + b1) + b2) + b3)
 // (sp = softplus; d = 64 -> 256 -> 256 -> 64) evaluated for a tile of 32 trajectories by one
-// 256-thread workgroup on MFMA, plus its vector-Jacobian product.
+// workgroup of NW = 4 or 8 waves on MFMA, plus its vector-Jacobian product.
 //
-// Layout of one tile (4 waves):
-//  - owner threads: thread t owns trajectory t/8 of the tile and state components
-//    (t%8)*8 .. +8, so a trajectory's 8 owners are adjacent lanes of one wave;
-//  - activations live in LDS, row-major [32 rows][K + PAD]; every MFMA reads its A fragment
-//    (32 rows x KSTEP) straight from there;
-//  - weights are read as MFMA B fragments from a host-packed copy (fragment (n_tile, k_step)
-//    is 64 lanes x KA contiguous elements, one coalesced load per lane);
-//  - layers 1 and 2: wave w produces output columns [64w, 64w + 64) (two 32x32 tiles);
-//    layer 3 (64 outputs, K = 256) is split over K: wave w reduces K in [64w, 64w + 64) and
-//    the four partial sums meet in LDS, where the owner threads add them in wave order.
+// Layout of one tile:
+//  - owner threads: 2 NW adjacent lanes of one wave own a trajectory, 32 / NW consecutive
+//    state components each;
+//  - activations live in LDS, row-major [32 rows][K + padding] (float32 with the columns of a
+//    fragment reordered, PolicyF32::pos); every MFMA reads its fragment (32 rows x KSTEP)
+//    straight from there;
+//  - weights come as MFMA fragments from a packed copy (dfx_mlp_pack; fragment (n_tile,
+//    k_step) is 64 lanes x KA contiguous elements, one coalesced load per lane).  In the
+//    solve's products they are the A operand and the activations B, so a lane's accumulators
+//    are runs of four outputs of one trajectory; where the adjoint writes row buffers it is
+//    the other way round (Gemm3's WA);
+//  - layers 1 and 2: each wave produces 256 / NW output columns; layer 3 (64 outputs, K = 256)
+//    is split over K in quarters, whose four partial sums meet in LDS, where the owner
+//    threads add them in order (MlpWaves).
 // Precision policies: three-piece BF16 operands with f32 accumulate
 // (v_mfma_f32_32x32x16_bf16), or f32 throughout (v_mfma_f32_32x32x2f32).  Activation
 // functions are evaluated in f32.
@@ -118,7 +122,7 @@ __device__ __forceinline__ Split4 split3x4(float a, float b, float c, float d) {
 // has no pieces (inf - inf), and a number near the largest rounds up to one.  Below the upper
 // bound no product, nor a sum of 4,096, overflows in either form.  A caller that finds a
 // value outside takes float32 MFMA: gradients of cotangents scaled by 2^-112 and 2^-116 were
-// off by 5e-6 and 7e-5 in pieces and by 5e-7 and 8e-7 that way.  Seven instructions for four
+// off by 5e-6 and 7e-5 in pieces and by 5e-7 and 8e-7 that way.  Eight instructions for four
 // values, beside thirty for their split.
 constexpr float SPLIT_MIN = 7.8886090522101181e-31f, SPLIT_END = 72057594037927936.0f;
 struct SplitRange {
@@ -589,7 +593,7 @@ __device__ __forceinline__ void mlp_forward_rows(const MlpWeights<PolicyBF16x3>&
 
 // Forward of the MLP on the tile: reads L.x (stage values), leaves softplus activations in
 // L.h1 / L.h2 and returns f for the owner's 32 / NW components in fout (NW waves per tile;
-// MlpWaves).  The three-piece bf16 form runs mlp_forward3.
+// MlpWaves).  The three-piece form takes its first branch.
 template <class P, int NW = 4, class Lds = MlpLds<P>>
 __device__ __forceinline__ void mlp_forward(const MlpWeights<P>& W, Lds& L, int wave,
                                             int lane, int owner_row, int owner_c0,
