@@ -48,8 +48,9 @@ struct AdjArgs {
   float* zs;
   int32_t* evals;  // out [tiles]: evaluations (row blocks) of each tile, negative where some
                    // value is outside the range of the three-piece products (SplitRange)
-  const int32_t* wflags;  // float32 form: nonzero where a weight is outside (kWeightFlags), and
-                          // such tiles are left to the float32 kernel; else null
+  const int32_t* wflags;  // float32 form: nonzero where a weight or bias is outside
+                          // (kWeightFlags), and marked tiles are left to the float32 kernel;
+                          // else null
   int64_t B, ts_stride;
   int32_t max_steps, n_ckpt, C, Cs, seg, n_ts, n_out, save_t0;
   double t0, t1;
@@ -161,6 +162,16 @@ __device__ __forceinline__ void pull_back_f32(const MlpWeights<PolicyF32>& W, Ml
 // P = PolicyF32, launched behind it by the float32 form: the tiles that the first pass marked,
 // because some weight, layer input or delta of theirs is outside the pieces' range
 // (SplitRange), from their start again on float32 MFMA; every other workgroup ends at once.
+// The first pass looks at what enters a product from outside (weights, biases, states, delta3)
+// and at what a pull-back gives, zb.  Their limits bound all the rest:
+//   above: h1 <= 64 2^10 2^24 = 2^40, h2 <= 256 2^10 2^40 = 2^58, delta2 <= 64 2^10 2^50 =
+//     2^66, delta1 <= 256 2^10 2^66 = 2^84, zb <= 2^102, and 4,096 rows of dW <= 2^120 (biases
+//     add little);
+//   below: a delta's pieces are off by 2^-134 at most, so a sum for delta1 by 256 2^10 2^-134 =
+//     2^-116 and one for zb by 2^-98, a quarter of 2^-24 of the least zb that passes.
+// Looking at every delta instead took 15 of 700 us; this is within the launch's spread (8,192
+// trajectories 709 us, without any test 721; 3,001 537 and 537).  In the bf16 form, which
+// evaluates in pieces anyway, the marks only choose the weight-gradient GEMM's arithmetic.
 // The row
 // buffers hold float32 values (layer inputs and deltas written before their split into
 // pieces) for the weight-gradient GEMM.  LDS: the forward planes;
@@ -175,13 +186,17 @@ __device__ __forceinline__ void pull_back_f32(const MlpWeights<PolicyF32>& W, Ml
 // weight-gradient GEMM sees one row block for both.  A tile runs as many steps as its
 // longest trajectory has; evals[tile] tells the GEMM how many of its E = 1 + 6 Cs slots
 // (block tile * E + slot) hold rows.
-// One segment of 8,192 trajectories and up to 4 steps: 0.70 ms (the range checks 0.01 of
-// it, and 5 us for the float32 launch that finds no tile marked); 0.92 ms with seven
+// One segment of 8,192 trajectories and up to 4 steps: 0.70 ms (and 5 us for the float32
+// launch that finds no tile marked); 0.92 ms with seven
 // pull-backs a step, idle steps run, and the products' loads waited for in the K loop (and
 // the GEMM 0.26 against 0.31 ms for the rows that went).  15 us per evaluation: MFMA, the
 // splits and the LDS stores of one column at a time, one after the other, bound it, not the
 // 1.3 GB of rows.
-constexpr int kWeightFlags = MLP_H * (2 * MLP_D + MLP_H) / 256;  // one per 256 weights
+constexpr float SPLIT_WEIGHT_END = 1024.0f, SPLIT_STATE_END = 16777216.0f,
+                SPLIT_DELTA_END = 1125899906842624.0f;  // 2^10, 2^24 (also of biases), 2^50
+// Flags of the weights, one per 256, then of the biases.
+constexpr int kMatrixFlags = MLP_H * (2 * MLP_D + MLP_H) / 256;
+constexpr int kWeightFlags = kMatrixFlags + (2 * MLP_H + MLP_D + 255) / 256;
 template <class P>
 using AdjLds = std::conditional_t<P::PIECES == 3, MlpLds<P>, MlpLdsBack>;
 
@@ -207,14 +222,15 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
   if (!Pieces && a.evals[tile] >= 0) return;
   int tile_steps = 0;
   while (__syncthreads_or(tile_steps < steps_here)) ++tile_steps;
-  const int evals = tile_steps > 0 ? 1 + 6 * tile_steps : 0;
+  int evals = tile_steps > 0 ? 1 + 6 * tile_steps : 0;
+  int32_t* mark = a.evals + tile;
+  int redo = a.wflags != nullptr;
   if (Pieces) {
-    const bool weights_out =
-        __syncthreads_or(a.wflags != nullptr && tid < kWeightFlags && a.wflags[tid] != 0);
-    if (tile_steps == 0 || weights_out) {
-      if (tid == 0) a.evals[tile] = -evals;
-      return;
-    }
+    const bool out = __syncthreads_or(redo && tid < kWeightFlags && a.wflags[tid] != 0);
+    if (tid == 0) *mark = out ? -evals : evals;
+    if (tile_steps == 0 || out) return;
+    // kept for the end in vector registers: scalar ones spill
+    asm("" : "+v"(evals), "+v"(mark), "+v"(redo));
   }
   SplitRange rng;
   const int dir = (a.t0 < a.t1) ? 1 : -1;
@@ -244,11 +260,13 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
                      float (&f)[CPT]) __attribute__((always_inline)) {
     put_cols(R.b[1], slot, z);
     store_inputs(L, orow, c0, z);
-    __syncthreads();
     if constexpr (Pieces) {
 #pragma unroll
       for (int j = 0; j < CPT; j += 4) rng.see(z[j], z[j + 1], z[j + 2], z[j + 3]);
-      mlp_forward_rows<NW>(W, L, wave, lane, orow, c0, f, R.b[3], R.b[5], slot, rng);
+    }
+    __syncthreads();
+    if constexpr (Pieces) {
+      mlp_forward_rows<NW>(W, L, wave, lane, orow, c0, f, R.b[3], R.b[5], slot);
     } else {
       mlp_forward<P, NW>(W, L, wave, lane, orow, c0, f);
       rows_out<MLP_H>(L.h1, L.LDH, R.b[3], slot);
@@ -320,23 +338,25 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
       };
       floatx16_t acc[NT];
       auto delta = [&](int t, int i) {
-        const float4 v = make_float4(acc[t][4 * i] * dsoftplus_from_value(h[t][i].x),
-                                     acc[t][4 * i + 1] * dsoftplus_from_value(h[t][i].y),
-                                     acc[t][4 * i + 2] * dsoftplus_from_value(h[t][i].z),
-                                     acc[t][4 * i + 3] * dsoftplus_from_value(h[t][i].w));
-        rng.see(v.x, v.y, v.z, v.w);
-        return v;
+        return make_float4(acc[t][4 * i] * dsoftplus_from_value(h[t][i].x),
+                           acc[t][4 * i + 1] * dsoftplus_from_value(h[t][i].y),
+                           acc[t][4 * i + 2] * dsoftplus_from_value(h[t][i].z),
+                           acc[t][4 * i + 3] * dsoftplus_from_value(h[t][i].w));
       };
       Gemm3<KS1, NT, false> g3;
       Gemm3<KS2, NT, false> g2;
       Gemm3<KS2, NT3> g1;
-#pragma unroll
-      for (int j = 0; j < CPT; j += 4) rng.see(d3[j], d3[j + 1], d3[j + 2], d3[j + 3]);
       g3.preload(W.w3t, W.plane3, NT * wave, 0, lane);
       load_h(R.b[5]);
       __builtin_amdgcn_sched_barrier(0);
       put_cols(R.b[4], slot, d3);
       store_inputs(L, orow, c0, d3);
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) {
+        constexpr float s = SPLIT_STATE_END / SPLIT_DELTA_END;
+        rng.most(s * d3[j], s * d3[j + 1], s * d3[j + 2], s * d3[j + 3]);
+        rng.least(d3[j], d3[j + 1], d3[j + 2], d3[j + 3]);
+      }
       __syncthreads();
       g3.template run<KS1>(L.x[0], MLP_TILE * MlpLds<P>::LDX, L.LDX, 0, acc, lane);
       g2.preload(W.w2t, W.plane2, NT * wave, 0, lane);
@@ -364,6 +384,8 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
         s += part[(3 * MLP_TILE + orow) * L.LDP + c];
         zb[j] = s;
       }
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) rng.least(zb[j], zb[j + 1], zb[j + 2], zb[j + 3]);
     }
   };
   // yb: cotangent of the state at the end of step q; fb: of f there, from the next step's
@@ -449,9 +471,10 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
   }
   pull_back(slot0, fb, zb);
   if constexpr (Pieces) {
-    const bool out = __syncthreads_or(rng.outside());
-    if (tid == 0) a.evals[tile] = out ? -evals : evals;
-    if (out && a.wflags) return;  // left to the float32 kernel
+    if (__syncthreads_or(rng.outside(SPLIT_STATE_END))) {
+      if (tid == 0) *mark = -evals;
+      if (redo) return;  // left to the float32 kernel
+    }
   }
   if (valid) {
 #pragma unroll
@@ -461,8 +484,12 @@ mlp_adj_segment_kernel(const AdjArgs a, const MlpWeights<P> W, const RowBufs R) 
 }
 
 // Three-piece planes (mlp_pack_layout(3)) of a float32 packed buffer (mlp_pack_layout(1)), and
-// per workgroup of the first three matrices whether a weight is outside the pieces' range.
+// the flags of the weights (by the workgroups of the first three matrices) and biases (by
+// those that follow).
 __global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __restrict__ packed,
+                                                               const float* __restrict__ b1,
+                                                               const float* __restrict__ b2,
+                                                               const float* __restrict__ b3,
                                                                __bf16* __restrict__ out,
                                                                int32_t* __restrict__ wflags) {
   int e = blockIdx.x * 256 + threadIdx.x, m, before;
@@ -474,10 +501,20 @@ __global__ void __launch_bounds__(256) mlp_split_packed_kernel(const float* __re
   const float v = packed[before + mlp_frag_index<PolicyF32>(n, k, sh.k)];
   __bf16* o = out + 3 * before + e;
   split3(v, o[0], o[sh.n * sh.k], o[2 * sh.n * sh.k]);
-  if (m < 3) {  // (whole workgroups: the matrices are multiples of 256)
+  if (blockIdx.x < kWeightFlags) {
     SplitRange rng;
-    rng.see(v);
-    const int outside = __syncthreads_or(rng.outside());
+    float end = SPLIT_WEIGHT_END;
+    if (m < 3) {  // (whole workgroups: the matrices are multiples of 256)
+      rng.see(v, v, v, v);
+    } else {
+      const int i = (int)(blockIdx.x - kMatrixFlags) * 256 + (int)threadIdx.x;
+      if (i < 2 * MLP_H + MLP_D) {
+        const float b = i < MLP_H ? b1[i] : (i < 2 * MLP_H ? b2[i - MLP_H] : b3[i - 2 * MLP_H]);
+        rng.most(b, b, b, b);
+      }
+      end = SPLIT_STATE_END;
+    }
+    const int outside = __syncthreads_or(rng.outside(end));
     if (threadIdx.x == 0) wflags[blockIdx.x] = outside;
   }
 }
@@ -610,7 +647,7 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
         rng.see(vb[x][i].x, vb[x][i].y, vb[x][i].z, vb[x][i].w);
       }
     }
-    return (bool)__any(rng.outside());
+    return (bool)__any(rng.outside(SPLIT_END));
   };
   auto add_columns = [&]() {
     if (col_sums) {
@@ -1154,10 +1191,10 @@ int run_segment(const dfx_mlp_problem* p, const void* packed, const float* b1, c
   const void* pieces = packed;
   if (f32) {
     int32_t* wflags = a.evals + (ntiles64 + 63) / 64 * 64;
-    __bf16* planes = reinterpret_cast<__bf16*>(wflags + kWeightFlags);
+    __bf16* planes = reinterpret_cast<__bf16*>(wflags + (kWeightFlags + 63) / 64 * 64);
     const unsigned nb = (unsigned)(mlp_pack_layout(1).total / 256);
     hipLaunchKernelGGL(mlp_split_packed_kernel, dim3(nb), dim3(256), 0, s,
-                       reinterpret_cast<const float*>(packed), planes, wflags);
+                       reinterpret_cast<const float*>(packed), b1, b2, b3, planes, wflags);
     pieces = planes;
     a.wflags = wflags;
   }
@@ -1191,7 +1228,8 @@ int dfx_mlp_adj_workspace(const dfx_mlp_problem* p, int32_t seg_steps, size_t* z
   *partial_bytes = (size_t)(partial_floats(ntiles * (1 + 6 * (int64_t)seg_steps)) +
                             (ntiles + 63) / 64 * 64) * sizeof(float);
   if (p->precision == DFX_F32)
-    *partial_bytes += kWeightFlags * sizeof(int32_t) + (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
+    *partial_bytes += (kWeightFlags + 63) / 64 * 64 * sizeof(int32_t) +
+                      (size_t)mlp_pack_layout(3).total * sizeof(__bf16);
   return DFX_OK;
 }
 

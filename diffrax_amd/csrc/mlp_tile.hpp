@@ -117,28 +117,32 @@ __device__ __forceinline__ Split4 split3x4(float a, float b, float c, float d) {
 }
 
 // Whether every value seen may be carried in three pieces in place of float32: zero, or of a
-// magnitude in [2^-100, 2^56).  Down to 2^-110 the pieces hold all 24 bits (a bfloat16 ends at
-// 2^-133; products and sums below 2^-126 are kept, the MFMA does not flush them); an infinity
-// has no pieces (inf - inf), and a number near the largest rounds up to one.  Below the upper
-// bound no product, nor a sum of 4,096, overflows in either form.  A caller that finds a
-// value outside takes float32 MFMA: gradients of cotangents scaled by 2^-112 and 2^-116 were
-// off by 5e-6 and 7e-5 in pieces and by 5e-7 and 8e-7 that way.  Eight instructions for four
-// values, beside thirty for their split.
-constexpr float SPLIT_MIN = 7.8886090522101181e-31f, SPLIT_END = 72057594037927936.0f;
+// magnitude from SPLIT_MIN up to a limit.  Down to 2^-110 the pieces hold all 24 bits (a
+// bfloat16 ends at 2^-133, so below that a piece sum is off by at most 2^-134; products and
+// sums below 2^-126 are kept, the MFMA does not flush them); an infinity has no pieces (inf -
+// inf), and a number near the largest rounds up to one.  A caller that finds a value outside
+// takes float32 MFMA: gradients of cotangents scaled by 2^-112 and 2^-116 were off by 5e-6 and
+// 7e-5 in pieces and by 5e-7 and 8e-7 that way.
+constexpr float SPLIT_MIN = 2.1175823681357508e-22f;   // 2^-72
+constexpr float SPLIT_END = 72057594037927936.0f;      // 2^56: no sum of 4,096 products overflows
 struct SplitRange {
   float hi = 0.0f;            // the largest magnitude
   unsigned lo = 0xffffffffu;  // the least 2 bits - 1 of the magnitudes (of zero: the most)
-  __device__ __forceinline__ void see_end(float a, float b, float c, float d) {
+  __device__ __forceinline__ void most(float a, float b, float c, float d) {
     hi = fmaxf(fmaxf(hi, fmaxf(fabsf(a), fabsf(b))), fmaxf(fabsf(c), fabsf(d)));
+    asm("" : "+v"(hi));
   }
-  __device__ __forceinline__ void see(float a, float b, float c, float d) {
-    see_end(a, b, c, d);
+  __device__ __forceinline__ void least(float a, float b, float c, float d) {
     auto key = [](float v) { return (__builtin_bit_cast(unsigned, v) << 1) - 1u; };
     lo = min(min(lo, min(key(a), key(b))), min(key(c), key(d)));
+    asm("" : "+v"(lo));  // (not split into comparisons whose masks fill the scalar registers)
   }
-  __device__ __forceinline__ void see(float v) { see(v, v, v, v); }
-  __device__ __forceinline__ bool outside() const {
-    return !(hi < SPLIT_END) || lo < (__builtin_bit_cast(unsigned, SPLIT_MIN) << 1) - 1u;
+  __device__ __forceinline__ void see(float a, float b, float c, float d) {
+    most(a, b, c, d);
+    least(a, b, c, d);
+  }
+  __device__ __forceinline__ bool outside(float limit) const {
+    return !(hi < limit) || lo < (__builtin_bit_cast(unsigned, SPLIT_MIN) << 1) - 1u;
   }
 };
 
@@ -548,13 +552,13 @@ __device__ __forceinline__ void put_rows(MlpLds<PolicyBF16x3>& L, __bf16* buf, f
 }
 
 // The forward of the three-piece form with its hidden activations kept in row buffers as well
-// (the adjoint's recompute): mlp_forward's bits.  rng sees the activations.
+// (the adjoint's recompute): mlp_forward's bits.
 template <int NW>
 __device__ __forceinline__ void mlp_forward_rows(const MlpWeights<PolicyBF16x3>& W,
                                                  MlpLds<PolicyBF16x3>& L, int wave, int lane,
                                                  int owner_row, int owner_c0,
                                                  float (&fout)[MlpWaves<NW>::CPT], float* h1_rows,
-                                                 float* h2_rows, int64_t block, SplitRange& rng) {
+                                                 float* h2_rows, int64_t block) {
   using WV = MlpWaves<NW>;
   using LD = MlpLds<PolicyBF16x3>;
   constexpr int NT = WV::NT12, NT3 = WV::NT3, KS1 = MLP_D / 16, KS2 = MLP_H / 16;
@@ -563,10 +567,8 @@ __device__ __forceinline__ void mlp_forward_rows(const MlpWeights<PolicyBF16x3>&
   auto hidden = [&](const float* bias) {
     return [&, bias](int t, int i) {
       const float b = bias[32 * (NT * wave + t) + (lane & 31)];
-      const float4 h = make_float4(softplus_f(acc[t][4 * i] + b), softplus_f(acc[t][4 * i + 1] + b),
-                                   softplus_f(acc[t][4 * i + 2] + b), softplus_f(acc[t][4 * i + 3] + b));
-      rng.see_end(h.x, h.y, h.z, h.w);  // (softplus_f is 0 or more than 2^-24)
-      return h;
+      return make_float4(softplus_f(acc[t][4 * i] + b), softplus_f(acc[t][4 * i + 1] + b),
+                         softplus_f(acc[t][4 * i + 2] + b), softplus_f(acc[t][4 * i + 3] + b));
     };
   };
   Gemm3<KS1, NT, false> g1;

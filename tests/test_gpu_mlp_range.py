@@ -76,3 +76,37 @@ def test_large_weight(cuda):
     want = _grads(cuda, "f32", W, y0, w)
     W[2][0, 7] = 3.4e38
     _close(_grads(cuda, "f32", W, y0, w), want)
+
+
+def test_large_bias(cuda):
+    """An activation whose leading piece is infinite, on weights that are zero: only its own
+    column of W3's gradient is large."""
+    W, (y0, w) = _weights(), _inputs()
+    w *= np.float32(2.0 ** -10)
+    W[4][:, 9] = 0.0
+    want = _grads(cuda, "f32", W, y0, w)
+    W[3][9] = 3.4e38
+    got = _grads(cuda, "f32", W, y0, w)
+    got[5][:, 9] = want[5][:, 9] = 0.0
+    _close(got, want)
+
+
+def test_one_small_trajectory(cuda):
+    """Cotangents near the least number in one trajectory of a tile: its own gradient keeps its
+    accuracy beside the others."""
+    W, (y0, w) = _weights(), _inputs()
+    want = _grads(cuda, "f32", W, y0, w)[0][5]
+    s = 2.0 ** -116
+    w[5] *= np.float32(s)
+    got = _grads(cuda, "f32", W, y0, w)[0][5] / s
+    assert float((got - want).abs().max() / want.abs().max()) < TOL
+
+
+def test_small_inside(cuda):
+    """Units whose slopes are near 2^-21 in both hidden layers: deltas near the least number from
+    cotangents that are not."""
+    W, (y0, w) = _weights(), _inputs()
+    W[1][:] = W[3][:] = -15.0
+    s = np.float32(2.0 ** -70)
+    got = _grads(cuda, "f32", W, y0, w * s)
+    _close([g / float(s) for g in got], _grads(cuda, "f32", W, y0, w))
