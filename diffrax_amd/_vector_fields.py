@@ -156,10 +156,10 @@ class MLPField(RegisteredVectorField):
     accumulate); the RK algebra is float32 in both and time / step control float64.  Gradient
     products are float32 too: in both forms those of RecursiveCheckpointAdjoint and every
     weight gradient run on three exact bfloat16 pieces of each operand (their errors against
-    float64 are half of float32 MFMA's), and on float32 MFMA where a value is outside the
-    pieces' range (nonzero below 2^-72; from 2^10 a weight, 2^24 a bias or state, 2^50 a
-    cotangent); with "bf16" the pull-backs of RecursiveCheckpointAdjoint stay in pieces there,
-    as its solve does."""
+    float64 are half of float32 MFMA's), and on float32 MFMA outside the pieces' range
+    (values that are nonzero below 2^-72; weights from 2^10, biases and states from 2^24,
+    cotangents from 2^50); with "bf16" the pull-backs of RecursiveCheckpointAdjoint stay in
+    pieces there, as its solve does."""
 
     vf_id = _lib.VF_MLP
     name = "mlp"

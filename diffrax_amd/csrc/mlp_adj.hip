@@ -47,7 +47,7 @@ struct AdjArgs {
   float* ybar;
   float* zs;
   int32_t* evals;  // out [tiles]: evaluations (row blocks) of each tile, negative where some
-                   // value is outside the range of the three-piece products (SplitRange)
+                   // value is outside the range of its three-piece products (SplitRange)
   const int32_t* wflags;  // float32 form: nonzero where a weight or bias is outside
                           // (kWeightFlags), and marked tiles are left to the float32 kernel;
                           // else null
@@ -171,7 +171,7 @@ __device__ __forceinline__ void pull_back_f32(const MlpWeights<PolicyF32>& W, Ml
 //     2^-116 and one for zb by 2^-98, a quarter of 2^-24 of the least zb that passes.
 // Looking at every delta instead took 15 of 700 us; this is within the launch's spread (8,192
 // trajectories 709 us, without any test 721; 3,001 537 and 537).  In the bf16 form, which
-// evaluates in pieces anyway, the marks only choose the weight-gradient GEMM's arithmetic.
+// evaluates in pieces anyway, nothing reads the marks.
 // The row
 // buffers hold float32 values (layer inputs and deltas written before their split into
 // pieces) for the weight-gradient GEMM.  LDS: the forward planes;
@@ -538,12 +538,13 @@ constexpr int kXcds = 8;
 
 // Chunks of row blocks the GEMM splits K into: 24 one-wave workgroups (64 x 64 output
 // pieces) each, two per SIMD of the chip resident at once, so 80 chunks (1,920 waves), but no
-// more than there are four-block chunks, and enough that none has more than 128 blocks: the
-// float32 accumulators' rounding grows with their 4,096 rows (8,192 trajectories and 64 steps,
-// 98,560 blocks: 770 chunks; with 80 the sums were off by 6e-6 of the largest, now by 1.4e-6).
+// more than there are four-block chunks, and as many times 80 as it takes that none has more
+// than 128 blocks: the float32 accumulators' rounding grows with their 4,096 rows (8,192
+// trajectories and 64 steps, 98,560 blocks: 800 chunks; with 80 the sums were off by 6e-6 of
+// the largest, now by 1.4e-6).
 __host__ __device__ inline int dw_chunks(int64_t blocks) {
-  const int64_t few = (blocks + 3) / 4, most = (blocks + 127) / 128;
-  const int64_t n = few < 80 ? few : (most > 80 ? most : 80);
+  const int64_t few = (blocks + 3) / 4, rounds = (blocks + 80 * 128 - 1) / (80 * 128);
+  const int64_t n = few < 80 ? few : 80 * rounds;
   return (int)(n < 1 ? 1 : n);
 }
 
@@ -556,9 +557,6 @@ __host__ __device__ inline int dw_chunks(int64_t blocks) {
 // Waves in the first piece column of a matrix also produce the chunk's column sums of A (the
 // bias gradient partials, partial_db: [chunk][db1 | db2 | db3]).
 // evals: of every `slots` blocks (a tile) only the first |evals[tile]| hold rows (null: all do).
-// A block with values outside the pieces' range (SplitRange) takes float32 MFMA, its rows as
-// the k of v_mfma_f32_32x32x2 (row 8i + j from lane half 0, 8i + 4 + j from half 1): blocks of
-// a tile with negative evals, or, with SC, found here.
 // SC: the rows of A are multiplied by rscale[row] (the backsolve's per-row weights dt * b_i,
 // zero for rejected steps and idle rows; a row of zero weight is dropped from both operands,
 // so a non-finite value in it contributes nothing).
@@ -610,16 +608,12 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
       }
     }
   };
-  // the first block with rows of tiles marked so, at or after blk (b1: none); lim: the end of
-  // its tile's; found: whether a block outside the pieces' range has been seen
+  // the first block with rows at or after blk (b1: none); lim: the end of its tile's
   int64_t lim = evals ? b0 : b1;
-  bool found = false;
-  auto next = [&](int64_t blk, bool marked) {
+  auto next = [&](int64_t blk) {
     while (blk >= lim && blk < b1) {
       const int64_t tile = blk / slots;
-      const int n = evals[tile];
-      found = found || n < 0;
-      lim = (n < 0) == marked ? min(tile * slots + abs(n), b1) : blk;
+      lim = min(tile * slots + abs(evals[tile]), b1);
       if (blk >= lim) {
         blk = min((tile + 1) * slots, b1);
         lim = blk;
@@ -627,12 +621,16 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
     }
     return blk;
   };
-  // the loaded block's rows times their weights (SC), and whether it is outside the range then
+  // the loaded block's rows times their weights (SC)
   auto scale = [&](int64_t blk) {
-    SplitRange rng;
+    float4 ws[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      ws[i] = *reinterpret_cast<const float4*>(rscale + blk * 32 + 8 * i + 4 * half);
+    __builtin_amdgcn_sched_barrier(0);  // one wait for the four loads
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float4 w = *reinterpret_cast<const float4*>(rscale + blk * 32 + 8 * i + 4 * half);
+      const float4 w = ws[i];
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         auto sc = [](float wt, float& da, float& db) {
@@ -643,11 +641,8 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
         sc(w.y, va[x][i].y, vb[x][i].y);
         sc(w.z, va[x][i].z, vb[x][i].z);
         sc(w.w, va[x][i].w, vb[x][i].w);
-        rng.see(va[x][i].x, va[x][i].y, va[x][i].z, va[x][i].w);
-        rng.see(vb[x][i].x, vb[x][i].y, vb[x][i].z, vb[x][i].w);
       }
     }
-    return (bool)__any(rng.outside(SPLIT_END));
   };
   auto add_columns = [&]() {
     if (col_sums) {
@@ -659,18 +654,12 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
       }
     }
   };
-  int64_t nxt = next(b0, false);
+  int64_t nxt = next(b0);
   if (nxt < b1) load(nxt);
   while (nxt < b1) {
     const int64_t blk = nxt;
-    nxt = next(blk + 1, false);
-    if constexpr (SC) {
-      if (scale(blk)) {  // left to the loop below
-        found = true;
-        if (nxt < b1) load(nxt);
-        continue;
-      }
-    }
+    nxt = next(blk + 1);
+    if constexpr (SC) scale(blk);
     add_columns();
     // k half s: the rows 16 s .. 16 s + 15 of the block, in the same order for both operands
     frag_t fa[2][2][3], fb[2][2][3];  // [s][x][piece]
@@ -705,14 +694,36 @@ mlp_dw_gemm_kernel(const RowBufs R, float* __restrict__ partial, float* __restri
       }
     }
   }
-  if (found) {  // the blocks outside the range (in a loop of their own: beside the pieces'
-                // registers they would spill)
-    lim = evals ? b0 : b1;
-    for (int64_t blk = next(b0, true); blk < b1; blk = next(blk + 1, true)) {
-      load(blk);
-      if constexpr (SC) {
-        if (!scale(blk)) continue;
+  // The sums tell whether the pieces could be trusted (SplitRange).  A value that has none, or a
+  // sum of theirs that overflows, leaves an accumulator that is not finite.  Pieces are off by
+  // 2^-134 at most, 4,096 products by 2^-112 for activations up to 2^10: less than 2^-24 of
+  // sums whose largest is SPLIT_MIN or more.  Else the chunk runs once more on float32 MFMA, its
+  // rows as the k of v_mfma_f32_32x32x2 (row 8i + j from lane half 0, 8i + 4 + j from half 1),
+  // in a loop of its own (beside the pieces' registers it would spill).
+  bool finite = true;
+  float most = 0.0f;
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        finite = finite && fabsf(acc[x][y][v]) < __builtin_inff();
+        most = fmaxf(most, fabsf(acc[x][y][v]));
       }
+    }
+  }
+  if (__any(!finite) || (__any(most > 0.0f) && !__any(most >= SPLIT_MIN))) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      acc[x][0] = floatx16_t{};
+      acc[x][1] = floatx16_t{};
+      csum[x] = 0.0f;
+    }
+    lim = evals ? b0 : b1;
+    for (int64_t blk = next(b0); blk < b1; blk = next(blk + 1)) {
+      load(blk);
+      if constexpr (SC) scale(blk);
       add_columns();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {

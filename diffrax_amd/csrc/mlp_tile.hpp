@@ -124,7 +124,6 @@ __device__ __forceinline__ Split4 split3x4(float a, float b, float c, float d) {
 // takes float32 MFMA: gradients of cotangents scaled by 2^-112 and 2^-116 were off by 5e-6 and
 // 7e-5 in pieces and by 5e-7 and 8e-7 that way.
 constexpr float SPLIT_MIN = 2.1175823681357508e-22f;   // 2^-72
-constexpr float SPLIT_END = 72057594037927936.0f;      // 2^56: no sum of 4,096 products overflows
 struct SplitRange {
   float hi = 0.0f;            // the largest magnitude
   unsigned lo = 0xffffffffu;  // the least 2 bits - 1 of the magnitudes (of zero: the most)

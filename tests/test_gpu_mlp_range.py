@@ -18,6 +18,11 @@ BACK = dfx.BacksolveAdjoint(stepsize_controller=dfx.PIDController(
     rtol=1e-5, atol=1e-7, norm=dfx.adjoint_rms_seminorm))
 
 
+# equal backward steps whatever the cotangents' size
+EVEN = dfx.BacksolveAdjoint(dt0=-0.125, stepsize_controller=dfx.PIDController(
+    rtol=1.0, atol=1.0, dtmax=0.125, norm=dfx.adjoint_rms_seminorm))
+
+
 def _grads(cuda, matmul, W, y0, w, adjoint=dfx.RecursiveCheckpointAdjoint()):
     P = [torch.tensor(a, dtype=torch.float32, device=cuda, requires_grad=True) for a in W]
     y0 = torch.tensor(y0, device=cuda, requires_grad=True)
@@ -41,13 +46,15 @@ def _inputs(B=70):
     return y0, rng.normal(size=(B, 5, 64)).astype(np.float32)
 
 
+@pytest.mark.parametrize("adjoint", [dfx.RecursiveCheckpointAdjoint(), EVEN],
+                         ids=["discrete", "backsolve"])
 @pytest.mark.parametrize("e", [-104, -112, -116])
-def test_small_cotangents(cuda, e):
+def test_small_cotangents(cuda, e, adjoint):
     """The gradient is linear in the cotangents, also where these are near the least number."""
     W, (y0, w) = _weights(), _inputs()
     s = np.float32(2.0 ** e)
-    got = _grads(cuda, "f32", W, y0, w * s)
-    _close([g / float(s) for g in got], _grads(cuda, "f32", W, y0, w))
+    got = _grads(cuda, "f32", W, y0, w * s, adjoint)
+    _close([g / float(s) for g in got], _grads(cuda, "f32", W, y0, w, adjoint))
 
 
 @pytest.mark.parametrize("adjoint", [dfx.RecursiveCheckpointAdjoint(), BACK],
